@@ -266,7 +266,7 @@ public:
         }
         for (void *p : {(void *) Xt, (void *) cellC, (void *) cellE, (void *) nearm, (void *) small, (void *) stamp,
                         (void *) qmark, (void *) entries, (void *) scratch, (void *) rank_perm,
-                        (void *) d_level})
+                        (void *) d_level, (void *) edges})
             if (p) dev_free(p);
         if (pin) host_free(pin);
     }
@@ -1018,19 +1018,19 @@ private:
     Pool store;     // weak-dense point lists of surviving trees, keep log (whole run)
     Pool lvl[2];    // frontier paths and counters of the current / next level
     Pool batch;     // one batch of child subspaces
-    // grid index sorts kept for later batches, by index dimensions (whole run)
-    struct KeptSort {
-        int *order, *pos, *off;
+    // grid index sorts and their sorted coordinate columns, by index dimensions:
+    // kept for the whole run while the budgets last (keptp, colp), else built
+    // in the batch's memory and forgotten with it
+    struct Sort {
+        int *order = nullptr, *pos = nullptr, *off = nullptr;
+        bool keep = false;
+        std::vector<float *> col;  // [d] kept columns, null until gathered
     };
-    std::unordered_map<uint64_t, KeptSort> kept;
-    Pool keptp;
-    size_t kept_used = 0, kept_budget = 0;
-    // sorted coordinate columns kept the same way, by index dimensions and
-    // dimension: (column, number of the batch that gathers it)
-    std::unordered_map<uint64_t, std::pair<float *, int>> kept_cols;
-    Pool colp;
-    size_t cols_used = 0;
-    int batch_no = 0;
+    std::unordered_map<uint64_t, Sort> kept, batch_sorts;
+    std::unordered_map<uint64_t, float *> batch_cols;  // columns of this batch only, by index and dimension
+    Pool keptp, colp;
+    size_t kept_used = 0, cols_used = 0, kept_budget = 0;
+    void index_of(std::vector<BatchSub> &hs, std::vector<const float *> &ctab);
     int cur_lvl = 0;
     HostBuf up, down;
     HostBuf emit_stage[2];
@@ -1038,6 +1038,7 @@ private:
     bool up_defer = false;                          // defer_uploads()
     char *pend_dst = nullptr;                       // the deferred copy: device place,
     size_t pend_src = 0, pend_bytes = 0;            // staging offset and bytes
+    float *edges = nullptr;                         // [ecells + 3] edges of the eps cells
     size_t batch_budget = 0;
     size_t max_batch = 0;  // child subspaces per batch
     bool phi_mode = false;          // rectangular = false
@@ -1063,6 +1064,7 @@ private:
     }
     void expand_level(const std::vector<int> &frontier, const int *counts);
     void process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1);
+    GridArg child_grid(const SubspaceArg &S) const;
     void replay_staged();
     std::vector<int> sup_flat;  // superset rows of every subspace (host copy of d_sup)
     static unsigned blocks_for_host(long long count) { return (unsigned) ((count + kBlockThreads - 1) / kBlockThreads); }

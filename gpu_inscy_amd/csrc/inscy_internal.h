@@ -134,32 +134,24 @@ struct KernelTimer {
 // pruned by the weak-density test).
 
 // One subspace of a batch.  Its per-subspace state (query flags, dense flags,
-// packed cells, sample edges, union-find parents) lives at [base, base + n).
-// Its grid index (keys, ranks, sorted order) lives at [obase, obase + n) with
-// grid cells at [hoff, hoff + ncell); the children S + {m} of one frontier
-// mask S (m is always the last dimension) share one index, built by the first
-// of them (rep = 1), and the coordinates of S's dimensions in sorted order.
-// Column t of the sorted coordinates and cells starts at mcoord for t == pos_m
-// (the child's own dimension), else at coord + t*n; pos_m = k when nothing is
-// shared.
+// union-find parents) lives at [base, base + n) of the batch's buffers, its
+// sample edges at [nbase, nbase + n).  Its grid index (order, pos, off) and its
+// coordinate columns in that order (col[t] for dimension t of S) are read where
+// they lie: kept for the whole run, or in the batch's own memory.
 constexpr int kMaxBounds = 8;
 struct BatchSub {
     SubspaceArg S;
     GridArg G;
-    long long base, coord, hoff, qoff;
-    long long obase, mcoord;
-    int pos_m, rep;
+    const int *order;   // [n + 4] point id at each sorted position
+    const int *pos;     // [n] sorted position of each point
+    const int *off;     // [cells + 1] first sorted position of each grid cell
+    const float *const *col;  // [k] coordinates in sorted order (n + 4 each)
+    long long base, nbase;
     int *cnt;           // [n] neighbour counts (capped), -1 = not counted
     const int *bound[kMaxBounds];  // [n] complete counts of subspaces S minus one dimension
     int *comp;          // [n] component roots (components pass)
     int *csize;         // [n] component sizes (components pass)
-    int nbound, ncell, cap, lo, thr_dense, qmax;
-    // cell test of the candidates: the first (up to 4) checked dimensions of
-    // S, packed 16 bits each into one word per sorted position; the others
-    // (restmask, positions in S) are tested one by one
-    int nchk4;
-    int chk[4];
-    uint64_t restmask;
+    int nbound, cap, lo, thr_dense, qmax;
     // phi mode (rectangular = false): dbit = 2 (dense = bit 1 of the stored
     // decision bits), thresholds of the weak and the dense test; count mode: dbit = 0
     int dbit;
@@ -168,16 +160,11 @@ struct BatchSub {
     // of S the neighbourhood tree walk matches in level order (all of S in
     // the identity order; ScyTreeNode.cu:910-915)
     uint64_t matchmask;
-    const uint16_t *cellE;  // [d][n] eps-grid cells by point (the query's own cells are read here)
 };
 
-// Device buffers of one batch's grid indexes.
+// Device buffers of one batch.
 struct BatchIndex {
-    int *keys, *rank;     // [B*n]
-    int *hist, *off;      // [nhist]
-    int *order;           // [B*n] point id at each sorted position
-    float *Ys;            // coordinates in sorted order
-    uint16_t *Es;         // eps-grid cells in sorted order (gathered only when a walk tests cells one by one)
+    const float *edge;    // [C + 3] edges of the eps cells (k_cell_edges)
     uint8_t *qflag;       // [B*n] query flag per (global) sorted position
     int *qlist;           // global sorted positions of the queries, ascending
     int *nsel;            // [1] number of queries
@@ -185,19 +172,27 @@ struct BatchIndex {
     void *select_temp;
     size_t select_bytes;
     int *nb;              // [B*n*kSampleEdges] first neighbours found by the count passes
-    uint64_t *sig;        // [B*n] packed cells of the checked dimensions per sorted position
-    uint64_t *sigS;       // [B*n] (index space) the same over the shared dimensions only
-    const int *reps;      // subspaces that build an index, in index order
-    int nrep;
     int2 *fb;             // phi mode: (subspace, point) pairs to recompute in leaf order
     int *nfb;             // [1] their number
     int fbcap;
     uint8_t *dsorted;     // [B*n] dense flag per sorted position
     int *par;             // [B*n] union-find parents (point ids within each subspace)
     int *giant;           // [B]
-    void *scan_temp;
-    size_t scan_bytes;
-    int nhist;            // sum of ncell + 1
+};
+
+// A grid index to sort: the points by their eps cells in dims[0..j), the last
+// one in F buckets per cell; its histogram cells start at hoff.
+struct SortJob {
+    int *order, *pos, *off;
+    long long hoff;
+    int dims[3];
+    int j, C, F, ncell;
+};
+// dst[i] = src[order[i]]: one coordinate column in an index's order
+struct ColJob {
+    const int *order;
+    const float *src;
+    float *dst;
 };
 
 // Tree whose s-connection paths set the merge flags of its dimensions >= first.
@@ -322,41 +317,16 @@ hipError_t launch_gather(const int *src, const int *idx, int count, int *out, hi
 hipError_t launch_iota(int *p, int n, hipStream_t st);
 hipError_t launch_root_paths(const dmask_t *nearm, int n, int *outx, uint64_t *outm, int mw, int *nout, hipStream_t st);
 
+// edges of the C eps cells, C + 3 floats (see k_cell_edges)
+hipError_t launch_cell_edges(int C, float *edge, hipStream_t st);
 // level-synchronous passes (blk_off: per-segment block offsets, nblk = blk_off[nseg])
 hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
                           int cells, int *flags, hipStream_t st);
-// grid indexes of nsub subspaces: keys, one scan over all grid cells, scatter
-// A grid index sort kept for later batches of the run (the same index
-// dimensions sort the points the same way): sorted point ids, each point's
-// sorted position and the cell offsets, all local to the index; with the
-// batch-side place of one index (obase, hoff) and its cell count.
-struct SortCopy {
-    int *order, *pos, *off;
-    long long obase, hoff;
-    int ncell;
-};
-
-// need_es: gather the sorted cell columns Es (a launch of the batch runs the
-// walk for any k, which tests cells one by one).  miss_reps: the indexes to
-// sort (positions in subs), placed first: their cells are the histogram's
-// first hmiss entries; stores: sorts to keep (filled from the batch after
-// sorting); hits: kept sorts copied in (after the stores, so an index repeated
-// within the batch reads the sort just kept).  After it X.keys holds every
-// point's local sorted position.
-// Sorted coordinate columns kept across batches (same index dimensions and
-// dimension): per index column (rep position * kmax + t) and per subspace's
-// own column, a kept column to read (src) or a slot to keep a gathered one
-// (store), either null.
-struct ColumnKeep {
-    const float *const *src;
-    float *const *store;
-    const float *const *own_src;
-    float *const *own_store;
-    int kmax;
-};
-hipError_t launch_b_index(const DevData &D, const BatchSub *subs, int nsub, const BatchIndex &X, bool need_es,
-                          const int *miss_reps, int nmiss, int hmiss, const SortCopy *stores, int nstore,
-                          const SortCopy *hits, int nhit, int max_cell, const ColumnKeep &cols, hipStream_t st);
+// grid indexes: keys and in-cell ranks, one scan over all grid cells, scatter.
+// keys, rank: [njob * n]; hist, off: [hmiss + 1]
+hipError_t launch_b_sort(const DevData &D, const SortJob *jobs, int njob, int hmiss, int max_cell, int *keys,
+                         int *rank, int *hist, int *off, void *scan_temp, size_t scan_bytes, hipStream_t st);
+hipError_t launch_b_gather(const ColJob *jobs, int njob, int n, hipStream_t st);
 // queries in sorted order: flag the points of the segments, compact per subspace
 hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySeg *segs, const int *blk_off,
                             int nseg, int nblk, const BatchIndex &X, hipStream_t st);
@@ -364,8 +334,8 @@ hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySe
 // uncounted point when blk_off is null (grid.y = subspace)
 // phi: rectangular = false, the stored values are decision bits (1 weak-dense,
 // 2 dense); points near a threshold are recomputed in leaf order (rank_order)
-// kfast in 1..7: every subspace of the launch has k = kfast and at most four
-// checked dimensions (the count kernel is then compiled for that k); else 0
+// kfast in 1..kMaxFastK: every subspace of the launch has k = kfast (the count
+// kernel is then compiled for that k); else 0
 hipError_t launch_b_count(const BatchSub *subs, int nsub, const int *blk_off, int nblk, int n, int kmax, int kfast,
                           const BatchIndex &X, float s_star, float eps, bool phi, bool phi_all_exact,
                           const DevData &D, const int *rank_order, unsigned long long *stat, const KernelTimer &tm,
@@ -482,6 +452,7 @@ hipError_t launch_tree_hits(const TreeHit *trees, const int *blk_off, int ntrees
 constexpr int kRangeWords = 31;      // per query in LDS: 9 range starts, 10 prefix sums, count, own run, 10 group sums
 constexpr int kBlockThreads = 256;   // threads per block of every pass
 constexpr int kQueriesPerBlock = 64;  // queries per block of the batched neighbour passes
+constexpr int kMaxFastK = 8;          // neighbour walks are compiled for each k up to this
 constexpr int kSampleEdges = 2;       // neighbours recorded per point by the count walk (Afforest's sample rounds)
 constexpr int kPartPerThread = 8;     // elements per thread of the batched partition passes
 

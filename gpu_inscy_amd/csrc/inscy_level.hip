@@ -80,11 +80,13 @@ void Engine::run_levels(inscy_result &out) {
     keptp.reset();
     kept_used = 0;
     kept_budget = keep_budget_override >= 0 ? (size_t) keep_budget_override : batch_budget;
-    kept_cols.clear();
     colp.reset();
     cols_used = 0;
-    batch_no = 0;
 
+    if (!edges) {
+        HIP_OK(dev_alloc(&edges, ((size_t) ecells + 3) * sizeof(float)));
+        HIP_OK(launch_cell_edges(ecells, edges, st));
+    }
     // the root tree: every point, the root s-connection paths
     Pool &L0 = lvl[cur_lvl];
     lvl[cur_lvl ^ 1].reset();
@@ -275,11 +277,12 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             SubspaceArg S = arg_of(c.s);
             GridArg G = grid_of(S, -1, true);
             const long long ncell = grid_cells(G);
-            // process_batch's takes per subspace: counts, keys, rank, order,
-            // query flags and list, two sample edges, packed cells (own and
-            // shared), dense flags and parents (50 bytes a point), k coordinate
-            // columns and cells (6k), the phi pass's queue (8), grid offsets
-            size_t est = (size_t) n * (50 + 6 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 8;
+            // process_batch's takes per subspace: counts, query flags and
+            // list, two sample edges, dense flags and parents (22 bytes a
+            // point), an index that is not kept (keys, rank, order, position:
+            // 16, k coordinate columns: 4k, grid histogram and offsets), the
+            // phi pass's queue (8)
+            size_t est = (size_t) n * (38 + 4 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 12;
             for (int a = c.t0; a < c.t1; ++a) {
                 if (!pair_on(a, c.m)) continue;
                 const LTree &t = lt[lv_act[a]];
@@ -297,177 +300,156 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
     }
 }
 
+// Grid index of the child subspace S | {m} (m its last dimension): S's own
+// index where it costs the neighbour passes little (S's index dimensions are at
+// most 25% less selective than the best ones of S | {m}; expected candidates
+// per query scale with the product of the index dimensions' selectivity
+// scores), so that the children of one frontier mask read one sort and one set
+// of columns.
+GridArg Engine::child_grid(const SubspaceArg &S) const {
+    const GridArg gopt = grid_of(S, -1, true);
+    const int kS = S.k - 1;
+    if (kS < 3 || __builtin_popcountll(match_of(S) & ((1ull << kS) - 1)) < 3) return gopt;
+    const GridArg gbest = grid_of(S, S.k - 1, true);
+    double cs = 1.0, co = 1.0;
+    for (int a = 0; a < gbest.j; ++a) cs *= std::max(score[S.dims[gbest.tI[a]]], 1.0);
+    for (int a = 0; a < gopt.j; ++a) co *= std::max(score[S.dims[gopt.tI[a]]], 1.0);
+    return gbest.j == gopt.j && cs <= 1.25 * co ? gbest : gopt;
+}
+
+// The grid indexes (order, pos, off) and coordinate columns of the subspaces
+// hs, whose S and G are set: a sort or column the run has kept is used where it
+// lies, the others are sorted and gathered here, into kept memory while the
+// budgets last, else into the batch's.  ctab receives the column pointers
+// (S.k per subspace, in order); the caller uploads it and sets hs[b].col.
+void Engine::index_of(std::vector<BatchSub> &hs, std::vector<const float *> &ctab) {
+    std::vector<SortJob> sorts;
+    std::vector<ColJob> cols;
+    long long hmiss = 0;
+    int max_cell = 0;
+    for (BatchSub &x : hs) {
+        uint64_t key = (uint64_t) x.G.j;
+        for (int a = 0; a < x.G.j; ++a) key |= (uint64_t) (x.S.dims[x.G.tI[a]] + 1) << (8 * (a + 1));
+        Sort *srt = nullptr;
+        auto it = kept.find(key);
+        if (it != kept.end()) {
+            srt = &it->second;
+            stats.sorts_kept++;
+        } else if (auto jt = batch_sorts.find(key); jt != batch_sorts.end()) {
+            srt = &jt->second;
+        } else {
+            const int ncell = (int) grid_cells(x.G);
+            const size_t need = ((size_t) 2 * n + ncell + 5) * sizeof(int) + 768;
+            const bool keep = kept_used + need <= kept_budget;
+            Pool &pool = keep ? keptp : batch;
+            Sort s;
+            s.keep = keep;
+            s.order = pool.take<int>((size_t) n + 4);  // the grouped walks read up to 3 ids past a run
+            s.pos = pool.take<int>(n);
+            s.off = pool.take<int>((size_t) ncell + 1);
+            if (keep) {
+                kept_used += need;
+                s.col.assign(d, nullptr);
+            }
+            SortJob j{};
+            j.order = s.order;
+            j.pos = s.pos;
+            j.off = s.off;
+            j.hoff = hmiss;
+            j.j = x.G.j;
+            j.C = x.G.C;
+            j.F = x.G.F;
+            j.ncell = ncell;
+            for (int a = 0; a < x.G.j; ++a) j.dims[a] = x.S.dims[x.G.tI[a]];
+            hmiss += ncell;
+            max_cell = std::max(max_cell, ncell);
+            sorts.push_back(j);
+            srt = &(keep ? kept : batch_sorts).emplace(key, std::move(s)).first->second;
+        }
+        x.order = srt->order;
+        x.pos = srt->pos;
+        x.off = srt->off;
+        for (int t = 0; t < x.S.k; ++t) {
+            const int dim = x.S.dims[t];
+            float *c = srt->keep ? srt->col[dim] : nullptr;
+            if (!c) {
+                const size_t need = ((size_t) n + 4) * sizeof(float) + 256;
+                const uint64_t ck = key | (uint64_t) (dim + 1) << 32;
+                if (srt->keep && cols_used + need <= kept_budget) {
+                    c = srt->col[dim] = colp.take<float>((size_t) n + 4);  // walks read up to 3 past the end
+                    cols_used += need;
+                    cols.push_back({srt->order, Xt + (size_t) dim * n, c});
+                } else {
+                    float *&bc = batch_cols[ck];
+                    if (!bc) {
+                        bc = batch.take<float>((size_t) n + 4);
+                        cols.push_back({srt->order, Xt + (size_t) dim * n, bc});
+                    }
+                    c = bc;
+                }
+            }
+            ctab.push_back(c);
+        }
+    }
+    if (sorts.empty() && cols.empty()) return;
+    const int ns = (int) sorts.size(), nc = (int) cols.size();
+    defer_uploads();
+    SortJob *ds = ns ? upload(batch, sorts) : nullptr;
+    ColJob *dc = nc ? upload(batch, cols) : nullptr;
+    flush_uploads();
+    if (ns) {
+        int *keys = batch.take<int>((size_t) ns * n), *rank = batch.take<int>((size_t) ns * n);
+        int *hist = batch.take<int>(hmiss + 1), *off = batch.take<int>(hmiss + 1);
+        const size_t sb = scan_temp_bytes((int) (hmiss + 1));
+        char *tmp = batch.take<char>(sb);
+        HIP_OK(launch_b_sort(D, ds, ns, (int) hmiss, max_cell, keys, rank, hist, off, tmp, sb, st));
+    }
+    if (nc) HIP_OK(launch_b_gather(dc, nc, n, st));
+}
+
 void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1) {
     Pool &nxt = lvl[cur_lvl ^ 1];
     batch.reset();
+    batch_sorts.clear();
+    batch_cols.clear();
     const int B = (int) (i1 - i0);
     const int QPB = kQueriesPerBlock;
 
     // ---- grid indexes of the batch's subspaces
-    // The children S + {m} of one frontier run whose S has at least three
-    // matched dimensions share one grid index over S's most selective ones
-    // (m, the last dimension, is then checked per candidate) and the sorted
-    // coordinates of S's dimensions; each adds its own column for m.
     std::vector<BatchSub> hs(B);
-    std::vector<int> reps;
-    long long coord = 0, hoff = 0, qoff = 0;
+    long long qoff = 0;
     int kmax = 1, kmin = 64;
-    bool all_packed = true;
-    int builder = -1;  // the index builder the next child of the same run may share
-    std::vector<int> shared_of(B, -1);  // the builder whose index a child shares
     int *cntB = batch.take<int>((size_t) B * n);
     for (int b = 0; b < B; ++b) {
         const ChildSub &c = cs[i0 + b];
         BatchSub &x = hs[b];
         std::memset(&x, 0, sizeof(x));
         x.S = arg_of(c.s);
-        const int kS = x.S.k - 1;
-        // shared where it costs the neighbour counts little: S's index
-        // dimensions are at most 25% less selective than the best index of
-        // S + {m} (expected candidates per query scale with the product of the
-        // index dimensions' selectivity scores)
-        bool shareable = kS >= 3 && __builtin_popcountll(match_of(x.S) & ((1ull << kS) - 1)) >= 3;
-        GridArg gbest{};
-        if (shareable) {
-            gbest = grid_of(x.S, x.S.k - 1, true);
-            const GridArg gopt = grid_of(x.S, -1, true);
-            double cs_ = 1.0, co_ = 1.0;
-            for (int a = 0; a < gbest.j; ++a) cs_ *= std::max(score[x.S.dims[gbest.tI[a]]], 1.0);
-            for (int a = 0; a < gopt.j; ++a) co_ *= std::max(score[x.S.dims[gopt.tI[a]]], 1.0);
-            shareable = gbest.j == gopt.j && cs_ <= 1.25 * co_;
-        }
-        long long ncell = 1;
-        if (shareable && builder >= 0 && cs[i0 + builder].t0 == c.t0 && cs[i0 + builder].t1 == c.t1 &&
-            hs[builder].G.j == gbest.j &&
-            std::equal(gbest.tI, gbest.tI + gbest.j, hs[builder].G.tI)) {
-            const BatchSub &r = hs[builder];
-            shared_of[b] = builder;
-            x.G = r.G;
-            x.obase = r.obase;
-            x.hoff = r.hoff;
-            x.coord = r.coord;
-            x.pos_m = x.S.k - 1;
-            x.mcoord = coord;
-            x.rep = 0;
-            coord += n;
-            ncell = grid_cells(x.G);
-        } else {
-            x.G = shareable ? grid_of(x.S, x.S.k - 1, true) : grid_of(x.S, -1, true);
-            ncell = grid_cells(x.G);
-            x.obase = (long long) reps.size() * n;
-            x.hoff = hoff;
-            hoff += ncell;
-            x.coord = coord;
-            x.pos_m = shareable ? x.S.k - 1 : x.S.k;
-            x.mcoord = shareable ? coord + (long long) (x.S.k - 1) * n : 0;
-            x.rep = 1;
-            coord += (long long) x.S.k * n;
-            reps.push_back(b);
-            if (shareable) builder = b;  // a later child of the same run may share it
-        }
+        x.G = child_grid(x.S);
         long long qmax = 0;
         for (int a = c.t0; a < c.t1; ++a)
             if (pair_on(a, c.m)) qmax += lt[lv_act[a]].nW;
         x.base = (long long) b * n;
-        x.qoff = qoff;
+        x.nbase = x.base;
         x.cnt = cntB + (size_t) b * n;
-        x.ncell = (int) ncell;
         x.cap = cap_of(x.S.k);
         x.thr_dense = dense_thr[x.S.k];
         x.qmax = (int) qmax;
         set_bounds(c.s, x);
         x.dbit = phi_mode ? 2 : 0;
         x.matchmask = match_of(x.S);
-        x.cellE = D.cellE;
         x.phi_w = phi_weak;
         x.phi_d = phi_dense[x.S.k];
-        x.nchk4 = 0;
-        x.restmask = 0;
-        for (int t = 0; t < x.S.k; ++t) {
-            if (!((x.G.checkmask >> t) & 1ull)) continue;
-            if (x.nchk4 < 4)
-                x.chk[x.nchk4++] = t;
-            else
-                x.restmask |= 1ull << t;
-        }
         qoff += qmax;
         kmax = std::max(kmax, x.S.k);
         kmin = std::min(kmin, x.S.k);
-        all_packed = all_packed && x.restmask == 0;
     }
-    const int kfast = (!generic_walk && kmin == kmax && kmax <= 7 && all_packed) ? kmax : 0;
+    const int kfast = (!generic_walk && kmin == kmax && kmax <= kMaxFastK) ? kmax : 0;
+    std::vector<const float *> ctab;
+    index_of(hs, ctab);
 
-    // index sorts kept from earlier batches of the run: the same index
-    // dimensions (in index order) sort the points the same way.  The indexes
-    // still to sort take the first places (obase, hoff), so the histogram
-    // scan covers only them; kept sorts are copied in behind.  A sort kept in
-    // this batch serves a later index of the same batch too.
-    std::vector<int> miss, hit_reps;
-    std::vector<KeptSort> hit_src, store_src;
-    int max_cell = 0;
-    auto cells_of = [&](const BatchSub &x) { return (int) grid_cells(x.G); };
-    for (int r : reps) {
-        const BatchSub &x = hs[r];
-        const int ncell = cells_of(x);
-        max_cell = std::max(max_cell, ncell);
-        uint64_t key = (uint64_t) x.G.j;
-        for (int a = 0; a < x.G.j; ++a) key |= (uint64_t) (x.S.dims[x.G.tI[a]] + 1) << (8 * (a + 1));
-        auto it = kept.find(key);
-        if (it != kept.end()) {
-            hit_reps.push_back(r);
-            hit_src.push_back(it->second);
-            continue;
-        }
-        miss.push_back(r);
-        const size_t need = ((size_t) 2 * n + ncell + 1) * sizeof(int) + 768;
-        KeptSort ks{nullptr, nullptr, nullptr};
-        if (kept_used + need <= kept_budget) {
-            ks = KeptSort{keptp.take<int>(n), keptp.take<int>(n), keptp.take<int>((size_t) ncell + 1)};
-            kept.emplace(key, ks);
-            kept_used += need;
-        }
-        store_src.push_back(ks);
-    }
-    long long hmiss = 0;
-    {
-        long long slot = 0, hpos = 0;
-        for (int r : miss) {
-            hs[r].obase = slot++ * n;
-            hs[r].hoff = hpos;
-            hpos += cells_of(hs[r]);
-        }
-        hmiss = hpos;
-        for (int r : hit_reps) {
-            hs[r].obase = slot++ * n;
-            hs[r].hoff = hpos;
-            hpos += cells_of(hs[r]);
-        }
-        for (int b = 0; b < B; ++b)
-            if (shared_of[b] >= 0) {
-                hs[b].obase = hs[shared_of[b]].obase;
-                hs[b].hoff = hs[shared_of[b]].hoff;
-            }
-    }
-    std::vector<SortCopy> hits, stores;
-    for (size_t u = 0; u < miss.size(); ++u)
-        if (store_src[u].order)
-            stores.push_back({store_src[u].order, store_src[u].pos, store_src[u].off, hs[miss[u]].obase,
-                              hs[miss[u]].hoff, cells_of(hs[miss[u]])});
-    for (size_t u = 0; u < hit_reps.size(); ++u)
-        hits.push_back({hit_src[u].order, hit_src[u].pos, hit_src[u].off, hs[hit_reps[u]].obase,
-                        hs[hit_reps[u]].hoff, cells_of(hs[hit_reps[u]])});
-    stats.sorts_kept += (int64_t) hits.size();
-    reps = miss;
-    reps.insert(reps.end(), hit_reps.begin(), hit_reps.end());
     BatchIndex X{};
-    X.nhist = (int) (hoff + 1);
-    X.keys = batch.take<int>((size_t) B * n);
-    X.rank = batch.take<int>((size_t) B * n);
-    X.order = batch.take<int>((size_t) B * n + 4);  // the grouped link walk reads up to 3 ids past a run
-    X.hist = batch.take<int>(X.nhist);
-    X.off = batch.take<int>(X.nhist);
-    X.Ys = batch.take<float>(coord + 4);  // the grouped walks read up to 3 past a column's end
-    X.Es = batch.take<uint16_t>(coord);
+    X.edge = edges;
     X.qflag = batch.take<uint8_t>(((size_t) B * n + 15) & ~(size_t) 15);  // read 16 bytes a lane
     X.qlist = batch.take<int>(std::max<long long>(qoff, 1));
     X.nsel = batch.take<int>(1);
@@ -475,75 +457,14 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     X.select_bytes = select_temp_bytes(B * n);
     X.select_temp = batch.take<char>(X.select_bytes);
     X.nb = batch.take<int>((size_t) kSampleEdges * B * n);
-    X.sig = batch.take<uint64_t>((size_t) B * n + 4);
-    X.sigS = batch.take<uint64_t>((size_t) reps.size() * n);
-    X.reps = upload(batch, reps);
-    X.nrep = (int) reps.size();
     X.nfb = batch.take<int>(1);
     X.fbcap = phi_mode ? B * n : 1;  // each point of each subspace is sent at most once per pass
     X.fb = batch.take<int2>(X.fbcap);
-    HIP_OK(launch_fill_i32(X.nb, -1, (size_t) kSampleEdges * B * n, st));
     X.dsorted = batch.take<uint8_t>((size_t) B * n + 8);  // the grouped link walk reads aligned words past the end
     X.par = batch.take<int>((size_t) B * n);
     X.giant = batch.take<int>(B);
-    X.scan_bytes = scan_temp_bytes(X.nhist);
-    X.scan_temp = batch.take<char>(X.scan_bytes);
+    HIP_OK(launch_fill_i32(X.nb, -1, (size_t) kSampleEdges * B * n, st));
     HIP_OK(launch_fill_i32(cntB, -1, (size_t) B * n, st));
-    BatchSub *dsubs = upload(batch, hs);
-    // sorted columns kept from earlier batches: the same index dimensions and
-    // dimension give the same column, in the order of the index's kept sort,
-    // so only an index whose sort is kept (copied in, or kept in this batch)
-    // keeps or reads columns: an index sorted again orders the points of a
-    // cell differently.  A column kept in this batch is read only from the
-    // next one on (the batch's gathers run in one launch).
-    ++batch_no;
-    auto sort_key = [&](const BatchSub &x) {
-        uint64_t key = (uint64_t) x.G.j;
-        for (int a = 0; a < x.G.j; ++a) key |= (uint64_t) (x.S.dims[x.G.tI[a]] + 1) << (8 * (a + 1));
-        return key;
-    };
-    auto column = [&](const BatchSub &x, int t, const float *&src, float *&dst) {
-        if (!kept.count(sort_key(x))) return;
-        const uint64_t ck = sort_key(x) | (uint64_t) (x.S.dims[t] + 1) << 32;
-        auto it = kept_cols.find(ck);
-        if (it != kept_cols.end()) {
-            if (it->second.second < batch_no) src = it->second.first;
-        } else if (cols_used + (size_t) n * sizeof(float) + 256 <= kept_budget) {
-            dst = colp.take<float>(n);
-            kept_cols.emplace(ck, std::make_pair(dst, batch_no));
-            cols_used += (size_t) n * sizeof(float) + 256;
-        }
-    };
-    std::vector<const float *> ysrc(reps.size() * kmax, nullptr), own_src(B, nullptr);
-    std::vector<float *> ystore(reps.size() * kmax, nullptr), own_store(B, nullptr);
-    for (size_t u = 0; u < reps.size(); ++u) {
-        const BatchSub &x = hs[reps[u]];
-        for (int t = 0; t < x.S.k; ++t)
-            if (t != x.pos_m) column(x, t, ysrc[u * kmax + t], ystore[u * kmax + t]);
-    }
-    for (int b = 0; b < B; ++b)
-        if (hs[b].pos_m < hs[b].S.k) column(hs[b], hs[b].pos_m, own_src[b], own_store[b]);
-    // the index tables of the batch in one copy
-    std::vector<char> blob;
-    auto add = [&blob](const auto &v) {
-        const size_t at = (blob.size() + 255) & ~(size_t) 255;
-        const size_t bytes = v.size() * sizeof(v[0]);
-        blob.resize(at + bytes);
-        if (bytes) std::memcpy(blob.data() + at, v.data(), bytes);
-        return at;
-    };
-    const size_t o_ysrc = add(ysrc), o_ystore = add(ystore), o_osrc = add(own_src), o_ostore = add(own_store);
-    const size_t o_miss = add(miss), o_stores = add(stores), o_hits = add(hits);
-    char *dblob = upload(batch, blob);
-    ColumnKeep cols{reinterpret_cast<const float *const *>(dblob + o_ysrc), reinterpret_cast<float *const *>(dblob + o_ystore),
-                    reinterpret_cast<const float *const *>(dblob + o_osrc),
-                    reinterpret_cast<float *const *>(dblob + o_ostore), kmax};
-    const int *dmiss = reinterpret_cast<const int *>(dblob + o_miss);
-    const SortCopy *dstores = reinterpret_cast<const SortCopy *>(dblob + o_stores);
-    const SortCopy *dhits = reinterpret_cast<const SortCopy *>(dblob + o_hits);
-    HIP_OK(launch_b_index(D, dsubs, B, X, kfast == 0, dmiss, (int) miss.size(), (int) hmiss, dstores,
-                          (int) stores.size(), dhits, (int) hits.size(), max_cell, cols, st));
-
 
     // ---- queries: the points of the trees each subspace refines, in sorted order
     std::vector<QuerySeg> qs;
@@ -557,14 +478,23 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             qblk.push_back(qblk.back() + nblocks(t.nW));
         }
     }
-    defer_uploads();
-    QuerySeg *dqs = upload(batch, qs);
-    int *dqb = upload(batch, qblk);
-    flush_uploads();
-    HIP_OK(launch_b_queries(dsubs, B, n, dqs, dqb, (int) qs.size(), qblk.back(), X, st));
     std::vector<int> cblk(B + 1, 0);
     for (int b = 0; b < B; ++b) cblk[b + 1] = cblk[b] + (hs[b].qmax + QPB - 1) / QPB;
+    defer_uploads();
+    const float *const *dcol = upload(batch, ctab);
+    {
+        size_t at = 0;
+        for (BatchSub &x : hs) {
+            x.col = dcol + at;
+            at += x.S.k;
+        }
+    }
+    BatchSub *dsubs = upload(batch, hs);
+    QuerySeg *dqs = upload(batch, qs);
+    int *dqb = upload(batch, qblk);
     int *dcb = upload(batch, cblk);
+    flush_uploads();
+    HIP_OK(launch_b_queries(dsubs, B, n, dqs, dqb, (int) qs.size(), qblk.back(), X, st));
     const bool dbg = batch_trace;
     std::chrono::steady_clock::time_point tq0, tq1;
     if (dbg) {

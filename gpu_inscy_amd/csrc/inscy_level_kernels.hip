@@ -48,161 +48,104 @@ __global__ void k_b_flags(const FlagTree *__restrict__ T, const int *__restrict_
     }
 }
 
-// ------------------------------------------------------------ grid indexes of a batch of subspaces
-// column t of subspace B's sorted coordinates / cells
-__device__ __forceinline__ long long col_of(const BatchSub &B, int t, int n) {
-    return t == B.pos_m ? B.mcoord : B.coord + (long long) t * n;
+// Edges of the eps cells: edge[i] is the smallest coordinate whose cell is at
+// least i - 1 (-inf for i <= 1, +inf past the last cell), i in [0, C + 3).  The
+// cell is monotone in the coordinate, so for a query in cell c the coordinates
+// whose cell is within one of c are exactly [edge[c], edge[c + 3]): the walks
+// test the cells of a candidate on its coordinate, without reading its cells.
+__global__ void k_cell_edges(int C, float *__restrict__ edge) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= C + 3) return;
+    const int target = i - 1;
+    float v = -__builtin_inff();
+    if (target >= C) {
+        v = __builtin_inff();
+    } else if (target > 0) {
+        const float ecs = ecell_width(C);
+        uint32_t lo = 0, hi = 0x3F800000u;  // cell(0) < target <= cell(1.0) = C - 1
+        while (hi - lo > 1) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if (ecell_of(__uint_as_float(mid), ecs, C) >= target)
+                hi = mid;
+            else
+                lo = mid;
+        }
+        v = __uint_as_float(hi);
+    }
+    edge[i] = v;
 }
 
-// grid keys and in-cell ranks of the subspaces that build an index (grid.y =
-// position in X.reps); one counting sort per such subspace
-__global__ void k_b_keys(DevData D, const BatchSub *__restrict__ subs, const int *__restrict__ reps,
-                         int *__restrict__ keys, int *__restrict__ rank, int *__restrict__ hist) {
-    const BatchSub &B = subs[reps[blockIdx.y]];
+// ------------------------------------------------------------ grid indexes of a batch of subspaces
+// grid keys and in-cell ranks (grid.y = index); one counting sort per index
+__global__ void k_b_keys(DevData D, const SortJob *__restrict__ jobs, int *__restrict__ keys, int *__restrict__ rank,
+                         int *__restrict__ hist) {
+    const SortJob &J = jobs[blockIdx.y];
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= D.n) return;
     int key = 0;
-    const int jl = B.G.j - 1;
-    for (int a = 0; a < jl; ++a) key = key * B.G.C + D.cellE[(size_t) B.S.dims[B.G.tI[a]] * D.n + p];
+    const int jl = J.j - 1;
+    for (int a = 0; a < jl; ++a) key = key * J.C + D.cellE[(size_t) J.dims[a] * D.n + p];
     // the last index dimension: its cell, or its bucket within the cell
-    const int dl = B.S.dims[B.G.tI[jl]];
-    if (B.G.F > 1)
-        key = key * (B.G.C * B.G.F) + fine_key(D.Xt[(size_t) dl * D.n + p], B.G.C, B.G.F);
+    const int dl = J.dims[jl];
+    if (J.F > 1)
+        key = key * (J.C * J.F) + fine_key(D.Xt[(size_t) dl * D.n + p], J.C, J.F);
     else
-        key = key * B.G.C + D.cellE[(size_t) dl * D.n + p];
-    keys[B.obase + p] = key;
-    rank[B.obase + p] = atomicAdd(&hist[B.hoff + key], 1);
+        key = key * J.C + D.cellE[(size_t) dl * D.n + p];
+    const size_t at = (size_t) blockIdx.y * D.n + p;
+    keys[at] = key;
+    rank[at] = atomicAdd(&hist[J.hoff + key], 1);
 }
 
 // `off` is one exclusive scan over the grid cells of every index of the
-// batch, so positions are global: index r holds [r*n, (r+1)*n).  The scatter
-// writes one int per point; the coordinates and cells are then gathered in
-// sorted order, so their writes are coalesced.
-__global__ void k_b_scatter(DevData D, const BatchSub *__restrict__ subs, const int *__restrict__ reps,
-                            int *__restrict__ keys, const int *__restrict__ rank, const int *__restrict__ off,
-                            int *__restrict__ order) {
-    const BatchSub &B = subs[reps[blockIdx.y]];
+// batch, so its positions are global: index u holds [u*n, (u+1)*n).  The
+// scatter writes the sorted ids, each point's sorted position and the index's
+// own cell offsets to where the index is kept.
+__global__ void k_b_scatter(int n, const SortJob *__restrict__ jobs, const int *__restrict__ keys,
+                            const int *__restrict__ rank, const int *__restrict__ off) {
+    const SortJob &J = jobs[blockIdx.y];
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= D.n) return;
-    const int at = off[B.hoff + keys[B.obase + p]] + rank[B.obase + p];
-    order[at] = p;
-    keys[B.obase + p] = at - (int) B.obase;  // from here on: the point's local sorted position
+    const int base = (int) ((long long) blockIdx.y * n);
+    if (p < n) {
+        const size_t src = (size_t) blockIdx.y * n + p;
+        const int at = off[J.hoff + keys[src]] + rank[src] - base;
+        J.order[at] = p;
+        J.pos[p] = at;
+    }
+    if (p <= J.ncell) J.off[p] = off[J.hoff + p] - base;
 }
 
-// the index builder's columns: every dimension but the child's own (all of
-// them when nothing is shared), and the packed cells of the checked ones
-// Sorted columns kept across batches: ysrc[c] (c = rep position * kmax + t
-// for the index columns, the subspace for its own column) is a kept copy of
-// the column, read in order instead of gathered; ystore[c] receives a newly
-// gathered column to keep.  Either may be null.
-__global__ void k_b_gather(DevData D, const BatchSub *__restrict__ subs, const int *__restrict__ reps,
-                           const int *__restrict__ order, float *__restrict__ Ys, uint16_t *__restrict__ Es,
-                           uint64_t *__restrict__ sigS, int need_es, const float *const *__restrict__ ysrc,
-                           float *const *__restrict__ ystore, int kmax) {
-    const BatchSub &B = subs[reps[blockIdx.y]];
-    const int n = D.n;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int p = order[B.obase + i];
-    const float ecs = ecell_width(D.ecells);
-    uint64_t w = 0;
-    for (int t = 0; t < B.S.k; ++t) {
-        if (t == B.pos_m) continue;
-        const int s = B.S.dims[t];
-        const float *src = ysrc[blockIdx.y * kmax + t];
-        float v;
-        if (src) {
-            v = src[i];
-        } else {
-            v = D.Xt[(size_t) s * n + p];
-            float *dst = ystore[blockIdx.y * kmax + t];
-            if (dst) dst[i] = v;
-        }
-        Ys[B.coord + (long long) t * n + i] = v;
-        // the cells from the coordinate itself (k_discretise's formula on the
-        // same value): no scattered read of the cell array
-        int f = -1;
-        for (int u = 0; u < B.nchk4; ++u)
-            if (B.chk[u] == t) f = u;
-        if (need_es || f >= 0) {
-            const int e = ecell_of(v, ecs, D.ecells);
-            if (need_es) Es[B.coord + (long long) t * n + i] = (uint16_t) e;
-            if (f >= 0) w |= (uint64_t) e << (16 * f);
-        }
+// coordinate columns in sorted order, four positions per thread
+constexpr int kGatherItems = 4;
+__global__ void k_b_gather(const ColJob *__restrict__ jobs, int n, int nblk) {
+    const int job = blockIdx.x / nblk, blk = blockIdx.x - job * nblk;
+    const ColJob J = jobs[job];
+    const int i0 = blk * kBlock * kGatherItems + threadIdx.x;
+    int p[kGatherItems];
+    float v[kGatherItems];
+#pragma unroll
+    for (int u = 0; u < kGatherItems; ++u) {
+        const int i = i0 + u * kBlock;
+        p[u] = i < n ? J.order[i] : 0;
     }
-    sigS[B.obase + i] = w;
-}
-
-// every subspace: its own column and its packed cells
-__global__ void k_b_gather_own(DevData D, const BatchSub *__restrict__ subs, const int *__restrict__ order,
-                               float *__restrict__ Ys, uint16_t *__restrict__ Es, const uint64_t *__restrict__ sigS,
-                               uint64_t *__restrict__ sig, int need_es, const float *const *__restrict__ ysrc,
-                               float *const *__restrict__ ystore) {
-    const BatchSub &B = subs[blockIdx.y];
-    const int n = D.n;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t w = sigS[B.obase + i];
-    if (B.pos_m < B.S.k) {
-        const int p = order[B.obase + i];
-        const int s = B.S.dims[B.pos_m];
-        const float *src = ysrc[blockIdx.y];
-        float v;
-        if (src) {
-            v = src[i];
-        } else {
-            v = D.Xt[(size_t) s * n + p];
-            if (float *dst = ystore[blockIdx.y]) dst[i] = v;
-        }
-        Ys[B.mcoord + i] = v;
-        bool own_checked = false;
-        for (int f = 0; f < B.nchk4; ++f) own_checked = own_checked || B.chk[f] == B.pos_m;
-        if (need_es || own_checked) {
-            const uint16_t e = (uint16_t) ecell_of(v, ecell_width(D.ecells), D.ecells);
-            if (need_es) Es[B.mcoord + i] = e;
-            for (int f = 0; f < B.nchk4; ++f)
-                if (B.chk[f] == B.pos_m) w |= (uint64_t) e << (16 * f);
-        }
+#pragma unroll
+    for (int u = 0; u < kGatherItems; ++u) v[u] = J.src[p[u]];
+#pragma unroll
+    for (int u = 0; u < kGatherItems; ++u) {
+        const int i = i0 + u * kBlock;
+        if (i < n) J.dst[i] = v[u];
     }
-    sig[B.base + i] = w;
 }
 
 // ------------------------------------------------------------ query lists in sorted order
-// pos: every point's local sorted position in its index
 __global__ void k_b_qmark(const BatchSub *__restrict__ subs, const QuerySeg *__restrict__ segs,
-                          const int *__restrict__ blk_off, int nseg, const int *__restrict__ pos,
-                          uint8_t *__restrict__ qflag) {
+                          const int *__restrict__ blk_off, int nseg, uint8_t *__restrict__ qflag) {
     const int s = seg_of(blk_off, nseg, blockIdx.x);
     const QuerySeg Q = segs[s];
     const int i = (blockIdx.x - blk_off[s]) * blockDim.x + threadIdx.x;
     if (i >= Q.len) return;
     const BatchSub &B = subs[Q.b];
     const int p = Q.P[i];
-    qflag[B.base + pos[B.obase + p]] = 1;
-}
-
-// kept sorts: copied in after the scan of the indexes still to sort; sorts
-// to keep are copied out of the batch after their scatter
-__global__ void k_b_sort_in(const SortCopy *__restrict__ cs, int n, int *__restrict__ order, int *__restrict__ pos,
-                            int *__restrict__ off) {
-    const SortCopy &c = cs[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        order[c.obase + i] = c.order[i];
-        pos[c.obase + i] = c.pos[i];
-    }
-    if (i <= c.ncell) off[c.hoff + i] = c.off[i] + (int) c.obase;
-}
-
-__global__ void k_b_sort_out(const SortCopy *__restrict__ cs, int n, const int *__restrict__ order,
-                             const int *__restrict__ pos, const int *__restrict__ off) {
-    const SortCopy &c = cs[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        c.order[i] = order[c.obase + i];
-        c.pos[i] = pos[c.obase + i];
-    }
-    if (i <= c.ncell) c.off[i] = off[c.hoff + i] - (int) c.obase;
+    qflag[B.base + B.pos[p]] = 1;
 }
 
 // qstart[b] = first index of the selected (ascending global) positions that is
@@ -238,16 +181,16 @@ __global__ void k_b_qstart(const int *__restrict__ qlist, const int *__restrict_
 // holds the query, so it is not empty).  q[21..30]: prefix sums of the runs'
 // lengths in groups of four (ceil(length / 4)), for the walks that take four
 // consecutive candidates of one run per lane.
-__device__ __forceinline__ void build_runs(const GridArg &G, const int *__restrict__ off, const int *qe,
-                                           const float *qy, int stride, float s_star, int base0, int *q) {
+__device__ __forceinline__ void build_runs(const GridArg &G, const int *__restrict__ off, const int *ci,
+                                           const float *qy, int stride, float s_star, int *q) {
     // rows r = 3 xi + yi over the cells within one of the query's in the first
     // (and second) index dimension, each a run of the last one's cells within
     // one; every row's two offsets are loaded before any is used, so the
     // set-up costs one memory round trip
     const int C = G.C;
-    const int c0 = qe[G.tI[0] * stride];
-    const int c1 = G.j == 3 ? qe[G.tI[1] * stride] : 0;
-    const int cl = qe[G.tI[G.j - 1] * stride];
+    const int c0 = ci[0];
+    const int c1 = G.j == 3 ? ci[1] : 0;
+    const int cl = ci[G.j - 1];
     const int F = G.F > 1 ? G.F : 1, CF = C * F;
     // a run: the buckets of the last dimension's cells within one of the
     // query's, less those farther than eps from the query's coordinate (a
@@ -281,7 +224,7 @@ __device__ __forceinline__ void build_runs(const GridArg &G, const int *__restri
     for (int r = 0; r < 9; ++r) {
         if (r / 3 < nx && r % 3 < ny && e[r] > a[r]) {
             if (r == own) q[20] = nr;
-            q[nr] = a[r] - base0;
+            q[nr] = a[r];
             acc += e[r] - a[r];
             gacc += (e[r] - a[r] + 3) >> 2;
             q[10 + nr] = acc;
@@ -297,37 +240,18 @@ __device__ __forceinline__ int run_pos(const int *q, int c, int &r) {
     return q[r] + (c - q[9 + r]);
 }
 
-constexpr int kFastDims = 8;
-
-// the packed cells of the checked dimensions lie within one cell of the query's
-__device__ __forceinline__ bool cells_near(uint64_t w, uint64_t qsig, int nc) {
-    bool ok = true;
-    for (int f = 0; f < nc; ++f) {
-        const int dc = (int) ((w >> (16 * f)) & 0xFFFFull) - (int) ((qsig >> (16 * f)) & 0xFFFFull);
-        ok = ok && dc >= -1 && dc <= 1;
-    }
-    return ok;
-}
-
-// Candidate at local sorted position jj against the staged query: cells of the
-// checked dimensions within one (packed word first), then the distance summed
-// in subspace order with separate multiplies and adds, compared with s_star.
-__device__ __forceinline__ bool cand_test(const BatchSub &B, int n, const float *__restrict__ Ys,
-                                          const uint16_t *__restrict__ Es, const uint64_t *__restrict__ sigb,
-                                          uint64_t qsig, const float *qy, const int *qe, int stride, int jj,
-                                          float s_star, float &acc_out) {
-    const int nc = B.nchk4;
-    if (nc > 0 && !cells_near(sigb[jj], qsig, nc)) return false;
-    const uint64_t rest = B.restmask;
+// Candidate at local sorted position jj against the staged query: the cells of
+// the checked dimensions within one of the query's (its coordinate between two
+// cell edges), then the distance summed in subspace order with separate
+// multiplies and adds, compared with s_star.
+__device__ __forceinline__ bool cand_test(const BatchSub &B, const float *qy, const float2 *qc, int stride, int jj, float s_star, float &acc_out) {
     const int k = B.S.k;
     float acc = 0.0f;
     for (int t = 0; t < k; ++t) {
-        const long long col = col_of(B, t, n);
-        if ((rest >> t) & 1ull) {
-            const int de = (int) Es[col + jj] - qe[t * stride];
-            if (de < -1 || de > 1) return false;
-        }
-        const float diff = qy[t * stride] - Ys[col + jj];
+        const float y = B.col[t][jj];
+        const float2 c = qc[t * stride];
+        if (!(y >= c.x && y < c.y)) return false;
+        const float diff = qy[t * stride] - y;
         const float sq = diff * diff;
         acc = acc + sq;
         if (acc > s_star) return false;
@@ -336,41 +260,57 @@ __device__ __forceinline__ bool cand_test(const BatchSub &B, int n, const float 
     return true;
 }
 
-// LDS of the neighbour passes: per query k coordinates, k cells, its packed
-// cells (2 words) and its runs
-__device__ __forceinline__ void lds_layout(char *smem, int k, float *&sy, int *&se, uint64_t *&qs, int *&qr) {
-    sy = reinterpret_cast<float *>(smem);
-    se = reinterpret_cast<int *>(smem + sizeof(float) * QPB * k);
-    qs = reinterpret_cast<uint64_t *>(smem + 8 * (size_t) QPB * k);
-    qr = reinterpret_cast<int *>(smem + 8 * (size_t) QPB * k + 8 * QPB);
+// LDS of the neighbour passes: per query k cell intervals, k coordinates and
+// its runs
+__device__ __forceinline__ void lds_layout(char *smem, int k, float2 *&sc, float *&sy, int *&qr) {
+    sc = reinterpret_cast<float2 *>(smem);
+    sy = reinterpret_cast<float *>(smem + sizeof(float2) * QPB * (size_t) k);
+    qr = reinterpret_cast<int *>(smem + (sizeof(float2) + sizeof(float)) * QPB * (size_t) k);
 }
 
-// the query's coordinates (sorted position i) and cells (point p) into LDS:
-// the first 8 dimensions' loads are all issued before any store (a store to
-// LDS through a generic pointer would otherwise order each load after the
-// previous store, one memory round trip per dimension)
+// the query's coordinates (sorted position i) and, per checked dimension, the
+// interval [lower, upper) of the coordinates whose eps cell is within one of
+// its own, into LDS: the first 8 dimensions' loads are all issued before any
+// store (a store to LDS through a generic pointer would otherwise order each
+// load after the previous store, one memory round trip per dimension)
 // (the cells are computed from the coordinates with the discretisation's
-// formula, G.C being the number of eps cells: no scattered read by point id)
-__device__ __forceinline__ void stage_query_b(const BatchSub &B, int n, const float *__restrict__ Ys, int p, int i,
-                                              float *sy, int *se, int stride) {
+// formula, G.C being the number of eps cells: no scattered read by point id;
+// the intervals come from the table of cell edges, see k_cell_edges)
+__device__ __forceinline__ void stage_query_b(const BatchSub &B, const float *__restrict__ edge, int i, float *sy,
+                                              float2 *sc, int stride, int *ci) {
     constexpr int kStage = 8;
     const int k = B.S.k;
     const float ecs = ecell_width(B.G.C);
-    (void) p;
+    const float inf = __builtin_inff();
     float y[kStage];
 #pragma unroll
-    for (int t = 0; t < kStage; ++t) y[t] = t < k ? Ys[col_of(B, t, n) + i] : 0.0f;
+    for (int t = 0; t < kStage; ++t) y[t] = t < k ? B.col[t][i] : 0.0f;
+    float2 c[kStage];
+#pragma unroll
+    for (int t = 0; t < kStage; ++t) {
+        c[t] = make_float2(-inf, inf);
+        if (t < k && ((B.G.checkmask >> t) & 1ull)) {
+            const int e = ecell_of(y[t], ecs, B.G.C);
+            c[t] = make_float2(edge[e], edge[e + 3]);
+        }
+    }
 #pragma unroll
     for (int t = 0; t < kStage; ++t)
         if (t < k) {
             sy[t * stride] = y[t];
-            se[t * stride] = ecell_of(y[t], ecs, B.G.C);
+            sc[t * stride] = c[t];
         }
     for (int t = kStage; t < k; ++t) {
-        const float v = Ys[col_of(B, t, n) + i];
+        const float v = B.col[t][i];
         sy[t * stride] = v;
-        se[t * stride] = ecell_of(v, ecs, B.G.C);
+        float2 cc = make_float2(-inf, inf);
+        if ((B.G.checkmask >> t) & 1ull) {
+            const int e = ecell_of(v, ecs, B.G.C);
+            cc = make_float2(edge[e], edge[e + 3]);
+        }
+        sc[t * stride] = cc;
     }
+    for (int a = 0; a < B.G.j; ++a) ci[a] = ecell_of(sy[B.G.tI[a] * stride], ecs, B.G.C);
 }
 
 // ------------------------------------------------------------ candidate walks of one query
@@ -384,13 +324,8 @@ struct QueryWalk {
     const BatchSub &B;
     int n, i, p;
     const int *q;    // the query's runs (LDS)
-    const float *qy; // its coordinates (LDS, stride QPB)
-    const int *qe;   // its cells (LDS, stride QPB)
-    uint64_t qsig;   // its packed cells
-    const int *__restrict__ order;
-    const float *__restrict__ Ys;
-    const uint16_t *__restrict__ Es;
-    const uint64_t *__restrict__ sigb;
+    const float *qy;   // its coordinates (LDS, stride QPB)
+    const float2 *qc;  // its cell intervals (LDS, stride QPB)
     float s_star, eps;
     double phirel;
     int *nbp;        // its two recorded neighbours
@@ -400,19 +335,6 @@ __device__ __forceinline__ int walk_rot(const QueryWalk &W, int total) {
     const int *q = W.q;
     const int cs0 = q[9 + q[20]], clen = q[10 + q[20]] - cs0;
     return total > 0 ? cs0 + (int) (((uint32_t) W.p * 2654435761u) % (uint32_t) max(clen, 1)) : 0;
-}
-
-// per 16-bit field (w - q + 1) mod 2^16 is 0, 1 or 2 exactly when the cells
-// differ by at most one (cells < 65535); fields beyond the checked
-// dimensions are zero in both words and pass
-__device__ __forceinline__ bool cells_near_packed(uint64_t w, uint64_t qsig) {
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    const u16x2 one = {1, 1};
-    const u16x2 d0 = __builtin_bit_cast(u16x2, (uint32_t) w) - __builtin_bit_cast(u16x2, (uint32_t) qsig) + one;
-    const u16x2 d1 =
-        __builtin_bit_cast(u16x2, (uint32_t) (w >> 32)) - __builtin_bit_cast(u16x2, (uint32_t) (qsig >> 32)) + one;
-    const u16x2 m = __builtin_elementwise_max(d0, d1);
-    return m.x <= 2 && m.y <= 2;
 }
 
 // neighbours found in one step: the first kSampleEdges are recorded (the sample edges
@@ -437,7 +359,7 @@ __device__ __forceinline__ void walk_tally(const QueryWalk &W, const int (&jj)[U
         const unsigned long long mine = (__ballot(hit[u]) >> gshift) & ((1ull << LPQ) - 1ull);
         if (hit[u] && found < kSampleEdges) {
             const int at = found + __popcll(mine & below);
-            if (at < kSampleEdges) W.nbp[at] = W.order[W.B.obase + jj[u]];
+            if (at < kSampleEdges) W.nbp[at] = W.B.order[jj[u]];
         }
         found += __popcll(mine);
     }
@@ -452,23 +374,44 @@ __device__ __forceinline__ bool walk_more(const QueryWalk &W, bool phi, int foun
     return found < W.B.cap;
 }
 
-// k = K dimensions, every checked one packed (the host checks), counts or
-// phi.  Each lane takes four consecutive candidates of one run per step, so a
-// step loads each coordinate column with one 16-byte load per lane (and the
-// packed cells with two) instead of four 4-byte loads.  The vector memory pipeline bounds
-// these walks (its address and data units are busy nearly all the time),
-// and its cost grows with the number of load instructions.  The runs are
+// The cell test of a step's hits.  A candidate within eps lies more than one
+// cell away only next to a cell edge, so the test runs on the few candidates
+// that passed the distance: its coordinates are read again there (they were
+// just loaded) rather than kept in registers for all of them.
+template <int U>
+__device__ __forceinline__ void cells_of_hits(const BatchSub &B, const float2 *qc, int stride, uint32_t checked,
+                                              int jj0, bool (&hit)[U]) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    static_assert(U == 4, "one 16-byte load per column");
+    if (!(hit[0] | hit[1] | hit[2] | hit[3])) return;
+    for (uint32_t m = checked; m; m &= m - 1) {
+        const int t = __builtin_ctz(m);
+        const float2 c = qc[t * stride];
+        const f4u y = *reinterpret_cast<const f4u *>(B.col[t] + (uint32_t) jj0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) hit[u] = hit[u] & (y[u] >= c.x) & (y[u] < c.y);
+    }
+}
+
+// k = K dimensions (the host checks), counts or phi.  Each lane takes four
+// consecutive candidates of one run per step, so a step loads each coordinate
+// column with one 16-byte load per lane instead of four 4-byte loads, and
+// nothing else: the eps cells of the checked dimensions are tested on the
+// coordinates of the step's hits (cells_of_hits).
+// The vector memory pipeline bounds these walks (its address and data units
+// are busy nearly all the time), and its cost grows with the number of load
+// instructions.  The runs are
 // concatenated in groups of four (q[21..30]); the last group of a run masks
 // the positions past the run's end, which are read (up to three past the
-// run: the batch's coordinate and packed-cell buffers end with padding) but
+// run: the batch's coordinate buffer ends with padding) but
 // never counted.  A lane's first group position is 4-byte aligned only;
 // dword-aligned multi-dword global loads are supported on gfx950.
 template <int K, bool PHI>
 __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double &dsum, bool &more, long long &seen) {
     typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-    typedef unsigned long long u2u __attribute__((ext_vector_type(2), aligned(8)));
     constexpr int LPQ = kBLanes, U = 4;
     const BatchSub &B = W.B;
+    const uint32_t checked = (uint32_t) B.G.checkmask;
     const int *q = W.q;
     const int sub = __lane_id() % LPQ;
     const int nr = q[19];
@@ -482,7 +425,7 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
     float qv[K];
 #pragma unroll
     for (int t = 0; t < K; ++t) {
-        col[t] = W.Ys + (t == B.pos_m ? B.mcoord : B.coord + (long long) t * W.n);
+        col[t] = B.col[t];
         qv[t] = W.qy[t * QPB];
     }
     for (int segm = 0; segm < 2; ++segm) {
@@ -499,14 +442,11 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
             const int len = q[10 + r] - q[9 + r];
             const int nv = g0 + sub < gend ? min(U, len - e0) : 0;  // its elements inside the run
             const int jj0 = q[r] + e0;
-            const u2u wa = *reinterpret_cast<const u2u *>(W.sigb + (uint32_t) jj0);
-            const u2u wb = *reinterpret_cast<const u2u *>(W.sigb + (uint32_t) jj0 + 2);
             f4u y[K];
 #pragma unroll
             for (int t = 0; t < K; ++t)
                 y[t] = *reinterpret_cast<const f4u *>(reinterpret_cast<const char *>(col[t]) +
                                                       ((uint32_t) jj0 << 2));
-            const uint64_t w[U] = {wa.x, wa.y, wb.x, wb.y};
             int jj[U];
             bool hit[U];
             float accs[U];
@@ -520,9 +460,10 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
                     acc = acc + sq;
                 }
                 jj[u] = jj0 + u;
-                hit[u] = (u < nv) & (jj[u] != W.i) & cells_near_packed(w[u], W.qsig) & (acc <= W.s_star);
+                hit[u] = (u < nv) & (jj[u] != W.i) & (acc <= W.s_star);
                 accs[u] = acc;
             }
+            if (checked) cells_of_hits<U>(B, W.qc, QPB, checked, jj0, hit);
             // the query's examined candidates of the step, summed over its
             // quad with two DPP moves
             int ex = nv;
@@ -557,79 +498,7 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
     }
 }
 
-// k <= kFastDims with every checked dimension packed, k known only at run
-// time (batches that mix dimensionalities): loads predicated on the packed
-// cell test, the sum over the first k of kFastDims terms
-template <bool PHI>
-__device__ __forceinline__ void walk_fast_rt(const QueryWalk &W, int &found, double &dsum, bool &more,
-                                             long long &seen) {
-    constexpr int LPQ = kBLanes, U = 4, STEP = LPQ * U;
-    const BatchSub &B = W.B;
-    const int *q = W.q;
-    const int sub = __lane_id() % LPQ;
-    const int total = q[9 + q[19]];
-    const int rot = walk_rot(W, total);
-    const int k = B.S.k, nc = B.nchk4, pm = B.pos_m;
-    const long long cb = B.coord, mc = B.mcoord;
-    float qv[kFastDims];
-#pragma unroll
-    for (int t = 0; t < kFastDims; ++t) qv[t] = t < k ? W.qy[t * QPB] : 0.0f;
-    int r = 0;
-    bool wrapped = false;
-    for (int c0 = 0; c0 < total && more; c0 += STEP) {
-        int jj[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int c = c0 + u * LPQ + sub;
-            jj[u] = -1;
-            if (c < total) {
-                int cr = c + rot;
-                if (cr >= total) {
-                    cr -= total;
-                    if (!wrapped) {
-                        wrapped = true;
-                        r = 0;
-                    }
-                }
-                jj[u] = run_pos(q, cr, r);
-            }
-        }
-        uint64_t w[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) w[u] = (jj[u] >= 0 && nc > 0) ? W.sigb[jj[u]] : 0ull;
-        bool ok[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) ok[u] = jj[u] >= 0 && jj[u] != W.i && cells_near(w[u], W.qsig, nc);
-        float y[U][kFastDims];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int t = 0; t < kFastDims; ++t)
-                y[u][t] = (ok[u] && t < k) ? W.Ys[(t == pm ? mc : cb + (long long) t * W.n) + jj[u]] : 0.0f;
-        bool hit[U];
-        float accs[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int t = 0; t < kFastDims; ++t) {
-                if (t < k) {
-                    const float diff = qv[t] - y[u][t];
-                    const float sq = diff * diff;
-                    acc = acc + sq;
-                }
-            }
-            hit[u] = ok[u] && acc <= W.s_star;
-            accs[u] = acc;
-        }
-        walk_tally<U, PHI>(W, jj, hit, accs, found, dsum);
-        seen += min(STEP, total - c0);
-        more = walk_more(W, PHI, found, dsum, total);
-    }
-}
-
-// any k, cells of the checked dimensions beyond the packed four compared one
-// by one (cand_test)
+// any k, one candidate per lane at a time (cand_test)
 template <bool PHI>
 __device__ __forceinline__ void walk_generic(const QueryWalk &W, int &found, double &dsum, bool &more,
                                              long long &seen) {
@@ -664,7 +533,7 @@ __device__ __forceinline__ void walk_generic(const QueryWalk &W, int &found, dou
         for (int u = 0; u < U; ++u) {
             accs[u] = 0.0f;
             hit[u] = jj[u] >= 0 && jj[u] != W.i &&
-                     cand_test(W.B, W.n, W.Ys, W.Es, W.sigb, W.qsig, W.qy, W.qe, QPB, jj[u], W.s_star, accs[u]);
+                     cand_test(W.B, W.qy, W.qc, QPB, jj[u], W.s_star, accs[u]);
         }
         walk_tally<U, PHI>(W, jj, hit, accs, found, dsum);
         seen += min(STEP, total - c0);
@@ -678,9 +547,7 @@ __device__ __forceinline__ void walk_generic(const QueryWalk &W, int &found, dou
 // count is still missing (components pass, with the subset bound).
 template <bool LIST, bool PHI, int K>
 __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__ subs, const int *__restrict__ blk_off,
-                                                    int nsub, int n, const int *__restrict__ off,
-                                                    const int *__restrict__ order, const float *__restrict__ Ys,
-                                                    const uint16_t *__restrict__ Es, const uint64_t *__restrict__ sig,
+                                                    int nsub, int n, const float *__restrict__ edge,
                                                     const int *__restrict__ qlist, const int *__restrict__ qstart,
                                                     float s_star, float eps, double phirel, int *__restrict__ nb,
                                                     int2 *__restrict__ fb, int *__restrict__ nfb, int fbcap,
@@ -697,10 +564,10 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
     }
     const BatchSub &B = subs[b];
     const int k = B.S.k;
+    float2 *sc;
     float *sy;
-    int *se, *qr;
-    uint64_t *qs;
-    lds_layout(smem, k, sy, se, qs, qr);
+    int *qr;
+    lds_layout(smem, k, sc, sy, qr);
     const int lq = threadIdx.x / LPQ, sub = threadIdx.x % LPQ;
     int i = 0;
     bool active;
@@ -712,9 +579,8 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
         i = blk * QPB + lq;
         active = i < n;
     }
-    const uint64_t *sigb = sig + B.base;
     int *cnt = B.cnt;
-    const int p = active ? order[B.obase + i] : 0;
+    const int p = active ? B.order[i] : 0;
     active = active && cnt[p] < 0;
     // N_S(p) is a subset of N_S'(p) for S' a subset of S: the smallest
     // complete count of the subspaces S minus one dimension, when below both
@@ -731,13 +597,11 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
             active = false;
         }
     }
-    const int base0 = (int) B.obase;
     int *q = qr + lq * kRangeWords;
     if (sub == 0 && active) {
-        const uint64_t qsg = sigb[i];
-        stage_query_b(B, n, Ys, p, i, sy + lq, se + lq, QPB);
-        qs[lq] = qsg;
-        build_runs(B.G, off + B.hoff, se + lq, sy + lq, QPB, s_star, base0, q);
+        int ci[3];
+        stage_query_b(B, edge, i, sy + lq, sc + lq, QPB, ci);
+        build_runs(B.G, B.off, ci, sy + lq, QPB, s_star, q);
     }
     __syncthreads();
     long long seen = 0;
@@ -745,14 +609,12 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
     if (active) {
         double dsum = 0.0;
         bool more = true;
-        const QueryWalk W{B, n, i, p, q, sy + lq, se + lq, qs[lq], order, Ys, Es, sigb, s_star, eps, phirel,
-                          nb + kSampleEdges * (B.base + p)};
-        // K > 0: every subspace of the launch has k = K with its checked
-        // dimensions packed (the host checks), so the walk is compiled for it
+        const QueryWalk W{B, n, i, p, q, sy + lq, sc + lq, s_star, eps, phirel,
+                          nb + kSampleEdges * (B.nbase + p)};
+        // K > 0: every subspace of the launch has k = K (the host checks), so
+        // the walk is compiled for it
         if constexpr (K > 0)
             walk_vec<K, PHI>(W, found, dsum, more, seen);
-        else if (k <= kFastDims && B.restmask == 0)
-            walk_fast_rt<PHI>(W, found, dsum, more, seen);
         else
             walk_generic<PHI>(W, found, dsum, more, seen);
         if (PHI) {
@@ -789,13 +651,12 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
     if (stat) {
         // per wave into one of 64 slot groups: [0] candidates examined, [1]
         // points counted, [2] algorithmic bytes (4k + 4 per point, 4 + 4k per
-        // neighbour established), [3] bytes of the examined candidates (their
-        // packed cells when packed, and k coordinates)
+        // neighbour established), [3] bytes of the examined candidates (k coordinates)
         const bool mine = sub == 0 && active;
         long long done = mine ? 1 : 0;
         long long abytes = mine ? (4ll * k + 4) + (long long) found * (4 + 4ll * k) : 0;
         if (sub != 0) seen = 0;
-        long long ebytes = seen * ((B.nchk4 > 0 ? 8ll : 0ll) + 4ll * k);
+        long long ebytes = seen * 4ll * k;
         for (int o = 32; o > 0; o >>= 1) {
             seen += __shfl_down(seen, o);
             done += __shfl_down(done, o);
@@ -814,14 +675,13 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
 
 // ------------------------------------------------------------ dense components of a batch
 // (k_dense_init .. k_uf_flatten per subspace; grid.y = subspace)
-__global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, const int *__restrict__ order,
-                               uint8_t *__restrict__ dsorted, int *__restrict__ par) {
+__global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, uint8_t *__restrict__ dsorted, int *__restrict__ par) {
     const BatchSub &B = subs[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     // i is a sorted position for the dense flag and a point id for the
     // parents and sizes, so every write is coalesced
-    const int p = order[B.obase + i];
+    const int p = B.order[i];
     dsorted[B.base + i] = meets(B.cnt[p], B.thr_dense, B.dbit) ? 1 : 0;
     par[B.base + i] = meets(B.cnt[i], B.thr_dense, B.dbit) ? i : -1;
     B.csize[i] = 0;
@@ -847,7 +707,7 @@ __global__ void k_b_link_sample(const BatchSub *__restrict__ subs, int n, const 
     if (pp < 0) return;
     // the recorded neighbours: min(count, kSampleEdges) of them, -1 after
     // (phi mode records them too)
-    const int q = nb[kSampleEdges * (B.base + p) + round];
+    const int q = nb[kSampleEdges * (B.nbase + p) + round];
     if (q < 0 || q >= n) return;
     // after the first round's compression every point's parent is its root:
     // equal parents are one set, decided without reading the root's own entry
@@ -893,62 +753,55 @@ __global__ void k_b_giant(const BatchSub *__restrict__ subs, int n, const int *_
 }
 
 // Full phase: every dense point outside the giant component links to all its
-// dense neighbours.  K > 0: every subspace of the launch has k = K with its
-// checked dimensions packed, and a step loads the dense flags, packed cells,
-// point ids and K coordinates of U candidates per lane at once (a lane past
-// the end re-reads the last candidate and is masked).
+// dense neighbours.  K > 0: every subspace of the launch has k = K, and a step
+// loads the dense flags, point ids and K coordinates of U candidates per lane
+// at once (a lane past the end re-reads the last candidate and is masked).
 template <int K>
 __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restrict__ subs, int n,
-                                                        const int *__restrict__ off, const int *__restrict__ order,
-                                                        const float *__restrict__ Ys, const uint16_t *__restrict__ Es,
-                                                        const uint64_t *__restrict__ sig,
+                                                        const float *__restrict__ edge,
                                                         const uint8_t *__restrict__ dsorted, float s_star,
                                                         const int *__restrict__ giant, int *__restrict__ par) {
     constexpr int LPQ = kBLanes;
     extern __shared__ char smem[];
     const BatchSub &B = subs[blockIdx.y];
     const int k = B.S.k;
+    float2 *sc;
     float *sy;
-    int *se, *qr;
-    uint64_t *qs;
-    lds_layout(smem, k, sy, se, qs, qr);
+    int *qr;
+    lds_layout(smem, k, sc, sy, qr);
     const int lq = threadIdx.x / LPQ, sub = threadIdx.x % LPQ;
     const int i = blockIdx.x * QPB + lq;
     const uint8_t *ds = dsorted + B.base;
-    const int *ord = order + B.obase;
-    const uint64_t *sigb = sig + B.base;
+    const int *ord = B.order;
     int *pr = par + B.base;
     bool active = i < n && ds[i];
     const int p = active ? ord[i] : 0;
     if (active && pr[p] == giant[blockIdx.y]) active = false;
     int *q = qr + lq * kRangeWords;
     if (sub == 0 && active) {
-        const uint64_t qsg = sigb[i];
-        stage_query_b(B, n, Ys, p, i, sy + lq, se + lq, QPB);
-        qs[lq] = qsg;
-        build_runs(B.G, off + B.hoff, se + lq, sy + lq, QPB, s_star, (int) B.obase, q);
+        int ci[3];
+        stage_query_b(B, edge, i, sy + lq, sc + lq, QPB, ci);
+        build_runs(B.G, B.off, ci, sy + lq, QPB, s_star, q);
     }
     __syncthreads();
     if (!active) return;
     const float *qy = sy + lq;
-    const int *qe = se + lq;
-    const uint64_t qsig = qs[lq];
+    const float2 *qcl = sc + lq;
     const int total = q[9 + q[19]];
     int rp = uf_find(pr, p);
     if constexpr (K > 0) {
         // each lane four consecutive candidates of one run per step (the
         // groups of walk_vec): per step one 16-byte load for the ids and each
-        // coordinate column, two for the packed cells and two aligned words
-        // for the four dense flags
+        // coordinate column, and two aligned words for the four dense flags
         typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
         typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
-        typedef unsigned long long u2u __attribute__((ext_vector_type(2), aligned(8)));
         constexpr int U = 4;
+        const uint32_t checked = (uint32_t) B.G.checkmask;
         const float *col[K];
         float qv[K];
 #pragma unroll
         for (int t = 0; t < K; ++t) {
-            col[t] = Ys + (t == B.pos_m ? B.mcoord : B.coord + (long long) t * n);
+            col[t] = B.col[t];
             qv[t] = qy[t * QPB];
         }
         const uint32_t *dw = reinterpret_cast<const uint32_t *>(dsorted);  // 256-byte aligned
@@ -967,14 +820,11 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
             const int jj0 = q[r] + e0;
             const size_t at = (size_t) B.base + (size_t) jj0;  // byte index of the first dense flag
             const uint32_t d0 = dw[at >> 2], d1 = dw[(at >> 2) + 1];
-            const u2u wa = *reinterpret_cast<const u2u *>(sigb + (uint32_t) jj0);
-            const u2u wb = *reinterpret_cast<const u2u *>(sigb + (uint32_t) jj0 + 2);
             const i4u qv4 = *reinterpret_cast<const i4u *>(ord + (uint32_t) jj0);
             f4u y[K];
 #pragma unroll
             for (int t = 0; t < K; ++t) y[t] = *reinterpret_cast<const f4u *>(col[t] + (uint32_t) jj0);
             const uint32_t dn4 = __builtin_amdgcn_alignbyte(d1, d0, (uint32_t) (at & 3));
-            const uint64_t w[U] = {wa.x, wa.y, wb.x, wb.y};
             const int qq[U] = {qv4.x, qv4.y, qv4.z, qv4.w};
             bool hit[U];
 #pragma unroll
@@ -986,9 +836,9 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
                     const float sq = diff * diff;
                     acc = acc + sq;
                 }
-                hit[u] = (u < nv) & (jj0 + u != i) & (((dn4 >> (8 * u)) & 0xFFu) != 0) &
-                         cells_near_packed(w[u], qsig) & (acc <= s_star);
+                hit[u] = (u < nv) & (jj0 + u != i) & (((dn4 >> (8 * u)) & 0xFFu) != 0) & (acc <= s_star);
             }
+            if (checked) cells_of_hits<U>(B, qcl, QPB, checked, jj0, hit);
             // parents only move up to roots: a parent equal to p's root is p's set
             int pq[U];
 #pragma unroll
@@ -1005,7 +855,7 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
         for (int c = sub; c < total; c += LPQ) {
             const int jj = run_pos(q, c, r);
             float acc;
-            if (jj == i || !ds[jj] || !cand_test(B, n, Ys, Es, sigb, qsig, qy, qe, QPB, jj, s_star, acc)) continue;
+            if (jj == i || !ds[jj] || !cand_test(B, qy, qcl, QPB, jj, s_star, acc)) continue;
             const int qq = ord[jj];
             // parents only move up to roots: a parent equal to p's root is p's set
             if (pr[qq] == rp || uf_find(pr, qq) == rp) continue;
@@ -1636,8 +1486,12 @@ static_assert(kBlockThreads == kBlock && kQueriesPerBlock == QPB, "launch geomet
 
 static unsigned query_blocks_n(int n) { return (unsigned) ((n + QPB - 1) / QPB); }
 static size_t count_lds(int kmax) {
-    return (sizeof(float) + sizeof(int)) * QPB * (size_t) (kmax > 0 ? kmax : 1) + 8 * QPB +
-           sizeof(int) * QPB * kRangeWords;
+    return (sizeof(float2) + sizeof(float)) * QPB * (size_t) (kmax > 0 ? kmax : 1) + sizeof(int) * QPB * kRangeWords;
+}
+
+hipError_t launch_cell_edges(int C, float *edge, hipStream_t st) {
+    LAUNCH(k_cell_edges, dim3(blocks_for((size_t) C + 3)), dim3(kBlock), 0, st, C, edge);
+    return hipGetLastError();
 }
 
 hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
@@ -1647,30 +1501,23 @@ hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nbl
     return hipGetLastError();
 }
 
-hipError_t launch_b_index(const DevData &D, const BatchSub *subs, int nsub, const BatchIndex &X, bool need_es,
-                          const int *miss_reps, int nmiss, int hmiss, const SortCopy *stores, int nstore,
-                          const SortCopy *hits, int nhit, int max_cell, const ColumnKeep &cols, hipStream_t st) {
-    if (nsub <= 0) return hipSuccess;
-    // the scan over the sorted indexes' cells ends with their total, the
-    // first position of the kept ones
-    const int nscan = hmiss + 1;
-    LAUNCH(k_b_fill<int>, dim3(fill_blocks((size_t) nscan, sizeof(int))), dim3(kBlock), 0, st, X.hist, 0, (size_t) nscan);
-    if (nmiss > 0)
-        LAUNCH(k_b_keys, dim3(blocks_for(D.n), nmiss), dim3(kBlock), 0, st, D, subs, miss_reps, X.keys, X.rank,
-               X.hist);
-    hipError_t e = launch_exclusive_sum(X.scan_temp, X.scan_bytes, X.hist, X.off, nscan, st);
+hipError_t launch_b_sort(const DevData &D, const SortJob *jobs, int njob, int hmiss, int max_cell, int *keys,
+                         int *rank, int *hist, int *off, void *scan_temp, size_t scan_bytes, hipStream_t st) {
+    if (njob <= 0) return hipSuccess;
+    const int nscan = hmiss + 1;  // the scan ends with the total
+    LAUNCH(k_b_fill<int>, dim3(fill_blocks((size_t) nscan, sizeof(int))), dim3(kBlock), 0, st, hist, 0, (size_t) nscan);
+    LAUNCH(k_b_keys, dim3(blocks_for(D.n), njob), dim3(kBlock), 0, st, D, jobs, keys, rank, hist);
+    hipError_t e = launch_exclusive_sum(scan_temp, scan_bytes, hist, off, nscan, st);
     if (e != hipSuccess) return e;
-    if (nmiss > 0)
-        LAUNCH(k_b_scatter, dim3(blocks_for(D.n), nmiss), dim3(kBlock), 0, st, D, subs, miss_reps, X.keys, X.rank,
-               X.off, X.order);
     const unsigned span = blocks_for((size_t) std::max(D.n, max_cell + 1));
-    if (nstore > 0)
-        LAUNCH(k_b_sort_out, dim3(span, nstore), dim3(kBlock), 0, st, stores, D.n, X.order, X.keys, X.off);
-    if (nhit > 0) LAUNCH(k_b_sort_in, dim3(span, nhit), dim3(kBlock), 0, st, hits, D.n, X.order, X.keys, X.off);
-    LAUNCH(k_b_gather, dim3(blocks_for(D.n), X.nrep), dim3(kBlock), 0, st, D, subs, X.reps, X.order, X.Ys, X.Es,
-           X.sigS, (int) need_es, cols.src, cols.store, cols.kmax);
-    LAUNCH(k_b_gather_own, dim3(blocks_for(D.n), nsub), dim3(kBlock), 0, st, D, subs, X.order, X.Ys, X.Es, X.sigS,
-           X.sig, (int) need_es, cols.own_src, cols.own_store);
+    LAUNCH(k_b_scatter, dim3(span, njob), dim3(kBlock), 0, st, D.n, jobs, keys, rank, off);
+    return hipGetLastError();
+}
+
+hipError_t launch_b_gather(const ColJob *jobs, int njob, int n, hipStream_t st) {
+    if (njob <= 0) return hipSuccess;
+    const int nblk = (n + kBlock * kGatherItems - 1) / (kBlock * kGatherItems);
+    LAUNCH(k_b_gather, dim3((unsigned) nblk * (unsigned) njob), dim3(kBlock), 0, st, jobs, n, nblk);
     return hipGetLastError();
 }
 
@@ -1786,7 +1633,7 @@ hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySe
     const size_t nb = (size_t) nsub * n;
     LAUNCH(k_b_fill<uint8_t>, dim3(fill_blocks(nb, 1)), dim3(kBlock), 0, st, X.qflag, (uint8_t) 0, nb);
     if (nblk > 0)
-        LAUNCH(k_b_qmark, dim3(nblk), dim3(kBlock), 0, st, subs, segs, blk_off, nseg, X.keys, X.qflag);
+        LAUNCH(k_b_qmark, dim3(nblk), dim3(kBlock), 0, st, subs, segs, blk_off, nseg, X.qflag);
     hipError_t e = launch_flag_compact(X.qflag, nb, X.select_temp, X.select_bytes, X.qlist, X.nsel, st);
     if (e != hipSuccess) return e;
     LAUNCH(k_b_qstart, dim3(blocks_for(nsub + 1)), dim3(kBlock), 0, st, X.qlist, X.nsel, nsub, n, X.qstart);
@@ -1799,20 +1646,20 @@ static void launch_count_k(const BatchSub *subs, int nsub, const int *blk_off, i
                            unsigned long long *stat, hipStream_t st) {
     if (blk_off) {
         if (phi)
-            LAUNCH((k_b_count<true, true, K>), dim3(nblk), dim3(kBlock), lds, st, subs, blk_off, nsub, n, X.off,
-                   X.order, X.Ys, X.Es, X.sig, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb, X.fbcap, stat);
+            LAUNCH((k_b_count<true, true, K>), dim3(nblk), dim3(kBlock), lds, st, subs, blk_off, nsub, n,
+                   X.edge, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb, X.fbcap, stat);
         else
-            LAUNCH((k_b_count<true, false, K>), dim3(nblk), dim3(kBlock), lds, st, subs, blk_off, nsub, n, X.off,
-                   X.order, X.Ys, X.Es, X.sig, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb, X.fbcap, stat);
+            LAUNCH((k_b_count<true, false, K>), dim3(nblk), dim3(kBlock), lds, st, subs, blk_off, nsub, n,
+                   X.edge, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb, X.fbcap, stat);
     } else {
         const dim3 grid(query_blocks_n(n), nsub);
         if (phi)
             LAUNCH((k_b_count<false, true, K>), grid, dim3(kBlock), lds, st, subs, (const int *) nullptr, nsub, n,
-                   X.off, X.order, X.Ys, X.Es, X.sig, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb,
+                   X.edge, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb,
                    X.fbcap, stat);
         else
             LAUNCH((k_b_count<false, false, K>), grid, dim3(kBlock), lds, st, subs, (const int *) nullptr, nsub, n,
-                   X.off, X.order, X.Ys, X.Es, X.sig, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb,
+                   X.edge, X.qlist, X.qstart, s_star, eps, phirel, X.nb, X.fb, X.nfb,
                    X.fbcap, stat);
     }
 }
@@ -1842,6 +1689,7 @@ hipError_t launch_b_count(const BatchSub *subs, int nsub, const int *blk_off, in
     case 5: launch_count_k<5>(subs, nsub, blk_off, nblk, n, lds, X, s_star, eps, phirel, phi, stat, st); break;
     case 6: launch_count_k<6>(subs, nsub, blk_off, nblk, n, lds, X, s_star, eps, phirel, phi, stat, st); break;
     case 7: launch_count_k<7>(subs, nsub, blk_off, nblk, n, lds, X, s_star, eps, phirel, phi, stat, st); break;
+    case 8: launch_count_k<8>(subs, nsub, blk_off, nblk, n, lds, X, s_star, eps, phirel, phi, stat, st); break;
     default: launch_count_k<0>(subs, nsub, blk_off, nblk, n, lds, X, s_star, eps, phirel, phi, stat, st); break;
     }
     if (tm.stop) (void) hipEventRecord(tm.stop, st);
@@ -1853,7 +1701,7 @@ hipError_t launch_b_count(const BatchSub *subs, int nsub, const int *blk_off, in
 hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, int kfast, const BatchIndex &X,
                                float s_star, hipStream_t st) {
     if (nsub <= 0) return hipSuccess;
-    LAUNCH(k_b_dense_init, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.order, X.dsorted, X.par);
+    LAUNCH(k_b_dense_init, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.dsorted, X.par);
     for (int round = 0; round < kSampleEdges; ++round) {
         LAUNCH(k_b_link_sample, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.nb, round, X.par);
         LAUNCH(k_b_uf_compress, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.par);
@@ -1862,7 +1710,7 @@ hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, 
     const dim3 grid(query_blocks_n(n), nsub);
     const size_t lds = count_lds(kmax);
 #define LINK_FULL(K)                                                                                                   \
-    LAUNCH(k_b_link_full<K>, grid, dim3(kBlock), lds, st, subs, n, X.off, X.order, X.Ys, X.Es, X.sig, X.dsorted,      \
+    LAUNCH(k_b_link_full<K>, grid, dim3(kBlock), lds, st, subs, n, X.edge, X.dsorted,      \
            s_star, X.giant, X.par)
     switch (kfast) {
     case 1: LINK_FULL(1); break;
@@ -1872,6 +1720,7 @@ hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, 
     case 5: LINK_FULL(5); break;
     case 6: LINK_FULL(6); break;
     case 7: LINK_FULL(7); break;
+    case 8: LINK_FULL(8); break;
     default: LINK_FULL(0); break;
     }
 #undef LINK_FULL

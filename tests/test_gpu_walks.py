@@ -1,0 +1,63 @@
+"""The level-synchronous driver's neighbour walks against the oracle on data
+whose coordinates sit on the edges of the eps cells (one float to either side,
+exactly on them, and half a cell away), where the cell rule and the distance
+disagree; whole results are compared, with per-tree traces."""
+
+import sys
+
+import numpy as np
+import pytest
+
+from gpu_inscy_amd import _lib, datagen
+from gpu_inscy_amd import inscy as INSCY
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    _lib.lib()
+
+
+def edge_data(seed, n, d, eps):
+    """Points of d-dimensional clumps on a lattice of half eps cells, moved by at
+    most one float in a third of the coordinates."""
+    rng = np.random.default_rng(seed)
+    C = int(np.ceil(1.0 / np.float64(np.float32(eps))))
+    centre = rng.integers(2, 2 * C - 2, size=(max(2, n // 60), d))
+    at = centre[rng.integers(0, len(centre), n)] + rng.integers(-2, 3, size=(n, d))
+    at = np.where(rng.random((n, d)) < 0.15, rng.integers(0, 2 * C + 1, size=(n, d)), at)
+    X = np.clip(at.astype(np.float64) / (2 * C), 0.0, 1.0).astype(np.float32)
+    step = rng.random((n, d))
+    X = np.where(step < 1 / 6, np.nextafter(X, np.float32(0)), X)
+    X = np.where(step > 5 / 6, np.nextafter(X, np.float32(1)), X)
+    return np.clip(X, 0.0, 1.0).astype(np.float32)
+
+
+# eps whose reciprocal is whole (cells of width eps up to rounding) and not
+# (cells narrower than eps: neighbours by distance in cells two apart)
+@pytest.mark.parametrize("rect", [True, False])
+@pytest.mark.parametrize("n,d,eps,num_obj", [(300, 4, 0.05, 3), (1201, 5, 0.05, 4), (1300, 6, 0.03, 3),
+                                             (700, 7, 0.125, 5), (257, 9, 0.11, 4)])
+def test_walks_on_cell_edges_match_oracle(n, d, eps, num_obj, rect):
+    print("cell edges", n, d, eps, num_obj, rect, flush=True)
+    sys.stdout.flush()
+    X = edge_data(n + d, n, d, eps)
+    args = (eps, 1.0, num_obj, max(4, n // 40), 1.0, 4, rect, 0)
+    ref = O.run_ref(X, *args[:7], 0, trace=True)
+    _lib.debug_trace(True)
+    try:
+        got = INSCY.run(X, *args, mode=_lib.MODE_BATCHED)
+        trace = _lib.debug_trace_rows()
+    finally:
+        _lib.debug_trace(False)
+    assert got.subspaces == ref.subspaces
+    for s, a, b in zip(ref.subspaces, ref.labels, got.labels):
+        assert np.array_equal(O.canonical(a), b), f"labels differ in subspace {s}"
+    assert np.array_equal(trace, ref.trace)
+    assert max(len(s) for s in got.subspaces) >= 3
