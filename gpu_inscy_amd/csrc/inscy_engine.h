@@ -383,7 +383,7 @@ public:
             sync();
         }
         arena.release(0);
-        D = DevData{Xt, cellC, cellE, d_level, d_level + d, n, d, cells, ecells};
+        D = DevData{d_X, Xt, cellC, cellE, d_level, d_level + d, n, d, cells, ecells};
     }
 
     // ---------------------------------------------------------- run
@@ -1063,7 +1063,8 @@ private:
         return dst;
     }
     void expand_level(const std::vector<int> &frontier, const int *counts);
-    void process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1);
+    void process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1, bool fan);
+    bool fan_level(const std::vector<ChildSub> &cs) const;
     GridArg child_grid(const SubspaceArg &S) const;
     void replay_staged();
     std::vector<int> sup_flat;  // superset rows of every subspace (host copy of d_sup)

@@ -64,6 +64,7 @@ struct SubspaceArg {
 // dimension-major ([d][n]) so that a wave reading one dimension of 64
 // consecutive points issues one coalesced load.
 struct DevData {
+    const float *X;         // [n][d] coordinates as given
     const float *Xt;        // [d][n] coordinates
     const uint8_t *cellC;   // [d][n] cell in the c-grid (ScyTreeNode.cu:100-102)
     const uint16_t *cellE;  // [d][n] cell in the ceil(1/eps)-grid (inscy_map.cpp:243-244)
@@ -352,6 +353,25 @@ hipError_t launch_subspace_phi(const DevData &D, const SubspaceArg &S, const Gri
 // matchmask, phi_w, phi_d and cnt)
 hipError_t launch_phi_exact(const DevData &D, const BatchSub *sub, const int2 *fb, const int *nfb, int fbcap,
                             const int *rank_order, float eps, float s_star, hipStream_t st);
+// neighbour counts of the children S | {m} of whole frontier masks S at once
+// (k_b_fan): one walk per point of S's trees serves every child.  jobs: at most
+// width (4, 8, 16, 32 or kFanMost) children of one group each, blk_off their
+// blocks of kFanQueries queries; kS: |S| of every group; cap: of kS + 1.  phi:
+// the caller clears *X.nfb before and recomputes the listed pairs after
+// (launch_phi_exact over the children)
+struct FanJob {
+    int g, ch0, nch, pad;  // group, its first child in the batch, number of children
+};
+struct FanTable {  // per child of the batch: its counts, dimension m and first sample edge
+    int *const *cnt;
+    const int *dim;
+    const long long *nbase;
+};
+constexpr int kFanMost = 64;  // children of one walk
+hipError_t launch_b_fan(const BatchSub *groups, const FanJob *jobs, const int *blk_off, int njob, int nblk, int width,
+                        int kS, const FanTable &T, const BatchIndex &X, float s_star, float eps, bool phi,
+                        bool phi_all_exact, int cap, float phi_w, float phi_d, const DevData &D,
+                        unsigned long long *stat, hipStream_t st);
 // dense components of nsub subspaces whose counts are complete
 hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, int kfast, const BatchIndex &X,
                                float s_star, hipStream_t st);
@@ -453,6 +473,8 @@ constexpr int kRangeWords = 31;      // per query in LDS: 9 range starts, 10 pre
 constexpr int kBlockThreads = 256;   // threads per block of every pass
 constexpr int kQueriesPerBlock = 64;  // queries per block of the batched neighbour passes
 constexpr int kMaxFastK = 8;          // neighbour walks are compiled for each k up to this
+constexpr int kFanLanes = 16;         // lanes per query of the fanned counts
+constexpr int kFanQueries = kBlockThreads / kFanLanes;  // queries per block
 constexpr int kSampleEdges = 2;       // neighbours recorded per point by the count walk (Afforest's sample rounds)
 constexpr int kPartPerThread = 8;     // elements per thread of the batched partition passes
 

@@ -267,6 +267,7 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
     }
 
     // batches bounded by memory, count and 32-bit positions
+    const bool fan = fan_level(cs);
     size_t i = 0;
     while (i < cs.size()) {
         size_t j = i;
@@ -283,6 +284,8 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             // 16, k coordinate columns: 4k, grid histogram and offsets), the
             // phi pass's queue (8)
             size_t est = (size_t) n * (38 + 4 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 12;
+            // the index and the queries of a fanned mask
+            if (fan && (j == i || cs[j - 1].t0 != c.t0)) est += (size_t) n * (21 + 4 * (size_t) S.k) + (size_t) ncell * 12;
             for (int a = c.t0; a < c.t1; ++a) {
                 if (!pair_on(a, c.m)) continue;
                 const LTree &t = lt[lv_act[a]];
@@ -295,7 +298,7 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             hsum += ncell;
             ++j;
         }
-        process_batch(cs, i, j);
+        process_batch(cs, i, j, fan);
         i = j;
     }
 }
@@ -407,102 +410,178 @@ void Engine::index_of(std::vector<BatchSub> &hs, std::vector<const float *> &cta
     if (nc) HIP_OK(launch_b_gather(dc, nc, n, st));
 }
 
-void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1) {
+// Whether the level's children are counted by one walk per frontier mask
+// (k_b_fan) instead of one per child: when the mask's own grid index has as
+// many dimensions as its children's, so that the walk meets no more candidates
+// than each child's would.  Where the children's index has one more (masks of
+// two dimensions whose cells cubed still fit the grid), a walk per child meets
+// far fewer: n=100,000 d=20, masks of two dimensions 16.8 ms by child, 39 ms by
+// mask; n=25,000 d=15, eps=0.015 (two index dimensions at most) 2.19 and 1.74.
+bool Engine::fan_level(const std::vector<ChildSub> &cs) const {
+    if (cs.empty() || (long long) n * d >= 1ll << 30) return false;  // 32-bit offsets into X
+    const SubspaceArg S = arg_of(cs[0].s & ~dbit(cs[0].m));
+    if (S.k < 1 || S.k > kMaxFastK) return false;
+    return grid_of(S, -1, true).j >= grid_of(arg_of(cs[0].s), -1, true).j;
+}
+
+void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1, bool fan) {
     Pool &nxt = lvl[cur_lvl ^ 1];
     batch.reset();
     batch_sorts.clear();
     batch_cols.clear();
     const int B = (int) (i1 - i0);
-    const int QPB = kQueriesPerBlock;
+    const int k = dcount(cs[i0].s);  // of every child: the level's trees restrict equally many dimensions
+    const int kfast = !generic_walk && k <= kMaxFastK ? k : 0;
 
-    // ---- grid indexes of the batch's subspaces
+    // ---- the batch's child subspaces
     std::vector<BatchSub> hs(B);
-    long long qoff = 0;
-    int kmax = 1, kmin = 64;
     int *cntB = batch.take<int>((size_t) B * n);
     for (int b = 0; b < B; ++b) {
         const ChildSub &c = cs[i0 + b];
         BatchSub &x = hs[b];
         std::memset(&x, 0, sizeof(x));
         x.S = arg_of(c.s);
-        x.G = child_grid(x.S);
-        long long qmax = 0;
-        for (int a = c.t0; a < c.t1; ++a)
-            if (pair_on(a, c.m)) qmax += lt[lv_act[a]].nW;
-        x.base = (long long) b * n;
-        x.nbase = x.base;
+        x.base = x.nbase = (long long) b * n;
         x.cnt = cntB + (size_t) b * n;
-        x.cap = cap_of(x.S.k);
-        x.thr_dense = dense_thr[x.S.k];
-        x.qmax = (int) qmax;
+        x.cap = cap_of(k);
+        x.thr_dense = dense_thr[k];
         set_bounds(c.s, x);
         x.dbit = phi_mode ? 2 : 0;
         x.matchmask = match_of(x.S);
         x.phi_w = phi_weak;
-        x.phi_d = phi_dense[x.S.k];
-        qoff += qmax;
-        kmax = std::max(kmax, x.S.k);
-        kmin = std::min(kmin, x.S.k);
+        x.phi_d = phi_dense[k];
+        if (!fan) x.G = child_grid(x.S);
     }
-    const int kfast = (!generic_walk && kmin == kmax && kmax <= kMaxFastK) ? kmax : 0;
+
+    // ---- the walked subspaces: every child, or with `fan` every frontier
+    // mask, whose walk serves all its children; their queries are the points
+    // of the trees refined, in sorted order
+    std::vector<BatchSub> gs;       // fan: the masks
+    constexpr int kWidths[] = {4, 8, 16, 32, kFanMost};
+    std::vector<FanJob> jobs[5];    // by the width of their walk
+    std::vector<QuerySeg> qs;
+    std::vector<int> qblk{0};
+    long long qoff = 0;
+    auto add_queries = [&](BatchSub &x, int w, int t0, int t1, int m) {  // m < 0: of any dimension
+        long long qmax = 0;
+        for (int a = t0; a < t1; ++a) {
+            const LTree &t = lt[lv_act[a]];
+            if (t.nW <= 0 || (m >= 0 && !pair_on(a, m))) continue;
+            qs.push_back({t.W, t.nW, w});
+            qblk.push_back(qblk.back() + nblocks(t.nW));
+            qmax += t.nW;
+        }
+        x.qmax = (int) qmax;
+        qoff += qmax;
+    };
+    if (fan) {
+        for (int b = 0; b < B;) {
+            const ChildSub &c = cs[i0 + b];
+            int e = b;
+            while (e < B && cs[i0 + e].t0 == c.t0) ++e;
+            BatchSub g;
+            std::memset(&g, 0, sizeof(g));
+            g.S = arg_of(c.s & ~dbit(c.m));
+            g.G = grid_of(g.S, -1, true);
+            g.base = (long long) gs.size() * n;
+            add_queries(g, (int) gs.size(), c.t0, c.t1, -1);
+            for (int at = b; at < e; at += kFanMost) {
+                const int nch = std::min(kFanMost, e - at);
+                int w = 0;
+                while (kWidths[w] < nch) ++w;
+                jobs[w].push_back({(int) gs.size(), at, nch, 0});
+            }
+            gs.push_back(g);
+            b = e;
+        }
+    } else {
+        for (int b = 0; b < B; ++b) add_queries(hs[b], b, cs[i0 + b].t0, cs[i0 + b].t1, cs[i0 + b].m);
+    }
+    std::vector<BatchSub> &ws = fan ? gs : hs;
+    const int nw = (int) ws.size();
     std::vector<const float *> ctab;
-    index_of(hs, ctab);
+    index_of(ws, ctab);
 
     BatchIndex X{};
     X.edge = edges;
-    X.qflag = batch.take<uint8_t>(((size_t) B * n + 15) & ~(size_t) 15);  // read 16 bytes a lane
+    X.qflag = batch.take<uint8_t>(((size_t) nw * n + 15) & ~(size_t) 15);  // read 16 bytes a lane
     X.qlist = batch.take<int>(std::max<long long>(qoff, 1));
     X.nsel = batch.take<int>(1);
-    X.qstart = batch.take<int>(B + 1);
-    X.select_bytes = select_temp_bytes(B * n);
+    X.qstart = batch.take<int>(nw + 1);
+    X.select_bytes = select_temp_bytes(nw * n);
     X.select_temp = batch.take<char>(X.select_bytes);
     X.nb = batch.take<int>((size_t) kSampleEdges * B * n);
     X.nfb = batch.take<int>(1);
     X.fbcap = phi_mode ? B * n : 1;  // each point of each subspace is sent at most once per pass
     X.fb = batch.take<int2>(X.fbcap);
-    X.dsorted = batch.take<uint8_t>((size_t) B * n + 8);  // the grouped link walk reads aligned words past the end
-    X.par = batch.take<int>((size_t) B * n);
-    X.giant = batch.take<int>(B);
     HIP_OK(launch_fill_i32(X.nb, -1, (size_t) kSampleEdges * B * n, st));
     HIP_OK(launch_fill_i32(cntB, -1, (size_t) B * n, st));
 
-    // ---- queries: the points of the trees each subspace refines, in sorted order
-    std::vector<QuerySeg> qs;
-    std::vector<int> qblk{0};
-    for (int b = 0; b < B; ++b) {
-        const ChildSub &c = cs[i0 + b];
-        for (int a = c.t0; a < c.t1; ++a) {
-            const LTree &t = lt[lv_act[a]];
-            if (t.nW <= 0 || !pair_on(a, c.m)) continue;
-            qs.push_back({t.W, t.nW, b});
-            qblk.push_back(qblk.back() + nblocks(t.nW));
-        }
-    }
-    std::vector<int> cblk(B + 1, 0);
-    for (int b = 0; b < B; ++b) cblk[b + 1] = cblk[b] + (hs[b].qmax + QPB - 1) / QPB;
-    defer_uploads();
-    const float *const *dcol = upload(batch, ctab);
-    {
+    auto columns = [&](std::vector<BatchSub> &v, const std::vector<const float *> &tab) {
+        const float *const *dcol = upload(batch, tab);
         size_t at = 0;
-        for (BatchSub &x : hs) {
+        for (BatchSub &x : v) {
             x.col = dcol + at;
             at += x.S.k;
         }
-    }
-    BatchSub *dsubs = upload(batch, hs);
+    };
+    std::vector<int> cblk{0};
+    FanTable ft{};
+    defer_uploads();
+    columns(ws, ctab);
+    BatchSub *dws = upload(batch, ws);
     QuerySeg *dqs = upload(batch, qs);
     int *dqb = upload(batch, qblk);
-    int *dcb = upload(batch, cblk);
+    FanJob *djobs[5] = {};
+    int *djb[5] = {}, njb[5] = {};
+    BatchSub *dsubs = nullptr;  // fan: the children, for the phi recomputation
+    int *dcb = nullptr;
+    if (fan) {
+        std::vector<int *> tc(B);
+        std::vector<int> td(B);
+        std::vector<long long> tbase(B);
+        for (int b = 0; b < B; ++b) {
+            tc[b] = hs[b].cnt;
+            td[b] = cs[i0 + b].m;
+            tbase[b] = hs[b].nbase;
+        }
+        ft = FanTable{upload(batch, tc), upload(batch, td), upload(batch, tbase)};
+        for (int w = 0; w < 5; ++w) {
+            if (jobs[w].empty()) continue;
+            std::vector<int> blk{0};
+            for (const FanJob &j : jobs[w]) blk.push_back(blk.back() + (gs[j.g].qmax + kFanQueries - 1) / kFanQueries);
+            djobs[w] = upload(batch, jobs[w]);
+            djb[w] = upload(batch, blk);
+            njb[w] = blk.back();
+        }
+        if (phi_mode) dsubs = upload(batch, hs);
+    } else {
+        for (int b = 0; b < B; ++b) cblk.push_back(cblk.back() + (hs[b].qmax + kQueriesPerBlock - 1) / kQueriesPerBlock);
+        dcb = upload(batch, cblk);
+    }
     flush_uploads();
-    HIP_OK(launch_b_queries(dsubs, B, n, dqs, dqb, (int) qs.size(), qblk.back(), X, st));
+    HIP_OK(launch_b_queries(dws, nw, n, dqs, dqb, (int) qs.size(), qblk.back(), X, st));
     const bool dbg = batch_trace;
     std::chrono::steady_clock::time_point tq0, tq1;
     if (dbg) {
         sync();
         tq0 = std::chrono::steady_clock::now();
     }
-    HIP_OK(launch_b_count(dsubs, B, dcb, cblk[B], n, kmax, kfast, X, s_star, prm.neighborhood_size, phi_mode, phi_all_exact, D, rank_perm,
-                          small + kStatAt, timer(), st));
+    if (fan) {
+        if (phi_mode) HIP_OK(launch_fill_i32(X.nfb, 0, 1, st));
+        const KernelTimer tm = timer();
+        if (tm.start) HIP_OK(hipEventRecord(tm.start, st));
+        for (int w = 0; w < 5; ++w)
+            HIP_OK(launch_b_fan(dws, djobs[w], djb[w], (int) jobs[w].size(), njb[w], kWidths[w], k - 1, ft, X, s_star,
+                                prm.neighborhood_size, phi_mode, phi_all_exact, cap_of(k), phi_weak, phi_dense[k], D,
+                                small + kStatAt, st));
+        if (tm.stop) HIP_OK(hipEventRecord(tm.stop, st));
+        if (phi_mode)
+            HIP_OK(launch_phi_exact(D, dsubs, X.fb, X.nfb, X.fbcap, rank_perm, prm.neighborhood_size, s_star, st));
+    } else {
+        HIP_OK(launch_b_count(dws, B, dcb, cblk.back(), n, k, kfast, X, s_star, prm.neighborhood_size, phi_mode,
+                              phi_all_exact, D, rank_perm, small + kStatAt, timer(), st));
+    }
     if (dbg) {
         sync();
         tq1 = std::chrono::steady_clock::now();
@@ -697,6 +776,8 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             if (!passing[b]) continue;
             const dmask_t s = cs[i0 + b].s;
             BatchSub x = hs[b];
+            x.base = (long long) ci * n;
+            if (fan) x.G = child_grid(x.S);
             x.cnt = cntP + (size_t) ci * n;
             x.comp = compP + (size_t) ci * n;
             x.csize = csizeP + (size_t) ci * n;
@@ -735,37 +816,39 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         HIP_OK(launch_b_stamp(dss, dsb, (int) stamps.size(), sbk.back(), st));
     }
     if (ncomp > 0) {
+        X.dsorted = batch.take<uint8_t>((size_t) ncomp * n + 8);  // the grouped link walk reads aligned words past the end
+        X.par = batch.take<int>((size_t) ncomp * n);
+        X.giant = batch.take<int>(ncomp);
+        std::vector<const float *> ctab2;
+        if (fan) index_of(hc, ctab2);
+        defer_uploads();
+        if (fan) columns(hc, ctab2);
         BatchSub *dhc = upload(batch, hc);
+        flush_uploads();
         std::chrono::steady_clock::time_point tc0, tc1, tc2;
         if (dbg) {
             sync();
             tc0 = std::chrono::steady_clock::now();
         }
-        HIP_OK(launch_b_count(dhc, ncomp, nullptr, 0, n, kmax, kfast, X, s_star, prm.neighborhood_size, phi_mode, phi_all_exact, D,
+        HIP_OK(launch_b_count(dhc, ncomp, nullptr, 0, n, k, kfast, X, s_star, prm.neighborhood_size, phi_mode, phi_all_exact, D,
                               rank_perm, small + kStatAt, timer(), st));
         if (dbg) {
             sync();
             tc1 = std::chrono::steady_clock::now();
         }
-        HIP_OK(launch_b_components(dhc, ncomp, n, kmax, kfast, X, s_star, st));
+        HIP_OK(launch_b_components(dhc, ncomp, n, k, kfast, X, s_star, st));
         if (dbg) {
             sync();
             tc2 = std::chrono::steady_clock::now();
-            int kmin = 64, kmx = 0;
             long long qs = 0;
-            for (int b = 0; b < B; ++b) {
-                kmin = std::min(kmin, hs[b].S.k);
-                kmx = std::max(kmx, hs[b].S.k);
-                qs += hs[b].qmax;
-            }
+            for (const BatchSub &x : ws) qs += x.qmax;
             auto ms = [](std::chrono::steady_clock::time_point a, std::chrono::steady_clock::time_point b) {
                 return std::chrono::duration<double, std::milli>(b - a).count();
             };
             std::fprintf(stderr,
-                         "[inscy batch] B=%d k=%d..%d cap=%d..%d queries<=%lld list_count=%.3fms "
+                         "[inscy batch] B=%d walked=%d k=%d cap=%d queries<=%lld list_count=%.3fms "
                          "comp=%d all_count=%.3fms components=%.3fms\n",
-                         B, kmin, kmx, cap_of(kmx), cap_of(kmin), qs, ms(tq0, tq1), ncomp, ms(tc0, tc1),
-                         ms(tc1, tc2));
+                         B, nw, k, cap_of(k), qs, ms(tq0, tq1), ncomp, ms(tc0, tc1), ms(tc1, tc2));
         }
         Entry *de = upload(batch, ents);
         HIP_OK(launch_b_entries(entries, nentries, de, ncomp, d_nE, st));

@@ -673,6 +673,305 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
     }
 }
 
+// ------------------------------------------------------------ neighbour counts of all children of a mask
+// The children S | {m} of a frontier mask S count the same points (those of
+// S's trees), and a neighbour in S | {m} is a neighbour in S whose coordinate
+// in m is near too; m is above every dimension of S, so the distance of the
+// child is S's running sum plus one last term.  One walk over the candidates of
+// S therefore serves all children: the kFanLanes lanes of a query test
+// kFanLanes * 4 candidates of S per step (the grouped loads of walk_vec) and
+// put the few neighbours found into LDS; then every lane, standing for NC
+// children and one of kFanLanes / CW slots, adds m's term of the slot's
+// neighbours: the lanes read consecutive coordinates of a neighbour's row of X.
+// The walk ends when every child is decided (cap, phi) or the runs are done.
+// The children's bounds (k_b_count) are not looked up: one undecided child
+// makes the walk anyway, and the look-up costs a scattered read per child and
+// bound (n=100,000 d=20, masks of three dimensions: 54 ms with it, 49 without).
+// Bound: about two fifths of the time is the set-up of the walks (a chain of
+// dependent loads per query), a quarter the candidates, a third VALU work on
+// the neighbours; hence slots for masks of few children instead of idle lanes
+// (49 -> 43 ms; by child, k_b_count took 63 ms).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <bool PHI, int K, int CW, int NC>
+__global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ groups, const FanJob *__restrict__ jobs,
+                                                  const int *__restrict__ blk_off, int njob, FanTable T, int d,
+                                                  const float *__restrict__ X, const float *__restrict__ edge,
+                                                  const int *__restrict__ qlist, const int *__restrict__ qstart,
+                                                  float s_star, float eps, double phirel, int cap, float phi_w,
+                                                  float phi_d, int *__restrict__ nb, int2 *__restrict__ fb,
+                                                  int *__restrict__ nfb, int fbcap,
+                                                  unsigned long long *__restrict__ stat) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int L = kFanLanes, Q = kFanQueries, U = 4;
+    constexpr int HS = L / CW;  // slots: neighbours of the step taken at once
+    __shared__ float sy[K][Q];
+    __shared__ float2 sc[K][Q];
+    __shared__ int rs[9][Q], rl[9][Q], rg[10][Q];  // runs: first position, length, groups of four before (rg[9]: all)
+    __shared__ uint2 hits[Q][L * U + U * HS];      // (row offset in X, sum over S) of the step's neighbours in S
+    const int ji = seg_of(blk_off, njob, blockIdx.x);
+    const FanJob J = jobs[ji];
+    const BatchSub &B = groups[J.g];
+    const int lq = threadIdx.x / L, l = threadIdx.x % L;
+    const int slot = l / CW, cl = l % CW;
+    const int gshift = __lane_id() & ~(L - 1);
+    const int qi = qstart[J.g] + (blockIdx.x - blk_off[ji]) * Q + lq;
+    const bool active = qi < qstart[J.g + 1];
+    int seen = 0, nhits = 0;
+    int found[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) found[c] = 0;
+    if (active) {
+        const int i = (int) (qlist[qi] - B.base);
+        const int p = B.order[i];
+        // the query's coordinates and cell intervals in S: lane t holds dimension t
+        const float inf = __builtin_inff();
+        const float ecs = ecell_width(B.G.C);
+        if (l < K) {
+            const float y = B.col[l][i];
+            float2 c = make_float2(-inf, inf);
+            if ((B.G.checkmask >> l) & 1ull) {
+                const int e = ecell_of(y, ecs, B.G.C);
+                c = make_float2(edge[e], edge[e + 3]);
+            }
+            sy[l][lq] = y;
+            sc[l][lq] = c;
+        }
+        // the lane's children: the query's coordinate in m and the interval of
+        // the cells around its own
+        int ch[NC], dim[NC];
+        float xq[NC], lo[NC], hi[NC];
+        double dsum[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            ch[c] = J.ch0 + min(cl + CW * c, J.nch - 1);
+            dim[c] = T.dim[ch[c]];
+            xq[c] = X[(size_t) p * d + dim[c]];
+            const int e = ecell_of(xq[c], ecs, B.G.C);
+            lo[c] = edge[e];
+            hi[c] = edge[e + 3];
+            dsum[c] = 0.0;
+        }
+        wave_sync();
+        // the runs of build_runs, lane r (of nine) row r
+        int gtotal, own, ogrp, olen, total;
+        {
+            const GridArg &G = B.G;
+            const int C = G.C;
+            const int c0 = ecell_of(sy[G.tI[0]][lq], ecs, C);
+            const int c1 = G.j == 3 ? ecell_of(sy[G.tI[1]][lq], ecs, C) : 0;
+            const float yl = sy[G.tI[G.j - 1]][lq];
+            const int cc = ecell_of(yl, ecs, C);
+            const int F = G.F > 1 ? G.F : 1, CF = C * F;
+            int clo = max(cc - 1, 0) * F, chi = min(cc + 1, C - 1) * F + F - 1;
+            if (F > 1) {
+                const double em = sqrt((double) s_star) * 1.001 + 1e-6;
+                clo = max(clo, fine_key(__double2float_rd((double) yl - em), C, F));
+                chi = min(chi, fine_key(__double2float_ru((double) yl + em), C, F));
+            }
+            const int x0 = max(c0 - 1, 0), nx = G.j == 1 ? 1 : min(c0 + 1, C - 1) - x0 + 1;
+            const int y0 = max(c1 - 1, 0), ny = G.j == 3 ? min(c1 + 1, C - 1) - y0 + 1 : 1;
+            own = G.j == 1 ? 0 : 3 * (c0 - x0) + (G.j == 3 ? c1 - y0 : 0);
+            const int xi = l / 3, yi = l % 3;
+            int a = 0, len = 0;
+            if (xi < nx && yi < ny) {
+                const int row = G.j == 1 ? 0 : G.j == 2 ? (x0 + xi) * CF : ((x0 + xi) * C + y0 + yi) * CF;
+                a = B.off[row + clo];
+                len = max(B.off[row + chi + 1] - a, 0);
+            }
+            const int g = (len + U - 1) / U;
+            int incl = g;
+            total = len;
+            for (int o = 1; o < L; o <<= 1) {
+                const int v = __shfl_up(incl, o, L);
+                if (l >= o) incl += v;
+                total += __shfl_xor(total, o, L);
+            }
+            if (l < 9) {
+                rs[l][lq] = a;
+                rl[l][lq] = len;
+                rg[l][lq] = incl - g;
+            }
+            if (l == 9) rg[9][lq] = incl;
+            gtotal = __shfl(incl, 9, L);
+            ogrp = __shfl(incl - g, own, L);
+            olen = __shfl(g, own, L);
+        }
+        wave_sync();
+        const float *col[K];
+        float qv[K];
+#pragma unroll
+        for (int t = 0; t < K; ++t) {
+            col[t] = B.col[t];
+            qv[t] = sy[t][lq];
+        }
+        const uint32_t checked = (uint32_t) B.G.checkmask;
+        const unsigned long long below = (1ull << l) - 1ull;
+        const uint2 none = make_uint2((uint32_t) p * (uint32_t) d, __float_as_uint(inf));
+        // start at a pseudo-random group of the query's own run (spreads the
+        // sample edges), walk to the end, then from the start to there
+        const int grot = gtotal > 0 ? ogrp + (int) (((uint32_t) p * 2654435761u) % (uint32_t) max(olen, 1)) : 0;
+        bool more = true;
+        for (int segm = 0; segm < 2; ++segm) {
+            const int gbeg = segm == 0 ? grot : 0, gend = segm == 0 ? gtotal : grot;
+            int r = segm == 0 ? own : 0;
+            for (int g0 = gbeg; g0 < gend && more; g0 += L) {
+                const int g = min(g0 + l, gend - 1);
+                while (g >= rg[r + 1][lq]) ++r;
+                const int e0 = (g - rg[r][lq]) * U;
+                const int nv = g0 + l < gend ? min(U, rl[r][lq] - e0) : 0;
+                const int jj0 = rs[r][lq] + e0;
+                f4u y[K];
+#pragma unroll
+                for (int t = 0; t < K; ++t) y[t] = *reinterpret_cast<const f4u *>(col[t] + (uint32_t) jj0);
+                bool hit[U];
+                float accs[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    float acc = 0.0f;
+#pragma unroll
+                    for (int t = 0; t < K; ++t) {
+                        const float diff = qv[t] - y[t][u];
+                        const float sq = diff * diff;
+                        acc = acc + sq;
+                    }
+                    hit[u] = (u < nv) & (jj0 + u != i) & (acc <= s_star);
+                    accs[u] = acc;
+                }
+                if (checked) cells_of_hits<U>(B, &sc[0][lq], Q, checked, jj0, hit);
+                seen += nv;
+                i4u id = {0, 0, 0, 0};
+                if (hit[0] | hit[1] | hit[2] | hit[3])
+                    id = *reinterpret_cast<const i4u *>(B.order + (uint32_t) jj0);
+                int nh = 0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const unsigned long long m = (__ballot(hit[u]) >> gshift) & 0xFFFFull;
+                    if (hit[u])
+                        hits[lq][nh + __popcll(m & below)] =
+                            make_uint2((uint32_t) id[u] * (uint32_t) d, __float_as_uint(accs[u]));
+                    nh += __popcll(m);
+                }
+                if (nh == 0) continue;  // uniform over the query's lanes
+                if (l < U * HS) hits[lq][nh + l] = none;  // past the last one: never near
+                wave_sync();
+                nhits += nh;
+                for (int h0 = 0; h0 < nh; h0 += U * HS) {
+                    uint2 e[U];
+                    float z[U][NC];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) e[u] = hits[lq][h0 + u * HS + slot];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) z[u][c] = X[e[u].x + (uint32_t) dim[c]];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) {
+                            const float diff = xq[c] - z[u][c];
+                            const float sq = diff * diff;
+                            const float acc = __uint_as_float(e[u].y) + sq;
+                            if (acc <= s_star && z[u][c] >= lo[c] && z[u][c] < hi[c]) {
+                                // sample edges: the first of slots 0 and 1, or the first two of the only slot
+                                if (cl + CW * c < J.nch &&
+                                    (HS > 1 ? (slot < kSampleEdges && found[c] == 0) : found[c] < kSampleEdges))
+                                    nb[kSampleEdges * (T.nbase[ch[c]] + p) + (HS > 1 ? slot : found[c])] =
+                                        (int) (e[u].x / (uint32_t) d);
+                                ++found[c];
+                                if (PHI) dsum[c] += phi_term(acc, eps);
+                            }
+                        }
+                }
+                // undecided children, over the slots
+                bool open = false;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    if (PHI) {
+                        double ds = dsum[c];
+                        for (int o = CW; o < L; o <<= 1) ds += __shfl_xor(ds, o);
+                        open |= (cl + CW * c < J.nch) &
+                                (ds * (1.0 - (double) total * phirel) < (double) fmaxf(phi_w, phi_d));
+                    } else {
+                        int f = found[c];
+                        for (int o = CW; o < L; o <<= 1) f += __shfl_xor(f, o);
+                        open |= (cl + CW * c < J.nch) & (f < cap);
+                    }
+                }
+                more = ((__ballot(open) >> gshift) & 0xFFFFull) != 0;
+                wave_sync();
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            for (int o = CW; o < L; o <<= 1) found[c] += __shfl_xor(found[c], o);
+            if (PHI)
+                for (int o = CW; o < L; o <<= 1) dsum[c] += __shfl_xor(dsum[c], o);
+            if (slot != 0 || cl + CW * c >= J.nch) {
+                found[c] = -1;  // counted by another lane
+                continue;
+            }
+            if (PHI) {
+                // as in k_b_count; a sum above both thresholds may be incomplete
+                const double tw = (double) phi_w, td = (double) phi_d;
+                const double sl = dsum[c] * (1.0 - (double) found[c] * phirel);
+                const double sh = dsum[c] * (1.0 + (double) found[c] * phirel);
+                int code = 0;
+                bool unsure = false;
+                double ub = -1.0;
+                if (!(dsum[c] * (1.0 - (double) total * phirel) < (double) fmaxf(phi_w, phi_d))) {
+                    code = 3;
+                } else {
+                    if (sl >= tw) code |= 1;
+                    else if (!(sh < tw)) unsure = true;
+                    if (sl >= td) code |= 2;
+                    else if (!(sh < td)) unsure = true;
+                    ub = sh * (1.0 + (double) found[c] * phirel);
+                }
+                T.cnt[ch[c]][p] = phi_code(code, ub);
+                if (unsure) {
+                    const int at = atomicAdd(nfb, 1);
+                    if (at < fbcap) fb[at] = make_int2(ch[c], p);
+                }
+            } else {
+                T.cnt[ch[c]][p] = found[c];
+            }
+        }
+    }
+    if (stat) {
+        // the slots of k_b_count: candidates of S examined, (child, point)
+        // pairs counted, their algorithmic bytes, bytes of the examined
+        // candidates (their K coordinates; a neighbour's id and its
+        // coordinates in the children's dimensions)
+        long long done = 0, abytes = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (active && found[c] >= 0) {
+                done += 1;
+                abytes += (4ll * (K + 1) + 4) + (long long) found[c] * (4 + 4ll * (K + 1));
+            }
+        long long sn = seen;
+        long long ebytes = sn * 4ll * K + (l == 0 ? (long long) nhits * (4 + 4ll * J.nch) : 0);
+        for (int o = 32; o > 0; o >>= 1) {
+            sn += __shfl_down(sn, o);
+            done += __shfl_down(done, o);
+            abytes += __shfl_down(abytes, o);
+            ebytes += __shfl_down(ebytes, o);
+        }
+        if (__lane_id() == 0 && done) {
+            unsigned long long *slot_at = stat + 16 * (blockIdx.x & 63);
+            atomicAdd(&slot_at[0], (unsigned long long) sn);
+            atomicAdd(&slot_at[1], (unsigned long long) done);
+            atomicAdd(&slot_at[2], (unsigned long long) abytes);
+            atomicAdd(&slot_at[3], (unsigned long long) ebytes);
+        }
+    }
+}
+
 // ------------------------------------------------------------ dense components of a batch
 // (k_dense_init .. k_uf_flatten per subspace; grid.y = subspace)
 __global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, uint8_t *__restrict__ dsorted, int *__restrict__ par) {
@@ -1695,6 +1994,54 @@ hipError_t launch_b_count(const BatchSub *subs, int nsub, const int *blk_off, in
     if (tm.stop) (void) hipEventRecord(tm.stop, st);
     if (phi)
         LAUNCH(k_b_phi_exact, dim3(1024), dim3(kBlock), 0, st, D, subs, X.fb, X.nfb, X.fbcap, rank_order, eps, s_star);
+    return hipGetLastError();
+}
+
+template <bool PHI, int K>
+static void launch_fan_width(int width, dim3 grid, hipStream_t st, const BatchSub *groups, const FanJob *jobs,
+                             const int *blk_off, int njob, const FanTable &T, const DevData &D, const BatchIndex &X,
+                             float s_star, float eps, double phirel, int cap, float phi_w, float phi_d,
+                             unsigned long long *stat) {
+#define FAN(CW, NC)                                                                                                    \
+    LAUNCH((k_b_fan<PHI, K, CW, NC>), grid, dim3(kBlock), 0, st, groups, jobs, blk_off, njob, T, D.d, D.X, X.edge,    \
+           X.qlist, X.qstart, s_star, eps, phirel, cap, phi_w, phi_d, X.nb, X.fb, X.nfb, X.fbcap, stat)
+    switch (width) {
+    case 4: FAN(4, 1); break;
+    case 8: FAN(8, 1); break;
+    case 16: FAN(8, 2); break;
+    case 32: FAN(16, 2); break;
+    default: FAN(16, 4); break;
+    }
+#undef FAN
+}
+
+hipError_t launch_b_fan(const BatchSub *groups, const FanJob *jobs, const int *blk_off, int njob, int nblk, int width,
+                        int kS, const FanTable &T, const BatchIndex &X, float s_star, float eps, bool phi,
+                        bool phi_all_exact, int cap, float phi_w, float phi_d, const DevData &D,
+                        unsigned long long *stat, hipStream_t st) {
+    if (njob <= 0 || nblk <= 0) return hipSuccess;
+    if (kS < 1 || kS > kMaxFastK || width > kFanMost) return hipErrorInvalidValue;
+    const double phirel = phi_all_exact ? 1e30 : kPhiRelDefault;
+#define FAN_K(K)                                                                                                       \
+    case K:                                                                                                            \
+        if (phi)                                                                                                       \
+            launch_fan_width<true, K>(width, dim3(nblk), st, groups, jobs, blk_off, njob, T, D, X, s_star, eps,       \
+                                      phirel, cap, phi_w, phi_d, stat);                                                \
+        else                                                                                                           \
+            launch_fan_width<false, K>(width, dim3(nblk), st, groups, jobs, blk_off, njob, T, D, X, s_star, eps,      \
+                                       phirel, cap, phi_w, phi_d, stat);                                               \
+        break
+    switch (kS) {
+        FAN_K(1);
+        FAN_K(2);
+        FAN_K(3);
+        FAN_K(4);
+        FAN_K(5);
+        FAN_K(6);
+        FAN_K(7);
+        FAN_K(8);
+    }
+#undef FAN_K
     return hipGetLastError();
 }
 

@@ -61,3 +61,35 @@ def test_walks_on_cell_edges_match_oracle(n, d, eps, num_obj, rect):
         assert np.array_equal(O.canonical(a), b), f"labels differ in subspace {s}"
     assert np.array_equal(trace, ref.trace)
     assert max(len(s) for s in got.subspaces) >= 3
+
+
+# masks whose children are counted by one walk: up to 3, 7, 15 and 31 children
+# (the widths of the walk; test_wide_dimensions_match_oracle has more than 64),
+# with points of clumps that stay dense over many dimensions (walks of 1 to 4)
+@pytest.mark.parametrize("n,d,eps,dims,rect", [(260, 5, 0.04, 5, True), (260, 5, 0.04, 5, False),
+                                               (350, 9, 0.04, 5, True), (350, 9, 0.04, 5, False),
+                                               (300, 17, 0.02, 4, True), (300, 17, 0.02, 4, False),
+                                               (301, 33, 0.02, 4, True)])
+def test_walks_serving_many_children_match_oracle(n, d, eps, dims, rect):
+    print("children", n, d, eps, dims, rect, flush=True)
+    rng = np.random.default_rng(n * d)
+    X = rng.random((n, d)).astype(np.float32)
+    for c in range(3):
+        rows = np.arange(c * n // 4, (c + 1) * n // 4)[:, None]
+        at = np.sort(rng.choice(d, dims, replace=False)) if c else np.r_[0:dims - 1, d - 1]
+        size = (c + 1) * n // 4 - c * n // 4
+        X[rows, at] = (rng.uniform(0.2, 0.8, dims) + 0.4 * eps * rng.standard_normal((size, dims))).astype(np.float32)
+    X = np.clip(X, 0.0, 1.0)
+    args = (eps, 1.0, 4, n // 6, 1.0, 4, rect, 0)
+    ref = O.run_ref(X, *args[:7], 0, trace=True)
+    _lib.debug_trace(True)
+    try:
+        got = INSCY.run(X, *args, mode=_lib.MODE_BATCHED)
+        trace = _lib.debug_trace_rows()
+    finally:
+        _lib.debug_trace(False)
+    assert got.subspaces == ref.subspaces
+    for s, a, b in zip(ref.subspaces, ref.labels, got.labels):
+        assert np.array_equal(O.canonical(a), b), f"labels differ in subspace {s}"
+    assert np.array_equal(trace, ref.trace)
+    assert max(len(s) for s in got.subspaces) >= dims - 1
