@@ -258,14 +258,34 @@ __device__ __forceinline__ uint64_t mix64(uint64_t h) {
     return h;
 }
 
-// a and b share their c-grid cells on every unrestricted dimension at SCY-tree
-// levels 0..upto (the regular-node prefix of the tree)
-__device__ __forceinline__ bool same_prefix(const DevData &D, dmask_t smask, int a, int b, int upto) {
+// Cells of a point are read as rows of 16 levels (one 16-byte load) wherever
+// many levels of one point are needed: the [d][n] array would cost one
+// scattered byte, and its cache line, per level.  Level masks: bit t for level t.
+struct CellRow {
+    uint64_t lo, hi;  // levels c0..c0+7 and c0+8..c0+15, one byte each
+    __device__ __forceinline__ int at(int t) const { return (int) (((t & 8) ? hi : lo) >> (8 * (t & 7))) & 0xFF; }
+};
+__device__ __forceinline__ CellRow load_row(const DevData &D, int p, int c0) {
+    const uint4 v = *reinterpret_cast<const uint4 *>(D.rows + (size_t) p * D.rs + c0);
+    return CellRow{(uint64_t) v.y << 32 | v.x, (uint64_t) v.w << 32 | v.z};
+}
+
+// bit i: byte i of x is not zero
+__device__ __forceinline__ uint32_t nonzero_bytes(uint64_t x) {
+    const uint64_t t = (((x & 0x7F7F7F7F7F7F7F7Full) + 0x7F7F7F7F7F7F7F7Full) | x) & 0x8080808080808080ull;
+    return (uint32_t) ((t >> 7) * 0x0102040810204080ull >> 56);
+}
+
+// a and b share their c-grid cells at the unrestricted levels 0..upto (the
+// regular-node prefix of the tree); restricted: level mask
+__device__ __forceinline__ bool same_prefix(const DevData &D, dmask_t restricted, int a, int b, int upto) {
     if (b < 0 || b >= D.n) return false;
-    for (int t = 0; t <= upto; ++t) {
-        const int k = D.level[t];
-        if (dhas(smask, k)) continue;
-        if (D.cellC[(size_t) k * D.n + a] != D.cellC[(size_t) k * D.n + b]) return false;
+    if (a == b) return true;
+    for (int c0 = 0; c0 <= upto; c0 += 16) {
+        const CellRow x = load_row(D, a, c0), y = load_row(D, b, c0);
+        const uint32_t diff = nonzero_bytes(x.lo ^ y.lo) | nonzero_bytes(x.hi ^ y.hi) << 8;
+        const uint32_t in = upto - c0 >= 15 ? 0xFFFFu : (2u << (upto - c0)) - 1u;
+        if (diff & in & ~(uint32_t) (restricted >> c0)) return false;
     }
     return true;
 }

@@ -266,7 +266,7 @@ public:
         }
         for (void *p : {(void *) Xt, (void *) cellC, (void *) cellE, (void *) nearm, (void *) small, (void *) stamp,
                         (void *) qmark, (void *) entries, (void *) scratch, (void *) rank_perm,
-                        (void *) d_level, (void *) edges})
+                        (void *) d_level, (void *) edges, (void *) rows})
             if (p) dev_free(p);
         if (pin) host_free(pin);
     }
@@ -295,6 +295,7 @@ public:
         HIP_OK(dev_alloc(&cellC, nd));
         HIP_OK(dev_alloc(&cellE, nd * sizeof(uint16_t)));
         HIP_OK(dev_alloc(&nearm, (size_t) n * sizeof(dmask_t)));
+        HIP_OK(dev_alloc(&rows, (size_t) n * cell_row_bytes(d)));
         HIP_OK(dev_alloc(&small, kSmallWords * sizeof(unsigned long long)));
         HIP_OK(dev_alloc(&stamp, (size_t) n * sizeof(int)));
         HIP_OK(dev_alloc(&qmark, (size_t) n * sizeof(int)));
@@ -319,7 +320,7 @@ public:
         int *hist = arena.take<int>((size_t) d * ecells);
         HIP_OK(launch_fill_i32(reinterpret_cast<int *>(small), 0, 2 * kSmallWords, st));
         HIP_OK(launch_discretise(d_X, n, d, cells, prm.neighborhood_size, Xt, cellC, cellE,
-                                 reinterpret_cast<uint64_t *>(nearm), 2, reinterpret_cast<int *>(small), st));
+                                 prm.entropy_order == 0 ? rows : nullptr, reinterpret_cast<uint64_t *>(nearm), 2, reinterpret_cast<int *>(small), st));
         HIP_OK(launch_hist1(cellE, n, d, ecells, hist, st));
         // c-grid occupancy: the input of the entropy order only
         int *histc = arena.take<int>((size_t) d * cells);
@@ -370,6 +371,7 @@ public:
         std::vector<int> both(level);
         both.insert(both.end(), lvl_of.begin(), lvl_of.end());
         HIP_OK(hipMemcpyAsync(d_level, both.data(), both.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        if (prm.entropy_order != 0) HIP_OK(launch_cell_rows(cellC, n, d, d_level, rows, st));
         sync();  // `both` is pageable and goes out of scope
         if (phi_mode) {
             // leaf order of the neighbourhood tree, whose levels follow the same order
@@ -383,7 +385,7 @@ public:
             sync();
         }
         arena.release(0);
-        D = DevData{d_X, Xt, cellC, cellE, d_level, d_level + d, n, d, cells, ecells};
+        D = DevData{d_X, Xt, cellC, cellE, rows, d_level, d_level + d, n, d, cells, ecells, cell_row_bytes(d)};
     }
 
     // ---------------------------------------------------------- run
@@ -975,6 +977,7 @@ private:
     float *Xt = nullptr;
     uint8_t *cellC = nullptr;
     uint16_t *cellE = nullptr;
+    uint8_t *rows = nullptr;  // cells by point and SCY-tree level
     dmask_t *nearm = nullptr;
     int mw = 1;  // words per path mask: 1 for d <= 64, else 2
     unsigned long long *small = nullptr;
@@ -1055,6 +1058,13 @@ private:
     int *lv_next_counts = nullptr;
     int lv_nslots = 0;
 
+    // dimension mask -> mask of their SCY-tree levels
+    dmask_t levels_of(dmask_t dims) const {
+        dmask_t m = 0;
+        for (int t = 0; t < d; ++t)
+            if (dhas(dims, level[t])) m |= dbit(t);
+        return m;
+    }
     void put(void *dst, const void *src, size_t bytes);
     template <class T>
     T *upload(Pool &pool, const std::vector<T> &v) {

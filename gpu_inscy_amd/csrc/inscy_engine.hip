@@ -518,7 +518,8 @@ int inscy_discretise(const float *d_X, int64_t n, int32_t d, int32_t cells, floa
         int *bad = nullptr;
         HIP_OK(hipMalloc(&bad, sizeof(int)));
         HIP_OK(hipMemset(bad, 0, sizeof(int)));
-        HIP_OK(launch_discretise(d_X, (int) n, d, cells, eps, nullptr, d_cell_c, d_cell_e, d_near_mask, (d + 63) / 64,
+        HIP_OK(launch_discretise(d_X, (int) n, d, cells, eps, nullptr, d_cell_c, d_cell_e, nullptr, d_near_mask,
+                                 (d + 63) / 64,
                                  bad, 0));
         int h = 0;
         HIP_OK(hipMemcpy(&h, bad, sizeof(int), hipMemcpyDeviceToHost));

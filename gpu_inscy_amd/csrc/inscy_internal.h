@@ -68,10 +68,14 @@ struct DevData {
     const float *Xt;        // [d][n] coordinates
     const uint8_t *cellC;   // [d][n] cell in the c-grid (ScyTreeNode.cu:100-102)
     const uint16_t *cellE;  // [d][n] cell in the ceil(1/eps)-grid (inscy_map.cpp:243-244)
+    const uint8_t *rows;    // [n][rs] c-grid cells of a point by SCY-tree level, zero past level d - 1
     const int *level;       // [d] dimension at each SCY-tree level (get_subspace_order, inscy_map.cpp:61-121)
     const int *lvl_of;      // [d] level of each dimension
-    int n, d, cells, ecells;
+    int n, d, cells, ecells, rs;
 };
+
+// bytes of a point's row of cells: one 16-byte load serves 16 levels
+inline int cell_row_bytes(int d) { return (d + 15) & ~15; }
 
 // Grid index of one subspace: the points are sorted by their eps-grid cells in
 // j (1..3) of the subspace's dimensions.
@@ -217,7 +221,7 @@ struct PartPair {
     const uint64_t *spm;  // mw words per path
     const int *gid;      // [cells]
     const int *weakcnt;  // counts of S ∪ {m}
-    int *cnt;            // [6G]: points, weak-dense points, paths per group; then cursors
+    int *cnt;            // [7G]: points, weak-dense points, paths per group; 3 cursors; the paths' branch levels
     int *outW;
     int *outx;
     uint64_t *outm;
@@ -267,8 +271,11 @@ hipError_t launch_flag_compact(const uint8_t *flags, size_t nb, void *temp, size
 // Launchers (all asynchronous on `st`; return the hipError_t of the launches).
 // discretise: the near-edge marks of point p are nw 64-bit words at nearw[p * nw]
 // (nw = 2 is dmask_t[n]; 1 suffices for d <= 64)
+// rows: the cells again as [n][cell_row_bytes(d)] in dimension order (may be null)
 hipError_t launch_discretise(const float *X, int n, int d, int cells, float eps, float *Xt, uint8_t *cellC,
-                             uint16_t *cellE, uint64_t *nearw, int nw, int *bad, hipStream_t st);
+                             uint16_t *cellE, uint8_t *rows, uint64_t *nearw, int nw, int *bad, hipStream_t st);
+// rows in `level` order (device array [d])
+hipError_t launch_cell_rows(const uint8_t *cellC, int n, int d, const int *level, uint8_t *rows, hipStream_t st);
 hipError_t launch_hist1(const uint16_t *cellE, int n, int d, int ecells, int *hist, hipStream_t st);
 // occupancy of the c-grid per dimension ([d][cells]), the input of the entropy order
 hipError_t launch_histc(const uint8_t *cellC, int n, int d, int cells, int *hist, hipStream_t st);

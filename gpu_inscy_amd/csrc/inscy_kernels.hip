@@ -28,14 +28,38 @@ namespace {
 // ------------------------------------------------------------ discretisation
 // get_cell_no (ScyTreeNode.cu:100-102): min((int)(x / (1/c)), c-1); the
 // s-connection test of construct_s_connection (:34-49): x >= (c+1)*(1/c) - eps.
+// cell of level t into the point's row, written 16 levels at a time
+__device__ __forceinline__ void put_cell(uint8_t *__restrict__ rows, int rs, int p, int t, int d, int c, uint64_t &lo,
+                                         uint64_t &hi) {
+    if (!rows) return;
+    const uint64_t v = (uint64_t) (uint8_t) c << (8 * (t & 7));
+    if (t & 8)
+        hi |= v;
+    else
+        lo |= v;
+    if ((t & 15) != 15 && t != d - 1) return;
+    *reinterpret_cast<uint4 *>(rows + (size_t) p * rs + (t & ~15)) =
+        make_uint4((uint32_t) lo, (uint32_t) (lo >> 32), (uint32_t) hi, (uint32_t) (hi >> 32));
+    lo = hi = 0;
+}
+
+__global__ void k_cell_rows(const uint8_t *__restrict__ cellC, int n, int d, const int *__restrict__ level,
+                            uint8_t *__restrict__ rows, int rs) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    uint64_t lo = 0, hi = 0;
+    for (int t = 0; t < d; ++t) put_cell(rows, rs, p, t, d, cellC[(size_t) level[t] * n + p], lo, hi);
+}
+
 __global__ void k_discretise(const float *__restrict__ X, int n, int d, int cells, float cs, int ecells,
                              float ecs, float eps, float *__restrict__ Xt, uint8_t *__restrict__ cellC,
-                             uint16_t *__restrict__ cellE, uint64_t *__restrict__ nearw, int nw,
-                             int *__restrict__ bad) {
+                             uint16_t *__restrict__ cellE, uint8_t *__restrict__ rows, int rs,
+                             uint64_t *__restrict__ nearw, int nw, int *__restrict__ bad) {
     int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     dmask_t nm = 0;
     bool out_of_range = false;
+    uint64_t lo = 0, hi = 0;  // the cells of 16 dimensions
     for (int k = 0; k < d; ++k) {
         float x = X[(size_t) p * d + k];
         if (!(x >= 0.0f && x <= 1.0f)) out_of_range = true;
@@ -45,6 +69,7 @@ __global__ void k_discretise(const float *__restrict__ X, int n, int d, int cell
         int e = min((int) __fdiv_rn(x, ecs), ecells - 1);
         cellC[(size_t) k * n + p] = (uint8_t) c;
         cellE[(size_t) k * n + p] = (uint16_t) e;
+        put_cell(rows, rs, p, k, d, c, lo, hi);
         float upper = __fmul_rn((float) (c + 1), cs);
         float bound = __fsub_rn(upper, eps);
         if (x >= bound) nm |= dbit(k);
@@ -504,10 +529,12 @@ __global__ void k_path_insert(DevData D, dmask_t smask, const int *__restrict__ 
     if (!need) return;
     int w = W[i];
     uint64_t h = 0x243F6A8885A308D3ull;
+    CellRow row{};
     for (int t = 0; t < D.d; ++t) {
-        const int k = D.level[t];
+        const int k = t;
+        if (!(t & 15)) row = load_row(D, w, t);
         if (dhas(smask, k)) continue;
-        h = mix64(h + D.cellC[(size_t) k * D.n + w] + 1);
+        h = mix64(h + row.at(t & 15) + 1);
         if (!dhas(need, k)) continue;
         uint64_t e = mix64(h ^ (0x9E3779B97F4A7C15ull * (uint64_t) (k + 1)));
         uint64_t entry = (e & 0xFFFFFFFF00000000ull) | (uint32_t) w;
@@ -541,10 +568,12 @@ __global__ void k_path_check(DevData D, dmask_t smask, const int *__restrict__ s
         if (stamp[x] != tid) {
             uint64_t h = 0x243F6A8885A308D3ull;
             dmask_t keep = 0;
+            CellRow row{};
             for (int t = 0; t < D.d; ++t) {
-                const int k = D.level[t];
+                const int k = t;
+                if (!(t & 15)) row = load_row(D, x, t);
                 if (dhas(smask, k)) continue;
-                h = mix64(h + D.cellC[(size_t) k * D.n + x] + 1);
+                h = mix64(h + row.at(t & 15) + 1);
                 if (!dhas(m, k)) continue;
                 uint64_t e = mix64(h ^ (0x9E3779B97F4A7C15ull * (uint64_t) (k + 1)));
                 uint64_t slot = e & tmask;
@@ -783,13 +812,18 @@ float sqrt_threshold(float eps) {
 
 #define LAUNCH(kernel, grid, block, lds, st, ...) hipLaunchKernelGGL(kernel, grid, block, lds, st, __VA_ARGS__)
 
+hipError_t launch_cell_rows(const uint8_t *cellC, int n, int d, const int *level, uint8_t *rows, hipStream_t st) {
+    LAUNCH(k_cell_rows, dim3(blocks_for(n)), dim3(kBlock), 0, st, cellC, n, d, level, rows, cell_row_bytes(d));
+    return hipGetLastError();
+}
+
 hipError_t launch_discretise(const float *X, int n, int d, int cells, float eps, float *Xt, uint8_t *cellC,
-                             uint16_t *cellE, uint64_t *nearw, int nw, int *bad, hipStream_t st) {
+                             uint16_t *cellE, uint8_t *rows, uint64_t *nearw, int nw, int *bad, hipStream_t st) {
     int ecells = (int) ceil(1.0 / (double) eps);
     float cs = 1.0f / (float) cells;
     float ecs = 1.0f / (float) ecells;
     LAUNCH(k_discretise, dim3(blocks_for(n)), dim3(kBlock), 0, st, X, n, d, cells, cs, ecells, ecs, eps, Xt, cellC,
-           cellE, nearw, nw, bad);
+           cellE, rows, cell_row_bytes(d), nearw, nw, bad);
     return hipGetLastError();
 }
 

@@ -26,6 +26,12 @@ namespace inscy {
 namespace {
 constexpr size_t kMaxBatch = 1024;  // child subspaces per batch (inscy_set_tuning, INSCY_MAX_BATCH override)
 constexpr uint64_t kEmptySlot = ~0ull;  // free slot of a path-prune table
+// slots of a path prune's table for at most `levels` prefixes, at most half full
+inline size_t path_slots(int levels) {
+    size_t s = 64;
+    while (s < 2 * (size_t) levels) s <<= 1;
+    return s;
+}
 inline int nblocks(long long count) { return (int) ((count + kBlockThreads - 1) / kBlockThreads); }
 }  // namespace
 
@@ -289,7 +295,8 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             for (int a = c.t0; a < c.t1; ++a) {
                 if (!pair_on(a, c.m)) continue;
                 const LTree &t = lt[lv_act[a]];
-                est += (size_t) t.nW * (8 + 32 * (size_t) (d - 1 - c.m)) + (size_t) t.nsp * 12 + 6 * 256 * 4;
+                // lists, and the path prune's table (a few branch levels per path)
+                est += (size_t) t.nW * 8 + (size_t) t.nsp * (12 + 32 * std::min<size_t>(d - 1 - c.m, 4)) + 7 * 256 * 4;
             }
             const bool fits = bytes + est <= batch_budget && (long long) (j - i + 1) * n < INT_MAX &&
                               hsum + ncell < INT_MAX;
@@ -600,7 +607,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             const LTree &t = lt[lv_act[a]];
             const int G = (int) lv_groups[a][c.m - t.first].size();
             pinfo.push_back({a, b, G, pc_total});
-            pc_total += 6 * G;
+            pc_total += 7 * G;
         }
     }
     const int np = (int) pinfo.size();
@@ -706,7 +713,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                         PruneChild pc;
                         std::memset(&pc, 0, sizeof(pc));
                         pc.smask = c.s;
-                        const size_t slots = table_slots(nW, d - 1 - c.m);
+                        const size_t slots = path_slots(c3[6 * G + g]);
                         pc.tmask = (uint64_t) (slots - 1);
                         pc.W = pairs[j].outW + offW;
                         pc.spx = pairs[j].outx + offS;

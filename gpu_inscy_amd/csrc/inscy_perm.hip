@@ -42,20 +42,21 @@ __device__ __forceinline__ int chain_end(uint64_t w) { return (int) ((w >> 8) & 
 __device__ __forceinline__ uint64_t chain_word(int b, int end) { return (uint64_t) b | ((uint64_t) end << 8); }
 
 constexpr uint64_t kSeed = 0x243F6A8885A308D3ull;
-__device__ __forceinline__ uint64_t level_salt(int k) { return 0x9E3779B97F4A7C15ull * (uint64_t) (k + 1); }
+__device__ __forceinline__ uint64_t level_salt(int t) { return 0x9E3779B97F4A7C15ull * (uint64_t) (t + 1); }
 
-// prefix of z through level index `upto` (unrestricted levels of smask)
-__device__ __forceinline__ uint64_t prefix_hash(const DevData &D, dmask_t smask, int z, int upto) {
+// Restricted levels are level masks (bit t for level t) throughout.
+// prefix of z through level `upto` (an unrestricted one)
+__device__ __forceinline__ uint64_t prefix_hash(const DevData &D, dmask_t restricted, int z, int upto) {
     uint64_t h = kSeed;
+    CellRow row{};
     for (int t = 0; t <= upto; ++t) {
-        const int k = D.level[t];
-        if (dhas(smask, k)) continue;
-        h = mix64(h + D.cellC[(size_t) k * D.n + z] + 1);
+        if (!(t & 15)) row = load_row(D, z, t);
+        if (!dhas(restricted, t)) h = mix64(h + row.at(t & 15) + 1);
     }
-    return mix64(h ^ level_salt(D.level[upto]));
+    return mix64(h ^ level_salt(upto));
 }
 
-__device__ void table_insert(const DevData &D, dmask_t smask, uint64_t *table, uint64_t tmask, uint64_t e, int z,
+__device__ void table_insert(const DevData &D, dmask_t restricted, uint64_t *table, uint64_t tmask, uint64_t e, int z,
                              int t) {
     const uint64_t entry = (e & 0xFFFFFFFF00000000ull) | (uint32_t) z;
     uint64_t slot = e & tmask;
@@ -66,18 +67,18 @@ __device__ void table_insert(const DevData &D, dmask_t smask, uint64_t *table, u
                             (unsigned long long) entry);
             if (cur == kEmpty) return;
         }
-        if ((cur >> 32) == (entry >> 32) && same_prefix(D, smask, z, (int) (uint32_t) cur, t)) return;
+        if ((cur >> 32) == (entry >> 32) && same_prefix(D, restricted, z, (int) (uint32_t) cur, t)) return;
         slot = (slot + 1) & tmask;
     }
 }
 
-__device__ bool table_has(const DevData &D, dmask_t smask, const uint64_t *table, uint64_t tmask, uint64_t e, int z,
-                          int t) {
+__device__ bool table_has(const DevData &D, dmask_t restricted, const uint64_t *table, uint64_t tmask, uint64_t e,
+                          int z, int t) {
     uint64_t slot = e & tmask;
     while (true) {
         const uint64_t cur = table[slot];  // complete: the inserts ran in an earlier launch
         if (cur == kEmpty) return false;
-        if ((cur >> 32) == (e >> 32) && same_prefix(D, smask, z, (int) (uint32_t) cur, t)) return true;
+        if ((cur >> 32) == (e >> 32) && same_prefix(D, restricted, z, (int) (uint32_t) cur, t)) return true;
         slot = (slot + 1) & tmask;
     }
 }
@@ -146,44 +147,47 @@ __global__ void k_perm_route(DevData D, dmask_t smask, int m, const int *__restr
     om[at] = chain_word(b, e);
 }
 
-// prefixes of the points at every unrestricted level whose dimension is in `need`
-__global__ void k_perm_insert_pts(DevData D, dmask_t smask, const int *__restrict__ pts, const int *__restrict__ npts,
-                                  dmask_t need, uint64_t *__restrict__ table, uint64_t tmask) {
+// prefixes of the points at every unrestricted level in `need`
+__global__ void k_perm_insert_pts(DevData D, dmask_t restricted, const int *__restrict__ pts,
+                                  const int *__restrict__ npts, dmask_t need, uint64_t *__restrict__ table,
+                                  uint64_t tmask) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= *npts || !need) return;
     const int z = pts[i];
     uint64_t h = kSeed;
+    CellRow row{};
     for (int t = 0; t < D.d; ++t) {
-        const int k = D.level[t];
-        if (dhas(smask, k)) continue;
-        h = mix64(h + D.cellC[(size_t) k * D.n + z] + 1);
-        if (dhas(need, k)) table_insert(D, smask, table, tmask, mix64(h ^ level_salt(k)), z, t);
+        if (!(t & 15)) row = load_row(D, z, t);
+        if (dhas(restricted, t)) continue;
+        h = mix64(h + row.at(t & 15) + 1);
+        if (dhas(need, t)) table_insert(D, restricted, table, tmask, mix64(h ^ level_salt(t)), z, t);
     }
 }
 
 // regular ancestors of the chains' first nodes: x's prefixes at the levels above b's
-__global__ void k_perm_insert_anchors(DevData D, dmask_t smask, const int *__restrict__ cx,
+__global__ void k_perm_insert_anchors(DevData D, dmask_t restricted, const int *__restrict__ cx,
                                       const uint64_t *__restrict__ cm, const int *__restrict__ nch,
                                       uint64_t *__restrict__ table, uint64_t tmask) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= *nch) return;
     const int z = cx[i], Lb = D.lvl_of[chain_b(cm[i])];
     uint64_t h = kSeed;
+    CellRow row{};
     for (int t = 0; t < Lb; ++t) {
-        const int k = D.level[t];
-        if (dhas(smask, k)) continue;
-        h = mix64(h + D.cellC[(size_t) k * D.n + z] + 1);
-        table_insert(D, smask, table, tmask, mix64(h ^ level_salt(k)), z, t);
+        if (!(t & 15)) row = load_row(D, z, t);
+        if (dhas(restricted, t)) continue;
+        h = mix64(h + row.at(t & 15) + 1);
+        table_insert(D, restricted, table, tmask, mix64(h ^ level_salt(t)), z, t);
     }
 }
 
 struct PermTables {
     const uint64_t *W, *P, *T, *A;
     uint64_t wmask, pmask, tmask, amask;
-    dmask_t cond;  // dimensions whose nodes above m's level a larger dimension id below keeps
+    dmask_t cond;  // levels whose nodes above m's level a larger dimension id below keeps
 };
 
-__global__ void k_perm_prune(DevData D, dmask_t smask, PermTables Tb, const int *__restrict__ cx,
+__global__ void k_perm_prune(DevData D, dmask_t restricted, PermTables Tb, const int *__restrict__ cx,
                              const uint64_t *__restrict__ cm, const int *__restrict__ nch, int *__restrict__ ox,
                              uint64_t *__restrict__ om, int *__restrict__ nout) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -193,13 +197,13 @@ __global__ void k_perm_prune(DevData D, dmask_t smask, PermTables Tb, const int 
     const int b = chain_b(w), Lb = D.lvl_of[b];
     // the regular parent: x's prefix through the last unrestricted level above b's
     int tp = Lb - 1;
-    while (tp >= 0 && dhas(smask, D.level[tp])) --tp;
-    if (tp >= 0 && !table_has(D, smask, Tb.W, Tb.wmask, prefix_hash(D, smask, z, tp), z, tp)) return;
-    const uint64_t e = prefix_hash(D, smask, z, Lb);
-    if (!table_has(D, smask, Tb.W, Tb.wmask, e, z, Lb)) {
-        const bool existed = table_has(D, smask, Tb.P, Tb.pmask, e, z, Lb) ||
-                             table_has(D, smask, Tb.A, Tb.amask, e, z, Lb) ||
-                             (dhas(Tb.cond, b) && table_has(D, smask, Tb.T, Tb.tmask, e, z, Lb));
+    while (tp >= 0 && dhas(restricted, tp)) --tp;
+    if (tp >= 0 && !table_has(D, restricted, Tb.W, Tb.wmask, prefix_hash(D, restricted, z, tp), z, tp)) return;
+    const uint64_t e = prefix_hash(D, restricted, z, Lb);
+    if (!table_has(D, restricted, Tb.W, Tb.wmask, e, z, Lb)) {
+        const bool existed = table_has(D, restricted, Tb.P, Tb.pmask, e, z, Lb) ||
+                             table_has(D, restricted, Tb.A, Tb.amask, e, z, Lb) ||
+                             (dhas(Tb.cond, Lb) && table_has(D, restricted, Tb.T, Tb.tmask, e, z, Lb));
         if (existed) return;  // the sibling lost its points: propergate_count2 erases the chain
     }
     const int at = atomicAdd(nout, 1);
@@ -207,11 +211,11 @@ __global__ void k_perm_prune(DevData D, dmask_t smask, PermTables Tb, const int 
     om[at] = w;
 }
 
-// the points of G's first cell mark their prefixes through level index tkey
+// the points of G's first cell mark their prefixes through level tkey
 // (tkey < 0: the root, flag[0])
-__global__ void k_perm_lo_mark(DevData D, dmask_t smask, const int *__restrict__ pts, const int *__restrict__ npts,
-                               int m, int lo, int tkey, uint64_t *__restrict__ table, uint64_t tmask,
-                               int *__restrict__ flag) {
+__global__ void k_perm_lo_mark(DevData D, dmask_t restricted, const int *__restrict__ pts,
+                               const int *__restrict__ npts, int m, int lo, int tkey, uint64_t *__restrict__ table,
+                               uint64_t tmask, int *__restrict__ flag) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= *npts) return;
     const int z = pts[i];
@@ -219,16 +223,18 @@ __global__ void k_perm_lo_mark(DevData D, dmask_t smask, const int *__restrict__
     if (tkey < 0)
         flag[0] = 1;
     else
-        table_insert(D, smask, table, tmask, prefix_hash(D, smask, z, tkey), z, tkey);
+        table_insert(D, restricted, table, tmask, prefix_hash(D, restricted, z, tkey), z, tkey);
 }
 
-__global__ void k_perm_lo_filter(DevData D, dmask_t smask, const int *__restrict__ in, const int *__restrict__ nin,
-                                 int tkey, const uint64_t *__restrict__ table, uint64_t tmask,
-                                 const int *__restrict__ flag, int *__restrict__ out, int *__restrict__ nout) {
+__global__ void k_perm_lo_filter(DevData D, dmask_t restricted, const int *__restrict__ in,
+                                 const int *__restrict__ nin, int tkey, const uint64_t *__restrict__ table,
+                                 uint64_t tmask, const int *__restrict__ flag, int *__restrict__ out,
+                                 int *__restrict__ nout) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= *nin) return;
     const int z = in[i];
-    const bool keep = tkey < 0 ? flag[0] != 0 : table_has(D, smask, table, tmask, prefix_hash(D, smask, z, tkey), z, tkey);
+    const bool keep = tkey < 0 ? flag[0] != 0
+                               : table_has(D, restricted, table, tmask, prefix_hash(D, restricted, z, tkey), z, tkey);
     if (keep) out[atomicAdd(nout, 1)] = z;
 }
 
@@ -325,13 +331,14 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
             else tabove = t;
         }
         const bool filt = !deeper && (tabove < 0 || level[tabove] > m);
-        // dimensions of nodes above m's level kept empty by a larger dimension id below
+        const dmask_t restricted = levels_of(smask);
+        // levels of nodes above m's level kept empty by a larger dimension id below
         dmask_t cond = 0;
         for (int t = 0; t < Lm; ++t) {
             const int k = level[t];
             if (dhas(T.smask, k)) continue;
             for (int u = t; u < Lm; ++u)
-                if (!dhas(T.smask, level[u]) && level[u] > m) cond |= dbit(k);
+                if (!dhas(T.smask, level[u]) && level[u] > m) cond |= dbit(t);
         }
         // the dimension's cluster marks, below every group's buffers (a
         // group's buffers are released while its kernels may still be queued:
@@ -357,12 +364,12 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
                 int *W2 = arena.take<int>(std::max(nW, 1));
                 HIP_OK(launch_fill_u64(table, kEmpty, slots, st));
                 HIP_OK(launch_fill_i32(flag, 0, 3, st));
-                LAUNCH(k_perm_lo_mark, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, smask, Pg, nPg, m, gs[g].lo,
+                LAUNCH(k_perm_lo_mark, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, m, gs[g].lo,
                        tabove, table, (uint64_t) (slots - 1), flag);
-                LAUNCH(k_perm_lo_filter, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, smask, Pg, nPg, tabove,
+                LAUNCH(k_perm_lo_filter, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, tabove,
                        table, (uint64_t) (slots - 1), flag, P2, flag + 1);
                 if (nW > 0)
-                    LAUNCH(k_perm_lo_filter, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, smask, Wg, nWg, tabove,
+                    LAUNCH(k_perm_lo_filter, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, restricted, Wg, nWg, tabove,
                            table, (uint64_t) (slots - 1), flag, W2, flag + 2);
                 HIP_OK(hipGetLastError());
                 HIP_OK(hipMemcpyAsync(pin, flag + 1, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -396,11 +403,11 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
                 LAUNCH(k_perm_route, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, T.smask, m,
                        d_gid + (size_t) (m - first) * cells, g, T.spx, T.chain, T.nsp, rx, rm, nr);
                 int free_dims = 0;
-                dmask_t need = 0;
-                for (int k = 0; k < d; ++k)
-                    if (!dhas(smask, k)) {
+                dmask_t need = 0;  // unrestricted levels
+                for (int t = 0; t < d; ++t)
+                    if (!dhas(restricted, t)) {
                         ++free_dims;
-                        need |= dbit(k);
+                        need |= dbit(t);
                     }
                 const size_t ws = slots_for((long long) nW * free_dims), ps = slots_for((long long) nPr * free_dims),
                              ts = slots_for((long long) T.nP_max * free_dims),
@@ -412,18 +419,18 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
                 HIP_OK(launch_fill_u64(tt, kEmpty, ts, st));
                 HIP_OK(launch_fill_u64(ta, kEmpty, as, st));
                 if (nW > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, smask, Wg, nWg, need, tw,
+                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, restricted, Wg, nWg, need, tw,
                            (uint64_t) (ws - 1));
                 if (nPr > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, smask, Pg, nPg, need, tp,
+                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, need, tp,
                            (uint64_t) (ps - 1));
                 if (cond && T.nP_max > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(T.nP_max)), dim3(kBlock), 0, st, D, smask, T.P, T.nP,
+                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(T.nP_max)), dim3(kBlock), 0, st, D, restricted, T.P, T.nP,
                            cond & need, tt, (uint64_t) (ts - 1));
-                LAUNCH(k_perm_insert_anchors, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, smask, rx, rm, nr,
+                LAUNCH(k_perm_insert_anchors, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, restricted, rx, rm, nr,
                        ta, (uint64_t) (as - 1));
                 const PermTables Tb{tw, tp, tt, ta, ws - 1, ps - 1, ts - 1, as - 1, cond};
-                LAUNCH(k_perm_prune, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, smask, Tb, rx, rm, nr, cx2,
+                LAUNCH(k_perm_prune, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, restricted, Tb, rx, rm, nr, cx2,
                        cm2, nc2);
                 HIP_OK(hipGetLastError());
             }
