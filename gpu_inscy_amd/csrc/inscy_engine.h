@@ -14,8 +14,9 @@
 // mergeWithNeighbors become one flag pass and one filter pass, the weak-density
 // prune is a neighbour-count pass plus compaction, and clustering works on the
 // dense components of S over the whole data set, computed once per subspace.
-// The host keeps the depth-first order of the reference because
-// pruneRedundancy and join read the partial result.
+// The level-synchronous driver (inscy_level.hip) serves the identity level
+// order, the depth-first one over s-connection chains (inscy_perm.hip) a
+// permuted order.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -228,16 +229,16 @@ struct HostBuf {
     }
 };
 
+// a tree of the permuted-order driver
 struct TreeRef {
     dmask_t smask;
     const int *P;      // device point ids
     const int *nP;     // device count
     int nP_max;        // host bound (exact where the host knows it)
-    const int *spx;    // device path origins
-    const uint64_t *spm;  // their masks, mw words each
+    const int *spx;    // origins of its s-connection chains
+    const uint64_t *chain;  // their chain words
     const int *nsp;
     int nsp_max;
-    const uint64_t *chain = nullptr;  // permuted-order driver: chain words instead of spm
 };
 
 // What the algorithm needs about one subspace S, computed on first use:
@@ -389,7 +390,7 @@ public:
     }
 
     // ---------------------------------------------------------- run
-    // level-synchronous driver (INSCY_MODE_BATCHED), same result
+    // level-synchronous driver (the identity level order)
     void run_levels(inscy_result &out);
     bool levels_mode = false;
     // permuted SCY-tree level order (entropy_order != 0): the depth-first
@@ -407,25 +408,6 @@ public:
     long long keep_budget_override = -1;  // test hook: bytes kept across batches (< 0: the batch budget)
     int mem_share = 1;  // engines running at once on the device (each budgets 1/mem_share of the free bytes)
     int max_batch_override = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
-
-    void run(inscy_result &out) {
-        int *P = arena.take<int>(n);
-        int *nP = arena.take<int>(1);
-        int *spx = arena.take<int>(n);
-        uint64_t *spm = arena.take<uint64_t>((size_t) n * mw);
-        int *nsp = arena.take<int>(1);
-        HIP_OK(launch_iota(P, n, st));
-        HIP_OK(launch_fill_i32(nP, n, 1, st));
-        HIP_OK(launch_root_paths(nearm, n, spx, spm, mw, nsp, st));
-        TreeRef root{(dmask_t) 0, P, nP, n, spx, spm, nsp, n};
-        auto t0 = std::chrono::steady_clock::now();
-        recurse(root, 0);
-        sync();
-        auto t1 = std::chrono::steady_clock::now();
-        emit(out);
-        stats.expand_seconds = std::chrono::duration<double>(t1 - t0).count();
-        stats.emit_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t1).count();
-    }
 
     // dense components of one subspace (kernel-level entry point)
     const Subspace &subspace(dmask_t smask) { return ensure_components(smask); }
@@ -701,137 +683,6 @@ private:
     };
 
     void recurse_perm(const TreeRef &T, int first);
-
-    void recurse(const TreeRef &T, int first) {
-        stats.calls++;
-        if (first >= d) return;
-        const int nd = d - first;
-        const size_t lvl_mark = arena.mark();
-
-        // restrict + mergeWithNeighbors for every dimension m >= first: the
-        // s-connected cells, then the cell groups (ScyTreeNode.cu:837-851)
-        int *flags = arena.take<int>((size_t) nd * cells);
-        HIP_OK(launch_fill_i32(flags, 0, (size_t) nd * cells, st));
-        HIP_OK(launch_flags_all(T.spx, T.spm, mw, T.nsp, T.nsp_max, cellC, n, first, cells, flags, st));
-        // the subspaces of the children are counted on this tree's points while
-        // the flags travel
-        const int markid = ++mark_id;
-        HIP_OK(launch_mark(T.P, T.nP, T.nP_max, qmark, markid, st));
-        for (int m = first; m < d; ++m) ensure_counts(T.smask | dbit(m), markid);
-        HIP_OK(hipMemcpyAsync(pin, flags, (size_t) nd * cells * sizeof(int), hipMemcpyDeviceToHost, st));
-        sync();
-        std::vector<std::vector<Group>> groups(nd);
-        std::vector<int> gid((size_t) nd * cells);
-        for (int m = first; m < d; ++m) {
-            const int *f = pin_i((size_t) (m - first) * cells);
-            auto &gs = groups[m - first];
-            for (int c = 0; c < cells; ++c) {
-                int lo = c;
-                while (f[c] && c < cells - 1) ++c;
-                for (int x = lo; x <= c; ++x) gid[(size_t) (m - first) * cells + x] = (int) gs.size();
-                gs.push_back({lo, c});
-            }
-        }
-        int *d_gid = arena.take<int>(gid.size());
-        std::copy(gid.begin(), gid.end(), pin_i());
-        HIP_OK(hipMemcpyAsync(d_gid, pin, gid.size() * sizeof(int), hipMemcpyHostToDevice, st));
-
-        // partition points, weak-dense points and paths by group, all dimensions
-        struct Part {
-            int *cnt, *P, *W, *x;
-            uint64_t *mk;
-        };
-        std::vector<Part> parts(nd);
-        for (int m = first; m < d; ++m) {
-            const int G = (int) groups[m - first].size();
-            Part &pt = parts[m - first];
-            pt.cnt = arena.take<int>((size_t) 6 * G);
-            pt.P = arena.take<int>(std::max(T.nP_max, 1));
-            pt.W = arena.take<int>(std::max(T.nP_max, 1));
-            pt.x = arena.take<int>(std::max(T.nsp_max, 1));
-            pt.mk = arena.take<uint64_t>((size_t) std::max(T.nsp_max, 1) * mw);
-            const Subspace &sub = subs[T.smask | dbit(m)];
-            HIP_OK(launch_partition(T.P, T.nP, T.nP_max, T.spx, T.spm, mw, T.nsp, T.nsp_max, cellC + (size_t) m * n,
-                                    d_gid + (size_t) (m - first) * cells, G, sub.cnt, weak_thr, 0, m, pt.cnt, pt.P,
-                                    pt.W, pt.x, pt.mk, st));
-        }
-        std::vector<size_t> cnt_at(nd);
-        size_t tot = 0;
-        for (int m = first; m < d; ++m) {
-            cnt_at[m - first] = tot;
-            tot += 3 * groups[m - first].size();
-        }
-        int *hostc = pin_i((size_t) nd * cells + 64);
-        for (int m = first; m < d; ++m)
-            HIP_OK(hipMemcpyAsync(hostc + cnt_at[m - first], parts[m - first].cnt,
-                                  3 * groups[m - first].size() * sizeof(int), hipMemcpyDeviceToHost, st));
-        sync();
-        std::vector<int> counts(hostc, hostc + tot);
-
-        for (int m = first; m < d; ++m) {
-            const dmask_t smask = T.smask | dbit(m);
-            const auto &gs = groups[m - first];
-            const int G = (int) gs.size();
-            const int *c3 = counts.data() + cnt_at[m - first];
-            const Part &pt = parts[m - first];
-            const size_t dim_mark = arena.mark();
-            uint8_t *lab = nullptr;
-            int offW = 0, offS = 0;
-            for (int g = 0; g < G; ++g) {
-                const int nPr = c3[g], nW = c3[G + g], nSP = c3[2 * G + g];
-                const int *W = pt.W + offW;
-                const int *spx = pt.x + offS;
-                const uint64_t *spm = pt.mk + (size_t) offS * mw;
-                offW += nW;
-                offS += nSP;
-                stats.trees++;
-                const bool pass = nW >= prm.min_size;
-                size_t at = trace.size();
-                if (trace_on) trace.push_back({(long long) dlo(smask), gs[g].lo, gs[g].hi, nPr, nW, pass ? 1 : 0, -1});
-                if (!pass) continue;
-                const size_t child_mark = arena.mark();
-                const int tid = ++tree_id;
-                // s-connection paths surviving the prune
-                int *spx2 = arena.take<int>(std::max(nSP, 1));
-                uint64_t *spm2 = arena.take<uint64_t>((size_t) std::max(nSP, 1) * mw);
-                int *nsp2 = arena.take<int>(1);
-                {
-                    size_t tmark = arena.mark();
-                    size_t slots = table_slots(nW, d - 1 - m);
-                    uint64_t *table = arena.take<uint64_t>(nSP > 0 ? slots : 1);
-                    HIP_OK(launch_path_prune(D, smask, W, pt.cnt + G + g, nW, spx, spm, mw, pt.cnt + 2 * G + g, nSP,
-                                             stamp, tid, reinterpret_cast<dmask_t *>(small + 16), table,
-                                             (uint64_t) (slots - 1), spx2, spm2, nsp2, st));
-                    arena.release(tmark);  // stream order keeps the table alive for the queued kernels
-                }
-                // components of S now: the children's counts are bounded by them
-                Subspace &sub = ensure_components(smask);
-                TreeRef child{smask, W, pt.cnt + G + g, nW, spx2, spm2, nsp2, nSP};
-                recurse(child, m + 1);
-                // pruneRedundancy then cluster, on the device in stream order
-                const int *nW_dev = pt.cnt + G + g;
-                if (!lab) {
-                    arena.release(child_mark);
-                    lab = arena.take<uint8_t>(n);  // survives until this dimension's join
-                    HIP_OK(launch_fill_u8(lab, 0, n, st));
-                    HIP_OK(launch_redundancy_seed(W, nW_dev, nW, stamp, ++tree_id, entries, d_nE, smask, sub.comp,
-                                                  d_list, d_nlist, d_mn, prm.r, d_keep, lab, st));
-                } else {
-                    HIP_OK(launch_redundancy_seed(W, nW_dev, nW, stamp, ++tree_id, entries, d_nE, smask, sub.comp,
-                                                  d_list, d_nlist, d_mn, prm.r, d_keep, lab, st));
-                    arena.release(child_mark);
-                }
-                if (trace_on) {
-                    HIP_OK(hipMemcpyAsync(pin, d_keep, sizeof(int), hipMemcpyDeviceToHost, st));
-                    sync();
-                    trace[at].redundant = pin_i()[0] ? 0 : 1;
-                }
-            }
-            if (lab) join(smask, lab);
-            arena.release(dim_mark);
-        }
-        arena.release(lvl_mark);
-    }
 
     // join (util.cu:655-743), on the device
     void join(dmask_t smask, const uint8_t *lab) {

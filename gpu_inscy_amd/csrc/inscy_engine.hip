@@ -120,9 +120,11 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.max_batch_override = g_max_batch;
             eng.profile_on = g_profile_on;
             eng.mem_share = mem_share;
-            // phi density (rectangular = false) is implemented in the
-            // level-synchronous driver only; it serves every mode
-            eng.levels_mode = (mode != INSCY_MODE_EXACT || p->rectangular == 0) && p->entropy_order == 0;
+            // one driver serves every mode of the identity order: the
+            // level-synchronous one gives the depth-first recursion's result,
+            // trees and decisions in a fraction of its launches (n=4,999 d=11:
+            // 12,556 dispatches and 58 ms one tree at a time, 240 and 3.9 ms)
+            eng.levels_mode = p->entropy_order == 0;
             eng.collect = mode == INSCY_MODE_COLLECT;
             if (mode == INSCY_MODE_LEARNED) {
                 eng.pruner = pruner_on_device(eng.prune_thr, eng.prune_min_depth);
@@ -131,10 +133,8 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.setup(d_X);
             if (p->entropy_order != 0)
                 eng.run_perm(*res);
-            else if (eng.levels_mode)
-                eng.run_levels(*res);
             else
-                eng.run(*res);
+                eng.run_levels(*res);
             res->stats = eng.stats;
             if (g_trace_on) g_trace = eng.trace;
         }

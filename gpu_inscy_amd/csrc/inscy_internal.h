@@ -292,16 +292,8 @@ hipError_t launch_subspace_components(const DevData &D, const SubspaceArg &S, co
                                       int *cnt, int *comp, int *csize, unsigned long long *stat,
                                       const KernelTimer &tm, hipStream_t st);
 hipError_t launch_mark(const int *P, const int *nP, int nP_max, int *mark, int markid, hipStream_t st);
-hipError_t launch_flags_all(const int *spx, const uint64_t *spm, int mw, const int *nsp, int nsp_max,
-                            const uint8_t *cellC, int n, int first, int cells, int *flags, hipStream_t st);
-hipError_t launch_partition(const int *P, const int *nP, int nP_max, const int *spx, const uint64_t *spm, int mw,
-                            const int *nsp, int nsp_max, const uint8_t *cellC_m, const int *gid, int G,
-                            const int *weakcnt, int thr, int wbit, int m, int *cnt, int *outP, int *outW, int *outx,
-                            uint64_t *outm, hipStream_t st);
-hipError_t launch_path_prune(const DevData &D, dmask_t smask, const int *W, const int *nW, int nW_max,
-                             const int *spx, const uint64_t *spm, int mw, const int *nsp, int nsp_max, int *stamp,
-                             int tid, dmask_t *bits, uint64_t *table, uint64_t tmask, int *outx, uint64_t *outm,
-                             int *nout, hipStream_t st);
+hipError_t launch_partition(const int *P, const int *nP, int nP_max, const uint8_t *cellC_m, const int *gid, int G,
+                            const int *weakcnt, int thr, int wbit, int *cnt, int *outP, int *outW, hipStream_t st);
 hipError_t launch_redundancy_seed(const int *W, const int *nW_dev, int nW, int *stamp, int tid, const Entry *E,
                                   const int *nE, dmask_t smask, const int *comp, int *list, int *nlist, int *mn,
                                   float r, int *keep, uint8_t *lab, hipStream_t st);

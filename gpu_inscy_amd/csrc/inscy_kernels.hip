@@ -96,70 +96,38 @@ __global__ void k_histc(const uint8_t *__restrict__ cellC, int n, int d, int cel
     atomicAdd(&hist[(size_t) k * cells + cellC[i]], 1);
 }
 
-// ------------------------------------------------------------ expansion of one tree
-// mergeWithNeighbors decision input (ScyTreeNode.cu:837-851 with the flag of
-// restrict_node :262-267): cell c of dimension b is s-connected iff a path
-// branching at b starts from a point in cell c.  One pass sets the flags of
-// every dimension b >= first.
-__global__ void k_flags_all(const int *__restrict__ spx, const uint64_t *__restrict__ spm, int mw,
-                            const int *__restrict__ nsp, const uint8_t *__restrict__ cellC, int n, int first,
-                            int cells, int *__restrict__ flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nsp) return;
-    int x = spx[i];
-    dmask_t m = mload(spm, i, mw) & dabove(first - 1);
-    while (m) {
-        const int b = dfirst(m);
-        m &= m - 1;
-        flags[(b - first) * cells + cellC[(size_t) b * n + x]] = 1;
-    }
-}
-
-// Counting-sort partition of a tree's points, weak-dense points and paths by
-// the cell group of dimension m (restrict + mergeWithNeighbors for every
-// group at once).  cnt[0..G): points, [G..2G): weak-dense points, [2G..3G):
-// paths that branch above m; [3G..6G): scatter cursors.
+// ------------------------------------------------------------ expansion of one tree (permuted level order)
+// Counting-sort partition of a tree's points and weak-dense points by the cell
+// group of dimension m (restrict + mergeWithNeighbors for every group at once).
+// cnt[0..G): points, [G..2G): weak-dense points; [2G..4G): scatter cursors.
 struct PartArg {
     const int *P;
     const int *nP;
-    const int *spx;
-    const uint64_t *spm;  // mw words per path
-    const int *nsp;
     const uint8_t *cellC_m;
     const int *gid;      // [cells] group of each cell of m
     const int *weakcnt;  // neighbour counts (or phi decision bits) of the subspace S ∪ {m}
-    int thr, m, G;
-    int nP_blocks, mw, wbit;
+    int thr, G, wbit;
 };
 
 __global__ void k_part_count(PartArg A, int *__restrict__ cnt) {
-    __shared__ int h[3 * 256];
-    for (int t = threadIdx.x; t < 3 * A.G; t += blockDim.x) h[t] = 0;
+    __shared__ int h[2 * 256];
+    for (int t = threadIdx.x; t < 2 * A.G; t += blockDim.x) h[t] = 0;
     __syncthreads();
-    if ((int) blockIdx.x < A.nP_blocks) {
-        int i = blockIdx.x * blockDim.x + threadIdx.x;
-        if (i < *A.nP) {
-            int p = A.P[i];
-            int g = A.gid[A.cellC_m[p]];
-            atomicAdd(&h[g], 1);
-            if (meets(A.weakcnt[p], A.thr, A.wbit)) atomicAdd(&h[A.G + g], 1);
-        }
-    } else {
-        int i = (blockIdx.x - A.nP_blocks) * blockDim.x + threadIdx.x;
-        if (i < *A.nsp) {
-            const dmask_t mk = mload(A.spm, i, A.mw) & dabove(A.m);
-            if (mk) atomicAdd(&h[2 * A.G + A.gid[A.cellC_m[A.spx[i]]]], 1);
-        }
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < *A.nP) {
+        int p = A.P[i];
+        int g = A.gid[A.cellC_m[p]];
+        atomicAdd(&h[g], 1);
+        if (meets(A.weakcnt[p], A.thr, A.wbit)) atomicAdd(&h[A.G + g], 1);
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < 3 * A.G; t += blockDim.x)
+    for (int t = threadIdx.x; t < 2 * A.G; t += blockDim.x)
         if (h[t]) atomicAdd(&cnt[t], h[t]);
 }
 
-__global__ void k_part_scatter(PartArg A, int *__restrict__ cnt, int *__restrict__ outP, int *__restrict__ outW,
-                               int *__restrict__ outx, uint64_t *__restrict__ outm) {
-    __shared__ int base[3 * 256];
-    if (threadIdx.x < 3) {
+__global__ void k_part_scatter(PartArg A, int *__restrict__ cnt, int *__restrict__ outP, int *__restrict__ outW) {
+    __shared__ int base[2 * 256];
+    if (threadIdx.x < 2) {
         int acc = 0;
         for (int g = 0; g < A.G; ++g) {
             base[threadIdx.x * A.G + g] = acc;
@@ -167,33 +135,16 @@ __global__ void k_part_scatter(PartArg A, int *__restrict__ cnt, int *__restrict
         }
     }
     __syncthreads();
-    int *cur = cnt + 3 * A.G;
-    if ((int) blockIdx.x < A.nP_blocks) {
-        int i = blockIdx.x * blockDim.x + threadIdx.x;
-        bool in = i < *A.nP;
-        int p = in ? A.P[i] : 0;
-        int g = in ? A.gid[A.cellC_m[p]] : 0;
-        bool weak = in && meets(A.weakcnt[p], A.thr, A.wbit);
-        int sp = wave_add_by_key(cur, g, in);
-        int sw = wave_add_by_key(cur + A.G, g, weak);
-        if (in) outP[base[g] + sp] = p;
-        if (weak) outW[base[A.G + g] + sw] = p;
-    } else {
-        int i = (blockIdx.x - A.nP_blocks) * blockDim.x + threadIdx.x;
-        dmask_t mk = 0;
-        int x = 0, g = 0;
-        if (i < *A.nsp) {
-            mk = mload(A.spm, i, A.mw) & dabove(A.m);
-            x = A.spx[i];
-            g = A.gid[A.cellC_m[x]];
-        }
-        int sx = wave_add_by_key(cur + 2 * A.G, g, mk != 0);
-        if (mk) {
-            int pos = base[2 * A.G + g] + sx;
-            outx[pos] = x;
-            mstore(outm, pos, mk, A.mw);
-        }
-    }
+    int *cur = cnt + 2 * A.G;
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    bool in = i < *A.nP;
+    int p = in ? A.P[i] : 0;
+    int g = in ? A.gid[A.cellC_m[p]] : 0;
+    bool weak = in && meets(A.weakcnt[p], A.thr, A.wbit);
+    int sp = wave_add_by_key(cur, g, in);
+    int sw = wave_add_by_key(cur + A.G, g, weak);
+    if (in) outP[base[g] + sp] = p;
+    if (weak) outW[base[A.G + g] + sw] = p;
 }
 
 // ------------------------------------------------------------ epsilon neighbourhood: subspace grid pass
@@ -496,105 +447,9 @@ __global__ void k_uf_flatten(int *__restrict__ par, int n, int *__restrict__ com
     if (i < n) comp[i] = c;
 }
 
-// ------------------------------------------------------------ s-connection paths after the prune
-// A path (b, x) survives the prune of tree R iff some surviving point w shares
-// x's cells on every unrestricted dimension <= b.  (propergate_count2,
-// ScyTreeNode.cu:446-467, erases the s-connection whose same-cell regular
-// sibling lost all its points; the regular node a path hangs from keeps a
-// point whenever that sibling does.)  Membership is answered by an
-// open-addressing table of 64-bit entries (32 hash bits | representative point
-// id); every hash match is confirmed by comparing the cells themselves, so the
-// test is exact.
-
-
 __global__ void k_stamp(const int *__restrict__ W, const int *__restrict__ nW, int *__restrict__ stamp, int tid) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < *nW) stamp[W[i]] = tid;
-}
-
-__global__ void k_path_bits(const int *__restrict__ spx, const uint64_t *__restrict__ spm, int mw,
-                            const int *__restrict__ nsp, const int *__restrict__ stamp, int tid,
-                            dmask_t *__restrict__ bits) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    dmask_t m = 0;
-    if (i < *nsp && stamp[spx[i]] != tid) m = mload(spm, i, mw);
-    wave_or_mask(m, bits);
-}
-
-__global__ void k_path_insert(DevData D, dmask_t smask, const int *__restrict__ W, const int *__restrict__ nW,
-                              const dmask_t *__restrict__ bits, uint64_t *__restrict__ table, uint64_t tmask) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nW) return;
-    const dmask_t need = *bits;
-    if (!need) return;
-    int w = W[i];
-    uint64_t h = 0x243F6A8885A308D3ull;
-    CellRow row{};
-    for (int t = 0; t < D.d; ++t) {
-        const int k = t;
-        if (!(t & 15)) row = load_row(D, w, t);
-        if (dhas(smask, k)) continue;
-        h = mix64(h + row.at(t & 15) + 1);
-        if (!dhas(need, k)) continue;
-        uint64_t e = mix64(h ^ (0x9E3779B97F4A7C15ull * (uint64_t) (k + 1)));
-        uint64_t entry = (e & 0xFFFFFFFF00000000ull) | (uint32_t) w;
-        uint64_t slot = e & tmask;
-        while (true) {
-            // a slot is written once, by the swap from empty: a plain load that
-            // still sees it empty is corrected by the failed swap, a full one is final
-            uint64_t cur = table[slot];
-            if (cur == kEmpty) {
-                cur = atomicCAS((unsigned long long *) &table[slot], (unsigned long long) kEmpty,
-                                (unsigned long long) entry);
-                if (cur == kEmpty) break;
-            }
-            if ((cur >> 32) == (entry >> 32) && same_prefix(D, smask, w, (int) (uint32_t) cur, t)) break;
-            slot = (slot + 1) & tmask;
-        }
-    }
-}
-
-__global__ void k_path_check(DevData D, dmask_t smask, const int *__restrict__ spx, const uint64_t *__restrict__ spm,
-                             int mw,
-                             const int *__restrict__ nsp, const int *__restrict__ stamp, int tid,
-                             const uint64_t *__restrict__ table, uint64_t tmask, int *__restrict__ outx,
-                             uint64_t *__restrict__ outm, int *__restrict__ nout) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int x = 0;
-    dmask_t m = 0;
-    if (i < *nsp) {
-        x = spx[i];
-        m = mload(spm, i, mw);
-        if (stamp[x] != tid) {
-            uint64_t h = 0x243F6A8885A308D3ull;
-            dmask_t keep = 0;
-            CellRow row{};
-            for (int t = 0; t < D.d; ++t) {
-                const int k = t;
-                if (!(t & 15)) row = load_row(D, x, t);
-                if (dhas(smask, k)) continue;
-                h = mix64(h + row.at(t & 15) + 1);
-                if (!dhas(m, k)) continue;
-                uint64_t e = mix64(h ^ (0x9E3779B97F4A7C15ull * (uint64_t) (k + 1)));
-                uint64_t slot = e & tmask;
-                while (true) {
-                    uint64_t cur = table[slot];  // complete: the inserts ran in an earlier launch
-                    if (cur == kEmpty) break;
-                    if ((cur >> 32) == (e >> 32) && same_prefix(D, smask, x, (int) (uint32_t) cur, t)) {
-                        keep |= dbit(k);
-                        break;
-                    }
-                    slot = (slot + 1) & tmask;
-                }
-            }
-            m = keep;
-        }
-    }
-    int slot = wave_slot(m != 0, nout);
-    if (m != 0) {
-        outx[slot] = x;
-        mstore(outm, slot, m, mw);
-    }
 }
 
 // ------------------------------------------------------------ redundancy and join on the device
@@ -913,42 +768,14 @@ hipError_t launch_mark(const int *P, const int *nP, int nP_max, int *mark, int m
     return hipGetLastError();
 }
 
-hipError_t launch_flags_all(const int *spx, const uint64_t *spm, int mw, const int *nsp, int nsp_max,
-                            const uint8_t *cellC, int n, int first, int cells, int *flags, hipStream_t st) {
-    if (nsp_max <= 0) return hipSuccess;
-    LAUNCH(k_flags_all, dim3(blocks_for(nsp_max)), dim3(kBlock), 0, st, spx, spm, mw, nsp, cellC, n, first, cells,
-           flags);
-    return hipGetLastError();
-}
-
-hipError_t launch_partition(const int *P, const int *nP, int nP_max, const int *spx, const uint64_t *spm, int mw,
-                            const int *nsp, int nsp_max, const uint8_t *cellC_m, const int *gid, int G,
-                            const int *weakcnt, int thr, int wbit, int m, int *cnt, int *outP, int *outW, int *outx,
-                            uint64_t *outm, hipStream_t st) {
-    int bp = (int) blocks_for(nP_max), bs = (int) blocks_for(nsp_max);
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 6 * G, sizeof(int))), dim3(kBlock), 0, st, cnt, 0, (size_t) 6 * G);
-    if (bp + bs == 0) return hipGetLastError();
-    PartArg A{P, nP, spx, spm, nsp, cellC_m, gid, weakcnt, thr, m, G, bp, mw, wbit};
-    LAUNCH(k_part_count, dim3(bp + bs), dim3(kBlock), 0, st, A, cnt);
-    LAUNCH(k_part_scatter, dim3(bp + bs), dim3(kBlock), 0, st, A, cnt, outP, outW, outx, outm);
-    return hipGetLastError();
-}
-
-hipError_t launch_path_prune(const DevData &D, dmask_t smask, const int *W, const int *nW, int nW_max,
-                             const int *spx, const uint64_t *spm, int mw, const int *nsp, int nsp_max, int *stamp,
-                             int tid, dmask_t *bits, uint64_t *table, uint64_t tmask, int *outx, uint64_t *outm,
-                             int *nout, hipStream_t st) {
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 1, sizeof(int))), dim3(kBlock), 0, st, nout, 0, (size_t) 1);
-    if (nsp_max <= 0) return hipGetLastError();
-    LAUNCH(k_fill<uint64_t>, dim3(fill_blocks((size_t) (tmask + 1), sizeof(uint64_t))), dim3(kBlock), 0, st, table, kEmpty, (size_t) (tmask + 1));
-    LAUNCH(k_fill<uint64_t>, dim3(fill_blocks((size_t) 2, sizeof(uint64_t))), dim3(kBlock), 0, st,
-           reinterpret_cast<uint64_t *>(bits), (uint64_t) 0, (size_t) 2);
-    if (nW_max > 0) LAUNCH(k_stamp, dim3(blocks_for(nW_max)), dim3(kBlock), 0, st, W, nW, stamp, tid);
-    LAUNCH(k_path_bits, dim3(blocks_for(nsp_max)), dim3(kBlock), 0, st, spx, spm, mw, nsp, stamp, tid, bits);
-    if (nW_max > 0)
-        LAUNCH(k_path_insert, dim3(blocks_for(nW_max)), dim3(kBlock), 0, st, D, smask, W, nW, bits, table, tmask);
-    LAUNCH(k_path_check, dim3(blocks_for(nsp_max)), dim3(kBlock), 0, st, D, smask, spx, spm, mw, nsp, stamp, tid,
-           table, tmask, outx, outm, nout);
+hipError_t launch_partition(const int *P, const int *nP, int nP_max, const uint8_t *cellC_m, const int *gid, int G,
+                            const int *weakcnt, int thr, int wbit, int *cnt, int *outP, int *outW, hipStream_t st) {
+    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 4 * G, sizeof(int))), dim3(kBlock), 0, st, cnt, 0, (size_t) 4 * G);
+    if (nP_max <= 0) return hipGetLastError();
+    const unsigned bp = blocks_for(nP_max);
+    PartArg A{P, nP, cellC_m, gid, weakcnt, thr, G, wbit};
+    LAUNCH(k_part_count, dim3(bp), dim3(kBlock), 0, st, A, cnt);
+    LAUNCH(k_part_scatter, dim3(bp), dim3(kBlock), 0, st, A, cnt, outP, outW);
     return hipGetLastError();
 }
 

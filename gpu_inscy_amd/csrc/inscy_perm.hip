@@ -263,7 +263,7 @@ void Engine::run_perm(inscy_result &out) {
     HIP_OK(hipMemcpyAsync(pin, nch, sizeof(int), hipMemcpyDeviceToHost, st));
     sync();
     const int nch_h = pin_i()[0];
-    TreeRef root{(dmask_t) 0, P, nP, n, cx, nullptr, nch, nch_h, cm};
+    TreeRef root{(dmask_t) 0, P, nP, n, cx, cm, nch, nch_h};
     auto t0 = std::chrono::steady_clock::now();
     recurse_perm(root, 0);
     sync();
@@ -310,13 +310,12 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
         const auto &gs = groups[m - first];
         const int G = (int) gs.size();
         const size_t dim_mark = arena.mark();
-        int *cnt = arena.take<int>((size_t) 6 * G);
+        int *cnt = arena.take<int>((size_t) 4 * G);
         int *PP = arena.take<int>(std::max(T.nP_max, 1));
         int *PW = arena.take<int>(std::max(T.nP_max, 1));
         const Subspace &sub = subs[smask];
-        HIP_OK(launch_partition(T.P, T.nP, T.nP_max, nullptr, nullptr, mw, nullptr, 0, cellC + (size_t) m * n,
-                                d_gid + (size_t) (m - first) * cells, G, sub.cnt, weak_thr, phi_mode ? 1 : 0, m, cnt, PP,
-                                PW, nullptr, nullptr, st));
+        HIP_OK(launch_partition(T.P, T.nP, T.nP_max, cellC + (size_t) m * n, d_gid + (size_t) (m - first) * cells, G,
+                                sub.cnt, weak_thr, phi_mode ? 1 : 0, cnt, PP, PW, st));
         HIP_OK(hipMemcpyAsync(pin, cnt, (size_t) 2 * G * sizeof(int), hipMemcpyDeviceToHost, st));
         sync();
         std::vector<int> c2(pin_i(), pin_i() + 2 * G);
@@ -435,7 +434,7 @@ void Engine::recurse_perm(const TreeRef &T, int first) {
                 HIP_OK(hipGetLastError());
             }
             Subspace &s2 = ensure_components(smask);
-            TreeRef child{smask, Wg, nWg, nW, cx2, nullptr, nc2, T.nsp_max, cm2};
+            TreeRef child{smask, Wg, nWg, nW, cx2, cm2, nc2, T.nsp_max};
             recurse_perm(child, m + 1);
             // pruneRedundancy then cluster, on the device in stream order
             if (!lab) {

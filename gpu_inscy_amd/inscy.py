@@ -12,7 +12,7 @@ marks are noise).
 
 Mapping of the reference's entry points:
   CPU (python/inscy.py:121-125)          -> exact mode (same results, on the GPU)
-  GPU (:189-192, run_gpu_4)              -> exact mode, one restricted tree at a time
+  GPU (:189-192, run_gpu_4)              -> exact mode (the same driver as batched mode)
   GPU5 (:194-197, run_gpu_5)             -> batched mode (same results)
   GPU3, GPU_star, GPU_memory, GPU_memory2 (:183-214) -> batched mode
   run_cpu, run_cpu_weak, run_gpu, run_gpu_* (7-argument ops, :110-186) -> exact

@@ -37,7 +37,7 @@ extern "C" {
 #define INSCY_ERR_UNSUPPORTED 4 /* a parameter combination this build does not implement */
 
 /* Engine modes. */
-#define INSCY_MODE_EXACT 1   /* one restricted tree at a time (reference GPU / GPU4 role) */
+#define INSCY_MODE_EXACT 1   /* the reference's GPU / GPU4 role: the driver and results of INSCY_MODE_BATCHED */
 #define INSCY_MODE_BATCHED 2 /* level-batched exact mode (reference GPU5 role); same results */
 #define INSCY_MODE_LEARNED 3 /* level-batched with the learned pruner (inscy_set_pruner): approximate */
 #define INSCY_MODE_COLLECT 4 /* level-batched exact, and records the pruner's training pairs (inscy_result_pairs) */
@@ -72,8 +72,8 @@ typedef struct inscy_stats {
     int64_t count_bytes;    /* its algorithmic bytes: per counted point 4k+4, per neighbour found 4+4k */
     /* wall time of the phases of the run (seconds): growing the restricted
      * trees (restrict, prunes, counts, dense components), the replay of
-     * pruneRedundancy and join (level-synchronous mode; inside the first
-     * phase in exact mode), and reading the result back */
+     * pruneRedundancy and join (inside the first phase with a permuted level
+     * order), and reading the result back */
     double expand_seconds;
     double replay_seconds;
     double emit_seconds;
