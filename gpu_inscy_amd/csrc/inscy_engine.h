@@ -298,8 +298,10 @@ public:
         HIP_OK(dev_alloc(&nearm, (size_t) n * sizeof(dmask_t)));
         HIP_OK(dev_alloc(&rows, (size_t) n * cell_row_bytes(d)));
         HIP_OK(dev_alloc(&small, kSmallWords * sizeof(unsigned long long)));
-        HIP_OK(dev_alloc(&stamp, (size_t) n * sizeof(int)));
-        HIP_OK(dev_alloc(&qmark, (size_t) n * sizeof(int)));
+        if (!levels_mode) {
+            HIP_OK(dev_alloc(&stamp, (size_t) n * sizeof(int)));
+            HIP_OK(dev_alloc(&qmark, (size_t) n * sizeof(int)));
+        }
         HIP_OK(host_alloc(&pin, pin_bytes()));
         grow_entries(1 << 12);
         // grid index size: C^j cells with j <= 3 and C^j <= max(8n, 4096)
@@ -319,18 +321,24 @@ public:
         arena.init(want);
 
         int *hist = arena.take<int>((size_t) d * ecells);
-        HIP_OK(launch_fill_i32(reinterpret_cast<int *>(small), 0, 2 * kSmallWords, st));
+        FillMany fill;
+        fill.add(small, 0, kSmallWords * sizeof(unsigned long long));
+        fill.add(hist, 0, (size_t) d * ecells * sizeof(int));
+        if (!levels_mode) {
+            fill.add(stamp, ~0u, (size_t) n * sizeof(int));
+            fill.add(qmark, ~0u, (size_t) n * sizeof(int));
+        }
+        HIP_OK(launch_fill_many(fill, st));
         HIP_OK(launch_discretise(d_X, n, d, cells, prm.neighborhood_size, Xt, cellC, cellE,
                                  prm.entropy_order == 0 ? rows : nullptr, reinterpret_cast<uint64_t *>(nearm), 2, reinterpret_cast<int *>(small), st));
         HIP_OK(launch_hist1(cellE, n, d, ecells, hist, st));
         // c-grid occupancy: the input of the entropy order only
         int *histc = arena.take<int>((size_t) d * cells);
         if (prm.entropy_order != 0) HIP_OK(launch_histc(cellC, n, d, cells, histc, st));
-        HIP_OK(launch_fill_i32(stamp, -1, n, st));
-        HIP_OK(launch_fill_i32(qmark, -1, n, st));
-        std::vector<int> h((size_t) d * ecells), hc((size_t) d * cells);
+        std::vector<int> hc((size_t) d * cells);
+        const int *h = reinterpret_cast<const int *>(down.get((size_t) d * ecells * sizeof(int)));
         HIP_OK(hipMemcpyAsync(pin, small, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipMemcpyAsync(h.data(), hist, h.size() * sizeof(int), hipMemcpyDeviceToHost, st));
+        HIP_OK(hipMemcpyAsync(down.p, hist, (size_t) d * ecells * sizeof(int), hipMemcpyDeviceToHost, st));
         if (prm.entropy_order != 0)
             HIP_OK(hipMemcpyAsync(hc.data(), histc, hc.size() * sizeof(int), hipMemcpyDeviceToHost, st));
         sync();
@@ -340,7 +348,7 @@ public:
         // query in the three-cell slab, sum_c h_c (h_{c-1} + h_c + h_{c+1})
         score.assign(d, 0.0);
         for (int k = 0; k < d; ++k) {
-            const int *hk = h.data() + (size_t) k * ecells;
+            const int *hk = h + (size_t) k * ecells;
             for (int c = 0; c < ecells; ++c) {
                 double nb = hk[c] + (c > 0 ? hk[c - 1] : 0) + (c + 1 < ecells ? hk[c + 1] : 0);
                 score[k] += (double) hk[c] * nb;
@@ -368,12 +376,14 @@ public:
         }
         lvl_of.assign(d, 0);
         for (int t = 0; t < d; ++t) lvl_of[level[t]] = t;
-        HIP_OK(dev_alloc(&d_level, (size_t) 2 * d * sizeof(int)));
-        std::vector<int> both(level);
-        both.insert(both.end(), lvl_of.begin(), lvl_of.end());
-        HIP_OK(hipMemcpyAsync(d_level, both.data(), both.size() * sizeof(int), hipMemcpyHostToDevice, st));
-        if (prm.entropy_order != 0) HIP_OK(launch_cell_rows(cellC, n, d, d_level, rows, st));
-        sync();  // `both` is pageable and goes out of scope
+        if (!levels_mode) {  // the level-synchronous driver knows its order: the identity
+            HIP_OK(dev_alloc(&d_level, (size_t) 2 * d * sizeof(int)));
+            std::vector<int> both(level);
+            both.insert(both.end(), lvl_of.begin(), lvl_of.end());
+            HIP_OK(hipMemcpyAsync(d_level, both.data(), both.size() * sizeof(int), hipMemcpyHostToDevice, st));
+            if (prm.entropy_order != 0) HIP_OK(launch_cell_rows(cellC, n, d, d_level, rows, st));
+            sync();  // `both` is pageable and goes out of scope
+        }
         if (phi_mode) {
             // leaf order of the neighbourhood tree, whose levels follow the same order
             HIP_OK(dev_alloc(&rank_perm, (size_t) n * sizeof(int)));
@@ -386,7 +396,7 @@ public:
             sync();
         }
         arena.release(0);
-        D = DevData{d_X, Xt, cellC, cellE, rows, d_level, d_level + d, n, d, cells, ecells, cell_row_bytes(d)};
+        D = DevData{d_X, Xt, cellC, cellE, rows, d_level, d_level ? d_level + d : nullptr, n, d, cells, ecells, cell_row_bytes(d)};
     }
 
     // ---------------------------------------------------------- run
@@ -436,7 +446,7 @@ public:
 
 private:
     // ---------------------------------------------------------- helpers
-    // `small` device words: [0] input check flag, [16..24) path-prune scratch,
+    // `small` device words (zeroed by the set-up): [0] input check flag, [1] the root's paths,
     // [kStatAt..) 64 slot pairs (16 words apart) of neighbour-count statistics
     static constexpr int kStatAt = 32;
     static constexpr int kSmallWords = kStatAt + 16 * 64;
@@ -503,6 +513,7 @@ private:
         keepf = reinterpret_cast<uint8_t *>(scratch + 8 + 2 * cap);
         dropf = keepf + n;
         freshf = dropf + n;
+        if (levels_mode) return;  // the scratch serves the permuted-order driver
         HIP_OK(launch_fill_i32(d_mn, INT_MAX, cap, st));
         HIP_OK(launch_fill_i32(d_nE, nentries, 1, st));
     }
@@ -696,9 +707,16 @@ private:
     // in chunks of rows straight into the result's contiguous label array.
     void emit(inscy_result &out) {
         out.n = n;
+        const size_t tab_bytes = ((size_t) nentries * sizeof(Entry) + 255) & ~(size_t) 255;
+        const size_t stat_bytes = 16 * 64 * sizeof(unsigned long long);
+        char *hb = down.get(tab_bytes + stat_bytes);
+        if (nentries)
+            HIP_OK(hipMemcpyAsync(hb, entries, (size_t) nentries * sizeof(Entry), hipMemcpyDeviceToHost, st));
+        // (no pass after this one counts into the statistics)
+        HIP_OK(hipMemcpyAsync(hb + tab_bytes, small + kStatAt, stat_bytes, hipMemcpyDeviceToHost, st));
         sync();
-        std::vector<Entry> tab(nentries);
-        if (nentries) HIP_OK(hipMemcpy(tab.data(), entries, (size_t) nentries * sizeof(Entry), hipMemcpyDeviceToHost));
+        const Entry *tab = reinterpret_cast<const Entry *>(hb);
+        const unsigned long long *h2 = reinterpret_cast<const unsigned long long *>(hb + tab_bytes);
         std::vector<int> rows;
         for (int e = 0; e < nentries; ++e)
             if (tab[e].nkept > 0) rows.push_back(e);
@@ -726,13 +744,12 @@ private:
             const size_t items = (size_t) R * n + 1;
             int *flags = batch.take<int>(items);
             int *idx = batch.take<int>(items);
-            char *lab = batch.take<char>((size_t) R * n * width);
-            int *cnts = batch.take<int>(R);
             const size_t sb = scan_temp_bytes((int) items);
             void *tmp = batch.take<char>(sb);
             // the row counts follow the labels at a 256-byte boundary
             auto cnt_at = [&](int r) { return ((size_t) r * n * width + 255) & ~(size_t) 255; };
             const size_t stage_bytes = cnt_at(R) + (size_t) R * sizeof(int);
+            char *lab = batch.take<char>(stage_bytes);
             char *stage[2] = {emit_stage[0].get(stage_bytes), emit_stage[1].get(stage_bytes)};
             hipEvent_t done[2];
             HIP_OK(event_pool().get(&done[0]));
@@ -780,10 +797,10 @@ private:
                 std::vector<EmitRow> er(r);
                 for (int t = 0; t < r; ++t) er[t] = EmitRow{tab[rows[c0 + t]].comp, tab[rows[c0 + t]].inres};
                 EmitRow *der = upload(batch, er);
-                HIP_OK(launch_emit(der, r, n, flags, idx, lab, width, cnts, tmp, sb, st));
-                HIP_OK(hipMemcpyAsync(stage[buf], lab, (size_t) r * n * width, hipMemcpyDeviceToHost, st));
-                HIP_OK(hipMemcpyAsync(stage[buf] + cnt_at(r), cnts, (size_t) r * sizeof(int),
-                                      hipMemcpyDeviceToHost, st));
+                HIP_OK(launch_emit(der, r, n, flags, idx, lab, width, reinterpret_cast<int *>(lab + cnt_at(r)), tmp,
+                                   sb, st));
+                HIP_OK(hipMemcpyAsync(stage[buf], lab, cnt_at(r) + (size_t) r * sizeof(int), hipMemcpyDeviceToHost,
+                                      st));
                 HIP_OK(hipEventRecord(done[buf], st));
                 if (prev_c0 >= 0) {
                     HIP_OK(hipEventSynchronize(done[prev_buf]));
@@ -802,8 +819,6 @@ private:
             event_pool().put(done[1]);
         }
         stats.subspaces = (int64_t) m;
-        std::vector<unsigned long long> h2(16 * 64);
-        HIP_OK(hipMemcpy(h2.data(), small + kStatAt, h2.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
         for (int b = 0; b < 64; ++b) {
             stats.candidates += (int64_t) h2[16 * b];
             stats.queries += (int64_t) h2[16 * b + 1];

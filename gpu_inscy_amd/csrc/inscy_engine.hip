@@ -488,7 +488,8 @@ int inscy_debug_flag_compact(const uint8_t *flags, int64_t nb, void *temp, int64
     if (!flags || !temp || !out || !nsel || nb <= 0 || nb >= INT_MAX ||
         temp_bytes < inscy_debug_flag_compact_temp(nb))
         return fail(INSCY_ERR_ARGUMENT, "invalid argument");
-    hipError_t e = launch_flag_compact(flags, (size_t) nb, temp, (size_t) temp_bytes, out, nsel, (hipStream_t) stream);
+    hipError_t e = launch_flag_compact(flags, (size_t) nb, temp, (size_t) temp_bytes, out, nsel, 1, nullptr,
+                                       (hipStream_t) stream);
     return e == hipSuccess ? INSCY_OK : fail(INSCY_ERR_DEVICE, hipGetErrorString(e));
 }
 

@@ -169,7 +169,7 @@ struct BatchSub {
 
 // Device buffers of one batch.
 struct BatchIndex {
-    const float *edge;    // [C + 3] edges of the eps cells (k_cell_edges)
+    const float *edge;    // [C + 3] edges of the eps cells (cell_edge)
     uint8_t *qflag;       // [B*n] query flag per (global) sorted position
     int *qlist;           // global sorted positions of the queries, ascending
     int *nsel;            // [1] number of queries
@@ -243,6 +243,7 @@ struct PruneChild {
     int nW, nsp, bw, mw;
 };
 
+// pad < 0: dst[i] = src[i]; else dst[src[i]] = pad (the tree stamps of the replay)
 struct CopySeg {
     const int *src;
     int *dst;
@@ -264,9 +265,10 @@ hipError_t launch_sort_pairs_u16(const uint16_t *keys, uint16_t *keys_tmp, uint1
 size_t select_temp_bytes(int items);
 // positions of the nonzero bytes of flags[0, nb) in order into out, their
 // number into *nsel; flags readable up to nb rounded up to 16 bytes, temp of
-// select_temp_bytes(nb) bytes
+// select_temp_bytes(nb) bytes; qstart (may be null, nb a multiple of n):
+// qstart[b] = flags set before position b * n, b in [0, nb / n]
 hipError_t launch_flag_compact(const uint8_t *flags, size_t nb, void *temp, size_t temp_bytes, int *out, int *nsel,
-                               hipStream_t st);
+                               int n, int *qstart, hipStream_t st);
 
 // Launchers (all asynchronous on `st`; return the hipError_t of the launches).
 // discretise: the near-edge marks of point p are nw 64-bit words at nearw[p * nw]
@@ -276,6 +278,7 @@ hipError_t launch_discretise(const float *X, int n, int d, int cells, float eps,
                              uint16_t *cellE, uint8_t *rows, uint64_t *nearw, int nw, int *bad, hipStream_t st);
 // rows in `level` order (device array [d])
 hipError_t launch_cell_rows(const uint8_t *cellC, int n, int d, const int *level, uint8_t *rows, hipStream_t st);
+// (hist zeroed by the caller)
 hipError_t launch_hist1(const uint16_t *cellE, int n, int d, int ecells, int *hist, hipStream_t st);
 // occupancy of the c-grid per dimension ([d][cells]), the input of the entropy order
 hipError_t launch_histc(const uint8_t *cellC, int n, int d, int cells, int *hist, hipStream_t st);
@@ -313,12 +316,32 @@ hipError_t launch_emit(const EmitRow *rows, int r, int n, int *flags, int *idx, 
                        void *scan_temp, size_t scan_bytes, hipStream_t st);
 hipError_t launch_fill_u8(uint8_t *p, uint8_t v, size_t count, hipStream_t st);
 hipError_t launch_fill_i32(int *p, int v, size_t count, hipStream_t st);
+// several arrays filled with 32-bit words in one launch (16-byte aligned; add
+// returns the array)
+struct FillMany {
+    static constexpr int kMost = 8;
+    uint32_t *p[kMost];
+    size_t words[kMost];
+    uint32_t v[kMost];
+    int n = 0;
+    template <class T>
+    T *add(T *dst, uint32_t word, size_t bytes) {
+        if (bytes) {
+            p[n] = reinterpret_cast<uint32_t *>(dst);
+            words[n] = (bytes + 3) / 4;  // whole words: the arrays' allocations are rounded to 256 bytes
+            v[n++] = word;
+        }
+        return dst;
+    }
+};
+hipError_t launch_fill_many(const FillMany &f, hipStream_t st);
 hipError_t launch_gather(const int *src, const int *idx, int count, int *out, hipStream_t st);
 hipError_t launch_iota(int *p, int n, hipStream_t st);
-hipError_t launch_root_paths(const dmask_t *nearm, int n, int *outx, uint64_t *outm, int mw, int *nout, hipStream_t st);
 
-// edges of the C eps cells, C + 3 floats (see k_cell_edges)
-hipError_t launch_cell_edges(int C, float *edge, hipStream_t st);
+// the root tree: points 0..n, its s-connection paths (their number added to
+// *nout), and the edges of the C eps cells (C + 3 floats, see cell_edge)
+hipError_t launch_b_root(const dmask_t *nearm, int n, int *P, int *outx, uint64_t *outm, int mw, int *nout, int C,
+                         float *edge, hipStream_t st);
 // level-synchronous passes (blk_off: per-segment block offsets, nblk = blk_off[nseg])
 hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
                           int cells, int *flags, hipStream_t st);
@@ -327,7 +350,8 @@ hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nbl
 hipError_t launch_b_sort(const DevData &D, const SortJob *jobs, int njob, int hmiss, int max_cell, int *keys,
                          int *rank, int *hist, int *off, void *scan_temp, size_t scan_bytes, hipStream_t st);
 hipError_t launch_b_gather(const ColJob *jobs, int njob, int n, hipStream_t st);
-// queries in sorted order: flag the points of the segments, compact per subspace
+// queries in sorted order: flag the points of the segments (X.qflag zeroed by the
+// caller), compact per subspace
 hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySeg *segs, const int *blk_off,
                             int nseg, int nblk, const BatchIndex &X, hipStream_t st);
 // neighbour counts of the listed queries (blk_off over subspaces), or of every
@@ -387,9 +411,6 @@ size_t rank_order_temp_bytes(int n);
 hipError_t launch_b_prune(const DevData &D, const PruneChild *C, int nc, const int *blk_w, int nblk_w,
                           const int *blk_p, int nblk_p, hipStream_t st);
 hipError_t launch_b_copy(const CopySeg *segs, const int *blk_off, int nseg, int nblk, hipStream_t st);
-hipError_t launch_b_entries(Entry *E, int at, const Entry *src, int count, int *nE, hipStream_t st);
-// dst[src[i]] = pad for every segment (the tree stamps of the replay)
-hipError_t launch_b_stamp(const CopySeg *segs, const int *blk_off, int nseg, int nblk, hipStream_t st);
 // replay: pruneRedundancy of one tree (keepv[tree] = decision; rowflag: 2 *
 // nlist zeroed words and done: one zeroed word, both left zeroed by the
 // launch), join of one (parent, dimension) pair (added: one scratch word)

@@ -586,6 +586,7 @@ __global__ void k_emit_roots(const EmitRow *__restrict__ rows, int n, int *__res
     const EmitRow R = rows[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (i == 0 && blockIdx.y == 0) flags[(size_t) gridDim.y * n] = 0;  // the scan's last entry is the total
     flags[(size_t) blockIdx.y * n + i] = (R.comp[i] == i && R.inres[i]) ? 1 : 0;
 }
 
@@ -593,24 +594,37 @@ __global__ void k_emit_roots(const EmitRow *__restrict__ rows, int n, int *__res
 // rows whose labels fit (the host reads them back at a quarter or half the bytes)
 template <class T>
 __global__ void k_emit_labels(const EmitRow *__restrict__ rows, int n, const int *__restrict__ idx,
-                              T *__restrict__ labels) {
+                              T *__restrict__ labels, int *__restrict__ counts) {
     const EmitRow R = rows[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const size_t row = (size_t) blockIdx.y * n;
+    if (i == 0) counts[blockIdx.y] = idx[row + n] - idx[row];
     const int c = R.comp[i];
     const int v = (c >= 0 && R.inres[c]) ? idx[row + c] - idx[row] : -1;
     labels[row + i] = (T) (sizeof(T) == sizeof(int) ? v : v + 1);
 }
 
-__global__ void k_emit_counts(const int *__restrict__ idx, int n, int r, int *__restrict__ counts) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < r) counts[t] = idx[(size_t) (t + 1) * n] - idx[(size_t) t * n];
-}
-
 template <class T>
 __global__ void k_fill(T *p, T v, size_t count) {
     fill_span(p, v, count);
+}
+
+struct FillArgs {
+    FillMany f;
+    int blk[FillMany::kMost + 1];  // first block of each array
+};
+constexpr int kFillVecs = 8;  // 16-byte stores per thread
+__global__ __launch_bounds__(kBlock) void k_fill_many(FillArgs a) {
+    int s = 0;
+    while (s + 1 < a.f.n && (int) blockIdx.x >= a.blk[s + 1]) ++s;
+    const uint32_t v = a.f.v[s];
+    const size_t words = a.f.words[s], nvec = words / 4;
+    uint4 *q = reinterpret_cast<uint4 *>(a.f.p[s]);
+    const size_t step = (size_t) (a.blk[s + 1] - a.blk[s]) * kBlock;
+    const size_t t0 = (size_t) (blockIdx.x - a.blk[s]) * kBlock + threadIdx.x;
+    for (size_t j = t0; j < nvec; j += step) q[j] = make_uint4(v, v, v, v);
+    if (t0 < words - 4 * nvec) a.f.p[s][4 * nvec + t0] = v;
 }
 
 __global__ void k_gather(const int *__restrict__ src, const int *__restrict__ idx, int count, int *__restrict__ out) {
@@ -627,18 +641,6 @@ __global__ void k_rank_keys(const uint16_t *__restrict__ cellE, int n, int dim, 
                             uint16_t *__restrict__ keys) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) keys[i] = cellE[(size_t) dim * n + perm[i]];
-}
-
-// Root s-connection paths: every point with at least one near-edge dimension.
-__global__ void k_root_paths(const dmask_t *__restrict__ nearm, int n, int *__restrict__ outx,
-                             uint64_t *__restrict__ outm, int mw, int *__restrict__ nout) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const dmask_t m = i < n ? nearm[i] : (dmask_t) 0;
-    int slot = wave_slot(m != 0, nout);
-    if (m != 0) {
-        outx[slot] = i;
-        mstore(outm, slot, m, mw);
-    }
 }
 
 }  // namespace
@@ -684,7 +686,6 @@ hipError_t launch_discretise(const float *X, int n, int d, int cells, float eps,
 
 hipError_t launch_hist1(const uint16_t *cellE, int n, int d, int ecells, int *hist, hipStream_t st) {
     size_t nd = (size_t) n * d;
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) d * ecells, sizeof(int))), dim3(kBlock), 0, st, hist, 0, (size_t) d * ecells);
     LAUNCH(k_hist1, dim3(blocks_for(nd)), dim3(kBlock), 0, st, cellE, n, d, ecells, hist);
     return hipGetLastError();
 }
@@ -810,20 +811,18 @@ hipError_t launch_emit(const EmitRow *rows, int r, int n, int *flags, int *idx, 
                        void *scan_temp, size_t scan_bytes, hipStream_t st) {
     if (r <= 0) return hipSuccess;
     const size_t items = (size_t) r * n + 1;
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 1, sizeof(int))), dim3(kBlock), 0, st, flags + (size_t) r * n, 0, (size_t) 1);
     LAUNCH(k_emit_roots, dim3(blocks_for(n), r), dim3(kBlock), 0, st, rows, n, flags);
     hipError_t e = launch_exclusive_sum(scan_temp, scan_bytes, flags, idx, (int) items, st);
     if (e != hipSuccess) return e;
     if (width == 1)
         LAUNCH(k_emit_labels<uint8_t>, dim3(blocks_for(n), r), dim3(kBlock), 0, st, rows, n, idx,
-               static_cast<uint8_t *>(labels));
+               static_cast<uint8_t *>(labels), counts);
     else if (width == 2)
         LAUNCH(k_emit_labels<uint16_t>, dim3(blocks_for(n), r), dim3(kBlock), 0, st, rows, n, idx,
-               static_cast<uint16_t *>(labels));
+               static_cast<uint16_t *>(labels), counts);
     else
         LAUNCH(k_emit_labels<int>, dim3(blocks_for(n), r), dim3(kBlock), 0, st, rows, n, idx,
-               static_cast<int *>(labels));
-    LAUNCH(k_emit_counts, dim3(blocks_for(r)), dim3(kBlock), 0, st, idx, n, r, counts);
+               static_cast<int *>(labels), counts);
     return hipGetLastError();
 }
 
@@ -842,6 +841,18 @@ hipError_t launch_fill_u64(uint64_t *p, uint64_t v, size_t count, hipStream_t st
 hipError_t launch_fill_i32(int *p, int v, size_t count, hipStream_t st) {
     if (!count) return hipSuccess;
     LAUNCH(k_fill<int>, dim3(fill_blocks(count, sizeof(int))), dim3(kBlock), 0, st, p, v, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_fill_many(const FillMany &f, hipStream_t st) {
+    if (f.n <= 0) return hipSuccess;
+    FillArgs a{f, {}};
+    a.blk[0] = 0;
+    for (int s = 0; s < f.n; ++s) {
+        const size_t b = (f.words[s] / 4 + kBlock * kFillVecs - 1) / (kBlock * kFillVecs);
+        a.blk[s + 1] = a.blk[s] + (int) std::max<size_t>(1, std::min<size_t>(b, 4096));
+    }
+    LAUNCH(k_fill_many, dim3(a.blk[f.n]), dim3(kBlock), 0, st, a);
     return hipGetLastError();
 }
 
@@ -885,12 +896,6 @@ hipError_t launch_rank_order(const uint16_t *cellE, int n, int d, int ecells, co
         hipError_t e = hipMemcpyAsync(perm, a, (size_t) n * sizeof(int), hipMemcpyDeviceToDevice, st);
         if (e != hipSuccess) return e;
     }
-    return hipGetLastError();
-}
-
-hipError_t launch_root_paths(const dmask_t *nearm, int n, int *outx, uint64_t *outm, int mw, int *nout, hipStream_t st) {
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 1, sizeof(int))), dim3(kBlock), 0, st, nout, 0, (size_t) 1);
-    LAUNCH(k_root_paths, dim3(blocks_for(n)), dim3(kBlock), 0, st, nearm, n, outx, outm, mw, nout);
     return hipGetLastError();
 }
 

@@ -25,8 +25,8 @@ namespace inscy {
 
 namespace {
 constexpr size_t kMaxBatch = 1024;  // child subspaces per batch (inscy_set_tuning, INSCY_MAX_BATCH override)
-constexpr uint64_t kEmptySlot = ~0ull;  // free slot of a path-prune table
-// slots of a path prune's table for at most `levels` prefixes, at most half full
+// slots of a path prune's table (all bits set when free) for at most `levels`
+// prefixes, at most half full
 inline size_t path_slots(int levels) {
     size_t s = 64;
     while (s < 2 * (size_t) levels) s <<= 1;
@@ -48,15 +48,16 @@ void Engine::put(void *dst, const void *src, size_t bytes) {
     std::memcpy(up.p + up_top, src, bytes);
     if (up_defer) {
         // pool takes and staging places are both rounded to 256 bytes, so a
-        // contiguous pair extends the pending copy (padding bytes included:
-        // they lie inside the take)
-        if (pend_bytes && static_cast<char *>(dst) == pend_dst + pend_bytes && up_top == pend_src + pend_bytes) {
-            pend_bytes += need;
+        // contiguous pair extends the pending copy (over the padding between
+        // them, which lies inside the earlier take)
+        const size_t padded = (pend_bytes + 255) & ~(size_t) 255;
+        if (pend_bytes && static_cast<char *>(dst) == pend_dst + padded && up_top == pend_src + padded) {
+            pend_bytes = padded + bytes;
         } else {
             if (pend_bytes) HIP_OK(hipMemcpyAsync(pend_dst, up.p + pend_src, pend_bytes, hipMemcpyHostToDevice, st));
             pend_dst = static_cast<char *>(dst);
             pend_src = up_top;
-            pend_bytes = need;
+            pend_bytes = bytes;
         }
     } else {
         HIP_OK(hipMemcpyAsync(dst, up.p + up_top, bytes, hipMemcpyHostToDevice, st));
@@ -89,16 +90,11 @@ void Engine::run_levels(inscy_result &out) {
     colp.reset();
     cols_used = 0;
 
-    if (!edges) {
-        HIP_OK(dev_alloc(&edges, ((size_t) ecells + 3) * sizeof(float)));
-        HIP_OK(launch_cell_edges(ecells, edges, st));
-    }
     // the root tree: every point, the root s-connection paths
     Pool &L0 = lvl[cur_lvl];
     lvl[cur_lvl ^ 1].reset();
     int *P = store.take<int>(n);
-    HIP_OK(launch_iota(P, n, st));
-    int *cnt0 = L0.take<int>(1);
+    int *cnt0 = reinterpret_cast<int *>(small + 1);  // zeroed by the set-up
     LTree root;
     root.first = 0;
     root.pass = true;
@@ -109,7 +105,8 @@ void Engine::run_levels(inscy_result &out) {
     root.spm = L0.take<uint64_t>((size_t) n * mw);
     root.nsp_max = n;
     root.slot = 0;
-    HIP_OK(launch_root_paths(nearm, n, root.spx, root.spm, mw, cnt0, st));
+    HIP_OK(dev_alloc(&edges, ((size_t) ecells + 3) * sizeof(float)));
+    HIP_OK(launch_b_root(nearm, n, P, root.spx, root.spm, mw, cnt0, ecells, edges, st));
     lt.push_back(std::move(root));
     stats.calls = 1;
 
@@ -209,7 +206,11 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
         fblk[a + 1] = fblk[a] + nblocks(t.nsp_max);
     }
     int *flags = cur.take<int>(ftot);
-    HIP_OK(launch_fill_i32(flags, 0, ftot, st));
+    lv_next_counts = nxt.take<int>(ftot);  // at most one child per cell
+    FillMany fill;
+    fill.add(flags, 0, (size_t) ftot * sizeof(int));
+    fill.add(lv_next_counts, 0, (size_t) ftot * sizeof(int));
+    HIP_OK(launch_fill_many(fill, st));
     defer_uploads();
     FlagTree *dft = upload(cur, ft);
     int *dfb = upload(cur, fblk);
@@ -231,7 +232,6 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
     // cell groups (restrict + mergeWithNeighbors, ScyTreeNode.cu:837-851)
     lv_groups.assign(na, {});
     std::vector<int> gid(ftot);
-    long long max_children = 0;
     for (int a = 0; a < na; ++a) {
         const LTree &t = lt[lv_act[a]];
         lv_groups[a].resize(d - t.first);
@@ -245,14 +245,11 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
                 for (int x = lo; x <= c; ++x) gm[x] = (int) gs.size();
                 gs.push_back({lo, c});
             }
-            max_children += (long long) gs.size();
         }
     }
     lv_gid = upload(cur, gid);
     lv_skip.clear();
     if (pruner || collect) score_pairs(na);
-    lv_next_counts = nxt.take<int>(std::max<long long>(max_children, 1));
-    HIP_OK(launch_fill_i32(lv_next_counts, 0, std::max<long long>(max_children, 1), st));
 
     // child subspaces: per run of frontier trees with one mask, S | {m} for m >= first
     std::vector<ChildSub> cs;
@@ -521,8 +518,30 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     X.nfb = batch.take<int>(1);
     X.fbcap = phi_mode ? B * n : 1;  // each point of each subspace is sent at most once per pass
     X.fb = batch.take<int2>(X.fbcap);
-    HIP_OK(launch_fill_i32(X.nb, -1, (size_t) kSampleEdges * B * n, st));
-    HIP_OK(launch_fill_i32(cntB, -1, (size_t) B * n, st));
+    // ---- (tree, dimension) pairs to partition by the cell groups
+    struct PairInfo {
+        int a, b, G, cnt_off;
+    };
+    std::vector<PairInfo> pinfo;
+    int pc_total = 0;
+    for (int b = 0; b < B; ++b) {
+        const ChildSub &c = cs[i0 + b];
+        for (int a = c.t0; a < c.t1; ++a) {
+            if (!pair_on(a, c.m)) continue;
+            const LTree &t = lt[lv_act[a]];
+            const int G = (int) lv_groups[a][c.m - t.first].size();
+            pinfo.push_back({a, b, G, pc_total});
+            pc_total += 7 * G;
+        }
+    }
+    int *pcnt = batch.take<int>(std::max(pc_total, 1));
+    FillMany fill;
+    fill.add(X.nb, ~0u, (size_t) kSampleEdges * B * n * sizeof(int));
+    fill.add(cntB, ~0u, (size_t) B * n * sizeof(int));
+    fill.add(X.qflag, 0, (size_t) nw * n);
+    fill.add(pcnt, 0, (size_t) pc_total * sizeof(int));
+    if (phi_mode && fan) fill.add(X.nfb, 0, sizeof(int));
+    HIP_OK(launch_fill_many(fill, st));
 
     auto columns = [&](std::vector<BatchSub> &v, const std::vector<const float *> &tab) {
         const float *const *dcol = upload(batch, tab);
@@ -575,7 +594,6 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         tq0 = std::chrono::steady_clock::now();
     }
     if (fan) {
-        if (phi_mode) HIP_OK(launch_fill_i32(X.nfb, 0, 1, st));
         const KernelTimer tm = timer();
         if (tm.start) HIP_OK(hipEventRecord(tm.start, st));
         for (int w = 0; w < 5; ++w)
@@ -595,24 +613,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     }
 
     // ---- partition of every (tree, dimension) pair by the cell groups
-    struct PairInfo {
-        int a, b, G, cnt_off;
-    };
-    std::vector<PairInfo> pinfo;
-    int pc_total = 0;
-    for (int b = 0; b < B; ++b) {
-        const ChildSub &c = cs[i0 + b];
-        for (int a = c.t0; a < c.t1; ++a) {
-            if (!pair_on(a, c.m)) continue;
-            const LTree &t = lt[lv_act[a]];
-            const int G = (int) lv_groups[a][c.m - t.first].size();
-            pinfo.push_back({a, b, G, pc_total});
-            pc_total += 7 * G;
-        }
-    }
     const int np = (int) pinfo.size();
-    int *pcnt = batch.take<int>(std::max(pc_total, 1));
-    HIP_OK(launch_fill_i32(pcnt, 0, std::max(pc_total, 1), st));
     std::vector<PartPair> pairs(np);
     std::vector<int> pblk(np + 1, 0);
     for (int j = 0; j < np; ++j) {
@@ -699,7 +700,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                 passing[pi.b] = 1;
                 int *Wst = store.take<int>(std::max(nW, 1));
                 if (nW > 0) {
-                    copies.push_back({pairs[j].outW + offW, Wst, nW, 0});
+                    copies.push_back({pairs[j].outW + offW, Wst, nW, -1});
                     stamps.push_back({pairs[j].outW + offW, nullptr, nW, (int) lt.size()});
                     stamp_b.push_back(pi.b);
                 }
@@ -740,42 +741,33 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         }
     }
 
-    // ---- path prune of the surviving children
-    if (!prune.empty()) {
-        const int nc = (int) prune.size();
-        uint64_t *tables = batch.take<uint64_t>(table_total);
-        dmask_t *bits = batch.take<dmask_t>(nc);
-        HIP_OK(launch_fill_u64(tables, kEmptySlot, table_total, st));
-        HIP_OK(launch_fill_u64(reinterpret_cast<uint64_t *>(bits), 0ull, (size_t) 2 * nc, st));
-        std::vector<int> bw(nc + 1, 0), bp(nc + 1, 0);
-        for (int c = 0; c < nc; ++c) {
+    // ---- path prune of the surviving children, their point lists, and the
+    // dense components of the subspaces that gained one: descriptors in one copy
+    FillMany post;
+    const int nprune = (int) prune.size();
+    std::vector<int> bw(nprune + 1, 0), bp(nprune + 1, 0);
+    if (nprune) {
+        uint64_t *tables = post.add(batch.take<uint64_t>(table_total), ~0u, table_total * sizeof(uint64_t));
+        dmask_t *bits = post.add(batch.take<dmask_t>(nprune), 0, (size_t) nprune * sizeof(dmask_t));
+        for (int c = 0; c < nprune; ++c) {
             prune[c].table = tables + prune_slots[c];
             prune[c].bits = bits + c;
             bw[c + 1] = bw[c] + nblocks(prune[c].nW);
             bp[c + 1] = bp[c] + nblocks(prune[c].nsp);
         }
-        defer_uploads();
-        PruneChild *dpc = upload(batch, prune);
-        int *dbw = upload(batch, bw);
-        int *dbp = upload(batch, bp);
-        flush_uploads();
-        HIP_OK(launch_b_prune(D, dpc, nc, dbw, bw[nc], dbp, bp[nc], st));
     }
-
-    // ---- dense components of the subspaces that gained a surviving tree
     std::vector<BatchSub> hc;
     std::vector<Entry> ents;
     int ncomp = 0;
     for (int b = 0; b < B; ++b) ncomp += passing[b];
+    std::vector<const float *> ctab2;
     if (ncomp > 0) {
         int *cntP = slabs.take<int>((size_t) ncomp * n);
         int *compP = slabs.take<int>((size_t) ncomp * n);
         int *csizeP = slabs.take<int>((size_t) ncomp * n);
         int *memP = slabs.take<int>((size_t) ncomp * n);
-        uint8_t *inresP = slabs.take<uint8_t>((size_t) ncomp * n);
-        int *stampP = slabs.take<int>((size_t) ncomp * n);
-        HIP_OK(launch_fill_u8(inresP, 0, (size_t) ncomp * n, st));
-        HIP_OK(launch_fill_i32(stampP, -1, (size_t) ncomp * n, st));
+        uint8_t *inresP = post.add(slabs.take<uint8_t>((size_t) ncomp * n), 0, (size_t) ncomp * n);
+        int *stampP = post.add(slabs.take<int>((size_t) ncomp * n), ~0u, (size_t) ncomp * n * sizeof(int));
         std::vector<int *> stamp_of(B, nullptr);
         grow_entries(nentries + ncomp);
         int ci = 0;
@@ -788,7 +780,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             x.cnt = cntP + (size_t) ci * n;
             x.comp = compP + (size_t) ci * n;
             x.csize = csizeP + (size_t) ci * n;
-            copies.push_back({hs[b].cnt, x.cnt, n, 0});
+            copies.push_back({hs[b].cnt, x.cnt, n, -1});
             hc.push_back(x);
             Subspace &sb = subs[s];
             sb.cnt = x.cnt;
@@ -802,36 +794,31 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             ents.push_back(Entry{s, sb.comp, sb.csize, sb.inres, memP + (size_t) ci * n, 0, 0});
             ++ci;
         }
-        for (size_t u = 0; u < stamps.size(); ++u) stamps[u].dst = stamp_of[stamp_b[u]];
-    }
-    if (!copies.empty()) {
-        std::vector<int> cb(copies.size() + 1, 0);
-        for (size_t c = 0; c < copies.size(); ++c) cb[c + 1] = cb[c] + nblocks(copies[c].len);
-        defer_uploads();
-        CopySeg *dcs = upload(batch, copies);
-        int *dcb2 = upload(batch, cb);
-        flush_uploads();
-        HIP_OK(launch_b_copy(dcs, dcb2, (int) copies.size(), cb.back(), st));
-    }
-    if (!stamps.empty()) {
-        std::vector<int> sbk(stamps.size() + 1, 0);
-        for (size_t c = 0; c < stamps.size(); ++c) sbk[c + 1] = sbk[c] + nblocks(stamps[c].len);
-        defer_uploads();
-        CopySeg *dss = upload(batch, stamps);
-        int *dsb = upload(batch, sbk);
-        flush_uploads();
-        HIP_OK(launch_b_stamp(dss, dsb, (int) stamps.size(), sbk.back(), st));
-    }
-    if (ncomp > 0) {
+        for (size_t u = 0; u < stamps.size(); ++u) {
+            stamps[u].dst = stamp_of[stamp_b[u]];
+            copies.push_back(stamps[u]);
+        }
         X.dsorted = batch.take<uint8_t>((size_t) ncomp * n + 8);  // the grouped link walk reads aligned words past the end
         X.par = batch.take<int>((size_t) ncomp * n);
         X.giant = batch.take<int>(ncomp);
-        std::vector<const float *> ctab2;
         if (fan) index_of(hc, ctab2);
-        defer_uploads();
-        if (fan) columns(hc, ctab2);
-        BatchSub *dhc = upload(batch, hc);
-        flush_uploads();
+    }
+    std::vector<int> cb(copies.size() + 1, 0);
+    for (size_t c = 0; c < copies.size(); ++c) cb[c + 1] = cb[c] + nblocks(copies[c].len);
+    defer_uploads();
+    PruneChild *dpc = nprune ? upload(batch, prune) : nullptr;
+    int *dbw = nprune ? upload(batch, bw) : nullptr;
+    int *dbp = nprune ? upload(batch, bp) : nullptr;
+    CopySeg *dcs = copies.empty() ? nullptr : upload(batch, copies);
+    int *dcb2 = copies.empty() ? nullptr : upload(batch, cb);
+    if (ncomp > 0 && fan) columns(hc, ctab2);
+    BatchSub *dhc = ncomp > 0 ? upload(batch, hc) : nullptr;
+    if (ncomp > 0) put(entries + nentries, ents.data(), ents.size() * sizeof(Entry));
+    flush_uploads();
+    HIP_OK(launch_fill_many(post, st));
+    if (nprune) HIP_OK(launch_b_prune(D, dpc, nprune, dbw, bw[nprune], dbp, bp[nprune], st));
+    if (!copies.empty()) HIP_OK(launch_b_copy(dcs, dcb2, (int) copies.size(), cb.back(), st));
+    if (ncomp > 0) {
         std::chrono::steady_clock::time_point tc0, tc1, tc2;
         if (dbg) {
             sync();
@@ -857,8 +844,6 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                          "comp=%d all_count=%.3fms components=%.3fms\n",
                          B, nw, k, cap_of(k), qs, ms(tq0, tq1), ncomp, ms(tc0, tc1), ms(tc1, tc2));
         }
-        Entry *de = upload(batch, ents);
-        HIP_OK(launch_b_entries(entries, nentries, de, ncomp, d_nE, st));
         nentries += ncomp;
         stats.components += ncomp;
     }
@@ -954,6 +939,8 @@ void Engine::replay_staged() {
     // per step: row flags (2 per superset row) and a block counter
     // (redundancy), the join's two words and its candidate list
     const size_t kScratchInts = (size_t) 64 << 20;  // per launch group
+    batch.reset();
+    size_t held = 0;  // scratch of the chunks in flight
     const int ccap = prm.min_size > 0 ? std::min(n, n / prm.min_size + 1) : n;
     for (int sg = 1; sg <= nst; ++sg) {
         const std::vector<int> &ids = by_stage[sg];
@@ -968,7 +955,12 @@ void Engine::replay_staged() {
                 ints += need;
                 ++b;
             }
-            batch.reset();
+            if (held > 0 && held + ints > kScratchInts) {
+                sync();  // the chunks in flight still use theirs
+                batch.reset();
+                held = 0;
+            }
+            held += ints + 65536;  // with its descriptors
             int *scr = batch.take<int>(std::max<size_t>(ints, 1));
             HIP_OK(launch_fill_i32(scr, 0, std::max<size_t>(ints, 1), st));
             std::vector<RepOp> ops(b - a);
@@ -1021,7 +1013,6 @@ void Engine::replay_staged() {
             flush_uploads();
             HIP_OK(launch_rep_stage(dops, no, dbr, br.back(), dbc, bc.back(), dbk, bk.back(), dbm, bm.back(), entries,
                                     prm.r, prm.min_size, n, keepv, st));
-            sync();  // the chunk's scratch and descriptors are reused by the next one
             a = b;
         }
     }

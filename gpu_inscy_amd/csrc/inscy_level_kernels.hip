@@ -53,26 +53,35 @@ __global__ void k_b_flags(const FlagTree *__restrict__ T, const int *__restrict_
 // cell is monotone in the coordinate, so for a query in cell c the coordinates
 // whose cell is within one of c are exactly [edge[c], edge[c + 3]): the walks
 // test the cells of a candidate on its coordinate, without reading its cells.
-__global__ void k_cell_edges(int C, float *__restrict__ edge) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= C + 3) return;
+__device__ __forceinline__ float cell_edge(int i, int C) {
     const int target = i - 1;
-    float v = -__builtin_inff();
-    if (target >= C) {
-        v = __builtin_inff();
-    } else if (target > 0) {
-        const float ecs = ecell_width(C);
-        uint32_t lo = 0, hi = 0x3F800000u;  // cell(0) < target <= cell(1.0) = C - 1
-        while (hi - lo > 1) {
-            const uint32_t mid = lo + (hi - lo) / 2;
-            if (ecell_of(__uint_as_float(mid), ecs, C) >= target)
-                hi = mid;
-            else
-                lo = mid;
-        }
-        v = __uint_as_float(hi);
+    if (target <= 0) return -__builtin_inff();
+    if (target >= C) return __builtin_inff();
+    const float ecs = ecell_width(C);
+    uint32_t lo = 0, hi = 0x3F800000u;  // cell(0) < target <= cell(1.0) = C - 1
+    while (hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (ecell_of(__uint_as_float(mid), ecs, C) >= target)
+            hi = mid;
+        else
+            lo = mid;
     }
-    edge[i] = v;
+    return __uint_as_float(hi);
+}
+
+// the root tree: every point, the path of every point with a near-edge
+// dimension; and the cell edges
+__global__ void k_b_root(const dmask_t *__restrict__ nearm, int n, int *__restrict__ P, int *__restrict__ outx,
+                         uint64_t *__restrict__ outm, int mw, int *__restrict__ nout, int C, float *__restrict__ edge) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < C + 3) edge[i] = cell_edge(i, C);
+    if (i < n) P[i] = i;
+    const dmask_t m = i < n ? nearm[i] : (dmask_t) 0;
+    const int slot = wave_slot(m != 0, nout);
+    if (m != 0) {
+        outx[slot] = i;
+        mstore(outm, slot, m, mw);
+    }
 }
 
 // ------------------------------------------------------------ grid indexes of a batch of subspaces
@@ -146,29 +155,6 @@ __global__ void k_b_qmark(const BatchSub *__restrict__ subs, const QuerySeg *__r
     const BatchSub &B = subs[Q.b];
     const int p = Q.P[i];
     qflag[B.base + B.pos[p]] = 1;
-}
-
-// qstart[b] = first index of the selected (ascending global) positions that is
-// >= b*n; qstart[nsub] = the number selected
-__global__ void k_b_qstart(const int *__restrict__ qlist, const int *__restrict__ nsel, int nsub, int n,
-                           int *__restrict__ qstart) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b > nsub) return;
-    const int total = *nsel;
-    if (b == nsub) {
-        qstart[b] = total;
-        return;
-    }
-    const long long key = (long long) b * n;
-    int lo = 0, hi = total;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (qlist[mid] < key)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    qstart[b] = lo;
 }
 
 // ------------------------------------------------------------ candidate walk
@@ -275,7 +261,7 @@ __device__ __forceinline__ void lds_layout(char *smem, int k, float2 *&sc, float
 // load after the previous store, one memory round trip per dimension)
 // (the cells are computed from the coordinates with the discretisation's
 // formula, G.C being the number of eps cells: no scattered read by point id;
-// the intervals come from the table of cell edges, see k_cell_edges)
+// the intervals come from the table of cell edges, see cell_edge)
 __device__ __forceinline__ void stage_query_b(const BatchSub &B, const float *__restrict__ edge, int i, float *sy,
                                               float2 *sc, int stride, int *ci) {
     constexpr int kStage = 8;
@@ -1780,25 +1766,17 @@ __global__ void k_rep_members_multi(const RepOp *__restrict__ ops, const int *__
         if (in[u]) mem[slot++] = i0 + u * kBlock + threadIdx.x;
 }
 
-__global__ void k_b_stamp(const CopySeg *__restrict__ segs, const int *__restrict__ blk_off, int ns) {
-    const int s = seg_of(blk_off, ns, blockIdx.x);
-    const CopySeg S = segs[s];
-    const int i = (blockIdx.x - blk_off[s]) * blockDim.x + threadIdx.x;
-    if (i < S.len) S.dst[S.src[i]] = S.pad;
-}
-
 // ------------------------------------------------------------ small helpers
 __global__ void k_b_copy(const CopySeg *__restrict__ segs, const int *__restrict__ blk_off, int ns) {
     const int s = seg_of(blk_off, ns, blockIdx.x);
     const CopySeg S = segs[s];
     const int i = (blockIdx.x - blk_off[s]) * blockDim.x + threadIdx.x;
-    if (i < S.len) S.dst[i] = S.src[i];
-}
-
-__global__ void k_b_entries(Entry *__restrict__ E, int at, const Entry *__restrict__ src, int count,
-                            int *__restrict__ nE) {
-    for (int i = threadIdx.x; i < count; i += blockDim.x) E[at + i] = src[i];
-    if (threadIdx.x == 0) *nE = at + count;
+    if (i >= S.len) return;
+    const int v = S.src[i];
+    if (S.pad < 0)
+        S.dst[i] = v;
+    else
+        S.dst[v] = S.pad;
 }
 
 template <class T>
@@ -1817,8 +1795,10 @@ static size_t count_lds(int kmax) {
     return (sizeof(float2) + sizeof(float)) * QPB * (size_t) (kmax > 0 ? kmax : 1) + sizeof(int) * QPB * kRangeWords;
 }
 
-hipError_t launch_cell_edges(int C, float *edge, hipStream_t st) {
-    LAUNCH(k_cell_edges, dim3(blocks_for((size_t) C + 3)), dim3(kBlock), 0, st, C, edge);
+hipError_t launch_b_root(const dmask_t *nearm, int n, int *P, int *outx, uint64_t *outm, int mw, int *nout, int C,
+                         float *edge, hipStream_t st) {
+    LAUNCH(k_b_root, dim3(blocks_for((size_t) std::max(n, C + 3))), dim3(kBlock), 0, st, nearm, n, P, outx, outm, mw,
+           nout, C, edge);
     return hipGetLastError();
 }
 
@@ -1897,7 +1877,8 @@ __global__ void __launch_bounds__(kBlock) k_b_flag_count(const uint8_t *__restri
 
 __global__ void __launch_bounds__(kBlock) k_b_flag_write(const uint8_t *__restrict__ qflag, size_t nb,
                                                           const int *__restrict__ toff, int ntile,
-                                                          int *__restrict__ qlist, int *__restrict__ nsel) {
+                                                          int *__restrict__ qlist, int *__restrict__ nsel, int n,
+                                                          int *__restrict__ qstart) {
     __shared__ int wsum[kBlock / 64];
     const size_t at = ((size_t) blockIdx.x * kBlock + threadIdx.x) * kFlagsPerLane;
     const uint4 v = lane_flags(qflag, at, nb);
@@ -1921,6 +1902,17 @@ __global__ void __launch_bounds__(kBlock) k_b_flag_write(const uint8_t *__restri
     __syncthreads();
     int o = toff[blockIdx.x] + x - c;
     for (int q = 0; q < (int) (threadIdx.x >> 6); ++q) o += wsum[q];
+    // qstart[b]: queries before position b * n (the first of subspace b)
+    if (qstart && at < nb) {
+        for (size_t b = (at + n - 1) / n; b * n < at + kFlagsPerLane && b * n < nb; ++b) {
+            const int off = (int) (b * n - at);
+            int before = o;
+            for (int q = 0; q < 4; ++q)
+                if (4 * q < off)
+                    before += __builtin_popcount((uint32_t) m[q] & (off - 4 * q >= 4 ? ~0u : (1u << (8 * (off - 4 * q))) - 1u));
+            qstart[b] = before;
+        }
+    }
     for (int q = 0; q < 4; ++q) {
         uint32_t mm = (uint32_t) m[q];
         while (mm) {
@@ -1929,7 +1921,10 @@ __global__ void __launch_bounds__(kBlock) k_b_flag_write(const uint8_t *__restri
             mm &= mm - 1;
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nsel = toff[ntile];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *nsel = toff[ntile];
+        if (qstart) qstart[nb / n] = toff[ntile];
+    }
 }
 
 static int flag_tiles(size_t items) { return (int) ((items + kFlagTile - 1) / kFlagTile); }
@@ -1942,7 +1937,7 @@ size_t select_temp_bytes(int items) {
 }
 
 hipError_t launch_flag_compact(const uint8_t *flags, size_t nb, void *temp, size_t temp_bytes, int *out, int *nsel,
-                               hipStream_t st) {
+                               int n, int *qstart, hipStream_t st) {
     const int nt = flag_tiles(nb);
     const size_t cnt_bytes = align256((size_t) (nt + 1) * sizeof(int));
     char *base = static_cast<char *>(temp);
@@ -1951,7 +1946,8 @@ hipError_t launch_flag_compact(const uint8_t *flags, size_t nb, void *temp, size
     LAUNCH(k_b_flag_count, dim3(nt), dim3(kBlock), 0, st, flags, nb, nt, tcnt);
     hipError_t e = launch_exclusive_sum(base + 2 * cnt_bytes, temp_bytes - 2 * cnt_bytes, tcnt, toff, nt + 1, st);
     if (e != hipSuccess) return e;
-    LAUNCH(k_b_flag_write, dim3(nt), dim3(kBlock), 0, st, flags, nb, toff, nt, out, nsel);
+    LAUNCH(k_b_flag_write, dim3(nt), dim3(kBlock), 0, st, flags, nb, toff, nt, out, nsel, n,
+           qstart);
     return hipGetLastError();
 }
 
@@ -1959,13 +1955,9 @@ hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySe
                             int nseg, int nblk, const BatchIndex &X, hipStream_t st) {
     if (nsub <= 0) return hipSuccess;
     const size_t nb = (size_t) nsub * n;
-    LAUNCH(k_b_fill<uint8_t>, dim3(fill_blocks(nb, 1)), dim3(kBlock), 0, st, X.qflag, (uint8_t) 0, nb);
     if (nblk > 0)
         LAUNCH(k_b_qmark, dim3(nblk), dim3(kBlock), 0, st, subs, segs, blk_off, nseg, X.qflag);
-    hipError_t e = launch_flag_compact(X.qflag, nb, X.select_temp, X.select_bytes, X.qlist, X.nsel, st);
-    if (e != hipSuccess) return e;
-    LAUNCH(k_b_qstart, dim3(blocks_for(nsub + 1)), dim3(kBlock), 0, st, X.qlist, X.nsel, nsub, n, X.qstart);
-    return hipGetLastError();
+    return launch_flag_compact(X.qflag, nb, X.select_temp, X.select_bytes, X.qlist, X.nsel, n, X.qstart, st);
 }
 
 template <int K>
@@ -2127,12 +2119,6 @@ hipError_t launch_b_copy(const CopySeg *segs, const int *blk_off, int nseg, int 
     return hipGetLastError();
 }
 
-hipError_t launch_b_stamp(const CopySeg *segs, const int *blk_off, int nseg, int nblk, hipStream_t st) {
-    if (nblk <= 0) return hipSuccess;
-    LAUNCH(k_b_stamp, dim3(nblk), dim3(kBlock), 0, st, segs, blk_off, nseg);
-    return hipGetLastError();
-}
-
 int rep_red_blocks(int nlist, int nW) { return std::max(1, std::min(nlist + nW / kChunk, 256)); }
 int rep_check_blocks(int nlist, int n) { return nlist > 0 ? std::min(nlist + n / kChunk, 256) : 0; }
 int rep_mem_blocks(int n) { return (n + kMemPerBlock - 1) / kMemPerBlock; }
@@ -2147,12 +2133,6 @@ hipError_t launch_rep_stage(const RepOp *ops, int nops, const int *blk_red, int 
     if (nblk_chk > 0) LAUNCH(k_rep_check_multi, dim3(nblk_chk), dim3(kBlock), 0, st, ops, blk_chk, nops, E, r);
     LAUNCH(k_rep_apply_multi, dim3(nops), dim3(kBlock), 0, st, ops, E);
     if (nblk_mem > 0) LAUNCH(k_rep_members_multi, dim3(nblk_mem), dim3(kBlock), 0, st, ops, blk_mem, nops, E, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_b_entries(Entry *E, int at, const Entry *src, int count, int *nE, hipStream_t st) {
-    if (count <= 0) return hipSuccess;
-    LAUNCH(k_b_entries, dim3(1), dim3(kBlock), 0, st, E, at, src, count, nE);
     return hipGetLastError();
 }
 
