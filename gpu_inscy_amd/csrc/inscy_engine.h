@@ -317,7 +317,8 @@ public:
         // the level-synchronous driver keeps its lists in pools; its arena holds
         // the replay's label flags (one per open dimension) and the emit buffers
         if (levels_mode) want = (size_t) n * (d + 8) + pass + (64u << 20);
-        if (const size_t free_b = device_available_bytes() / (size_t) mem_share) want = std::min(want, free_b / 3);
+        available = device_available_bytes() / (size_t) mem_share;
+        if (available) want = std::min(want, available / 3);
         arena.init(want);
 
         int *hist = arena.take<int>((size_t) d * ecells);
@@ -908,6 +909,7 @@ private:
     char *pend_dst = nullptr;                       // the deferred copy: device place,
     size_t pend_src = 0, pend_bytes = 0;            // staging offset and bytes
     float *edges = nullptr;                         // [ecells + 3] edges of the eps cells
+    size_t available = 0;  // device bytes this run may take, at its set-up
     size_t batch_budget = 0;
     size_t max_batch = 0;  // child subspaces per batch
     bool phi_mode = false;          // rectangular = false

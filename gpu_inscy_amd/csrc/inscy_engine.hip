@@ -107,7 +107,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
     bool own = false;
     try {
         if (!st) {
-            HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+            HIP_OK(stream_pool().get(&st));
             own = true;
         }
         auto res = std::make_unique<inscy_result>();
@@ -138,13 +138,13 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             res->stats = eng.stats;
             if (g_trace_on) g_trace = eng.trace;
         }
-        if (own) (void) hipStreamDestroy(st);
+        if (own) stream_pool().put(st);
         res->stats.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         *out = res.release();
         g_error.clear();
         return INSCY_OK;
     } catch (...) {
-        if (own) (void) hipStreamDestroy(st);
+        if (own) stream_pool().put(st);
         return fail_current();
     }
 }
@@ -174,7 +174,7 @@ static int run_many_impl(const float *const *X, const int64_t *n, const int32_t 
     auto work = [&]() {
         if (hipSetDevice(dev) != hipSuccess) return;
         hipStream_t st = nullptr;
-        if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return;
+        if (stream_pool().get(&st) != hipSuccess) return;
         for (int q = next++; q < count; q = next++) {
             const int i = order[q];
             if (host_input) {
@@ -198,7 +198,7 @@ static int run_many_impl(const float *const *X, const int64_t *n, const int32_t 
             }
             if (rc[i] != INSCY_OK) msg[i] = g_error;
         }
-        (void) hipStreamDestroy(st);
+        stream_pool().put(st);
     };
     std::vector<std::thread> th;
     th.reserve(workers);
@@ -271,16 +271,28 @@ int inscy_run(const float *X, int64_t n, int32_t d, const inscy_params *params, 
     int rc = check_params(n, d, params, mode);
     if (rc) return rc;
     if (!X) return fail(INSCY_ERR_ARGUMENT, "X is NULL");
+    // a small input goes through pinned memory (a pageable copy waits for the
+    // device), either way on the run's own stream
+    constexpr size_t kStaged = (size_t) 1 << 20;
     float *dX = nullptr;
-    size_t bytes = (size_t) n * d * sizeof(float);
+    void *pinned = nullptr;
+    hipStream_t st = nullptr;
+    const size_t bytes = (size_t) n * d * sizeof(float);
     hipError_t e = dev_alloc(&dX, bytes);
     if (e != hipSuccess) return fail(INSCY_ERR_MEMORY, std::string("device allocation: ") + hipGetErrorString(e));
-    e = hipMemcpy(dX, X, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        dev_free(dX);
-        return fail(INSCY_ERR_DEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
+    e = stream_pool().get(&st);
+    const void *src = X;
+    if (e == hipSuccess && bytes <= kStaged && host_alloc(&pinned, kStaged) == hipSuccess) {
+        std::memcpy(pinned, X, bytes);
+        src = pinned;
     }
-    rc = run_impl(dX, n, d, params, mode, nullptr, out);
+    if (e == hipSuccess) e = hipMemcpyAsync(dX, src, bytes, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+        rc = run_impl(dX, n, d, params, mode, st, out);
+    else
+        rc = fail(INSCY_ERR_DEVICE, std::string("input copy: ") + hipGetErrorString(e));
+    stream_pool().put(st);  // waits for the stream: the buffers below are idle then
+    if (pinned) host_free(pinned);
     dev_free(dX);
     return rc;
 }
@@ -380,6 +392,7 @@ int inscy_mlp_round(const float *d_master, uint16_t *d_params, void *stream) {
 }
 
 int inscy_release_memory(void) {
+    stream_pool().release();
     device_cache().release(-1);
     host_cache().release(-1);
     return INSCY_OK;

@@ -81,8 +81,7 @@ void Engine::run_levels(inscy_result &out) {
     if (const char *e = std::getenv("INSCY_MAX_BATCH")) max_batch = (size_t) std::max(1, std::atoi(e));
     if (max_batch_override > 0) max_batch = (size_t) max_batch_override;
     batch_budget = (size_t) 2 << 30;
-    if (const size_t free_b = device_available_bytes() / (size_t) mem_share)
-        batch_budget = std::min<size_t>(std::max<size_t>(free_b / 8, (size_t) 256 << 20), (size_t) 8 << 30);
+    if (available) batch_budget = std::min<size_t>(std::max<size_t>(available / 8, (size_t) 256 << 20), (size_t) 8 << 30);
     kept.clear();
     keptp.reset();
     kept_used = 0;

@@ -156,6 +156,59 @@ inline EventPool &event_pool() {
     return *p;
 }
 
+// Streams of the runs that bring none: creating and destroying one costs as much
+// as twenty launches.  A stream comes back idle (its run has synchronised it); a
+// device keeps at most kMost of them, and inscy_release_memory() gives them back.
+class StreamPool {
+public:
+    static constexpr size_t kMost = 16;
+    hipError_t get(hipStream_t *s) {
+        const int dev = device();
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            auto &fl = free_[dev];
+            if (!fl.empty()) {
+                *s = fl.back();
+                fl.pop_back();
+                return hipSuccess;
+            }
+        }
+        return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+    }
+    void put(hipStream_t s) {
+        if (!s) return;
+        if (hipStreamSynchronize(s) == hipSuccess) {
+            std::lock_guard<std::mutex> g(mu_);
+            auto &fl = free_[device()];
+            if (fl.size() < kMost) {
+                fl.push_back(s);
+                return;
+            }
+        }
+        (void) hipStreamDestroy(s);
+    }
+    void release() {
+        std::lock_guard<std::mutex> g(mu_);
+        for (auto &kv : free_) {
+            for (hipStream_t s : kv.second) (void) hipStreamDestroy(s);
+            kv.second.clear();
+        }
+    }
+
+private:
+    static int device() {
+        int d = 0;
+        (void) hipGetDevice(&d);
+        return d;
+    }
+    std::mutex mu_;
+    std::unordered_map<int, std::vector<hipStream_t>> free_;
+};
+inline StreamPool &stream_pool() {
+    static StreamPool *p = new StreamPool;
+    return *p;
+}
+
 // Device memory a run can still take: what the runtime reports free plus the
 // cached blocks no run holds (an earlier run's buffers stay cached and would
 // otherwise shrink every later run's budgets).
