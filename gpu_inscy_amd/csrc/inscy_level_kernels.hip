@@ -1496,10 +1496,11 @@ struct RowPlan {
     uint8_t by_mem[kSegRows];
 };
 
-// loads rows [seg, seg + ns) of the list and their chunk prefix; returns the
-// number of chunks.  by_mem: walk the row's members (else the tree's points,
-// when nW is shorter; nW < 0 walks members always)
-__device__ int plan_rows(const Entry *__restrict__ E, const int *__restrict__ list, int seg, int ns, int nW,
+// loads rows [seg, seg + ns) of the list and their chunk prefix (of the items
+// past the first `head`); returns the number of chunks.  by_mem: walk the row's
+// members (else the tree's points, when nW is shorter; nW < 0 walks members
+// always)
+__device__ int plan_rows(const Entry *__restrict__ E, const int *__restrict__ list, int seg, int ns, int nW, int head,
                          RowPlan &R, int *wtmp) {
     for (int i = threadIdx.x; i < ns; i += blockDim.x) {
         const Entry e = E[list[seg + i]];
@@ -1514,7 +1515,7 @@ __device__ int plan_rows(const Entry *__restrict__ E, const int *__restrict__ li
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
         const int i = threadIdx.x * PER + u;
-        c[u] = i < ns ? (R.len[i] + kChunk - 1) / kChunk : 0;
+        c[u] = i < ns ? (max(R.len[i] - head, 0) + kChunk - 1) / kChunk : 0;
         sum += c[u];
     }
     int incl = sum;
@@ -1560,8 +1561,12 @@ __device__ __forceinline__ int flag_cand(int J) { return -(2 + 3 * J); }
 __device__ __forceinline__ int flag_drop(int J) { return -(3 + 3 * J); }
 __device__ __forceinline__ int flag_fresh(int J) { return -(4 + 3 * J); }
 
-// pruneRedundancy of every step with a tree (the body of k_rep_redundancy,
-// with the step's own block range standing for the grid)
+// pruneRedundancy of every step with a tree (the step's own block range stands
+// for the grid).  A row is decided by one touched cluster smaller than |T| r, and
+// most rows that the tree touches show one among their first items: every row
+// is probed first, a wave per row, and only the rows left over are walked on
+// in chunks.
+constexpr int kProbe = 256;
 __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__restrict__ blk_off, int nops,
                                 const Entry *__restrict__ E, float r, int *__restrict__ keepv) {
     __shared__ RowPlan R;
@@ -1575,9 +1580,40 @@ __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__rest
     const int *list = Op.list;
     int *rowflag = Op.rowflag;
     const double lhs = (double) ((float) nW * r);
+    // item t of a row: (touch, small)
+    auto item = [&](const Entry &e, bool by_mem, int t, bool &touch, bool &small) {
+        if (by_mem) {
+            const int q = e.mem[t];
+            if (Op.tstamp[q] == tree) {
+                touch = true;
+                small |= lhs > (double) e.csize[e.comp[q]];
+            }
+        } else {
+            const int K = e.comp[Op.W[t]];
+            if (K >= 0 && e.inres[K]) {
+                touch = true;
+                small |= lhs > (double) e.csize[K];
+            }
+        }
+    };
     for (int seg = 0; seg < nlist; seg += kSegRows) {
         const int ns = min(kSegRows, nlist - seg);
-        const int total = plan_rows(E, list, seg, ns, nW, R, wtmp);
+        const int total = plan_rows(E, list, seg, ns, nW, kProbe, R, wtmp);
+        constexpr int W = kBlock / 64;
+        for (int i = bi * W + (int) (threadIdx.x / 64); i < ns; i += nb * W) {
+            const int len = min(R.len[i], kProbe);
+            if (len == 0) continue;
+            const Entry e = E[list[seg + i]];
+            const bool by_mem = R.by_mem[i];
+            bool touch = false, small = false;
+            for (int t = __lane_id(); t < len; t += 64) item(e, by_mem, t, touch, small);
+            const bool any_touch = __any(touch), any_small = __any(small);
+            if (__lane_id() == 0) {
+                if (any_touch) st_relaxed(&rowflag[2 * (seg + i)], 1);
+                if (any_small) st_relaxed(&rowflag[2 * (seg + i) + 1], 1);
+            }
+        }
+        __syncthreads();
         for (int w = bi; w < total; w += nb) {
             const int i = row_of(R, ns, w);
             const int h = seg + i;
@@ -1587,30 +1623,15 @@ __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__rest
             __syncthreads();
             if (sk) continue;
             const Entry e = E[list[h]];
-            const int t0 = (w - R.pre[i]) * kChunk, t1 = min(R.len[i], t0 + kChunk);
+            const bool by_mem = R.by_mem[i];
+            const int t0 = kProbe + (w - R.pre[i]) * kChunk, t1 = min(R.len[i], t0 + kChunk);
             bool touch = false, small = false;
-            if (R.by_mem[i]) {
-                for (int t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-                    const int q = e.mem[t];
-                    if (Op.tstamp[q] == tree) {
-                        touch = true;
-                        small |= lhs > (double) e.csize[e.comp[q]];
-                    }
-                }
-            } else {
-                for (int t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-                    const int K = e.comp[Op.W[t]];
-                    if (K >= 0 && e.inres[K]) {
-                        touch = true;
-                        small |= lhs > (double) e.csize[K];
-                    }
-                }
-            }
+            for (int t = t0 + threadIdx.x; t < t1; t += blockDim.x) item(e, by_mem, t, touch, small);
             touch = __syncthreads_or(touch);
             small = __syncthreads_or(small);
             if (threadIdx.x == 0) {
-                if (touch && !ld_relaxed(&rowflag[2 * h])) atomicOr(&rowflag[2 * h], 1);
-                if (small) atomicOr(&rowflag[2 * h + 1], 1);
+                if (touch) st_relaxed(&rowflag[2 * h], 1);
+                if (small) st_relaxed(&rowflag[2 * h + 1], 1);
             }
         }
         __syncthreads();
@@ -1675,7 +1696,7 @@ __global__ void k_rep_check_multi(const RepOp *__restrict__ ops, const int *__re
     const int cj = flag_cand(Op.J), dj = flag_drop(Op.J);
     for (int seg = 0; seg < Op.nlist; seg += kSegRows) {
         const int ns = min(kSegRows, Op.nlist - seg);
-        const int total = plan_rows(E, Op.list, seg, ns, -1, R, wtmp);
+        const int total = plan_rows(E, Op.list, seg, ns, -1, 0, R, wtmp);
         for (int w = bi; w < total; w += nb) {
             const int i = row_of(R, ns, w);
             const Entry e = E[Op.list[seg + i]];
