@@ -183,6 +183,7 @@ struct BatchIndex {
     uint8_t *dsorted;     // [B*n] dense flag per sorted position
     int *par;             // [B*n] union-find parents (point ids within each subspace)
     int *giant;           // [B]
+    int *fit;             // [B] the subspace's sample phase ran in LDS (k_b_sample)
 };
 
 // A grid index to sort: the points by their eps cells in dims[0..j), the last

@@ -800,6 +800,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         X.dsorted = batch.take<uint8_t>((size_t) ncomp * n + 8);  // the grouped link walk reads aligned words past the end
         X.par = batch.take<int>((size_t) ncomp * n);
         X.giant = batch.take<int>(ncomp);
+        X.fit = batch.take<int>(ncomp);
         if (fan) index_of(hc, ctab2);
     }
     std::vector<int> cb(copies.size() + 1, 0);

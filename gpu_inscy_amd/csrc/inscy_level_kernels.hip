@@ -960,7 +960,246 @@ __global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ g
 
 // ------------------------------------------------------------ dense components of a batch
 // (k_dense_init .. k_uf_flatten per subspace; grid.y = subspace)
-__global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, uint8_t *__restrict__ dsorted, int *__restrict__ par) {
+
+// The whole sample phase of one subspace (its dense flags, the unions of the
+// sample edges, compressed parents, the giant component) in one block, with the
+// union-find in LDS: a device-scope swap goes past the XCD's L2 and their rate
+// bounded the same unions on global parents (n=100,000 d=20, 27 batches: 41.5 ms
+// there, 29.5 ms here, bound by the chains of dependent reads of one block; four
+// points a thread in flight, one took 32.0 ms).
+// Above kUfCap points every point first takes the smallest of itself and its
+// dense sample neighbours as parent (each thread writes its own entry, a forest
+// without a swap, about a third of the points are left as roots), and the roots
+// are numbered in id order for the LDS (smaller number = smaller id, so roots
+// stay the smallest ids); a subspace with more roots than fit clears fit[s] and
+// is left to the global passes.
+constexpr int kUfCap = 39936;
+constexpr int kUfThreads = 1024, kUfWaves = kUfThreads / 64, kUfItems = 4;
+__device__ __forceinline__ int lds_find(volatile int *up, int x) {
+    int p = up[x];
+    while (p != x) {
+        const int g = up[p];
+        if (g != p) up[x] = g;
+        x = p;
+        p = g;
+    }
+    return x;
+}
+__device__ __forceinline__ void lds_union(int *up, int a, int b) {
+    while (true) {
+        a = lds_find(up, a);
+        b = lds_find(up, b);
+        if (a == b) return;
+        if (a > b) {
+            const int t = a;
+            a = b;
+            b = t;
+        }
+        const int old = atomicCAS(&up[b], b, a);
+        if (old == b) return;
+        b = old;
+    }
+}
+// point i's first parent: the smallest of itself and its dense sample neighbours
+// (-1 when it is not dense)
+__device__ __forceinline__ int hooked(const BatchSub &B, const int *__restrict__ nb, int i) {
+    if (!meets(B.cnt[i], B.thr_dense, B.dbit)) return -1;
+    int root = i;
+#pragma unroll
+    for (int e = 0; e < kSampleEdges; ++e) {
+        const int q = nb[kSampleEdges * (B.nbase + i) + e];
+        if (q >= 0 && q < root && meets(B.cnt[q], B.thr_dense, B.dbit)) root = q;
+    }
+    return root;
+}
+
+__global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restrict__ subs, int n,
+                                                         const int *__restrict__ nb, uint8_t *__restrict__ dsorted,
+                                                         int *__restrict__ par, int *__restrict__ giant,
+                                                         int *__restrict__ fit) {
+    __shared__ int up[kUfCap];
+    __shared__ int wcnt[kUfWaves + 1];
+    const BatchSub &B = subs[blockIdx.x];
+    const int t = threadIdx.x, lane = __lane_id(), wv = t >> 6;
+    int *pr = par + B.base;
+    const bool numbered = n > kUfCap;  // uniform over the launch
+    // every pass takes kUfItems points per thread at once: one block holds the
+    // whole subspace, so its loads in flight bound it
+    constexpr int M = kUfItems, STEP = kUfThreads * M;
+    const int2 *nb2 = reinterpret_cast<const int2 *>(nb) + B.nbase;
+    static_assert(kSampleEdges == 2, "a point's sample edges are one int2");
+    for (int i0 = t; i0 < n; i0 += STEP) {
+        int c[M], o[M], co[M];
+        int2 q[M];
+        int cq[M][2];
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            const int i = min(i0 + u * kUfThreads, n - 1);
+            c[u] = B.cnt[i];
+            o[u] = B.order[i];
+            q[u] = numbered ? nb2[i] : make_int2(-1, -1);
+        }
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            co[u] = B.cnt[o[u]];
+            cq[u][0] = q[u].x >= 0 && q[u].x < n ? B.cnt[q[u].x] : 0;
+            cq[u][1] = q[u].y >= 0 && q[u].y < n ? B.cnt[q[u].y] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            const int i = i0 + u * kUfThreads;
+            if (i >= n) continue;
+            dsorted[B.base + i] = meets(co[u], B.thr_dense, B.dbit) ? 1 : 0;
+            int root = -1;
+            if (meets(c[u], B.thr_dense, B.dbit)) {
+                root = i;
+                if (q[u].x >= 0 && q[u].x < root && meets(cq[u][0], B.thr_dense, B.dbit)) root = q[u].x;
+                if (q[u].y >= 0 && q[u].y < root && meets(cq[u][1], B.thr_dense, B.dbit)) root = q[u].y;
+                if (!numbered) up[i] = i;
+            }
+            pr[i] = root;
+        }
+    }
+    if (numbered) {
+        __syncthreads();
+        for (int i0 = t; i0 < n; i0 += STEP) {
+            int r[M], p[M];
+#pragma unroll
+            for (int u = 0; u < M; ++u) r[u] = i0 + u * kUfThreads < n ? pr[i0 + u * kUfThreads] : -1;
+            bool moved = true;
+            while (moved) {
+                moved = false;
+#pragma unroll
+                for (int u = 0; u < M; ++u) p[u] = r[u] >= 0 ? pr[r[u]] : -1;
+#pragma unroll
+                for (int u = 0; u < M; ++u) {
+                    moved |= p[u] != r[u];
+                    r[u] = p[u];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+                if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
+        }
+        __syncthreads();
+        // roots of the wave's share (a multiple of 64), then their numbers:
+        // csize[root] = number, comp[number] = root
+        const int share = ((n + kUfWaves - 1) / kUfWaves + 63) & ~63;
+        const int w0 = min(n, wv * share), w1 = min(n, w0 + share);
+        int c = 0;
+        for (int i = w0 + lane; i - lane < w1; i += 64) c += __popcll(__ballot(i < w1 && pr[i] == i));
+        if (lane == 0) wcnt[wv] = c;
+        __syncthreads();
+        if (t == 0) {
+            int acc = 0;
+            for (int w = 0; w < kUfWaves; ++w) {
+                const int v = wcnt[w];
+                wcnt[w] = acc;
+                acc += v;
+            }
+            wcnt[kUfWaves] = acc;
+            fit[blockIdx.x] = acc <= kUfCap;
+        }
+        __syncthreads();
+        if (wcnt[kUfWaves] > kUfCap) return;
+        int at = wcnt[wv];
+        for (int i = w0 + lane; i - lane < w1; i += 64) {
+            const bool root = i < w1 && pr[i] == i;
+            const unsigned long long m = __ballot(root);
+            const int num = at + __popcll(m & ((1ull << lane) - 1ull));
+            at += __popcll(m);
+            if (root) {
+                up[num] = num;
+                B.csize[i] = num;
+                B.comp[num] = i;
+            }
+        }
+        __syncthreads();
+        for (int i0 = t; i0 < n; i0 += STEP) {
+            int r[M];
+#pragma unroll
+            for (int u = 0; u < M; ++u) r[u] = i0 + u * kUfThreads < n ? pr[i0 + u * kUfThreads] : -1;
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+                if (r[u] >= 0) r[u] = B.csize[r[u]];
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+                if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
+        }
+    }
+    __syncthreads();
+    for (int i0 = t; i0 < n; i0 += STEP) {
+        int a[M], b[M][2];
+        int2 q[M];
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            const int i = i0 + u * kUfThreads;
+            a[u] = i < n ? pr[i] : -1;
+            q[u] = i < n ? nb2[i] : make_int2(-1, -1);
+        }
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            b[u][0] = a[u] >= 0 && q[u].x >= 0 && q[u].x < n ? pr[q[u].x] : -1;
+            b[u][1] = a[u] >= 0 && q[u].y >= 0 && q[u].y < n ? pr[q[u].y] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < M; ++u)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                if (b[u][e] >= 0 && b[u][e] != a[u]) lds_union(up, a[u], b[u][e]);
+    }
+    __syncthreads();
+    for (int i0 = t; i0 < n; i0 += STEP) {
+        int r[M];
+#pragma unroll
+        for (int u = 0; u < M; ++u) r[u] = i0 + u * kUfThreads < n ? pr[i0 + u * kUfThreads] : -1;
+#pragma unroll
+        for (int u = 0; u < M; ++u)
+            if (r[u] >= 0) r[u] = lds_find(up, r[u]);
+        if (numbered) {
+#pragma unroll
+            for (int u = 0; u < M; ++u)
+                if (r[u] >= 0) r[u] = B.comp[r[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < M; ++u)
+            if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
+    }
+    __syncthreads();  // the ids by number are read, the parents written
+    for (int i = t; i < n; i += kUfThreads) B.csize[i] = 0;
+    if (t < 256) {
+        const int p = (int) (((long long) t * n) / 256);
+        up[t] = p < n ? pr[p] : -1;
+    }
+    __syncthreads();
+    if (t < 64) {
+        // the most frequent of the 256 roots, the smaller id on a tie (k_b_giant)
+        int bc = 0, br = -1;
+        for (int u = t; u < 256; u += 64) {
+            const int r = up[u];
+            int c = 0;
+            if (r >= 0)
+                for (int v = 0; v < 256; ++v) c += up[v] == r;
+            if (c > bc || (c == bc && c > 0 && r < br)) {
+                bc = c;
+                br = r;
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const int c2 = __shfl_down(bc, o), r2 = __shfl_down(br, o);
+            if (c2 > bc || (c2 == bc && c2 > 0 && r2 < br)) {
+                bc = c2;
+                br = r2;
+            }
+        }
+        if (t == 0) giant[blockIdx.x] = bc > 0 ? br : -1;
+    }
+}
+
+// The same on global parents, for the subspaces that do not fit (fit null: all).
+__global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, const int *__restrict__ nb,
+                               const int *__restrict__ fit, uint8_t *__restrict__ dsorted, int *__restrict__ par) {
+    if (fit && fit[blockIdx.y]) return;
     const BatchSub &B = subs[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -968,41 +1207,44 @@ __global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, uint8_t
     // parents and sizes, so every write is coalesced
     const int p = B.order[i];
     dsorted[B.base + i] = meets(B.cnt[p], B.thr_dense, B.dbit) ? 1 : 0;
-    par[B.base + i] = meets(B.cnt[i], B.thr_dense, B.dbit) ? i : -1;
+    par[B.base + i] = hooked(B, nb, i);
     B.csize[i] = 0;
 }
 
 // Sample phase of the components: every dense point links to the dense ones
 // among the first kSampleEdges neighbours its count pass recorded (any edges would do:
 // the full phase below links every point outside the giant component to all
-// its dense neighbours, so the result does not depend on the sample).
-// One round per recorded neighbour, with the roots compressed in between, so
-// that the finds of the second round walk short paths (Afforest's rounds).
-__global__ void k_b_link_sample(const BatchSub *__restrict__ subs, int n, const int *__restrict__ nb, int round,
-                                int *__restrict__ par) {
+// its dense neighbours, so the result does not depend on the sample).  It runs
+// on compressed parents, so most edges are decided by two equal parents.
+__global__ void k_b_link_sample(const BatchSub *__restrict__ subs, int n, const int *__restrict__ nb,
+                                const int *__restrict__ fit, int *__restrict__ par) {
+    if (fit && fit[blockIdx.y]) return;
     const BatchSub &B = subs[blockIdx.y];
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     // a point is dense exactly when its parent is set (k_b_dense_init gives
-    // dense points themselves, the others -1, and unions only move roots to
+    // dense points an ancestor, the others -1, and unions only move roots to
     // smaller roots), so the parents answer both density tests without the
     // counts
     int *pr = par + B.base;
     const int pp = pr[p];
     if (pp < 0) return;
-    // the recorded neighbours: min(count, kSampleEdges) of them, -1 after
-    // (phi mode records them too)
-    const int q = nb[kSampleEdges * (B.nbase + p) + round];
-    if (q < 0 || q >= n) return;
-    // after the first round's compression every point's parent is its root:
+    // the recorded neighbours: -1 where there is none (phi mode records them too)
+    int q[kSampleEdges], pq[kSampleEdges];
+#pragma unroll
+    for (int e = 0; e < kSampleEdges; ++e) q[e] = nb[kSampleEdges * (B.nbase + p) + e];
+#pragma unroll
+    for (int e = 0; e < kSampleEdges; ++e) pq[e] = q[e] >= 0 && q[e] < n ? pr[q[e]] : -1;
     // equal parents are one set, decided without reading the root's own entry
     // (which every point of a large component would read at once)
-    const int pq = pr[q];
-    if (pq < 0 || pq == pp) return;
-    uf_union(pr, p, q);
+#pragma unroll
+    for (int e = 0; e < kSampleEdges; ++e)
+        if (pq[e] >= 0 && pq[e] != pp) uf_union(pr, p, q[e]);
 }
 
-__global__ void k_b_uf_compress(const BatchSub *__restrict__ subs, int n, int *__restrict__ par) {
+__global__ void k_b_uf_compress(const BatchSub *__restrict__ subs, int n, const int *__restrict__ fit,
+                                int *__restrict__ par) {
+    if (fit && fit[blockIdx.y]) return;
     int *pr = par + subs[blockIdx.y].base;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n && pr[i] >= 0) pr[i] = uf_find(pr, i);
@@ -1010,8 +1252,9 @@ __global__ void k_b_uf_compress(const BatchSub *__restrict__ subs, int n, int *_
 
 // one block of 256 per subspace: the most frequent root among 256 evenly
 // spaced points
-__global__ void k_b_giant(const BatchSub *__restrict__ subs, int n, const int *__restrict__ par,
-                          int *__restrict__ giant) {
+__global__ void k_b_giant(const BatchSub *__restrict__ subs, int n, const int *__restrict__ fit,
+                          const int *__restrict__ par, int *__restrict__ giant) {
+    if (fit && fit[blockIdx.x]) return;
     __shared__ int roots[256];
     __shared__ int best_c[256];
     __shared__ int best_r[256];
@@ -1565,7 +1808,7 @@ __device__ __forceinline__ int flag_fresh(int J) { return -(4 + 3 * J); }
 // for the grid).  A row is decided by one touched cluster smaller than |T| r, and
 // most rows that the tree touches show one among their first items: every row
 // is probed first, a wave per row, and only the rows left over are walked on
-// in chunks.
+// in chunks (n=100,000 d=20: 25.4 -> 20.7 ms a run; n=10,000 d=15: 1.15 -> 1.09).
 constexpr int kProbe = 256;
 __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__restrict__ blk_off, int nops,
                                 const Entry *__restrict__ E, float r, int *__restrict__ keepv) {
@@ -2090,12 +2333,23 @@ hipError_t launch_b_fan(const BatchSub *groups, const FanJob *jobs, const int *b
 hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, int kfast, const BatchIndex &X,
                                float s_star, hipStream_t st) {
     if (nsub <= 0) return hipSuccess;
-    LAUNCH(k_b_dense_init, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.dsorted, X.par);
-    for (int round = 0; round < kSampleEdges; ++round) {
-        LAUNCH(k_b_link_sample, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.nb, round, X.par);
-        LAUNCH(k_b_uf_compress, dim3(blocks_for(n), nsub), dim3(kBlock), 0, st, subs, n, X.par);
+    // In LDS (one block per subspace) while one block's pass over a subspace is
+    // shorter than the swaps of all blocks on global parents.  Whole runs, d=8,
+    // about 100 subspaces, LDS against global: n=10,000 2.4 / 2.6 ms, 39,936
+    // 6.0 / 7.4, 60,000 9.5 / 11.3, 100,000 21.8 / 24.7, 150,000 39.1 / 41.4,
+    // 200,000 67.1 / 62.3
+    const bool lds_pass = n <= 4 * kUfCap;
+    const int *fit = lds_pass ? X.fit : nullptr;
+    if (lds_pass)
+        LAUNCH(k_b_sample, dim3(nsub), dim3(kUfThreads), 0, st, subs, n, X.nb, X.dsorted, X.par, X.giant, X.fit);
+    if (n > kUfCap) {
+        const dim3 all(blocks_for(n), nsub);
+        LAUNCH(k_b_dense_init, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.dsorted, X.par);
+        LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
+        LAUNCH(k_b_link_sample, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.par);
+        LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
+        LAUNCH(k_b_giant, dim3(nsub), dim3(256), 0, st, subs, n, fit, X.par, X.giant);
     }
-    LAUNCH(k_b_giant, dim3(nsub), dim3(256), 0, st, subs, n, X.par, X.giant);
     const dim3 grid(query_blocks_n(n), nsub);
     const size_t lds = count_lds(kmax);
 #define LINK_FULL(K)                                                                                                   \

@@ -93,3 +93,37 @@ def test_walks_serving_many_children_match_oracle(n, d, eps, dims, rect):
         assert np.array_equal(O.canonical(a), b), f"labels differ in subspace {s}"
     assert np.array_equal(trace, ref.trace)
     assert max(len(s) for s in got.subspaces) >= dims - 1
+
+
+def groups(n, per):
+    """n points in tight groups of `per` on a grid, and each point's group, line and
+    column: n / per groups in the pair of columns (their number decides whether
+    its first parents fit the LDS), the square root of that in either one."""
+    rng = np.random.default_rng(n + per)
+    k = n // per
+    g = int(np.ceil(np.sqrt(k)))
+    at = rng.permutation(np.minimum(np.arange(n) // per, k - 1))
+    X = np.stack([at // g, at % g], 1) + 0.4 + rng.uniform(0, 0.11, (n, 2))
+    return (X / g).astype(np.float32), 0.25 / g, (at // g, at % g, at)
+
+
+# k_b_sample's rules at 39,936 points (ids in LDS up to there) and four times
+# that (global parents above); groups of 3 leave more first parents than fit
+# from 119,808 points on
+@pytest.mark.parametrize("n,per", [(75, 3), (1025, 3), (39936, 3), (39937, 3), (159744, 3), (159744, 4),
+                                   (159745, 3)])
+def test_sample_phase_sizes(n, per):
+    print("sample phase", n, per, flush=True)
+    X, eps, want = groups(n, per)
+    args = (eps, 1.0, 1, 2, 1.0, 4, True)
+    if n < 40000:
+        # groups are the oracle's clusters: every pair in one is within eps,
+        # every other is not
+        ref = O.run_ref(X, *args)
+        assert ref.subspaces == [[0], [1], [0, 1]]
+        for a, b in zip(ref.labels, want):
+            assert np.array_equal(O.canonical(a), O.canonical(b))
+    got = INSCY.run(torch.from_numpy(X).cuda(), *args, 0, mode=_lib.MODE_BATCHED)
+    assert got.subspaces == [[0], [1], [0, 1]]
+    for a, b in zip(got.labels, want):
+        assert np.array_equal(a, O.canonical(b))
