@@ -290,4 +290,25 @@ __device__ __forceinline__ bool same_prefix(const DevData &D, dmask_t restricted
     return true;
 }
 
+// Edges of the eps cells: edge[i] is the smallest coordinate whose cell is at
+// least i - 1 (-inf for i <= 1, +inf past the last cell), i in [0, C + 3).  The
+// cell is monotone in the coordinate, so for a query in cell c the coordinates
+// whose cell is within one of c are exactly [edge[c], edge[c + 3]): the walks
+// test the cells of a candidate on its coordinate, without reading its cells.
+__device__ __forceinline__ float cell_edge(int i, int C) {
+    const int target = i - 1;
+    if (target <= 0) return -__builtin_inff();
+    if (target >= C) return __builtin_inff();
+    const float ecs = ecell_width(C);
+    uint32_t lo = 0, hi = 0x3F800000u;  // cell(0) < target <= cell(1.0) = C - 1
+    while (hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (ecell_of(__uint_as_float(mid), ecs, C) >= target)
+            hi = mid;
+        else
+            lo = mid;
+    }
+    return __uint_as_float(hi);
+}
+
 }  // namespace inscy

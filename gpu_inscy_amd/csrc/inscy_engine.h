@@ -14,9 +14,9 @@
 // mergeWithNeighbors become one flag pass and one filter pass, the weak-density
 // prune is a neighbour-count pass plus compaction, and clustering works on the
 // dense components of S over the whole data set, computed once per subspace.
-// The level-synchronous driver (inscy_level.hip) serves the identity level
-// order, the depth-first one over s-connection chains (inscy_perm.hip) a
-// permuted order.
+// The level-synchronous driver (inscy_level.hip) grows the trees; in a permuted
+// level order they hold s-connection chains in place of the paths
+// (inscy_perm.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -229,18 +229,6 @@ struct HostBuf {
     }
 };
 
-// a tree of the permuted-order driver
-struct TreeRef {
-    dmask_t smask;
-    const int *P;      // device point ids
-    const int *nP;     // device count
-    int nP_max;        // host bound (exact where the host knows it)
-    const int *spx;    // origins of its s-connection chains
-    const uint64_t *chain;  // their chain words
-    const int *nsp;
-    int nsp_max;
-};
-
 // What the algorithm needs about one subspace S, computed on first use:
 // neighbour counts of every point (the prune reads them for its region), then,
 // once a tree of S survives its prune, the dense components of S over the
@@ -265,11 +253,10 @@ public:
             event_pool().put(t.start);
             event_pool().put(t.stop);
         }
-        for (void *p : {(void *) Xt, (void *) cellC, (void *) cellE, (void *) nearm, (void *) small, (void *) stamp,
-                        (void *) qmark, (void *) entries, (void *) scratch, (void *) rank_perm,
+        for (void *p : {(void *) Xt, (void *) cellC, (void *) cellE, (void *) nearm, (void *) small,
+                        (void *) entries, (void *) rank_perm,
                         (void *) d_level, (void *) edges, (void *) rows})
             if (p) dev_free(p);
-        if (pin) host_free(pin);
     }
 
     // ---------------------------------------------------------- set-up
@@ -291,6 +278,8 @@ public:
                 std::max(prm.F * alpha_thr(k, prm.neighborhood_size, n), (float) prm.num_obj * omega_thr(k)));
 
         mw = d <= 64 ? 1 : 2;
+        permuted = prm.entropy_order != 0;
+        pw = permuted ? 1 : mw;
         size_t nd = (size_t) n * d;
         HIP_OK(dev_alloc(&Xt, nd * sizeof(float)));
         HIP_OK(dev_alloc(&cellC, nd));
@@ -298,25 +287,15 @@ public:
         HIP_OK(dev_alloc(&nearm, (size_t) n * sizeof(dmask_t)));
         HIP_OK(dev_alloc(&rows, (size_t) n * cell_row_bytes(d)));
         HIP_OK(dev_alloc(&small, kSmallWords * sizeof(unsigned long long)));
-        if (!levels_mode) {
-            HIP_OK(dev_alloc(&stamp, (size_t) n * sizeof(int)));
-            HIP_OK(dev_alloc(&qmark, (size_t) n * sizeof(int)));
-        }
-        HIP_OK(host_alloc(&pin, pin_bytes()));
         grow_entries(1 << 12);
         // grid index size: C^j cells with j <= 3 and C^j <= max(8n, 4096)
         grid_cap = std::max<long long>(8LL * n, 4096);
         grid_cap = std::max<long long>(std::min<long long>(grid_cap, 1LL << 24), ecells);
         scan_bytes = scan_temp_bytes((int) grid_cap + 1);
-        // arena: per recursion level the partitions of all children of one tree
-        // (points, weak-dense points, paths) plus one child's pruned paths,
-        // and the scratch of one subspace grid pass
-        size_t per_level = (size_t) 24 * d * n + (size_t) 64 * n;
-        size_t pass = (size_t) n * (32 + (size_t) d * 6) + (size_t) (grid_cap + 1) * 8 + scan_bytes + (1u << 20);
-        size_t want = per_level * (size_t) (d + 2) + table_bytes_max() + pass + (size_t) n * 16 + (64u << 20);
-        // the level-synchronous driver keeps its lists in pools; its arena holds
-        // the replay's label flags (one per open dimension) and the emit buffers
-        if (levels_mode) want = (size_t) n * (d + 8) + pass + (64u << 20);
+        // arena: the scratch of the set-up and of one subspace grid pass (the
+        // driver keeps its lists in pools)
+        const size_t pass = (size_t) n * (32 + (size_t) d * 6) + (size_t) (grid_cap + 1) * 8 + scan_bytes + (1u << 20);
+        size_t want = (size_t) n * (d + 8) + pass + (64u << 20);
         available = device_available_bytes() / (size_t) mem_share;
         if (available) want = std::min(want, available / 3);
         arena.init(want);
@@ -325,10 +304,6 @@ public:
         FillMany fill;
         fill.add(small, 0, kSmallWords * sizeof(unsigned long long));
         fill.add(hist, 0, (size_t) d * ecells * sizeof(int));
-        if (!levels_mode) {
-            fill.add(stamp, ~0u, (size_t) n * sizeof(int));
-            fill.add(qmark, ~0u, (size_t) n * sizeof(int));
-        }
         HIP_OK(launch_fill_many(fill, st));
         HIP_OK(launch_discretise(d_X, n, d, cells, prm.neighborhood_size, Xt, cellC, cellE,
                                  prm.entropy_order == 0 ? rows : nullptr, reinterpret_cast<uint64_t *>(nearm), 2, reinterpret_cast<int *>(small), st));
@@ -337,13 +312,14 @@ public:
         int *histc = arena.take<int>((size_t) d * cells);
         if (prm.entropy_order != 0) HIP_OK(launch_histc(cellC, n, d, cells, histc, st));
         std::vector<int> hc((size_t) d * cells);
-        const int *h = reinterpret_cast<const int *>(down.get((size_t) d * ecells * sizeof(int)));
-        HIP_OK(hipMemcpyAsync(pin, small, sizeof(int), hipMemcpyDeviceToHost, st));
+        const int *h = reinterpret_cast<const int *>(down.get(((size_t) d * ecells + 1) * sizeof(int)));
+        const int *bad = h + (size_t) d * ecells;
+        HIP_OK(hipMemcpyAsync(const_cast<int *>(bad), small, sizeof(int), hipMemcpyDeviceToHost, st));
         HIP_OK(hipMemcpyAsync(down.p, hist, (size_t) d * ecells * sizeof(int), hipMemcpyDeviceToHost, st));
         if (prm.entropy_order != 0)
             HIP_OK(hipMemcpyAsync(hc.data(), histc, hc.size() * sizeof(int), hipMemcpyDeviceToHost, st));
         sync();
-        if (reinterpret_cast<int *>(pin)[0] != 0)
+        if (*bad != 0)
             throw Failure(INSCY_ERR_ARGUMENT, "X must be finite with every value in [0, 1] (normalize first)");
         // selectivity of each dimension as an index: expected candidates of a
         // query in the three-cell slab, sum_c h_c (h_{c-1} + h_c + h_{c+1})
@@ -377,12 +353,12 @@ public:
         }
         lvl_of.assign(d, 0);
         for (int t = 0; t < d; ++t) lvl_of[level[t]] = t;
-        if (!levels_mode) {  // the level-synchronous driver knows its order: the identity
+        if (permuted) {
             HIP_OK(dev_alloc(&d_level, (size_t) 2 * d * sizeof(int)));
             std::vector<int> both(level);
             both.insert(both.end(), lvl_of.begin(), lvl_of.end());
             HIP_OK(hipMemcpyAsync(d_level, both.data(), both.size() * sizeof(int), hipMemcpyHostToDevice, st));
-            if (prm.entropy_order != 0) HIP_OK(launch_cell_rows(cellC, n, d, d_level, rows, st));
+            HIP_OK(launch_cell_rows(cellC, n, d, d_level, rows, st));
             sync();  // `both` is pageable and goes out of scope
         }
         if (phi_mode) {
@@ -401,12 +377,8 @@ public:
     }
 
     // ---------------------------------------------------------- run
-    // level-synchronous driver (the identity level order)
+    // level-synchronous driver (inscy_level.hip)
     void run_levels(inscy_result &out);
-    bool levels_mode = false;
-    // permuted SCY-tree level order (entropy_order != 0): the depth-first
-    // driver over s-connection chains (inscy_perm.hip)
-    void run_perm(inscy_result &out);
     // learned pruner (INSCY_MODE_LEARNED): device bf16 parameters, the score
     // below which a (tree, dimension) pair is skipped, and the smallest |S| of
     // a tree whose pairs may be skipped; pair collection (INSCY_MODE_COLLECT)
@@ -421,7 +393,18 @@ public:
     int max_batch_override = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
 
     // dense components of one subspace (kernel-level entry point)
-    const Subspace &subspace(dmask_t smask) { return ensure_components(smask); }
+    const int *components(dmask_t smask) {
+        Subspace &s = sub_of(smask);
+        SubspaceArg S = arg_of(smask);
+        GridArg G = grid_of(S);
+        s.comp = slabs.take<int>(n);
+        s.csize = slabs.take<int>(n);
+        size_t mk = arena.mark();
+        GridBuffers B = grid_buffers(S, G);
+        HIP_OK(launch_subspace_components(D, S, G, s_star, cap_of(S.k), dense_thr[S.k], B, s.cnt, s.comp, s.csize, st));
+        arena.release(mk);
+        return s.comp;
+    }
 
     // exact |N_S(p)| of every point, without the threshold cap (kernel-level entry point)
     const int *exact_counts(dmask_t smask) {
@@ -430,7 +413,7 @@ public:
         GridArg G = grid_of(S);
         size_t mk = arena.mark();
         GridBuffers B = grid_buffers(S, G);
-        HIP_OK(launch_subspace_counts(D, S, G, s_star, INT_MAX, B, nullptr, 0, s.cnt, nullptr, KernelTimer{}, st));
+        HIP_OK(launch_subspace_counts(D, S, G, s_star, INT_MAX, B, s.cnt, st));
         arena.release(mk);
         return s.cnt;
     }
@@ -451,18 +434,6 @@ private:
     // [kStatAt..) 64 slot pairs (16 words apart) of neighbour-count statistics
     static constexpr int kStatAt = 32;
     static constexpr int kSmallWords = kStatAt + 16 * 64;
-    size_t pin_bytes() const {
-        return std::max<size_t>((size_t) n * 8 + (size_t) 2 * d * 256 * 8 + (1u << 16), 1u << 20);
-    }
-    static size_t table_slots(int nW, int bits) {
-        size_t want = (size_t) std::max(1, nW) * (size_t) std::max(1, bits) * 2;
-        size_t s = 1024;
-        while (s < want) s <<= 1;
-        return s;
-    }
-    size_t table_bytes_max() const { return table_slots(n, d) * sizeof(uint64_t); }
-    int *pin_i(size_t off = 0) { return reinterpret_cast<int *>(pin) + off; }
-
     void sync() {
         flush_uploads();
         HIP_OK(hipStreamSynchronize(st));
@@ -493,30 +464,14 @@ private:
         if (want <= ecap) return;
         int cap = std::max(want, 2 * ecap);
         Entry *ne = nullptr;
-        int *ns = nullptr;
         HIP_OK(dev_alloc(&ne, (size_t) cap * sizeof(Entry)));
-        // scratch: nE, nlist, keep, pad | list[cap] | mn[cap] | keepf[n], drop[n], fresh[n] (bytes)
-        HIP_OK(dev_alloc(&ns, (size_t) (8 + 2 * cap) * sizeof(int) + (size_t) 3 * n + 256));
         if (entries) {
             sync();
             HIP_OK(hipMemcpy(ne, entries, (size_t) nentries * sizeof(Entry), hipMemcpyDeviceToDevice));
             dev_free(entries);
-            dev_free(scratch);
         }
         entries = ne;
-        scratch = ns;
         ecap = cap;
-        d_nE = scratch;
-        d_nlist = scratch + 1;
-        d_keep = scratch + 2;
-        d_list = scratch + 8;
-        d_mn = scratch + 8 + cap;
-        keepf = reinterpret_cast<uint8_t *>(scratch + 8 + 2 * cap);
-        dropf = keepf + n;
-        freshf = dropf + n;
-        if (levels_mode) return;  // the scratch serves the permuted-order driver
-        HIP_OK(launch_fill_i32(d_mn, INT_MAX, cap, st));
-        HIP_OK(launch_fill_i32(d_nE, nentries, 1, st));
     }
 
     SubspaceArg arg_of(dmask_t smask) const {
@@ -601,107 +556,10 @@ private:
         return s;
     }
 
-    // phi mode (rectangular = false): the decision bits of the points of S
-    // without a value, stamped markid when mark is given (the permuted-order
-    // driver's density): the grid pass decides a point whose thresholds lie
-    // outside the rounding band of its double scan-order sum (2^-22 per term,
-    // as in the level-synchronous passes); the others are summed again in the
-    // neighbourhood tree's leaf order
-    void phi_points(dmask_t smask, Subspace &s, const int *mark, int markid) {
-        BatchSub x;
-        std::memset(&x, 0, sizeof(x));
-        x.S = arg_of(smask);
-        x.matchmask = match_of(x.S);
-        x.phi_w = phi_weak;
-        x.phi_d = phi_dense[x.S.k];
-        x.dbit = 2;
-        x.cnt = s.cnt;
-        const GridArg G = grid_of(x.S);
-        size_t mk = arena.mark();
-        BatchSub *dx = arena.take<BatchSub>(1);
-        put(dx, &x, sizeof(x));
-        int2 *fb = arena.take<int2>(n);
-        int *nfb = arena.take<int>(1);
-        GridBuffers B = grid_buffers(x.S, G);
-        flush_uploads();
-        const double phirel = phi_all_exact ? 1e30 : 1.0 / 4194304.0;
-        HIP_OK(launch_subspace_phi(D, x.S, G, B, s_star, prm.neighborhood_size, phirel, x.phi_w, x.phi_d, mark, markid,
-                                   s.cnt, fb, nfb, n, st));
-        HIP_OK(launch_phi_exact(D, dx, fb, nfb, n, rank_perm, prm.neighborhood_size, s_star, st));
-        arena.release(mk);  // stream order keeps the buffers for the queued kernels
-    }
-
-    // |N_S(p)| of the points stamped with markid that are not counted yet
-    // (phi mode: their decision bits).
-    Subspace &ensure_counts(dmask_t smask, int markid) {
-        Subspace &s = sub_of(smask);
-        if (s.entry >= 0) return s;  // all points counted by the components pass
-        if (phi_mode) {
-            phi_points(smask, s, qmark, markid);
-            return s;
-        }
-        SubspaceArg S = arg_of(smask);
-        GridArg G = grid_of(S);
-        size_t mk = arena.mark();
-        GridBuffers B = grid_buffers(S, G);
-        HIP_OK(launch_subspace_counts(D, S, G, s_star, cap_of(S.k), B, qmark, markid, s.cnt, small + kStatAt, timer(),
-                                      st));
-        arena.release(mk);
-        return s;
-    }
-
-    // Dense components of S (counting every point not yet counted) and its
-    // result-table row, once per subspace.
-    Subspace &ensure_components(dmask_t smask) {
-        Subspace &s = sub_of(smask);
-        if (s.entry >= 0) return s;
-        SubspaceArg S = arg_of(smask);
-        GridArg G = grid_of(S);
-        s.comp = slabs.take<int>(n);
-        s.csize = slabs.take<int>(n);
-        s.inres = slabs.take<uint8_t>(n);
-        int *mem = slabs.take<int>(n);
-        // a subspace S' = S minus one dimension whose counts are complete bounds
-        // the counts of S from above (exact where below its own cap); phi
-        // mode decides every remaining point in leaf order first
-        const int *bound = nullptr;
-        int lo = std::min(weak_thr, dense_thr[S.k]);
-        if (phi_mode) phi_points(smask, s, nullptr, 0);
-        for (int t = 0; t < S.k && !bound && !phi_mode; ++t) {
-            const dmask_t sub = smask & ~dbit(S.dims[t]);
-            auto it = subs.find(sub);
-            if (sub && it != subs.end() && it->second.entry >= 0) {
-                bound = it->second.cnt;
-                lo = std::min(lo, cap_of(S.k - 1));
-            }
-        }
-        size_t mk = arena.mark();
-        GridBuffers B = grid_buffers(S, G);
-        HIP_OK(launch_subspace_components(D, S, G, s_star, cap_of(S.k), lo, dense_thr[S.k], phi_mode ? 2 : 0, B, bound,
-                                          s.cnt, s.comp, s.csize, small + kStatAt, timer(), st));
-        arena.release(mk);
-        HIP_OK(launch_fill_u8(s.inres, 0, n, st));
-        grow_entries(nentries + 1);
-        Entry e{smask, s.comp, s.csize, s.inres, mem, 0, 0};
-        s.entry = nentries++;
-        HIP_OK(launch_set_entry(entries, s.entry, e, d_nE, nentries, st));
-        stats.components++;
-        return s;
-    }
-
-    // ---------------------------------------------------------- recursion
     struct Group {
         int lo, hi;
     };
 
-    void recurse_perm(const TreeRef &T, int first);
-
-    // join (util.cu:655-743), on the device
-    void join(dmask_t smask, const uint8_t *lab) {
-        Subspace &s = ensure_components(smask);
-        HIP_OK(launch_join(lab, n, s.comp, s.csize, prm.min_size, prm.r, entries, d_nE, smask, s.entry, s.inres,
-                           d_list, d_nlist, keepf, dropf, freshf, st));
-    }
 
     // Result in the reference's order (ascending bitmask == vec_cmp,
     // util.cu:633-653) with canonical labels computed on the device, read back
@@ -847,11 +705,9 @@ private:
     uint8_t *rows = nullptr;  // cells by point and SCY-tree level
     dmask_t *nearm = nullptr;
     int mw = 1;  // words per path mask: 1 for d <= 64, else 2
+    bool permuted = false;  // levels in entropy order: trees hold chains (inscy_perm.hip)
+    int pw = 1;             // words per path: a mask, or one chain word
     unsigned long long *small = nullptr;
-    int *stamp = nullptr;
-    int *qmark = nullptr;  // [n] stamp of the tree whose points are being counted
-    int mark_id = 0;
-    void *pin = nullptr;
     std::vector<double> score;  // per-dimension index selectivity (lower is better)
     long long grid_cap = 0;
     size_t scan_bytes = 0;
@@ -861,11 +717,7 @@ private:
     std::unordered_map<dmask_t, Subspace, DMaskHash> subs;
     // device result table
     Entry *entries = nullptr;
-    int *scratch = nullptr;
     int ecap = 0, nentries = 0;
-    int *d_nE = nullptr, *d_nlist = nullptr, *d_keep = nullptr, *d_list = nullptr, *d_mn = nullptr;
-    uint8_t *keepf = nullptr, *dropf = nullptr, *freshf = nullptr;
-    int tree_id = 0;
 
     // ---------------------------------------------------------- level-synchronous driver state
     struct LTree {
@@ -954,6 +806,7 @@ private:
     int *keepv = nullptr;
     int rep_join = 0;  // number of the last join
     void set_bounds(dmask_t s, BatchSub &x);
+    PermStep perm_step(dmask_t s, int m) const;
     void trace_tree(int f, const std::vector<int> &keep);
     std::vector<KernelTimer> timers;
     // pairs of the level: first pair of each active tree, pruner decisions

@@ -48,9 +48,9 @@ static int check_params(int64_t n, int32_t d, const inscy_params *p, int32_t mod
     if (p->number_of_cells < 1 || p->number_of_cells > 255)
         return fail(INSCY_ERR_ARGUMENT, "number_of_cells must be in [1, 255]");
     if (mode < INSCY_MODE_EXACT || mode > INSCY_MODE_COLLECT) return fail(INSCY_ERR_ARGUMENT, "unknown mode");
-    // A permuted SCY-tree level order runs the depth-first driver over
-    // s-connection chains (inscy_perm.hip), with neighbour-count density or,
-    // for rectangular = false, phi summed in the neighbourhood tree's leaf order.
+    // A permuted SCY-tree level order has its trees hold s-connection chains
+    // (inscy_perm.hip), with neighbour-count density or, for rectangular =
+    // false, phi summed in the neighbourhood tree's leaf order.
     if (p->entropy_order != 0) {
         if (mode == INSCY_MODE_LEARNED || mode == INSCY_MODE_COLLECT)
             return fail(INSCY_ERR_UNSUPPORTED, "entropy_order != 0 runs the exact drivers only");
@@ -120,21 +120,17 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.max_batch_override = g_max_batch;
             eng.profile_on = g_profile_on;
             eng.mem_share = mem_share;
-            // one driver serves every mode of the identity order: the
-            // level-synchronous one gives the depth-first recursion's result,
-            // trees and decisions in a fraction of its launches (n=4,999 d=11:
-            // 12,556 dispatches and 58 ms one tree at a time, 240 and 3.9 ms)
-            eng.levels_mode = p->entropy_order == 0;
+            // one driver serves every mode and level order: the level-synchronous
+            // one gives the depth-first recursion's result, trees and decisions
+            // in a fraction of its launches (n=4,999 d=11: 12,556 dispatches and
+            // 58 ms one tree at a time, 240 and 3.9 ms)
             eng.collect = mode == INSCY_MODE_COLLECT;
             if (mode == INSCY_MODE_LEARNED) {
                 eng.pruner = pruner_on_device(eng.prune_thr, eng.prune_min_depth);
                 if (!eng.pruner) throw Failure(INSCY_ERR_ARGUMENT, "INSCY_MODE_LEARNED needs a network (inscy_set_pruner)");
             }
             eng.setup(d_X);
-            if (p->entropy_order != 0)
-                eng.run_perm(*res);
-            else
-                eng.run_levels(*res);
+            eng.run_levels(*res);
             res->stats = eng.stats;
             if (g_trace_on) g_trace = eng.trace;
         }
@@ -611,7 +607,7 @@ int inscy_dense_components(const float *d_X, int64_t n, int32_t d, const inscy_p
     try {
         Engine eng(*p, (int) n, d, nullptr);
         eng.setup(d_X);
-        const int *comp = eng.subspace(mask_from(dims, k, d)).comp;
+        const int *comp = eng.components(mask_from(dims, k, d));
         HIP_OK(hipMemcpyAsync(d_comp, comp, (size_t) n * sizeof(int), hipMemcpyDeviceToDevice, nullptr));
         HIP_OK(hipDeviceSynchronize());
         return INSCY_OK;

@@ -34,6 +34,10 @@ __host__ __device__ __forceinline__ int dcount(dmask_t m) {
 __host__ __device__ __forceinline__ int dfirst(dmask_t m) {
     return dlo(m) ? __builtin_ctzll(dlo(m)) : 64 + __builtin_ctzll(dhi(m));
 }
+// highest dimension of a mask, -1 when it is empty
+__host__ __device__ __forceinline__ int dlast(dmask_t m) {
+    return dhi(m) ? 127 - __builtin_clzll(dhi(m)) : dlo(m) ? 63 - __builtin_clzll(dlo(m)) : -1;
+}
 static_assert(sizeof(dmask_t) == 16 && alignof(dmask_t) == 16, "one layout on host and device");
 // Arrays of s-connection path masks hold mw 64-bit words per entry: 1 when
 // d <= 64 (half the bytes of the partitions and path lists), 2 above.
@@ -222,6 +226,7 @@ struct PartPair {
     const uint64_t *spm;  // mw words per path
     const int *gid;      // [cells]
     const int *weakcnt;  // counts of S ∪ {m}
+    const uint8_t *keep; // [nP] the points that count (null: all)
     int *cnt;            // [7G]: points, weak-dense points, paths per group; 3 cursors; the paths' branch levels
     int *outW;
     int *outx;
@@ -242,6 +247,59 @@ struct PruneChild {
     uint64_t *outm;
     int *nout;
     int nW, nsp, bw, mw;
+};
+
+// Permuted level order (inscy_perm.hip): what the restriction of a tree of mask S
+// on dimension m does to its nodes, as level masks (bit t for level t).
+struct PermStep {
+    dmask_t tree;        // levels S restricts
+    dmask_t restricted;  // and m's
+    dmask_t big;         // levels free in S, not m's, of a dimension above m
+    dmask_t cond;        // levels above m's kept empty by a larger dimension id below them
+    int m, Lm;           // the dimension and its level
+    int tkey;            // deepest free level above m's (-1: none)
+    int filt;            // a merged group keeps the points under a prefix of its first cell only
+};
+// the chains of one (tree, dimension) pair, counted by where they go: in[g],
+// group g of their cell; out[g], every group but g
+struct PermPair {
+    PermStep s;
+    const int *spx;
+    const uint64_t *chain;
+    const int *gid;
+    int *in, *out;
+    int nsp, G;
+};
+// the point filter of one pair whose step has `filt`
+struct PermFilter {
+    PermStep s;
+    const int *P;
+    const int *gid;
+    uint64_t *table;
+    uint64_t tmask;
+    uint8_t *keep;  // [nP]
+    int nP;
+};
+// a surviving child's chains: routed out of its parent's, then pruned
+struct PermChild {
+    PermStep s;
+    dmask_t *bits;       // levels of the prefixes asked for
+    const int *spx;      // the parent's chains
+    const uint64_t *chain;
+    const int *gid;
+    const int *P;        // the parent's points
+    const uint8_t *keep;
+    const int *weakcnt;
+    uint64_t *table;     // prefixes asked for
+    uint64_t tmask;
+    uint8_t *marks;      // [2 * slots]: a weak-dense point, an existing node
+    int *rx;             // [nr] routed chains
+    uint64_t *rw;
+    int *nr_at;
+    int *outx;
+    uint64_t *outw;
+    int *nout;
+    int nsp, nP, nr, g;
 };
 
 // pad < 0: dst[i] = src[i]; else dst[src[i]] = pad (the tree stamps of the replay)
@@ -283,28 +341,13 @@ hipError_t launch_cell_rows(const uint8_t *cellC, int n, int d, const int *level
 hipError_t launch_hist1(const uint16_t *cellE, int n, int d, int ecells, int *hist, hipStream_t st);
 // occupancy of the c-grid per dimension ([d][cells]), the input of the entropy order
 hipError_t launch_histc(const uint8_t *cellC, int n, int d, int cells, int *hist, hipStream_t st);
-// |N_S(p)| (capped at `cap`) of the points with cnt == -1 and, when mark is
-// given, mark[p] == markid (stat: candidates examined, points counted)
+// |N_S(p)| (capped at `cap`) of the points with cnt == -1
 hipError_t launch_subspace_counts(const DevData &D, const SubspaceArg &S, const GridArg &G, float s_star, int cap,
-                                  const GridBuffers &B, const int *mark, int markid, int *cnt,
-                                  unsigned long long *stat, const KernelTimer &tm, hipStream_t st);
-// remaining counts, then the dense components of S (comp = smallest member id or -1)
-// (bound: complete counts of a subspace of S, or null; lo: the smaller threshold of S)
-// dbit != 0: cnt holds phi decision bits and bit dbit is the dense test
+                                  const GridBuffers &B, int *cnt, hipStream_t st);
+// counts, then the dense components of S (comp = smallest member id or -1)
 hipError_t launch_subspace_components(const DevData &D, const SubspaceArg &S, const GridArg &G, float s_star,
-                                      int cap, int lo, int thr_dense, int dbit, const GridBuffers &B, const int *bound,
-                                      int *cnt, int *comp, int *csize, unsigned long long *stat,
-                                      const KernelTimer &tm, hipStream_t st);
-hipError_t launch_mark(const int *P, const int *nP, int nP_max, int *mark, int markid, hipStream_t st);
-hipError_t launch_partition(const int *P, const int *nP, int nP_max, const uint8_t *cellC_m, const int *gid, int G,
-                            const int *weakcnt, int thr, int wbit, int *cnt, int *outP, int *outW, hipStream_t st);
-hipError_t launch_redundancy_seed(const int *W, const int *nW_dev, int nW, int *stamp, int tid, const Entry *E,
-                                  const int *nE, dmask_t smask, const int *comp, int *list, int *nlist, int *mn,
-                                  float r, int *keep, uint8_t *lab, hipStream_t st);
-hipError_t launch_join(const uint8_t *lab, int n, const int *compS, const int *csizeS, int min_size, float r,
-                       Entry *E, const int *nE, dmask_t smask, int eS, uint8_t *inresS, int *list, int *nlist,
-                       uint8_t *keepf, uint8_t *drop, uint8_t *fresh, hipStream_t st);
-hipError_t launch_set_entry(Entry *E, int idx, const Entry &e, int *nE, int count, hipStream_t st);
+                                      int cap, int thr_dense, const GridBuffers &B, int *cnt, int *comp, int *csize,
+                                      hipStream_t st);
 // canonical labels of r result subspaces: flags and idx hold r*n + 1 ints,
 // labels r*n, counts r (clusters per row)
 struct EmitRow {
@@ -315,7 +358,6 @@ struct EmitRow {
 // uint8 / uint16, for rows with at most 255 / 65535 clusters)
 hipError_t launch_emit(const EmitRow *rows, int r, int n, int *flags, int *idx, void *labels, int width, int *counts,
                        void *scan_temp, size_t scan_bytes, hipStream_t st);
-hipError_t launch_fill_u8(uint8_t *p, uint8_t v, size_t count, hipStream_t st);
 hipError_t launch_fill_i32(int *p, int v, size_t count, hipStream_t st);
 // several arrays filled with 32-bit words in one launch (16-byte aligned; add
 // returns the array)
@@ -337,12 +379,21 @@ struct FillMany {
 };
 hipError_t launch_fill_many(const FillMany &f, hipStream_t st);
 hipError_t launch_gather(const int *src, const int *idx, int count, int *out, hipStream_t st);
-hipError_t launch_iota(int *p, int n, hipStream_t st);
 
 // the root tree: points 0..n, its s-connection paths (their number added to
 // *nout), and the edges of the C eps cells (C + 3 floats, see cell_edge)
 hipError_t launch_b_root(const dmask_t *nearm, int n, int *P, int *outx, uint64_t *outm, int mw, int *nout, int C,
                          float *edge, hipStream_t st);
+// the same in a permuted level order: one chain per near-edge dimension of a point
+hipError_t launch_p_root(const dmask_t *nearm, int n, int d, int *P, int *cx, uint64_t *cw, int *nout, int C,
+                         float *edge, hipStream_t st);
+hipError_t launch_p_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
+                          int cells, int *flags, hipStream_t st);
+hipError_t launch_p_filter(const DevData &D, const PermFilter *F, const int *blk_off, int nf, int nblk, hipStream_t st);
+hipError_t launch_p_count(const DevData &D, const PermPair *P, const int *blk_off, int np, int nblk, hipStream_t st);
+hipError_t launch_p_prune(const DevData &D, const PermChild *C, int nc, const int *blk_route, int nblk_route,
+                          const int *blk_mark, int nblk_mark, const int *blk_check, int nblk_check, int thr, int wbit,
+                          hipStream_t st);
 // level-synchronous passes (blk_off: per-segment block offsets, nblk = blk_off[nseg])
 hipError_t launch_b_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
                           int cells, int *flags, hipStream_t st);
@@ -365,13 +416,6 @@ hipError_t launch_b_count(const BatchSub *subs, int nsub, const int *blk_off, in
                           const BatchIndex &X, float s_star, float eps, bool phi, bool phi_all_exact,
                           const DevData &D, const int *rank_order, unsigned long long *stat, const KernelTimer &tm,
                           hipStream_t st);
-// phi decision bits of the points of one subspace without a value (cnt ==
-// -1; stamped markid when mark is given), from the grid pass of S: decided
-// where a threshold lies outside the rounding band (phirel per term), the
-// others listed in fb (capacity fbcap, count in nfb) as (0, point)
-hipError_t launch_subspace_phi(const DevData &D, const SubspaceArg &S, const GridArg &G, const GridBuffers &B,
-                              float s_star, float eps, double phirel, float phi_w, float phi_d, const int *mark,
-                              int markid, int *cnt, int2 *fb, int *nfb, int fbcap, hipStream_t st);
 // the listed points' phi summed in the neighbourhood tree's leaf order
 // (rank_order), stored in sub's cnt (sub: one device BatchSub with S,
 // matchmask, phi_w, phi_d and cnt)

@@ -96,57 +96,6 @@ __global__ void k_histc(const uint8_t *__restrict__ cellC, int n, int d, int cel
     atomicAdd(&hist[(size_t) k * cells + cellC[i]], 1);
 }
 
-// ------------------------------------------------------------ expansion of one tree (permuted level order)
-// Counting-sort partition of a tree's points and weak-dense points by the cell
-// group of dimension m (restrict + mergeWithNeighbors for every group at once).
-// cnt[0..G): points, [G..2G): weak-dense points; [2G..4G): scatter cursors.
-struct PartArg {
-    const int *P;
-    const int *nP;
-    const uint8_t *cellC_m;
-    const int *gid;      // [cells] group of each cell of m
-    const int *weakcnt;  // neighbour counts (or phi decision bits) of the subspace S ∪ {m}
-    int thr, G, wbit;
-};
-
-__global__ void k_part_count(PartArg A, int *__restrict__ cnt) {
-    __shared__ int h[2 * 256];
-    for (int t = threadIdx.x; t < 2 * A.G; t += blockDim.x) h[t] = 0;
-    __syncthreads();
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < *A.nP) {
-        int p = A.P[i];
-        int g = A.gid[A.cellC_m[p]];
-        atomicAdd(&h[g], 1);
-        if (meets(A.weakcnt[p], A.thr, A.wbit)) atomicAdd(&h[A.G + g], 1);
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < 2 * A.G; t += blockDim.x)
-        if (h[t]) atomicAdd(&cnt[t], h[t]);
-}
-
-__global__ void k_part_scatter(PartArg A, int *__restrict__ cnt, int *__restrict__ outP, int *__restrict__ outW) {
-    __shared__ int base[2 * 256];
-    if (threadIdx.x < 2) {
-        int acc = 0;
-        for (int g = 0; g < A.G; ++g) {
-            base[threadIdx.x * A.G + g] = acc;
-            acc += cnt[threadIdx.x * A.G + g];
-        }
-    }
-    __syncthreads();
-    int *cur = cnt + 2 * A.G;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool in = i < *A.nP;
-    int p = in ? A.P[i] : 0;
-    int g = in ? A.gid[A.cellC_m[p]] : 0;
-    bool weak = in && meets(A.weakcnt[p], A.thr, A.wbit);
-    int sp = wave_add_by_key(cur, g, in);
-    int sw = wave_add_by_key(cur + A.G, g, weak);
-    if (in) outP[base[g] + sp] = p;
-    if (weak) outW[base[A.G + g] + sw] = p;
-}
-
 // ------------------------------------------------------------ epsilon neighbourhood: subspace grid pass
 // Candidate rule of get_possible_neighbors_from (ScyTreeNode.cu:896-946) on
 // the ceil(1/eps)-grid: |cell_e(q) - cell_e(p)| <= 1 in every dimension of S;
@@ -186,16 +135,13 @@ __global__ void k_grid_scatter(DevData D, SubspaceArg S, const int *__restrict__
 }
 
 
-// |N_S(p)| of the points still uncounted (cnt == -1) and, when `mark` is
-// given, stamped with `markid`.  Counting stops once `cap` neighbours are
-// found: every comparison the algorithm makes with a count is against a
+// |N_S(p)| of the points still uncounted (cnt == -1).  Counting stops once
+// `cap` neighbours are found: every comparison made with a count is against a
 // threshold <= cap, so min(|N_S(p)|, cap)-or-more decides them all.
 __global__ __launch_bounds__(kBlock) void k_grid_count(int n, SubspaceArg S, GridArg G, const int *__restrict__ off,
                                                        const int *__restrict__ order, const float *__restrict__ Ys,
                                                        const uint16_t *__restrict__ Es, float s_star, int cap,
-                                                       const int *__restrict__ mark, int markid,
-                                                       const int *__restrict__ bound, int lo, int *__restrict__ cnt,
-                                                       unsigned long long *__restrict__ stat) {
+                                                       int *__restrict__ cnt) {
     constexpr int LPQ = kLanesPerQuery, QPB = kBlock / LPQ;
     extern __shared__ char smem[];
     float *sy = reinterpret_cast<float *>(smem);
@@ -203,20 +149,9 @@ __global__ __launch_bounds__(kBlock) void k_grid_count(int n, SubspaceArg S, Gri
     const int lq = threadIdx.x / LPQ, sub = threadIdx.x % LPQ;
     const int i = blockIdx.x * QPB + lq;
     int p = i < n ? order[i] : 0;
-    bool active = i < n && cnt[p] < 0 && (!mark || mark[p] == markid);
-    // N_S(p) is a subset of N_S'(p) for S' a subset of S (the rounded distance
-    // sum only grows with more dimensions), so a complete count of a subspace
-    // of S below both thresholds of S decides p without a scan.
-    if (active && bound) {
-        int b = bound[p];
-        if (b >= 0 && b < lo) {
-            if (sub == 0) cnt[p] = b;
-            active = false;
-        }
-    }
+    const bool active = i < n && cnt[p] < 0;
     if (sub == 0 && active) stage_query(S, n, Ys, Es, i, sy + lq, se + lq, QPB);
     __syncthreads();
-    long long seen = 0;
     int found = 0;
     if (active) {
         const float *qy = sy + lq;
@@ -227,109 +162,20 @@ __global__ __launch_bounds__(kBlock) void k_grid_count(int n, SubspaceArg S, Gri
                 int jj = base + sub;
                 bool hit = jj < b && jj != i && is_neighbour(S, G, n, Ys, Es, qy, qe, QPB, jj, s_star);
                 found += __popcll((__ballot(hit) >> gshift) & ((1ull << LPQ) - 1ull));
-                seen += min(LPQ, b - base);
             }
         });
         if (sub == 0) cnt[p] = found;
-    }
-    if (stat) {
-        // per wave, into one of 64 slot groups (16 words apart): [0] candidates
-        // examined, [1] points counted, [2] algorithmic bytes = per point the
-        // query's k coordinates and its count (4k + 4) plus, per neighbour
-        // established, its id and k coordinates (4 + 4k)
-        const bool mine = sub == 0 && active;
-        long long done = mine ? 1 : 0;
-        long long abytes = mine ? (4ll * S.k + 4) + (long long) found * (4 + 4ll * S.k) : 0;
-        if (sub != 0) seen = 0;
-        for (int o = 32; o > 0; o >>= 1) {
-            seen += __shfl_down(seen, o);
-            done += __shfl_down(done, o);
-            abytes += __shfl_down(abytes, o);
-        }
-        if (__lane_id() == 0 && done) {
-            unsigned long long *slot = stat + 16 * (blockIdx.x & 63);
-            atomicAdd(&slot[0], (unsigned long long) seen);
-            atomicAdd(&slot[1], (unsigned long long) done);
-            atomicAdd(&slot[2], (unsigned long long) abytes);
-        }
-    }
-}
-
-// phi mode (rectangular = false): the decision bits of the points without a
-// value (cnt == -1; stamped markid when mark is given).  The lanes of a query
-// sum its phi terms in double in scan order; a threshold outside the rounding
-// band of the reference's float leaf-order sum (phirel per term) is decided
-// here, and a point with a threshold inside it goes to fb for the leaf-order
-// recomputation.  Stored like the level-synchronous passes: phi_code(bits, U).
-__global__ __launch_bounds__(kBlock) void k_grid_phi(int n, SubspaceArg S, GridArg G, const int *__restrict__ off,
-                                                     const int *__restrict__ order, const float *__restrict__ Ys,
-                                                     const uint16_t *__restrict__ Es, float s_star, float eps,
-                                                     double phirel, float phi_w, float phi_d,
-                                                     const int *__restrict__ mark, int markid, int *__restrict__ cnt,
-                                                     int2 *__restrict__ fb, int *__restrict__ nfb, int fbcap) {
-    constexpr int LPQ = kLanesPerQuery, QPB = kBlock / LPQ;
-    extern __shared__ char smem[];
-    float *sy = reinterpret_cast<float *>(smem);
-    int *se = reinterpret_cast<int *>(smem + sizeof(float) * QPB * S.k);
-    const int lq = threadIdx.x / LPQ, sub = threadIdx.x % LPQ;
-    const int i = blockIdx.x * QPB + lq;
-    const int p = i < n ? order[i] : 0;
-    const bool active = i < n && cnt[p] < 0 && (!mark || mark[p] == markid);
-    if (sub == 0 && active) stage_query(S, n, Ys, Es, i, sy + lq, se + lq, QPB);
-    __syncthreads();
-    if (!active) return;  // the walk's ballots below span only active query groups
-    const float *qy = sy + lq;
-    const int *qe = se + lq;
-    const int gshift = (__lane_id() / LPQ) * LPQ;
-    int found = 0;
-    double dsum = 0.0;
-    for_ranges(G, off, qe, QPB, [&](int a, int b) {
-        for (int base = a; base < b; base += LPQ) {
-            const int jj = base + sub;
-            float acc = 0.0f;
-            bool hit = jj < b && jj != i;
-            for (int t = 0; t < S.k && hit; ++t) {
-                if ((G.checkmask >> t) & 1ull) {
-                    const int de = (int) Es[(size_t) t * n + jj] - qe[t * QPB];
-                    if (de < -1 || de > 1) hit = false;
-                }
-                if (hit) {
-                    const float diff = qy[t * QPB] - Ys[(size_t) t * n + jj];
-                    const float sq = diff * diff;
-                    acc = acc + sq;
-                    if (acc > s_star) hit = false;
-                }
-            }
-            if (hit) dsum += phi_term(acc, eps);
-            found += __popcll((__ballot(hit) >> gshift) & ((1ull << LPQ) - 1ull));
-        }
-    });
-    for (int o = LPQ / 2; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o);
-    if (sub != 0) return;
-    const double lo = dsum * (1.0 - (double) found * phirel);
-    const double hi = dsum * (1.0 + (double) found * phirel);
-    const double tw = (double) phi_w, td = (double) phi_d;
-    int code = 0;
-    bool unsure = false;
-    if (lo >= tw) code |= 1;
-    else if (!(hi < tw)) unsure = true;
-    if (lo >= td) code |= 2;
-    else if (!(hi < td)) unsure = true;
-    cnt[p] = phi_code(code, hi * (1.0 + (double) found * phirel));
-    if (unsure) {
-        const int at = atomicAdd(nfb, 1);
-        if (at < fbcap) fb[at] = make_int2(0, p);
     }
 }
 
 // dense flag per sorted position, union-find roots, zeroed component sizes
 __global__ void k_dense_init(const int *__restrict__ order, int n, const int *__restrict__ cnt, int thr_dense,
-                             int dbit, uint8_t *__restrict__ dsorted, int *__restrict__ par, int *__restrict__ csize) {
+                             uint8_t *__restrict__ dsorted, int *__restrict__ par, int *__restrict__ csize) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     // i: a sorted position for the dense flag, a point id for the rest
-    dsorted[i] = meets(cnt[order[i]], thr_dense, dbit) ? 1 : 0;
-    par[i] = meets(cnt[i], thr_dense, dbit) ? i : -1;
+    dsorted[i] = cnt[order[i]] >= thr_dense ? 1 : 0;
+    par[i] = cnt[i] >= thr_dense ? i : -1;
     csize[i] = 0;
 }
 
@@ -445,137 +291,6 @@ __global__ void k_uf_flatten(int *__restrict__ par, int n, int *__restrict__ com
     if (i < n && par[i] >= 0) c = uf_find(par, i);
     wave_add_by_key(csize, c, c >= 0);
     if (i < n) comp[i] = c;
-}
-
-__global__ void k_stamp(const int *__restrict__ W, const int *__restrict__ nW, int *__restrict__ stamp, int tid) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < *nW) stamp[W[i]] = tid;
-}
-
-// ------------------------------------------------------------ redundancy and join on the device
-// The result lives on the device as a table of subspace entries; an entry is
-// in the result while nkept > 0.  The decisions run in stream order, which is
-// the reference's depth-first order, without any host round trip.
-
-// entries e whose mask contains smask (subspace_of, util.cu:619-631) and that
-// are in the result now
-__global__ void k_select(const Entry *__restrict__ E, const int *__restrict__ nE, dmask_t smask, int *__restrict__ list,
-                         int *__restrict__ nlist) {
-    __shared__ int cnt;
-    if (threadIdx.x == 0) cnt = 0;
-    __syncthreads();
-    const int ne = *nE;
-    for (int e = threadIdx.x; e < ne; e += blockDim.x)
-        if ((E[e].mask & smask) == smask && E[e].nkept > 0) list[atomicAdd(&cnt, 1)] = e;
-    __syncthreads();
-    if (threadIdx.x == 0) *nlist = cnt;
-}
-
-// pruneRedundancy (ScyTreeNode.cu:669-734): per listed superspace H, the
-// smallest result cluster of H holding a point of the region.  The members of
-// H's result clusters are listed, the region's points are stamped with `tid`.
-__global__ void k_redundancy(const int *__restrict__ stamp, int tid, const Entry *__restrict__ E,
-                             const int *__restrict__ list, const int *__restrict__ nlist, int *__restrict__ mn) {
-    const int nl = *nlist;
-    const int stride = gridDim.x * blockDim.x;
-    for (int h = 0; h < nl; ++h) {
-        const Entry e = E[list[h]];
-        int best = INT_MAX;
-        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < e.nmem; t += stride) {
-            int q = e.mem[t];
-            if (stamp[q] == tid) best = min(best, e.csize[e.comp[q]]);
-        }
-        for (int o = 32; o > 0; o >>= 1) best = min(best, __shfl_down(best, o));
-        if (__lane_id() == 0 && best != INT_MAX) atomicMin(&mn[h], best);
-    }
-}
-
-// keep iff no superspace cluster touches the region or |W| * r > max_h min_h
-__global__ void k_decide(const int *__restrict__ nlist, int *__restrict__ mn, int nW, float r,
-                         int *__restrict__ keep) {
-    if (threadIdx.x != 0) return;
-    const int nl = *nlist;
-    int max_min = 0;
-    for (int h = 0; h < nl; ++h) {
-        if (mn[h] != INT_MAX && mn[h] > max_min) max_min = mn[h];
-        mn[h] = INT_MAX;
-    }
-    float lhs = (float) nW * r;
-    *keep = (max_min == 0 || (double) lhs > (double) max_min) ? 1 : 0;
-}
-
-// cluster (ClusteringCpu.cu:317-389): a BFS from region point w labels w's
-// dense component; here the component is marked labelled.
-__global__ void k_seed_if(const int *__restrict__ W, int nW, const int *__restrict__ comp, const int *__restrict__ keep,
-                          uint8_t *__restrict__ lab) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nW || !*keep) return;
-    int c = comp[W[i]];
-    if (c >= 0) lab[c] = 1;
-}
-
-// join (util.cu:655-743), step 1: labelled components of at least min_size
-__global__ void k_join_keep(const uint8_t *__restrict__ lab, int n, const int *__restrict__ csize, int min_size,
-                            uint8_t *__restrict__ keepf, uint8_t *__restrict__ drop) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    keepf[k] = (lab[k] && csize[k] >= min_size) ? 1 : 0;
-    drop[k] = 0;
-}
-
-// step 2: drop K when one of its points lies in a result cluster of a
-// superspace H larger than |K| * r (walking the members of H's clusters)
-__global__ void k_join_check(const int *__restrict__ compS, const uint8_t *__restrict__ keepf,
-                             const int *__restrict__ csizeS, float r, const Entry *__restrict__ E,
-                             const int *__restrict__ list, const int *__restrict__ nlist, uint8_t *__restrict__ drop) {
-    const int nl = *nlist;
-    const int stride = gridDim.x * blockDim.x;
-    for (int h = 0; h < nl; ++h) {
-        const Entry e = E[list[h]];
-        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < e.nmem; t += stride) {
-            int q = e.mem[t];
-            int K = compS[q];
-            if (K < 0 || !keepf[K]) continue;
-            if ((float) csizeS[K] * r < (float) e.csize[e.comp[q]]) drop[K] = 1;
-        }
-    }
-}
-
-// step 3: insert the survivors into the result of S
-__global__ void k_join_apply(const uint8_t *__restrict__ keepf, const uint8_t *__restrict__ drop, int n,
-                             uint8_t *__restrict__ inres, uint8_t *__restrict__ fresh, Entry *__restrict__ E, int eS) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    int added = 0;
-    if (k < n) {
-        fresh[k] = 0;
-        if (keepf[k] && !drop[k] && !inres[k]) {
-            inres[k] = 1;
-            fresh[k] = 1;
-            added = 1;
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) added += __shfl_down(added, o);
-    if (__lane_id() == 0 && added) atomicAdd(&E[eS].nkept, added);
-}
-
-// step 4: append the members of the newly inserted clusters to S's member list
-__global__ void k_join_members(const int *__restrict__ compS, int n, const uint8_t *__restrict__ fresh,
-                               Entry *__restrict__ E, int eS) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool in = false;
-    if (i < n) {
-        int K = compS[i];
-        in = K >= 0 && fresh[K];
-    }
-    int slot = wave_slot(in, &E[eS].nmem);
-    if (in) E[eS].mem[slot] = i;
-}
-
-__global__ void k_set_entry(Entry *__restrict__ E, int idx, Entry e, int *__restrict__ nE, int count) {
-    if (threadIdx.x == 0) {
-        E[idx] = e;
-        *nE = count;
-    }
 }
 
 // Canonical labels of a chunk of result subspaces (grid.y = row): clusters
@@ -718,40 +433,23 @@ static unsigned query_blocks(int n) {
 static size_t query_lds(const SubspaceArg &S) { return (sizeof(float) + sizeof(int)) * (kBlock / kLanesPerQuery) * S.k; }
 
 hipError_t launch_subspace_counts(const DevData &D, const SubspaceArg &S, const GridArg &G, float s_star, int cap,
-                                  const GridBuffers &B, const int *mark, int markid, int *cnt,
-                                  unsigned long long *stat, const KernelTimer &tm, hipStream_t st) {
+                                  const GridBuffers &B, int *cnt, hipStream_t st) {
     hipError_t e = build_grid(D, S, G, B, st);
     if (e != hipSuccess) return e;
-    if (tm.start) (void) hipEventRecord(tm.start, st);
     LAUNCH(k_grid_count, dim3(query_blocks(D.n)), dim3(kBlock), query_lds(S), st, D.n, S, G, B.off, B.order, B.Ys,
-           B.Es, s_star, cap, mark, markid, (const int *) nullptr, 0, cnt, stat);
-    if (tm.stop) (void) hipEventRecord(tm.stop, st);
-    return hipGetLastError();
-}
-
-hipError_t launch_subspace_phi(const DevData &D, const SubspaceArg &S, const GridArg &G, const GridBuffers &B,
-                              float s_star, float eps, double phirel, float phi_w, float phi_d, const int *mark,
-                              int markid, int *cnt, int2 *fb, int *nfb, int fbcap, hipStream_t st) {
-    hipError_t e = build_grid(D, S, G, B, st);
-    if (e != hipSuccess) return e;
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 1, sizeof(int))), dim3(kBlock), 0, st, nfb, 0, (size_t) 1);
-    LAUNCH(k_grid_phi, dim3(query_blocks(D.n)), dim3(kBlock), query_lds(S), st, D.n, S, G, B.off, B.order, B.Ys, B.Es,
-           s_star, eps, phirel, phi_w, phi_d, mark, markid, cnt, fb, nfb, fbcap);
+           B.Es, s_star, cap, cnt);
     return hipGetLastError();
 }
 
 hipError_t launch_subspace_components(const DevData &D, const SubspaceArg &S, const GridArg &G, float s_star,
-                                      int cap, int lo, int thr_dense, int dbit, const GridBuffers &B, const int *bound,
-                                      int *cnt, int *comp, int *csize, unsigned long long *stat,
-                                      const KernelTimer &tm, hipStream_t st) {
+                                      int cap, int thr_dense, const GridBuffers &B, int *cnt, int *comp,
+                                      int *csize, hipStream_t st) {
     hipError_t e = build_grid(D, S, G, B, st);
     if (e != hipSuccess) return e;
     const int n = D.n;
-    if (tm.start) (void) hipEventRecord(tm.start, st);
     LAUNCH(k_grid_count, dim3(query_blocks(n)), dim3(kBlock), query_lds(S), st, n, S, G, B.off, B.order, B.Ys, B.Es,
-           s_star, cap, (const int *) nullptr, 0, bound, lo, cnt, stat);
-    if (tm.stop) (void) hipEventRecord(tm.stop, st);
-    LAUNCH(k_dense_init, dim3(blocks_for(n)), dim3(kBlock), 0, st, B.order, n, cnt, thr_dense, dbit, B.dsorted, B.par,
+           s_star, cap, cnt);
+    LAUNCH(k_dense_init, dim3(blocks_for(n)), dim3(kBlock), 0, st, B.order, n, cnt, thr_dense, B.dsorted, B.par,
            csize);
     LAUNCH(k_link_sample, dim3(query_blocks(n)), dim3(kBlock), query_lds(S), st, n, S, G, B.off, B.order, B.Ys, B.Es,
            B.dsorted, s_star, B.par);
@@ -760,50 +458,6 @@ hipError_t launch_subspace_components(const DevData &D, const SubspaceArg &S, co
     LAUNCH(k_link_full, dim3(query_blocks(n)), dim3(kBlock), query_lds(S), st, n, S, G, B.off, B.order, B.Ys, B.Es,
            B.dsorted, s_star, B.giant, B.par);
     LAUNCH(k_uf_flatten, dim3(blocks_for(n)), dim3(kBlock), 0, st, B.par, n, comp, csize);
-    return hipGetLastError();
-}
-
-hipError_t launch_mark(const int *P, const int *nP, int nP_max, int *mark, int markid, hipStream_t st) {
-    if (nP_max <= 0) return hipSuccess;
-    LAUNCH(k_stamp, dim3(blocks_for(nP_max)), dim3(kBlock), 0, st, P, nP, mark, markid);
-    return hipGetLastError();
-}
-
-hipError_t launch_partition(const int *P, const int *nP, int nP_max, const uint8_t *cellC_m, const int *gid, int G,
-                            const int *weakcnt, int thr, int wbit, int *cnt, int *outP, int *outW, hipStream_t st) {
-    LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) 4 * G, sizeof(int))), dim3(kBlock), 0, st, cnt, 0, (size_t) 4 * G);
-    if (nP_max <= 0) return hipGetLastError();
-    const unsigned bp = blocks_for(nP_max);
-    PartArg A{P, nP, cellC_m, gid, weakcnt, thr, G, wbit};
-    LAUNCH(k_part_count, dim3(bp), dim3(kBlock), 0, st, A, cnt);
-    LAUNCH(k_part_scatter, dim3(bp), dim3(kBlock), 0, st, A, cnt, outP, outW);
-    return hipGetLastError();
-}
-
-hipError_t launch_redundancy_seed(const int *W, const int *nW_dev, int nW, int *stamp, int tid, const Entry *E,
-                                  const int *nE, dmask_t smask, const int *comp, int *list, int *nlist, int *mn,
-                                  float r, int *keep, uint8_t *lab, hipStream_t st) {
-    LAUNCH(k_select, dim3(1), dim3(kBlock), 0, st, E, nE, smask, list, nlist);
-    if (nW > 0) LAUNCH(k_stamp, dim3(blocks_for(nW)), dim3(kBlock), 0, st, W, nW_dev, stamp, tid);
-    LAUNCH(k_redundancy, dim3(256), dim3(kBlock), 0, st, stamp, tid, E, list, nlist, mn);
-    LAUNCH(k_decide, dim3(1), dim3(64), 0, st, nlist, mn, nW, r, keep);
-    if (nW > 0) LAUNCH(k_seed_if, dim3(blocks_for(nW)), dim3(kBlock), 0, st, W, nW, comp, keep, lab);
-    return hipGetLastError();
-}
-
-hipError_t launch_join(const uint8_t *lab, int n, const int *compS, const int *csizeS, int min_size, float r,
-                       Entry *E, const int *nE, dmask_t smask, int eS, uint8_t *inresS, int *list, int *nlist,
-                       uint8_t *keepf, uint8_t *drop, uint8_t *fresh, hipStream_t st) {
-    LAUNCH(k_join_keep, dim3(blocks_for(n)), dim3(kBlock), 0, st, lab, n, csizeS, min_size, keepf, drop);
-    LAUNCH(k_select, dim3(1), dim3(kBlock), 0, st, E, nE, smask, list, nlist);
-    LAUNCH(k_join_check, dim3(256), dim3(kBlock), 0, st, compS, keepf, csizeS, r, E, list, nlist, drop);
-    LAUNCH(k_join_apply, dim3(blocks_for(n)), dim3(kBlock), 0, st, keepf, drop, n, inresS, fresh, E, eS);
-    LAUNCH(k_join_members, dim3(blocks_for(n)), dim3(kBlock), 0, st, compS, n, fresh, E, eS);
-    return hipGetLastError();
-}
-
-hipError_t launch_set_entry(Entry *E, int idx, const Entry &e, int *nE, int count, hipStream_t st) {
-    LAUNCH(k_set_entry, dim3(1), dim3(64), 0, st, E, idx, e, nE, count);
     return hipGetLastError();
 }
 
@@ -823,12 +477,6 @@ hipError_t launch_emit(const EmitRow *rows, int r, int n, int *flags, int *idx, 
     else
         LAUNCH(k_emit_labels<int>, dim3(blocks_for(n), r), dim3(kBlock), 0, st, rows, n, idx,
                static_cast<int *>(labels), counts);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_u8(uint8_t *p, uint8_t v, size_t count, hipStream_t st) {
-    if (!count) return hipSuccess;
-    LAUNCH(k_fill<uint8_t>, dim3(fill_blocks(count, sizeof(uint8_t))), dim3(kBlock), 0, st, p, v, count);
     return hipGetLastError();
 }
 
@@ -859,12 +507,6 @@ hipError_t launch_fill_many(const FillMany &f, hipStream_t st) {
 hipError_t launch_gather(const int *src, const int *idx, int count, int *out, hipStream_t st) {
     if (count <= 0) return hipSuccess;
     LAUNCH(k_gather, dim3(blocks_for(count)), dim3(kBlock), 0, st, src, idx, count, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_iota(int *p, int n, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    LAUNCH(k_iota, dim3(blocks_for(n)), dim3(kBlock), 0, st, p, n);
     return hipGetLastError();
 }
 

@@ -100,12 +100,17 @@ void Engine::run_levels(inscy_result &out) {
     root.W = P;
     root.nW = n;
     root.pre = n;
-    root.spx = L0.take<int>(n);
-    root.spm = L0.take<uint64_t>((size_t) n * mw);
-    root.nsp_max = n;
+    // identity order: a path per point; permuted: a chain per near-edge dimension
+    const size_t most = permuted ? std::min<size_t>((size_t) n * d, INT_MAX) : (size_t) n;
+    root.spx = L0.take<int>(most);
+    root.spm = L0.take<uint64_t>(most * pw);
+    root.nsp_max = (int) most;
     root.slot = 0;
     HIP_OK(dev_alloc(&edges, ((size_t) ecells + 3) * sizeof(float)));
-    HIP_OK(launch_b_root(nearm, n, P, root.spx, root.spm, mw, cnt0, ecells, edges, st));
+    if (permuted)
+        HIP_OK(launch_p_root(nearm, n, d, P, root.spx, root.spm, cnt0, ecells, edges, st));
+    else
+        HIP_OK(launch_b_root(nearm, n, P, root.spx, root.spm, mw, cnt0, ecells, edges, st));
     lt.push_back(std::move(root));
     stats.calls = 1;
 
@@ -214,7 +219,7 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
     FlagTree *dft = upload(cur, ft);
     int *dfb = upload(cur, fblk);
     flush_uploads();
-    HIP_OK(launch_b_flags(dft, dfb, na, fblk[na], cellC, n, cells, flags, st));
+    HIP_OK((permuted ? launch_p_flags : launch_b_flags)(dft, dfb, na, fblk[na], cellC, n, cells, flags, st));
     const int nf = (int) frontier.size();
     char *h = down.get((size_t) (ftot + nf) * sizeof(int));
     HIP_OK(hipMemcpyAsync(h, flags, (size_t) ftot * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -293,6 +298,8 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
                 const LTree &t = lt[lv_act[a]];
                 // lists, and the path prune's table (a few branch levels per path)
                 est += (size_t) t.nW * 8 + (size_t) t.nsp * (12 + 32 * std::min<size_t>(d - 1 - c.m, 4)) + 7 * 256 * 4;
+                // the point filter's table and flags, the routed chains and their table
+                if (permuted) est += (size_t) t.nW * 33 + (size_t) t.nsp * 96;
             }
             const bool fits = bytes + est <= batch_budget && (long long) (j - i + 1) * n < INT_MAX &&
                               hsum + ncell < INT_MAX;
@@ -422,6 +429,7 @@ void Engine::index_of(std::vector<BatchSub> &hs, std::vector<const float *> &cta
 // mask; n=25,000 d=15, eps=0.015 (two index dimensions at most) 2.19 and 1.74.
 bool Engine::fan_level(const std::vector<ChildSub> &cs) const {
     if (cs.empty() || (long long) n * d >= 1ll << 30) return false;  // 32-bit offsets into X
+    if (permuted) return false;  // the children match different dimensions of one mask
     const SubspaceArg S = arg_of(cs[0].s & ~dbit(cs[0].m));
     if (S.k < 1 || S.k > kMaxFastK) return false;
     return grid_of(S, -1, true).j >= grid_of(arg_of(cs[0].s), -1, true).j;
@@ -535,6 +543,38 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     }
     int *pcnt = batch.take<int>(std::max(pc_total, 1));
     FillMany fill;
+    // permuted order: the restriction of every pair, and the point filters
+    std::vector<PermStep> steps;
+    std::vector<PermFilter> filters;
+    std::vector<int> filter_of(permuted ? pinfo.size() : 0, -1), fltblk{0};
+    if (permuted) {
+        size_t slots_total = 0;
+        std::vector<size_t> slots_at;
+        for (size_t j = 0; j < pinfo.size(); ++j) {
+            const ChildSub &c = cs[i0 + pinfo[j].b];
+            const LTree &t = lt[lv_act[pinfo[j].a]];
+            steps.push_back(perm_step(t.smask, c.m));
+            // groups of one cell each keep every point
+            if (!steps.back().filt || pinfo[j].G == cells || t.nW <= 0) continue;
+            PermFilter f;
+            std::memset(&f, 0, sizeof(f));
+            f.s = steps.back();
+            f.P = t.W;
+            f.nP = t.nW;
+            f.gid = lv_gid + lv_gidoff[pinfo[j].a] + (c.m - t.first) * cells;
+            f.keep = batch.take<uint8_t>(t.nW);
+            const size_t slots = path_slots(t.nW);
+            f.tmask = (uint64_t) (slots - 1);
+            slots_at.push_back(slots_total);
+            slots_total += slots;
+            filter_of[j] = (int) filters.size();
+            filters.push_back(f);
+            fltblk.push_back(fltblk.back() + nblocks(t.nW));
+        }
+        uint64_t *tables = batch.take<uint64_t>(slots_total);
+        fill.add(tables, ~0u, slots_total * sizeof(uint64_t));
+        for (size_t f = 0; f < filters.size(); ++f) filters[f].table = tables + slots_at[f];
+    }
     fill.add(X.nb, ~0u, (size_t) kSampleEdges * B * n * sizeof(int));
     fill.add(cntB, ~0u, (size_t) B * n * sizeof(int));
     fill.add(X.qflag, 0, (size_t) nw * n);
@@ -623,25 +663,48 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         std::memset(&pp, 0, sizeof(pp));
         pp.P = t.W;
         pp.nP = t.nW;
-        pp.spx = t.spx;
-        pp.spm = t.spm;
-        pp.nsp = t.nsp;
+        if (!permuted) {
+            pp.spx = t.spx;
+            pp.spm = t.spm;
+            pp.nsp = t.nsp;
+        } else if (filter_of[j] >= 0) {
+            pp.keep = filters[filter_of[j]].keep;
+        }
         pp.gid = lv_gid + lv_gidoff[pi.a] + (c.m - t.first) * cells;
         pp.weakcnt = hs[pi.b].cnt;
         pp.cnt = pcnt + pi.cnt_off;
         pp.outW = batch.take<int>(std::max(t.nW, 1));
-        pp.outx = batch.take<int>(std::max(t.nsp, 1));
-        pp.outm = batch.take<uint64_t>((size_t) std::max(t.nsp, 1) * mw);
+        if (!permuted) {
+            pp.outx = batch.take<int>(std::max(t.nsp, 1));
+            pp.outm = batch.take<uint64_t>((size_t) std::max(t.nsp, 1) * mw);
+        }
         pp.mw = mw;
         pp.m = c.m;
         pp.G = pi.G;
         pp.bp = nblocks((t.nW + kPartPerThread - 1) / kPartPerThread);
-        pblk[j + 1] = pblk[j] + pp.bp + nblocks((t.nsp + kPartPerThread - 1) / kPartPerThread);
+        pblk[j + 1] = pblk[j] + pp.bp + nblocks((pp.nsp + kPartPerThread - 1) / kPartPerThread);
+    }
+    std::vector<PermPair> ppairs(permuted ? np : 0);
+    std::vector<int> ppblk(1, 0);
+    for (int j = 0; j < (int) ppairs.size(); ++j) {
+        const LTree &t = lt[lv_act[pinfo[j].a]];
+        PermPair &pp = ppairs[j];
+        pp = PermPair{steps[j], t.spx, t.spm, pairs[j].gid, pairs[j].cnt + 2 * pinfo[j].G, pairs[j].cnt + 6 * pinfo[j].G,
+                      t.nsp, pinfo[j].G};
+        ppblk.push_back(ppblk.back() + nblocks(t.nsp));
     }
     defer_uploads();
     PartPair *dpairs = upload(batch, pairs);
     int *dpb = upload(batch, pblk);
+    PermFilter *dflt = permuted ? upload(batch, filters) : nullptr;
+    int *dfltb = permuted ? upload(batch, fltblk) : nullptr;
+    PermPair *dpp = permuted ? upload(batch, ppairs) : nullptr;
+    int *dppb = permuted ? upload(batch, ppblk) : nullptr;
     flush_uploads();
+    if (permuted) {
+        HIP_OK(launch_p_filter(D, dflt, dfltb, (int) filters.size(), fltblk.back(), st));
+        HIP_OK(launch_p_count(D, dpp, dppb, np, ppblk.back(), st));
+    }
     HIP_OK(launch_b_partition(dpairs, dpb, np, pblk[np], cellC, n, weak_thr, phi_mode ? 1 : 0, prm.min_size, st));
     char *h = down.get((size_t) std::max(pc_total, 1) * sizeof(int));
     HIP_OK(hipMemcpyAsync(h, pcnt, (size_t) std::max(pc_total, 1) * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -653,6 +716,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     std::vector<CopySeg> stamps;  // W points -> tree index, into the subspace's stamp array
     std::vector<int> stamp_b;
     std::vector<PruneChild> prune;
+    std::vector<PermChild> pprune;
     std::vector<size_t> prune_slots;
     std::vector<char> passing(B, 0);
     size_t table_total = 0;
@@ -681,9 +745,12 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             col_G[gp] = G;
         }
         const int *c3 = hcnt.data() + pi.cnt_off;
-        int offW = 0, offS = 0;
+        int offW = 0, offS = 0, others = 0;
+        for (int g = 0; permuted && g < G; ++g) others += c3[6 * G + g];
         for (int g = 0; g < G; ++g) {
-            const int nPr = c3[g], nW = c3[G + g], nSP = c3[2 * G + g];
+            const int nPr = c3[g], nW = c3[G + g];
+            // permuted: the chains of the group's cells and of every other group's
+            const int nSP = c3[2 * G + g] + (permuted ? others - c3[6 * G + g] : 0);
             LTree ch;
             ch.smask = c.s;
             ch.first = c.m + 1;
@@ -708,8 +775,33 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                     ch.slot = lv_nslots++;
                     ch.nsp_max = nSP;
                     ch.spx = nxt.take<int>(std::max(nSP, 1));
-                    ch.spm = nxt.take<uint64_t>((size_t) std::max(nSP, 1) * mw);
-                    if (nSP > 0) {
+                    ch.spm = nxt.take<uint64_t>((size_t) std::max(nSP, 1) * pw);
+                    if (nSP > 0 && permuted) {
+                        const LTree &t = lt[tparent];
+                        PermChild pc;
+                        std::memset(&pc, 0, sizeof(pc));
+                        pc.s = steps[j];
+                        pc.spx = t.spx;
+                        pc.chain = t.spm;
+                        pc.gid = pairs[j].gid;
+                        pc.P = t.W;
+                        pc.keep = pairs[j].keep;
+                        pc.weakcnt = pairs[j].weakcnt;
+                        const size_t slots = path_slots(2 * nSP);
+                        pc.tmask = (uint64_t) (slots - 1);
+                        pc.rx = batch.take<int>(nSP);
+                        pc.rw = batch.take<uint64_t>(nSP);
+                        pc.outx = ch.spx;
+                        pc.outw = ch.spm;
+                        pc.nout = lv_next_counts + ch.slot;
+                        pc.nsp = t.nsp;
+                        pc.nP = t.nW;
+                        pc.nr = nSP;
+                        pc.g = g;
+                        prune_slots.push_back(table_total);
+                        table_total += slots;
+                        pprune.push_back(pc);
+                    } else if (nSP > 0) {
                         PruneChild pc;
                         std::memset(&pc, 0, sizeof(pc));
                         pc.smask = c.s;
@@ -743,8 +835,24 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     // ---- path prune of the surviving children, their point lists, and the
     // dense components of the subspaces that gained one: descriptors in one copy
     FillMany post;
-    const int nprune = (int) prune.size();
-    std::vector<int> bw(nprune + 1, 0), bp(nprune + 1, 0);
+    const int nprune = (int) prune.size(), npprune = (int) pprune.size();
+    std::vector<int> bw(nprune + npprune + 1, 0), bp(nprune + npprune + 1, 0), br(npprune + 1, 0);
+    if (npprune) {
+        uint64_t *tables = post.add(batch.take<uint64_t>(table_total), ~0u, table_total * sizeof(uint64_t));
+        uint8_t *marks = post.add(batch.take<uint8_t>(2 * table_total), 0, 2 * table_total);
+        dmask_t *bits = post.add(batch.take<dmask_t>(npprune), 0, (size_t) npprune * sizeof(dmask_t));
+        int *nr = post.add(batch.take<int>(npprune), 0, (size_t) npprune * sizeof(int));
+        for (int c = 0; c < npprune; ++c) {
+            PermChild &pc = pprune[c];
+            pc.table = tables + prune_slots[c];
+            pc.marks = marks + 2 * prune_slots[c];
+            pc.bits = bits + c;
+            pc.nr_at = nr + c;
+            br[c + 1] = br[c] + nblocks(pc.nsp);
+            bw[c + 1] = bw[c] + nblocks((long long) pc.nP + pc.nr);
+            bp[c + 1] = bp[c] + nblocks(pc.nr);
+        }
+    }
     if (nprune) {
         uint64_t *tables = post.add(batch.take<uint64_t>(table_total), ~0u, table_total * sizeof(uint64_t));
         dmask_t *bits = post.add(batch.take<dmask_t>(nprune), 0, (size_t) nprune * sizeof(dmask_t));
@@ -807,8 +915,10 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     for (size_t c = 0; c < copies.size(); ++c) cb[c + 1] = cb[c] + nblocks(copies[c].len);
     defer_uploads();
     PruneChild *dpc = nprune ? upload(batch, prune) : nullptr;
-    int *dbw = nprune ? upload(batch, bw) : nullptr;
-    int *dbp = nprune ? upload(batch, bp) : nullptr;
+    PermChild *dpch = npprune ? upload(batch, pprune) : nullptr;
+    int *dbr = npprune ? upload(batch, br) : nullptr;
+    int *dbw = nprune + npprune ? upload(batch, bw) : nullptr;
+    int *dbp = nprune + npprune ? upload(batch, bp) : nullptr;
     CopySeg *dcs = copies.empty() ? nullptr : upload(batch, copies);
     int *dcb2 = copies.empty() ? nullptr : upload(batch, cb);
     if (ncomp > 0 && fan) columns(hc, ctab2);
@@ -816,6 +926,9 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     if (ncomp > 0) put(entries + nentries, ents.data(), ents.size() * sizeof(Entry));
     flush_uploads();
     HIP_OK(launch_fill_many(post, st));
+    if (npprune)
+        HIP_OK(launch_p_prune(D, dpch, npprune, dbr, br[npprune], dbw, bw[npprune], dbp, bp[npprune], weak_thr,
+                              phi_mode ? 1 : 0, st));
     if (nprune) HIP_OK(launch_b_prune(D, dpc, nprune, dbw, bw[nprune], dbp, bp[nprune], st));
     if (!copies.empty()) HIP_OK(launch_b_copy(dcs, dcb2, (int) copies.size(), cb.back(), st));
     if (ncomp > 0) {
@@ -849,6 +962,32 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     }
 }
 
+// The restriction of a tree of mask s on dimension m, permuted level order.
+PermStep Engine::perm_step(dmask_t s, int m) const {
+    PermStep p;
+    std::memset(&p, 0, sizeof(p));
+    p.m = m;
+    p.Lm = lvl_of[m];
+    p.tree = levels_of(s);
+    p.restricted = p.tree | dbit(p.Lm);
+    p.tkey = -1;
+    bool deeper = false, kept_below = false;
+    for (int t = d - 1; t >= 0; --t) {
+        if (dhas(p.restricted, t)) continue;
+        if (level[t] > m) p.big |= dbit(t);
+        if (t > p.Lm) {
+            deeper = true;
+        } else {
+            if (p.tkey < 0) p.tkey = t;
+            kept_below |= level[t] > m;
+            if (kept_below) p.cond |= dbit(t);
+        }
+    }
+    // m's level the deepest free one, and none above it or a larger dimension's
+    p.filt = !deeper && (p.tkey < 0 || level[p.tkey] > m);
+    return p;
+}
+
 // The subspaces S minus one dimension whose counts are complete (their
 // dense components were built) bound the counts of S from above; a bound
 // decides a point only below both thresholds of S and below the cap of the
@@ -861,7 +1000,18 @@ void Engine::set_bounds(dmask_t s, BatchSub &x) {
     for (int t = 0; t < k && x.nbound < kMaxBounds; ++t) {
         const dmask_t sub = s & ~dbit(x.S.dims[t]);
         auto it = subs.find(sub);
-        if (sub && it != subs.end() && it->second.entry >= 0) x.bound[x.nbound++] = it->second.cnt;
+        if (!sub || it == subs.end() || it->second.entry < 0) continue;
+        if (permuted) {
+            // the cells of a dimension that only S minus t matches do not
+            // restrict the neighbours in S
+            const SubspaceArg Q = arg_of(sub);
+            uint64_t mq = match_of(Q), ms = match_of(x.S);
+            bool inside = true;
+            for (int u = 0; u < Q.k; ++u)
+                if ((mq >> u) & 1) inside &= (ms >> (u < t ? u : u + 1)) & 1;
+            if (!inside) continue;
+        }
+        x.bound[x.nbound++] = it->second.cnt;
     }
     // counts are exact below the cap of |S| - 1 (phi: the stored values carry
     // an upper bound, used in the kernel)

@@ -48,27 +48,6 @@ __global__ void k_b_flags(const FlagTree *__restrict__ T, const int *__restrict_
     }
 }
 
-// Edges of the eps cells: edge[i] is the smallest coordinate whose cell is at
-// least i - 1 (-inf for i <= 1, +inf past the last cell), i in [0, C + 3).  The
-// cell is monotone in the coordinate, so for a query in cell c the coordinates
-// whose cell is within one of c are exactly [edge[c], edge[c + 3]): the walks
-// test the cells of a candidate on its coordinate, without reading its cells.
-__device__ __forceinline__ float cell_edge(int i, int C) {
-    const int target = i - 1;
-    if (target <= 0) return -__builtin_inff();
-    if (target >= C) return __builtin_inff();
-    const float ecs = ecell_width(C);
-    uint32_t lo = 0, hi = 0x3F800000u;  // cell(0) < target <= cell(1.0) = C - 1
-    while (hi - lo > 1) {
-        const uint32_t mid = lo + (hi - lo) / 2;
-        if (ecell_of(__uint_as_float(mid), ecs, C) >= target)
-            hi = mid;
-        else
-            lo = mid;
-    }
-    return __uint_as_float(hi);
-}
-
 // the root tree: every point, the path of every point with a near-edge
 // dimension; and the cell edges
 __global__ void k_b_root(const dmask_t *__restrict__ nearm, int n, int *__restrict__ P, int *__restrict__ outx,
@@ -1420,7 +1399,7 @@ __global__ void k_b_part_count(const PartPair *__restrict__ pairs, const int *__
     if (blk < A.bp) {
         for (int u = 0; u < kPartPerThread; ++u) {
             const int i = (blk * kPartPerThread + u) * blockDim.x + threadIdx.x;
-            if (i < A.nP) {
+            if (i < A.nP && (!A.keep || A.keep[i])) {
                 const int p = A.P[i];
                 const int g = A.gid[cm[p]];
                 atomicAdd(&h[g], 1);
@@ -1487,7 +1466,7 @@ __global__ void k_b_part_scatter(const PartPair *__restrict__ pairs, const int *
         mk[u] = 0;
         if (pts) {
             const int i = (blk * kPartPerThread + u) * blockDim.x + threadIdx.x;
-            if (i < A.nP) {
+            if (i < A.nP && (!A.keep || A.keep[i])) {
                 const int p = A.P[i];
                 const int g = A.gid[cm[p]];
                 if (A.cnt[G + g] >= min_size && meets(A.weakcnt[p], thr, wbit)) {

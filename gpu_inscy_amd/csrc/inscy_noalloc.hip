@@ -144,7 +144,7 @@ hipError_t launch_neighbour_counts_noalloc(unsigned char *base, const float *X, 
     Sk.k = k;
     for (int t = 0; t < k; ++t) Sk.dims[t] = t;
     const DevData D{nullptr, Xt, nullptr, cellE, nullptr, nullptr, nullptr, n, k, 1, ecells, 0};
-    e = launch_subspace_counts(D, Sk, G, s_star, INT_MAX, B, nullptr, 0, cnt, nullptr, KernelTimer{}, st);
+    e = launch_subspace_counts(D, Sk, G, s_star, INT_MAX, B, cnt, st);
     if (e != hipSuccess) return e;
     if (nq > 0) {
         k_gather_checked<<<(unsigned) ((nq + bs - 1) / bs), bs, 0, st>>>(cnt, n, queries, nq, out);

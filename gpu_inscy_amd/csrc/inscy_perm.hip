@@ -1,5 +1,6 @@
 // Permuted SCY-tree level order (entropy_order != 0, get_subspace_order,
-// inscy_map.cpp:61-121): the depth-first driver over s-connection chains.
+// inscy_map.cpp:61-121): the tree passes of the level-synchronous driver over
+// s-connection chains.
 //
 // With the levels in a permuted order, restrict_node (ScyTreeNode.cu:227-320)
 // keeps every node whose dimension id exceeds the restricted one, so a
@@ -27,9 +28,14 @@
 //    an ancestor of one of its chains, or a node above m's level kept because
 //    a level between it and m's has a dimension id above m) and lost its
 //    weak-dense points.
-// Prefix membership tests use open-addressing tables of (32 hash bits |
-// representative point), every hit confirmed by comparing cells.
-#include "inscy_engine.h"
+// The prefixes that a child's prune asks about (two per routed chain: its parent
+// and its sibling) go into an open-addressing table of (25 hash bits | level |
+// point), every hit confirmed by comparing cells; the tree's points and chains
+// look theirs up and mark the ones found.  Every pass serves all (tree,
+// dimension) pairs or children of a batch in one launch: one tree at a time the
+// launches were the bound (n=3,001 d=9: 4,666 launches and 26.5 ms a run, 166 and
+// 2.0 ms in this form).
+#include "inscy_internal.h"
 
 #include "inscy_device.h"
 
@@ -43,417 +49,287 @@ __device__ __forceinline__ uint64_t chain_word(int b, int end) { return (uint64_
 
 constexpr uint64_t kSeed = 0x243F6A8885A308D3ull;
 __device__ __forceinline__ uint64_t level_salt(int t) { return 0x9E3779B97F4A7C15ull * (uint64_t) (t + 1); }
+// levels from..to (empty when to < from)
+__device__ __forceinline__ dmask_t levels_in(int from, int to) { return dabove(from - 1) & ~dabove(to); }
 
-// Restricted levels are level masks (bit t for level t) throughout.
-// prefix of z through level `upto` (an unrestricted one)
-__device__ __forceinline__ uint64_t prefix_hash(const DevData &D, dmask_t restricted, int z, int upto) {
+// f(t, hash) for the prefix of z through every level t of `want` (unrestricted ones)
+template <class F>
+__device__ __forceinline__ void prefixes(const DevData &D, dmask_t restricted, int z, dmask_t want, F f) {
     uint64_t h = kSeed;
     CellRow row{};
-    for (int t = 0; t <= upto; ++t) {
+    for (int t = 0; want && t < D.d; ++t) {
         if (!(t & 15)) row = load_row(D, z, t);
-        if (!dhas(restricted, t)) h = mix64(h + row.at(t & 15) + 1);
+        if (dhas(restricted, t)) continue;
+        h = mix64(h + row.at(t & 15) + 1);
+        if (!dhas(want, t)) continue;
+        want &= ~dbit(t);
+        f(t, mix64(h ^ level_salt(t)));
     }
-    return mix64(h ^ level_salt(upto));
 }
 
-__device__ void table_insert(const DevData &D, dmask_t restricted, uint64_t *table, uint64_t tmask, uint64_t e, int z,
-                             int t) {
-    const uint64_t entry = (e & 0xFFFFFFFF00000000ull) | (uint32_t) z;
+// a table entry: 25 hash bits | level | point (n < 2^30, so never kEmpty)
+__device__ __forceinline__ uint64_t table_entry(uint64_t e, int z, int t) {
+    return (e >> 39) << 39 | (uint64_t) t << 32 | (uint32_t) z;
+}
+// slot of the prefix e of z through level t, inserted when it is not there
+// (insert false: -1 then); accept(point) decides beyond the cells
+template <bool INSERT, class F>
+__device__ __forceinline__ long long table_slot(const DevData &D, dmask_t restricted, uint64_t *table, uint64_t tmask,
+                                                uint64_t e, int z, int t, F accept) {
+    const uint64_t entry = table_entry(e, z, t);
     uint64_t slot = e & tmask;
     while (true) {
+        // a slot is written once, by the swap from empty: a plain load that
+        // still sees it empty is corrected by the failed swap, a full one is final
         uint64_t cur = table[slot];
         if (cur == kEmpty) {
+            if (!INSERT) return -1;
             cur = atomicCAS((unsigned long long *) &table[slot], (unsigned long long) kEmpty,
                             (unsigned long long) entry);
-            if (cur == kEmpty) return;
+            if (cur == kEmpty) return (long long) slot;
         }
-        if ((cur >> 32) == (entry >> 32) && same_prefix(D, restricted, z, (int) (uint32_t) cur, t)) return;
+        if ((cur >> 32) == (entry >> 32) && accept((int) (uint32_t) cur) &&
+            same_prefix(D, restricted, z, (int) (uint32_t) cur, t))
+            return (long long) slot;
         slot = (slot + 1) & tmask;
     }
 }
+struct AnyPoint {
+    __device__ __forceinline__ bool operator()(int) const { return true; }
+};
 
-__device__ bool table_has(const DevData &D, dmask_t restricted, const uint64_t *table, uint64_t tmask, uint64_t e,
-                          int z, int t) {
-    uint64_t slot = e & tmask;
-    while (true) {
-        const uint64_t cur = table[slot];  // complete: the inserts ran in an earlier launch
-        if (cur == kEmpty) return false;
-        if ((cur >> 32) == (e >> 32) && same_prefix(D, restricted, z, (int) (uint32_t) cur, t)) return true;
-        slot = (slot + 1) & tmask;
+// the root tree: every point, a chain to the deepest level for every near-edge
+// dimension of a point; and the cell edges
+__global__ void k_p_root(const dmask_t *__restrict__ nearm, int n, int d, int *__restrict__ P, int *__restrict__ cx,
+                         uint64_t *__restrict__ cw, int *__restrict__ nout, int C, float *__restrict__ edge) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < C + 3) edge[i] = cell_edge(i, C);
+    if (i < n) P[i] = i;
+    dmask_t m = i < n ? nearm[i] : (dmask_t) 0;
+    const int lane = __lane_id();
+    int at = dcount(m);
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(at, o);
+        if (lane >= o) at += v;
     }
-}
-
-__global__ void k_perm_root(const dmask_t *__restrict__ nearm, int n, int d, int *__restrict__ cx,
-                            uint64_t *__restrict__ cm, int *__restrict__ nout) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    dmask_t m = nearm[p];
-    if (!m) return;
-    int at = atomicAdd(nout, dcount(m));
+    int base = 0;
+    if (lane == 63 && at) base = atomicAdd(nout, at);
+    at += __shfl(base, 63) - dcount(m);
     while (m) {
         const int b = dfirst(m);
         m &= m - 1;
-        cx[at] = p;
-        cm[at] = chain_word(b, d - 1);
-        ++at;
+        cx[at] = i;
+        cw[at++] = chain_word(b, d - 1);
     }
 }
 
-__global__ void k_perm_flags(const int *__restrict__ cx, const uint64_t *__restrict__ cm, const int *__restrict__ nch,
-                             const uint8_t *__restrict__ cellC, int n, int first, int cells, int *__restrict__ flags) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nch) return;
-    const int b = chain_b(cm[i]);
-    if (b < first) return;
-    flags[(size_t) (b - first) * cells + cellC[(size_t) b * n + cx[i]]] = 1;
+// merge flags of every dimension >= first of every tree
+__global__ void k_p_flags(const FlagTree *__restrict__ T, const int *__restrict__ blk_off, int nt,
+                          const uint8_t *__restrict__ cellC, int n, int cells, int *__restrict__ flags) {
+    const int t = seg_of(blk_off, nt, blockIdx.x);
+    const FlagTree F = T[t];
+    const int i = (blockIdx.x - blk_off[t]) * blockDim.x + threadIdx.x;
+    if (i >= *F.nsp) return;
+    const int b = chain_b(F.spm[i]);
+    if (b < F.first) return;
+    flags[F.flag_off + (b - F.first) * cells + cellC[(size_t) b * n + F.spx[i]]] = 1;
 }
 
-// the chains of group g after the restriction of T (smask) on m
-__global__ void k_perm_route(DevData D, dmask_t smask, int m, const int *__restrict__ gid, int g,
-                             const int *__restrict__ cx, const uint64_t *__restrict__ cm, const int *__restrict__ nch,
-                             int *__restrict__ ox, uint64_t *__restrict__ om, int *__restrict__ nout) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nch) return;
-    const uint64_t w = cm[i];
-    const int b = chain_b(w), end = chain_end(w);
-    if (b == m) return;
-    const int x = cx[i];
-    const bool cell_in = gid[D.cellC[(size_t) m * D.n + x]] == g;
-    const int Lb = D.lvl_of[b], Lm = D.lvl_of[m];
-    auto deepest = [&](int from, int to) {  // deepest unrestricted level in [from, to], not m's, dimension > m
-        int best = -1;
-        for (int t = from; t <= to; ++t) {
-            const int k = D.level[t];
-            if (t != Lm && !dhas(smask, k) && k > m) best = t;
+// end of a chain after the step, in the group of x's cell (in) or in another
+// one; -1 where the chain does not pass
+__device__ __forceinline__ int route(const PermStep &s, int Lb, int end, bool in) {
+    if (Lb > s.Lm) return in ? dlast(s.big & levels_in(Lb, end)) : -1;
+    if (end >= s.Lm && in) {
+        const int e = dlast(s.big & levels_in(s.Lm + 1, end));
+        // else the chain node above the restricted level
+        return e >= 0 ? e : max(Lb, dlast(~s.tree & levels_in(Lb, s.Lm - 1)));
+    }
+    return dlast(s.big & levels_in(Lb, min(end, s.Lm - 1)));
+}
+
+// how many chains of every pair go to each of its groups
+__global__ void k_p_count(DevData D, const PermPair *__restrict__ pairs, const int *__restrict__ blk_off, int np) {
+    __shared__ int h[2 * 256];
+    const int j = seg_of(blk_off, np, blockIdx.x);
+    const PermPair &A = pairs[j];
+    const int G = A.G;
+    for (int t = threadIdx.x; t < 2 * G; t += blockDim.x) h[t] = 0;
+    __syncthreads();
+    const int i = (blockIdx.x - blk_off[j]) * blockDim.x + threadIdx.x;
+    if (i < A.nsp) {
+        const uint64_t w = A.chain[i];
+        const int b = chain_b(w), end = chain_end(w);
+        if (b != A.s.m) {
+            const int Lb = D.lvl_of[b], g = A.gid[D.cellC[(size_t) A.s.m * D.n + A.spx[i]]];
+            if (route(A.s, Lb, end, true) >= 0) atomicAdd(&h[g], 1);
+            if (route(A.s, Lb, end, false) >= 0) atomicAdd(&h[G + g], 1);
         }
-        return best;
-    };
-    int e;
-    if (Lb > Lm) {
-        if (!cell_in) return;
-        e = deepest(Lb, end);
-    } else if (end >= Lm && cell_in) {
-        e = deepest(Lm + 1, end);
-        if (e < 0) {
-            e = Lm - 1;  // the chain node above the restricted level
-            while (e > Lb && dhas(smask, D.level[e])) --e;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < 2 * G; t += blockDim.x)
+        if (h[t]) atomicAdd(t < G ? &A.in[t] : &A.out[t - G], h[t]);
+}
+
+// The points of every group's first cell enter their prefixes (through the
+// deepest free level above m's), then every point looks its own up among its
+// group's.
+template <bool MARK>
+__global__ void k_p_filter(DevData D, const PermFilter *__restrict__ filters, const int *__restrict__ blk_off, int nf) {
+    const int j = seg_of(blk_off, nf, blockIdx.x);
+    const PermFilter &F = filters[j];
+    const int i = (blockIdx.x - blk_off[j]) * blockDim.x + threadIdx.x;
+    if (i >= F.nP) return;
+    const int z = F.P[i];
+    const uint8_t *cm = D.cellC + (size_t) F.s.m * D.n;
+    const int c = cm[z], g = F.gid[c];
+    const bool lo = c == 0 || F.gid[c - 1] != g;
+    if (MARK && !lo) return;
+    bool found = lo;
+    if (MARK || !lo) {
+        const int tk = F.s.tkey;
+        uint64_t e = kSeed;
+        if (tk >= 0) prefixes(D, F.s.restricted, z, dbit(tk), [&](int, uint64_t h) { e = h; });
+        e = mix64(e + (uint64_t) g);
+        found = table_slot<MARK>(D, F.s.restricted, F.table, F.tmask, e, z, tk < 0 ? 0 : tk, [&](int y) {
+                    return y >= 0 && y < D.n && F.gid[cm[y]] == g;
+                }) >= 0;
+    }
+    if (!MARK) F.keep[i] = found;
+}
+
+// a child's chains out of its parent's, and the prefixes its prune asks about:
+// x's through the last free level above b's (the chain's regular parent) and
+// through b's (its regular sibling)
+__global__ void k_p_route(DevData D, const PermChild *__restrict__ C, const int *__restrict__ blk_off, int nc) {
+    const int c = seg_of(blk_off, nc, blockIdx.x);
+    const PermChild &P = C[c];
+    const int i = (blockIdx.x - blk_off[c]) * blockDim.x + threadIdx.x;
+    int x = 0, b = 0, e = -1, Lb = 0;
+    if (i < P.nsp) {
+        const uint64_t w = P.chain[i];
+        b = chain_b(w);
+        x = P.spx[i];
+        if (b != P.s.m) {
+            Lb = D.lvl_of[b];
+            e = route(P.s, Lb, chain_end(w), P.gid[D.cellC[(size_t) P.s.m * D.n + x]] == P.g);
         }
-    } else {
-        e = deepest(Lb, min(end, Lm - 1));
     }
-    if (e < 0) return;
-    const int at = atomicAdd(nout, 1);
-    ox[at] = x;
-    om[at] = chain_word(b, e);
-}
-
-// prefixes of the points at every unrestricted level in `need`
-__global__ void k_perm_insert_pts(DevData D, dmask_t restricted, const int *__restrict__ pts,
-                                  const int *__restrict__ npts, dmask_t need, uint64_t *__restrict__ table,
-                                  uint64_t tmask) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *npts || !need) return;
-    const int z = pts[i];
-    uint64_t h = kSeed;
-    CellRow row{};
-    for (int t = 0; t < D.d; ++t) {
-        if (!(t & 15)) row = load_row(D, z, t);
-        if (dhas(restricted, t)) continue;
-        h = mix64(h + row.at(t & 15) + 1);
-        if (dhas(need, t)) table_insert(D, restricted, table, tmask, mix64(h ^ level_salt(t)), z, t);
+    const int at = wave_slot(e >= 0, P.nr_at);
+    dmask_t want = 0;
+    if (e >= 0) {
+        P.rx[at] = x;
+        P.rw[at] = chain_word(b, e);
+        const int tp = dlast(~P.s.restricted & levels_in(0, Lb - 1));
+        want = dbit(Lb) | (tp >= 0 ? dbit(tp) : (dmask_t) 0);
     }
+    wave_or_mask(want, P.bits);
+    if (!want) return;
+    prefixes(D, P.s.restricted, x, want, [&](int t, uint64_t h) {
+        table_slot<true>(D, P.s.restricted, P.table, P.tmask, h, x, t, AnyPoint{});
+    });
 }
 
-// regular ancestors of the chains' first nodes: x's prefixes at the levels above b's
-__global__ void k_perm_insert_anchors(DevData D, dmask_t restricted, const int *__restrict__ cx,
-                                      const uint64_t *__restrict__ cm, const int *__restrict__ nch,
-                                      uint64_t *__restrict__ table, uint64_t tmask) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nch) return;
-    const int z = cx[i], Lb = D.lvl_of[chain_b(cm[i])];
-    uint64_t h = kSeed;
-    CellRow row{};
-    for (int t = 0; t < Lb; ++t) {
-        if (!(t & 15)) row = load_row(D, z, t);
-        if (dhas(restricted, t)) continue;
-        h = mix64(h + row.at(t & 15) + 1);
-        table_insert(D, restricted, table, tmask, mix64(h ^ level_salt(t)), z, t);
+// Marks of the prefixes asked for.  The parent's points: in the child, the node
+// existed and, weak-dense, still holds a point; elsewhere it existed at the
+// levels of `cond`.  Then the routed chains: their regular ancestors existed.
+__global__ void k_p_mark(DevData D, const PermChild *__restrict__ C, const int *__restrict__ blk_off, int nc, int thr,
+                         int wbit) {
+    const int c = seg_of(blk_off, nc, blockIdx.x);
+    const PermChild &P = C[c];
+    const int i = (blockIdx.x - blk_off[c]) * blockDim.x + threadIdx.x;
+    const dmask_t need = *P.bits;
+    dmask_t exist = 0;
+    int z = 0;
+    bool weak = false;
+    if (i < P.nP) {
+        z = P.P[i];
+        if (P.gid[D.cellC[(size_t) P.s.m * D.n + z]] == P.g && (!P.keep || P.keep[i])) {
+            exist = need;
+            weak = meets(P.weakcnt[z], thr, wbit);
+        } else {
+            exist = need & P.s.cond;
+        }
+    } else if (i < P.nP + P.nr) {
+        z = P.rx[i - P.nP];
+        exist = need & levels_in(0, D.lvl_of[chain_b(P.rw[i - P.nP])] - 1);
     }
+    prefixes(D, P.s.restricted, z, exist, [&](int t, uint64_t h) {
+        const long long at = table_slot<false>(D, P.s.restricted, P.table, P.tmask, h, z, t, AnyPoint{});
+        if (at < 0) return;
+        // every marker writes the same byte
+        if (weak && !P.marks[2 * at]) P.marks[2 * at] = 1;
+        if (!P.marks[2 * at + 1]) P.marks[2 * at + 1] = 1;
+    });
 }
 
-struct PermTables {
-    const uint64_t *W, *P, *T, *A;
-    uint64_t wmask, pmask, tmask, amask;
-    dmask_t cond;  // levels whose nodes above m's level a larger dimension id below keeps
-};
-
-__global__ void k_perm_prune(DevData D, dmask_t restricted, PermTables Tb, const int *__restrict__ cx,
-                             const uint64_t *__restrict__ cm, const int *__restrict__ nch, int *__restrict__ ox,
-                             uint64_t *__restrict__ om, int *__restrict__ nout) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nch) return;
-    const int z = cx[i];
-    const uint64_t w = cm[i];
-    const int b = chain_b(w), Lb = D.lvl_of[b];
-    // the regular parent: x's prefix through the last unrestricted level above b's
-    int tp = Lb - 1;
-    while (tp >= 0 && dhas(restricted, tp)) --tp;
-    if (tp >= 0 && !table_has(D, restricted, Tb.W, Tb.wmask, prefix_hash(D, restricted, z, tp), z, tp)) return;
-    const uint64_t e = prefix_hash(D, restricted, z, Lb);
-    if (!table_has(D, restricted, Tb.W, Tb.wmask, e, z, Lb)) {
-        const bool existed = table_has(D, restricted, Tb.P, Tb.pmask, e, z, Lb) ||
-                             table_has(D, restricted, Tb.A, Tb.amask, e, z, Lb) ||
-                             (dhas(Tb.cond, Lb) && table_has(D, restricted, Tb.T, Tb.tmask, e, z, Lb));
-        if (existed) return;  // the sibling lost its points: propergate_count2 erases the chain
+__global__ void k_p_check(DevData D, const PermChild *__restrict__ C, const int *__restrict__ blk_off, int nc) {
+    const int c = seg_of(blk_off, nc, blockIdx.x);
+    const PermChild &P = C[c];
+    const int i = (blockIdx.x - blk_off[c]) * blockDim.x + threadIdx.x;
+    int x = 0;
+    uint64_t w = 0;
+    bool keep = false;
+    if (i < P.nr) {
+        x = P.rx[i];
+        w = P.rw[i];
+        const int Lb = D.lvl_of[chain_b(w)];
+        const int tp = dlast(~P.s.restricted & levels_in(0, Lb - 1));
+        keep = true;
+        prefixes(D, P.s.restricted, x, dbit(Lb) | (tp >= 0 ? dbit(tp) : (dmask_t) 0), [&](int t, uint64_t h) {
+            const long long at = table_slot<false>(D, P.s.restricted, P.table, P.tmask, h, x, t, AnyPoint{});
+            const bool holds = at >= 0 && P.marks[2 * at], was = at >= 0 && P.marks[2 * at + 1];
+            // the parent holds no point, or the sibling lost its points
+            // (propergate_count2 erases the chain)
+            if (!holds && (t != Lb || was)) keep = false;
+        });
     }
-    const int at = atomicAdd(nout, 1);
-    ox[at] = z;
-    om[at] = w;
-}
-
-// the points of G's first cell mark their prefixes through level tkey
-// (tkey < 0: the root, flag[0])
-__global__ void k_perm_lo_mark(DevData D, dmask_t restricted, const int *__restrict__ pts,
-                               const int *__restrict__ npts, int m, int lo, int tkey, uint64_t *__restrict__ table,
-                               uint64_t tmask, int *__restrict__ flag) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *npts) return;
-    const int z = pts[i];
-    if (D.cellC[(size_t) m * D.n + z] != lo) return;
-    if (tkey < 0)
-        flag[0] = 1;
-    else
-        table_insert(D, restricted, table, tmask, prefix_hash(D, restricted, z, tkey), z, tkey);
-}
-
-__global__ void k_perm_lo_filter(DevData D, dmask_t restricted, const int *__restrict__ in,
-                                 const int *__restrict__ nin, int tkey, const uint64_t *__restrict__ table,
-                                 uint64_t tmask, const int *__restrict__ flag, int *__restrict__ out,
-                                 int *__restrict__ nout) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *nin) return;
-    const int z = in[i];
-    const bool keep = tkey < 0 ? flag[0] != 0
-                               : table_has(D, restricted, table, tmask, prefix_hash(D, restricted, z, tkey), z, tkey);
-    if (keep) out[atomicAdd(nout, 1)] = z;
-}
-
-#define LAUNCH(kernel, grid, block, lds, st, ...) hipLaunchKernelGGL(kernel, grid, block, lds, st, __VA_ARGS__)
-
-size_t slots_for(long long items) {
-    size_t want = (size_t) std::max<long long>(items, 1) * 2, s = 256;
-    while (s < want) s <<= 1;
-    return s;
+    const int at = wave_slot(keep, P.nout);
+    if (keep) {
+        P.outx[at] = x;
+        P.outw[at] = w;
+    }
 }
 
 }  // namespace
 
-void Engine::run_perm(inscy_result &out) {
-    int *P = arena.take<int>(n);
-    int *nP = arena.take<int>(1);
-    const size_t cap = (size_t) n * d;
-    int *cx = arena.take<int>(std::max<size_t>(cap, 1));
-    uint64_t *cm = arena.take<uint64_t>(std::max<size_t>(cap, 1));
-    int *nch = arena.take<int>(1);
-    HIP_OK(launch_iota(P, n, st));
-    HIP_OK(launch_fill_i32(nP, n, 1, st));
-    HIP_OK(launch_fill_i32(nch, 0, 1, st));
-    LAUNCH(k_perm_root, dim3(blocks_for(n)), dim3(kBlock), 0, st, nearm, n, d, cx, cm, nch);
-    HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(pin, nch, sizeof(int), hipMemcpyDeviceToHost, st));
-    sync();
-    const int nch_h = pin_i()[0];
-    TreeRef root{(dmask_t) 0, P, nP, n, cx, cm, nch, nch_h};
-    auto t0 = std::chrono::steady_clock::now();
-    recurse_perm(root, 0);
-    sync();
-    auto t1 = std::chrono::steady_clock::now();
-    emit(out);
-    stats.expand_seconds = std::chrono::duration<double>(t1 - t0).count();
-    stats.emit_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t1).count();
+#define LAUNCH(kernel, grid, block, lds, st, ...) hipLaunchKernelGGL(kernel, grid, block, lds, st, __VA_ARGS__)
+
+hipError_t launch_p_root(const dmask_t *nearm, int n, int d, int *P, int *cx, uint64_t *cw, int *nout, int C,
+                         float *edge, hipStream_t st) {
+    LAUNCH(k_p_root, dim3(blocks_for((size_t) std::max(n, C + 3))), dim3(kBlock), 0, st, nearm, n, d, P, cx, cw, nout, C,
+           edge);
+    return hipGetLastError();
 }
 
-void Engine::recurse_perm(const TreeRef &T, int first) {
-    stats.calls++;
-    if (first >= d) return;
-    const int nd = d - first;
-    const size_t lvl_mark = arena.mark();
-    int *flags = arena.take<int>((size_t) nd * cells);
-    HIP_OK(launch_fill_i32(flags, 0, (size_t) nd * cells, st));
-    if (T.nsp_max > 0)
-        LAUNCH(k_perm_flags, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, T.spx, T.chain, T.nsp, cellC, n, first,
-               cells, flags);
-    HIP_OK(hipGetLastError());
-    const int markid = ++mark_id;
-    HIP_OK(launch_mark(T.P, T.nP, T.nP_max, qmark, markid, st));
-    for (int m = first; m < d; ++m) ensure_counts(T.smask | dbit(m), markid);
-    HIP_OK(hipMemcpyAsync(pin, flags, (size_t) nd * cells * sizeof(int), hipMemcpyDeviceToHost, st));
-    sync();
-    std::vector<std::vector<Group>> groups(nd);
-    std::vector<int> gid((size_t) nd * cells);
-    for (int m = first; m < d; ++m) {
-        const int *f = pin_i((size_t) (m - first) * cells);
-        auto &gs = groups[m - first];
-        for (int c = 0; c < cells; ++c) {
-            int lo = c;
-            while (f[c] && c < cells - 1) ++c;
-            for (int x = lo; x <= c; ++x) gid[(size_t) (m - first) * cells + x] = (int) gs.size();
-            gs.push_back({lo, c});
-        }
-    }
-    int *d_gid = arena.take<int>(gid.size());
-    std::copy(gid.begin(), gid.end(), pin_i());
-    HIP_OK(hipMemcpyAsync(d_gid, pin, gid.size() * sizeof(int), hipMemcpyHostToDevice, st));
+hipError_t launch_p_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
+                          int cells, int *flags, hipStream_t st) {
+    if (nblk <= 0) return hipSuccess;
+    LAUNCH(k_p_flags, dim3(nblk), dim3(kBlock), 0, st, T, blk_off, nt, cellC, n, cells, flags);
+    return hipGetLastError();
+}
 
-    for (int m = first; m < d; ++m) {
-        const dmask_t smask = T.smask | dbit(m);
-        const auto &gs = groups[m - first];
-        const int G = (int) gs.size();
-        const size_t dim_mark = arena.mark();
-        int *cnt = arena.take<int>((size_t) 4 * G);
-        int *PP = arena.take<int>(std::max(T.nP_max, 1));
-        int *PW = arena.take<int>(std::max(T.nP_max, 1));
-        const Subspace &sub = subs[smask];
-        HIP_OK(launch_partition(T.P, T.nP, T.nP_max, cellC + (size_t) m * n, d_gid + (size_t) (m - first) * cells, G,
-                                sub.cnt, weak_thr, phi_mode ? 1 : 0, cnt, PP, PW, st));
-        HIP_OK(hipMemcpyAsync(pin, cnt, (size_t) 2 * G * sizeof(int), hipMemcpyDeviceToHost, st));
-        sync();
-        std::vector<int> c2(pin_i(), pin_i() + 2 * G);
-        // m's level the deepest unrestricted one, and the level above it:
-        // the point filter of merged groups
-        const int Lm = lvl_of[m];
-        int deeper = 0, tabove = -1;
-        for (int t = 0; t < d; ++t) {
-            const int k = level[t];
-            if (dhas(T.smask, k) || k == m) continue;
-            if (t > Lm) deeper = 1;
-            else tabove = t;
-        }
-        const bool filt = !deeper && (tabove < 0 || level[tabove] > m);
-        const dmask_t restricted = levels_of(smask);
-        // levels of nodes above m's level kept empty by a larger dimension id below
-        dmask_t cond = 0;
-        for (int t = 0; t < Lm; ++t) {
-            const int k = level[t];
-            if (dhas(T.smask, k)) continue;
-            for (int u = t; u < Lm; ++u)
-                if (!dhas(T.smask, level[u]) && level[u] > m) cond |= dbit(t);
-        }
-        // the dimension's cluster marks, below every group's buffers (a
-        // group's buffers are released while its kernels may still be queued:
-        // later launches on the stream reuse the memory only after them)
-        uint8_t *lab_buf = arena.take<uint8_t>(n);
-        uint8_t *lab = nullptr;
-        int offP = 0, offW = 0;
-        for (int g = 0; g < G; ++g) {
-            int nPr = c2[g], nW = c2[G + g];
-            const int *Pg = PP + offP, *Wg = PW + offW;
-            offP += nPr;
-            offW += nW;
-            const size_t group_mark = arena.mark();
-            int *nPg = arena.take<int>(2);
-            int *nWg = nPg + 1;
-            HIP_OK(launch_fill_i32(nPg, nPr, 1, st));
-            HIP_OK(launch_fill_i32(nWg, nW, 1, st));
-            if (filt && gs[g].hi > gs[g].lo && nPr > 0) {
-                const size_t slots = slots_for(nPr);
-                uint64_t *table = arena.take<uint64_t>(slots);
-                int *flag = arena.take<int>(3);
-                int *P2 = arena.take<int>(std::max(nPr, 1));
-                int *W2 = arena.take<int>(std::max(nW, 1));
-                HIP_OK(launch_fill_u64(table, kEmpty, slots, st));
-                HIP_OK(launch_fill_i32(flag, 0, 3, st));
-                LAUNCH(k_perm_lo_mark, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, m, gs[g].lo,
-                       tabove, table, (uint64_t) (slots - 1), flag);
-                LAUNCH(k_perm_lo_filter, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, tabove,
-                       table, (uint64_t) (slots - 1), flag, P2, flag + 1);
-                if (nW > 0)
-                    LAUNCH(k_perm_lo_filter, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, restricted, Wg, nWg, tabove,
-                           table, (uint64_t) (slots - 1), flag, W2, flag + 2);
-                HIP_OK(hipGetLastError());
-                HIP_OK(hipMemcpyAsync(pin, flag + 1, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
-                sync();
-                nPr = pin_i()[0];
-                nW = pin_i()[1];
-                Pg = P2;
-                Wg = W2;
-                HIP_OK(launch_fill_i32(nPg, nPr, 1, st));
-                HIP_OK(launch_fill_i32(nWg, nW, 1, st));
-            }
-            stats.trees++;
-            const bool pass = nW >= prm.min_size;
-            const size_t at = trace.size();
-            if (trace_on) trace.push_back({(long long) dlo(smask), gs[g].lo, gs[g].hi, nPr, nW, pass ? 1 : 0, -1});
-            if (!pass) {
-                arena.release(group_mark);
-                continue;
-            }
-            // the group's chains, then their prune
-            const int cap = std::max(T.nsp_max, 1);
-            int *rx = arena.take<int>(cap);
-            uint64_t *rm = arena.take<uint64_t>(cap);
-            int *nr = arena.take<int>(1);
-            int *cx2 = arena.take<int>(cap);
-            uint64_t *cm2 = arena.take<uint64_t>(cap);
-            int *nc2 = arena.take<int>(1);
-            HIP_OK(launch_fill_i32(nr, 0, 1, st));
-            HIP_OK(launch_fill_i32(nc2, 0, 1, st));
-            if (T.nsp_max > 0) {
-                LAUNCH(k_perm_route, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, T.smask, m,
-                       d_gid + (size_t) (m - first) * cells, g, T.spx, T.chain, T.nsp, rx, rm, nr);
-                int free_dims = 0;
-                dmask_t need = 0;  // unrestricted levels
-                for (int t = 0; t < d; ++t)
-                    if (!dhas(restricted, t)) {
-                        ++free_dims;
-                        need |= dbit(t);
-                    }
-                const size_t ws = slots_for((long long) nW * free_dims), ps = slots_for((long long) nPr * free_dims),
-                             ts = slots_for((long long) T.nP_max * free_dims),
-                             as = slots_for((long long) T.nsp_max * free_dims);
-                uint64_t *tw = arena.take<uint64_t>(ws), *tp = arena.take<uint64_t>(ps), *tt = arena.take<uint64_t>(ts),
-                         *ta = arena.take<uint64_t>(as);
-                HIP_OK(launch_fill_u64(tw, kEmpty, ws, st));
-                HIP_OK(launch_fill_u64(tp, kEmpty, ps, st));
-                HIP_OK(launch_fill_u64(tt, kEmpty, ts, st));
-                HIP_OK(launch_fill_u64(ta, kEmpty, as, st));
-                if (nW > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nW)), dim3(kBlock), 0, st, D, restricted, Wg, nWg, need, tw,
-                           (uint64_t) (ws - 1));
-                if (nPr > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(nPr)), dim3(kBlock), 0, st, D, restricted, Pg, nPg, need, tp,
-                           (uint64_t) (ps - 1));
-                if (cond && T.nP_max > 0)
-                    LAUNCH(k_perm_insert_pts, dim3(blocks_for(T.nP_max)), dim3(kBlock), 0, st, D, restricted, T.P, T.nP,
-                           cond & need, tt, (uint64_t) (ts - 1));
-                LAUNCH(k_perm_insert_anchors, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, restricted, rx, rm, nr,
-                       ta, (uint64_t) (as - 1));
-                const PermTables Tb{tw, tp, tt, ta, ws - 1, ps - 1, ts - 1, as - 1, cond};
-                LAUNCH(k_perm_prune, dim3(blocks_for(T.nsp_max)), dim3(kBlock), 0, st, D, restricted, Tb, rx, rm, nr, cx2,
-                       cm2, nc2);
-                HIP_OK(hipGetLastError());
-            }
-            Subspace &s2 = ensure_components(smask);
-            TreeRef child{smask, Wg, nWg, nW, cx2, cm2, nc2, T.nsp_max};
-            recurse_perm(child, m + 1);
-            // pruneRedundancy then cluster, on the device in stream order
-            if (!lab) {
-                lab = lab_buf;
-                HIP_OK(launch_fill_u8(lab, 0, n, st));
-            }
-            HIP_OK(launch_redundancy_seed(Wg, nWg, nW, stamp, ++tree_id, entries, d_nE, smask, s2.comp, d_list,
-                                          d_nlist, d_mn, prm.r, d_keep, lab, st));
-            if (trace_on) {
-                HIP_OK(hipMemcpyAsync(pin, d_keep, sizeof(int), hipMemcpyDeviceToHost, st));
-                sync();
-                trace[at].redundant = pin_i()[0] ? 0 : 1;
-            }
-            arena.release(group_mark);
-        }
-        if (lab) join(smask, lab);
-        arena.release(dim_mark);
-    }
-    arena.release(lvl_mark);
+hipError_t launch_p_filter(const DevData &D, const PermFilter *F, const int *blk_off, int nf, int nblk,
+                           hipStream_t st) {
+    if (nblk <= 0) return hipSuccess;
+    LAUNCH(k_p_filter<true>, dim3(nblk), dim3(kBlock), 0, st, D, F, blk_off, nf);
+    LAUNCH(k_p_filter<false>, dim3(nblk), dim3(kBlock), 0, st, D, F, blk_off, nf);
+    return hipGetLastError();
+}
+
+hipError_t launch_p_count(const DevData &D, const PermPair *P, const int *blk_off, int np, int nblk, hipStream_t st) {
+    if (nblk <= 0) return hipSuccess;
+    LAUNCH(k_p_count, dim3(nblk), dim3(kBlock), 0, st, D, P, blk_off, np);
+    return hipGetLastError();
+}
+
+hipError_t launch_p_prune(const DevData &D, const PermChild *C, int nc, const int *blk_route, int nblk_route,
+                          const int *blk_mark, int nblk_mark, const int *blk_check, int nblk_check, int thr, int wbit,
+                          hipStream_t st) {
+    if (nc <= 0) return hipSuccess;
+    if (nblk_route > 0) LAUNCH(k_p_route, dim3(nblk_route), dim3(kBlock), 0, st, D, C, blk_route, nc);
+    if (nblk_mark > 0) LAUNCH(k_p_mark, dim3(nblk_mark), dim3(kBlock), 0, st, D, C, blk_mark, nc, thr, wbit);
+    if (nblk_check > 0) LAUNCH(k_p_check, dim3(nblk_check), dim3(kBlock), 0, st, D, C, blk_check, nc);
+    return hipGetLastError();
 }
 
 }  // namespace inscy

@@ -127,3 +127,26 @@ def test_sample_phase_sizes(n, per):
     assert got.subspaces == [[0], [1], [0, 1]]
     for a, b in zip(got.labels, want):
         assert np.array_equal(a, O.canonical(b))
+
+
+# the permuted level orders' passes over one pair, a few and all pairs of a level at once
+@pytest.mark.parametrize("order", [1, -1])
+@pytest.mark.parametrize("max_batch", [1, 3, 0])
+def test_permuted_order_in_batches_matches_oracle(max_batch, order):
+    for n, d, eps, num_obj, rect in ((257, 5, 0.11, 4, True), (1201, 4, 0.05, 4, False), (1031, 7, 0.07, 2, True)):
+        print("permuted batches", max_batch, order, n, d, flush=True)
+        X = edge_data(n + d, n, d, eps)
+        args = (eps, 1.0, num_obj, max(4, n // 40), 1.0, 3, rect)
+        ref = O.run_ref(X, *args, order, trace=True)
+        _lib.set_tuning(max_batch=max_batch)
+        _lib.debug_trace(True)
+        try:
+            got = INSCY.run(torch.from_numpy(X).cuda(), *args, order, mode=_lib.MODE_BATCHED)
+            trace = _lib.debug_trace_rows()
+        finally:
+            _lib.debug_trace(False)
+            _lib.set_tuning()
+        assert got.subspaces == ref.subspaces
+        for a, b in zip(ref.labels, got.labels):
+            assert np.array_equal(O.canonical(a), b)
+        assert np.array_equal(trace, ref.trace)
