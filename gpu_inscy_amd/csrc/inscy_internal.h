@@ -184,7 +184,7 @@ struct BatchIndex {
     int2 *fb;             // phi mode: (subspace, point) pairs to recompute in leaf order
     int *nfb;             // [1] their number
     int fbcap;
-    uint8_t *dsorted;     // [B*n] dense flag per sorted position
+    int *rootpos;         // [B*n] root of the sample phase per sorted position, -1 where not dense
     int *par;             // [B*n] union-find parents (point ids within each subspace)
     int *giant;           // [B]
     int *fit;             // [B] the subspace's sample phase ran in LDS (k_b_sample)

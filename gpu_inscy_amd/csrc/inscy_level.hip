@@ -286,11 +286,11 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             GridArg G = grid_of(S, -1, true);
             const long long ncell = grid_cells(G);
             // process_batch's takes per subspace: counts, query flags and
-            // list, two sample edges, dense flags and parents (22 bytes a
+            // list, two sample edges, sample-phase roots and parents (25 bytes a
             // point), an index that is not kept (keys, rank, order, position:
             // 16, k coordinate columns: 4k, grid histogram and offsets), the
             // phi pass's queue (8)
-            size_t est = (size_t) n * (38 + 4 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 12;
+            size_t est = (size_t) n * (41 + 4 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 12;
             // the index and the queries of a fanned mask
             if (fan && (j == i || cs[j - 1].t0 != c.t0)) est += (size_t) n * (21 + 4 * (size_t) S.k) + (size_t) ncell * 12;
             for (int a = c.t0; a < c.t1; ++a) {
@@ -905,7 +905,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             stamps[u].dst = stamp_of[stamp_b[u]];
             copies.push_back(stamps[u]);
         }
-        X.dsorted = batch.take<uint8_t>((size_t) ncomp * n + 8);  // the grouped link walk reads aligned words past the end
+        X.rootpos = batch.take<int>((size_t) ncomp * n + 4);  // the grouped link walk reads up to 3 past a run
         X.par = batch.take<int>((size_t) ncomp * n);
         X.giant = batch.take<int>(ncomp);
         X.fit = batch.take<int>(ncomp);

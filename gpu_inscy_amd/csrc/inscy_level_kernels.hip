@@ -993,7 +993,7 @@ __device__ __forceinline__ int hooked(const BatchSub &B, const int *__restrict__
 }
 
 __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restrict__ subs, int n,
-                                                         const int *__restrict__ nb, uint8_t *__restrict__ dsorted,
+                                                         const int *__restrict__ nb, int *__restrict__ rootpos,
                                                          int *__restrict__ par, int *__restrict__ giant,
                                                          int *__restrict__ fit) {
     __shared__ int up[kUfCap];
@@ -1008,19 +1008,17 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
     const int2 *nb2 = reinterpret_cast<const int2 *>(nb) + B.nbase;
     static_assert(kSampleEdges == 2, "a point's sample edges are one int2");
     for (int i0 = t; i0 < n; i0 += STEP) {
-        int c[M], o[M], co[M];
+        int c[M];
         int2 q[M];
         int cq[M][2];
 #pragma unroll
         for (int u = 0; u < M; ++u) {
             const int i = min(i0 + u * kUfThreads, n - 1);
             c[u] = B.cnt[i];
-            o[u] = B.order[i];
             q[u] = numbered ? nb2[i] : make_int2(-1, -1);
         }
 #pragma unroll
         for (int u = 0; u < M; ++u) {
-            co[u] = B.cnt[o[u]];
             cq[u][0] = q[u].x >= 0 && q[u].x < n ? B.cnt[q[u].x] : 0;
             cq[u][1] = q[u].y >= 0 && q[u].y < n ? B.cnt[q[u].y] : 0;
         }
@@ -1028,7 +1026,6 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
         for (int u = 0; u < M; ++u) {
             const int i = i0 + u * kUfThreads;
             if (i >= n) continue;
-            dsorted[B.base + i] = meets(co[u], B.thr_dense, B.dbit) ? 1 : 0;
             int root = -1;
             if (meets(c[u], B.thr_dense, B.dbit)) {
                 root = i;
@@ -1145,7 +1142,20 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
             if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
     }
     __syncthreads();  // the ids by number are read, the parents written
-    for (int i = t; i < n; i += kUfThreads) B.csize[i] = 0;
+    for (int i0 = t; i0 < n; i0 += STEP) {
+        int o[M];
+#pragma unroll
+        for (int u = 0; u < M; ++u) o[u] = B.order[min(i0 + u * kUfThreads, n - 1)];
+#pragma unroll
+        for (int u = 0; u < M; ++u) o[u] = pr[o[u]];
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            const int i = i0 + u * kUfThreads;
+            if (i >= n) continue;
+            rootpos[B.base + i] = o[u];
+            B.csize[i] = 0;
+        }
+    }
     if (t < 256) {
         const int p = (int) (((long long) t * n) / 256);
         up[t] = p < n ? pr[p] : -1;
@@ -1177,15 +1187,11 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
 
 // The same on global parents, for the subspaces that do not fit (fit null: all).
 __global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, const int *__restrict__ nb,
-                               const int *__restrict__ fit, uint8_t *__restrict__ dsorted, int *__restrict__ par) {
+                               const int *__restrict__ fit, int *__restrict__ par) {
     if (fit && fit[blockIdx.y]) return;
     const BatchSub &B = subs[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    // i is a sorted position for the dense flag and a point id for the
-    // parents and sizes, so every write is coalesced
-    const int p = B.order[i];
-    dsorted[B.base + i] = meets(B.cnt[p], B.thr_dense, B.dbit) ? 1 : 0;
     par[B.base + i] = hooked(B, nb, i);
     B.csize[i] = 0;
 }
@@ -1229,6 +1235,15 @@ __global__ void k_b_uf_compress(const BatchSub *__restrict__ subs, int n, const 
     if (i < n && pr[i] >= 0) pr[i] = uf_find(pr, i);
 }
 
+// the parents in sorted order, for the full phase
+__global__ void k_b_rootpos(const BatchSub *__restrict__ subs, int n, const int *__restrict__ fit,
+                            const int *__restrict__ par, int *__restrict__ rootpos) {
+    if (fit && fit[blockIdx.y]) return;
+    const BatchSub &B = subs[blockIdx.y];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) rootpos[B.base + i] = par[B.base + B.order[i]];
+}
+
 // one block of 256 per subspace: the most frequent root among 256 evenly
 // spaced points
 __global__ void k_b_giant(const BatchSub *__restrict__ subs, int n, const int *__restrict__ fit,
@@ -1260,13 +1275,19 @@ __global__ void k_b_giant(const BatchSub *__restrict__ subs, int n, const int *_
 }
 
 // Full phase: every dense point outside the giant component links to all its
-// dense neighbours.  K > 0: every subspace of the launch has k = K, and a step
-// loads the dense flags, point ids and K coordinates of U candidates per lane
-// at once (a lane past the end re-reads the last candidate and is masked).
+// dense neighbours.  Nearly all candidates are in the point's own set after the
+// sample phase, so a step reads the roots of that phase first (rootpos, by
+// sorted position, -1 where not dense: kLinkGroups groups of four per lane in
+// flight), and only a group with a root of another set is tested on its ids,
+// coordinates and cells (tested first, every candidate cost K + 2 loads:
+// n=100,000 d=20 38.3 -> 34.2 ms a run, n=25,000 d=15 1.6 -> 1.2; one group in
+// flight 36.1).  The staging of a query is what bounds it now.
+// K > 0: every subspace of the launch has k = K.
+constexpr int kLinkGroups = 4;
 template <int K>
 __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restrict__ subs, int n,
                                                         const float *__restrict__ edge,
-                                                        const uint8_t *__restrict__ dsorted, float s_star,
+                                                        const int *__restrict__ rootpos, float s_star,
                                                         const int *__restrict__ giant, int *__restrict__ par) {
     constexpr int LPQ = kBLanes;
     extern __shared__ char smem[];
@@ -1278,13 +1299,15 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
     lds_layout(smem, k, sc, sy, qr);
     const int lq = threadIdx.x / LPQ, sub = threadIdx.x % LPQ;
     const int i = blockIdx.x * QPB + lq;
-    const uint8_t *ds = dsorted + B.base;
+    const int *rts = rootpos + B.base;
     const int *ord = B.order;
     int *pr = par + B.base;
-    bool active = i < n && ds[i];
-    const int p = active ? ord[i] : 0;
-    if (active && pr[p] == giant[blockIdx.y]) active = false;
+    const int r0 = i < n ? rts[i] : -1;  // the point's set after the sample phase
+    const bool active = r0 >= 0 && r0 != giant[blockIdx.y];
     int *q = qr + lq * kRangeWords;
+    // r0 stands for the point in every union: its parent is read while the
+    // query is staged
+    int rp = active ? uf_find(pr, r0) : -1;
     if (sub == 0 && active) {
         int ci[3];
         stage_query_b(B, edge, i, sy + lq, sc + lq, QPB, ci);
@@ -1295,66 +1318,65 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
     const float *qy = sy + lq;
     const float2 *qcl = sc + lq;
     const int total = q[9 + q[19]];
-    int rp = uf_find(pr, p);
     if constexpr (K > 0) {
-        // each lane four consecutive candidates of one run per step (the
-        // groups of walk_vec): per step one 16-byte load for the ids and each
-        // coordinate column, and two aligned words for the four dense flags
+        // each lane four consecutive candidates of one run per group (the
+        // groups of walk_vec)
         typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
         typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
-        constexpr int U = 4;
+        constexpr int U = 4, W = kLinkGroups;
         const uint32_t checked = (uint32_t) B.G.checkmask;
-        const float *col[K];
-        float qv[K];
-#pragma unroll
-        for (int t = 0; t < K; ++t) {
-            col[t] = B.col[t];
-            qv[t] = qy[t * QPB];
-        }
-        const uint32_t *dw = reinterpret_cast<const uint32_t *>(dsorted);  // 256-byte aligned
         const int nr = q[19];
         const int gtotal = q[21 + nr];
         int r = 0, rgend = q[22];
-        for (int g0 = 0; g0 < gtotal; g0 += LPQ) {
-            const int g = min(g0 + sub, gtotal - 1);
-            while (g >= rgend) {
-                ++r;
-                rgend = q[22 + r];
+        for (int g0 = 0; g0 < gtotal; g0 += W * LPQ) {
+            int at[W], nv[W];
+            i4u rt[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int gw = g0 + w * LPQ + sub;
+                const int g = min(gw, gtotal - 1);
+                while (g >= rgend) {
+                    ++r;
+                    rgend = q[22 + r];
+                }
+                const int e0 = (g - q[21 + r]) << 2;
+                nv[w] = gw < gtotal ? min(U, q[10 + r] - q[9 + r] - e0) : 0;
+                at[w] = q[r] + e0;
+                rt[w] = *reinterpret_cast<const i4u *>(rts + (uint32_t) at[w]);
             }
-            const int e0 = (g - q[21 + r]) << 2;
-            const int len = q[10 + r] - q[9 + r];
-            const int nv = g0 + sub < gtotal ? min(U, len - e0) : 0;
-            const int jj0 = q[r] + e0;
-            const size_t at = (size_t) B.base + (size_t) jj0;  // byte index of the first dense flag
-            const uint32_t d0 = dw[at >> 2], d1 = dw[(at >> 2) + 1];
-            const i4u qv4 = *reinterpret_cast<const i4u *>(ord + (uint32_t) jj0);
-            f4u y[K];
 #pragma unroll
-            for (int t = 0; t < K; ++t) y[t] = *reinterpret_cast<const f4u *>(col[t] + (uint32_t) jj0);
-            const uint32_t dn4 = __builtin_amdgcn_alignbyte(d1, d0, (uint32_t) (at & 3));
-            const int qq[U] = {qv4.x, qv4.y, qv4.z, qv4.w};
-            bool hit[U];
+            for (int w = 0; w < W; ++w) {
+                bool other[U], any = false;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                float acc = 0.0f;
+                for (int u = 0; u < U; ++u) {
+                    other[u] = (u < nv[w]) & (rt[w][u] >= 0) & (rt[w][u] != r0);
+                    any |= other[u];
+                }
+                if (!any) continue;
+                const int jj0 = at[w];
+                const i4u id = *reinterpret_cast<const i4u *>(ord + (uint32_t) jj0);
+                float acc[U] = {};
 #pragma unroll
                 for (int t = 0; t < K; ++t) {
-                    const float diff = qv[t] - y[t][u];
-                    const float sq = diff * diff;
-                    acc = acc + sq;
+                    const f4u y = *reinterpret_cast<const f4u *>(B.col[t] + (uint32_t) jj0);
+                    const float qv = qy[t * QPB];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const float diff = qv - y[u];
+                        const float sq = diff * diff;
+                        acc[u] = acc[u] + sq;
+                    }
                 }
-                hit[u] = (u < nv) & (jj0 + u != i) & (((dn4 >> (8 * u)) & 0xFFu) != 0) & (acc <= s_star);
-            }
-            if (checked) cells_of_hits<U>(B, qcl, QPB, checked, jj0, hit);
-            // parents only move up to roots: a parent equal to p's root is p's set
-            int pq[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) pq[u] = hit[u] ? pr[qq[u]] : rp;
+                for (int u = 0; u < U; ++u) other[u] &= acc[u] <= s_star;
+                if (checked) cells_of_hits<U>(B, qcl, QPB, checked, jj0, other);
+                // parents only move up to roots: a parent equal to p's root is p's set
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (!hit[u] || pq[u] == rp || uf_find(pr, qq[u]) == rp) continue;
-                uf_union(pr, p, qq[u]);
-                rp = uf_find(pr, p);
+                for (int u = 0; u < U; ++u) {
+                    if (!other[u] || pr[id[u]] == rp || uf_find(pr, id[u]) == rp) continue;
+                    uf_union(pr, r0, id[u]);
+                    rp = uf_find(pr, r0);
+                }
             }
         }
     } else {
@@ -1362,12 +1384,12 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
         for (int c = sub; c < total; c += LPQ) {
             const int jj = run_pos(q, c, r);
             float acc;
-            if (jj == i || !ds[jj] || !cand_test(B, qy, qcl, QPB, jj, s_star, acc)) continue;
+            if (rts[jj] < 0 || rts[jj] == r0 || !cand_test(B, qy, qcl, QPB, jj, s_star, acc)) continue;
             const int qq = ord[jj];
             // parents only move up to roots: a parent equal to p's root is p's set
             if (pr[qq] == rp || uf_find(pr, qq) == rp) continue;
-            uf_union(pr, p, qq);
-            rp = uf_find(pr, p);
+            uf_union(pr, r0, qq);
+            rp = uf_find(pr, r0);
         }
     }
 }
@@ -2320,19 +2342,20 @@ hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, 
     const bool lds_pass = n <= 4 * kUfCap;
     const int *fit = lds_pass ? X.fit : nullptr;
     if (lds_pass)
-        LAUNCH(k_b_sample, dim3(nsub), dim3(kUfThreads), 0, st, subs, n, X.nb, X.dsorted, X.par, X.giant, X.fit);
+        LAUNCH(k_b_sample, dim3(nsub), dim3(kUfThreads), 0, st, subs, n, X.nb, X.rootpos, X.par, X.giant, X.fit);
     if (n > kUfCap) {
         const dim3 all(blocks_for(n), nsub);
-        LAUNCH(k_b_dense_init, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.dsorted, X.par);
+        LAUNCH(k_b_dense_init, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.par);
         LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
         LAUNCH(k_b_link_sample, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.par);
         LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
+        LAUNCH(k_b_rootpos, all, dim3(kBlock), 0, st, subs, n, fit, X.par, X.rootpos);
         LAUNCH(k_b_giant, dim3(nsub), dim3(256), 0, st, subs, n, fit, X.par, X.giant);
     }
     const dim3 grid(query_blocks_n(n), nsub);
     const size_t lds = count_lds(kmax);
 #define LINK_FULL(K)                                                                                                   \
-    LAUNCH(k_b_link_full<K>, grid, dim3(kBlock), lds, st, subs, n, X.edge, X.dsorted,      \
+    LAUNCH(k_b_link_full<K>, grid, dim3(kBlock), lds, st, subs, n, X.edge, X.rootpos,      \
            s_star, X.giant, X.par)
     switch (kfast) {
     case 1: LINK_FULL(1); break;
