@@ -27,7 +27,7 @@ import numpy as np
 from . import _lib, datagen
 from . import inscy as INSCY
 
-BATCHES = (256, 512, 1024, 2048)
+BATCHES = (256, 512, 1024, 2048, 4096)
 WORKERS = (2, 4, 8)
 
 

@@ -146,7 +146,7 @@ int inscy_profile(int on);
 
 /* Tuning of later calls of this process (no counterpart in the reference;
  * gpu_inscy_amd/autotune.py measures and applies it): max_batch child
- * subspaces per level-synchronous batch (default 1024, still bounded by
+ * subspaces per level-synchronous batch (default 4096, still bounded by
  * memory), workers streams of inscy_run_many (default 8); 0 restores a
  * default.  INSCY_ERR_ARGUMENT outside [0, 65536] and [0, 64].  Results do
  * not depend on either. */
