@@ -534,7 +534,7 @@ struct TreeHit {
 };
 hipError_t launch_tree_hits(const TreeHit *trees, const int *blk_off, int ntrees, int nblk, int *hit, hipStream_t st);
 
-constexpr int kRangeWords = 31;      // per query in LDS: 9 range starts, 10 prefix sums, count, own run, 10 group sums
+constexpr int kRangeWords = 31;      // per query in LDS: 9 run starts, 10 prefix sums, own run, 10 group sums; odd for the banks
 constexpr int kBlockThreads = 256;   // threads per block of every pass
 constexpr int kQueriesPerBlock = 64;  // queries per block of the batched neighbour passes
 constexpr int kMaxFastK = 8;          // neighbour walks are compiled for each k up to this

@@ -140,22 +140,37 @@ __global__ void k_b_qmark(const BatchSub *__restrict__ subs, const QuerySeg *__r
 // The candidates of a query are up to 9 runs of sorted positions (grid cells
 // of the index dimensions).  They are concatenated into one index space
 // [0, total): q[0..8] run starts (local positions), q[9..18] prefix sums of
-// the run lengths, q[19] the number of runs.  A lane maps its candidate
+// the run lengths (empty runs stay in place).  A lane maps its candidate
 // number to a position with a run pointer that only moves forward.
-// q[20]: the run of the query's own cells in the first index dimensions (it
-// holds the query, so it is not empty).  q[21..30]: prefix sums of the runs'
+// q[19]: the run of the query's own cells in the first index dimensions (it
+// holds the query, so it is not empty).  q[20..29]: prefix sums of the runs'
 // lengths in groups of four (ceil(length / 4)), for the walks that take four
 // consecutive candidates of one run per lane.
-__device__ __forceinline__ void build_runs(const GridArg &G, const int *__restrict__ off, const int *ci,
-                                           const float *qy, int stride, float s_star, int *q) {
-    // rows r = 3 xi + yi over the cells within one of the query's in the first
-    // (and second) index dimension, each a run of the last one's cells within
-    // one; every row's two offsets are loaded before any is used, so the
-    // set-up costs one memory round trip
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// inclusive sum over the lanes of a quad (all four active)
+__device__ __forceinline__ int quad_scan(int v, int sub) {
+    int o = __builtin_amdgcn_update_dpp(0, v, 0x90, 0xF, 0xF, false);  // quad_perm [0,0,1,2]
+    v += sub >= 1 ? o : 0;
+    o = __builtin_amdgcn_update_dpp(0, v, 0x44, 0xF, 0xF, false);  // quad_perm [0,1,0,1]
+    return v + (sub >= 2 ? o : 0);
+}
+
+// rows r = 3 xi + yi over the cells within one of the query's in the first
+// (and second) index dimension, each a run of the last one's cells within one:
+// lane `sub` of the query's quad takes rows sub, sub + 4 and 8; every row's two
+// offsets are loaded before any is used, so the runs cost one memory round trip
+__device__ __forceinline__ void build_runs(const GridArg &G, const int *__restrict__ off, const float *qy, int stride,
+                                           int sub, float s_star, int *q) {
     const int C = G.C;
-    const int c0 = ci[0];
-    const int c1 = G.j == 3 ? ci[1] : 0;
-    const int cl = ci[G.j - 1];
+    const float ecs = ecell_width(C);
+    const int c0 = ecell_of(qy[G.tI[0] * stride], ecs, C);
+    const int c1 = G.j == 3 ? ecell_of(qy[G.tI[1] * stride], ecs, C) : 0;
+    const float yl = qy[G.tI[G.j - 1] * stride];
+    const int cl = ecell_of(yl, ecs, C);
     const int F = G.F > 1 ? G.F : 1, CF = C * F;
     // a run: the buckets of the last dimension's cells within one of the
     // query's, less those farther than eps from the query's coordinate (a
@@ -163,41 +178,43 @@ __device__ __forceinline__ void build_runs(const GridArg &G, const int *__restri
     // rounded outwards and the bucket map is monotone, so no neighbour is lost)
     int lo = max(cl - 1, 0) * F, hi = min(cl + 1, C - 1) * F + F - 1;
     if (F > 1) {
-        const double xq = (double) qy[G.tI[G.j - 1] * stride];
+        const double xq = (double) yl;
         const double em = sqrt((double) s_star) * 1.001 + 1e-6;
         lo = max(lo, fine_key(__double2float_rd(xq - em), C, F));
         hi = min(hi, fine_key(__double2float_ru(xq + em), C, F));
     }
     const int x0 = max(c0 - 1, 0), nx = G.j == 1 ? 1 : min(c0 + 1, C - 1) - x0 + 1;
     const int y0 = max(c1 - 1, 0), ny = G.j == 3 ? min(c1 + 1, C - 1) - y0 + 1 : 1;
-    const int own = G.j == 1 ? 0 : 3 * (c0 - x0) + (G.j == 3 ? c1 - y0 : 0);
-    int a[9], e[9];
+    int a[3], e[3];
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
+    for (int w = 0; w < 3; ++w) {
         // rows past the edge of the grid load a row inside it (no branch
-        // around the loads) and are dropped below
+        // around the loads) and are emptied below
+        const int r = min(sub + 4 * w, 8);
         const int xi = min(r / 3, nx - 1), yi = min(r % 3, ny - 1);
         const int row = G.j == 1 ? 0 : G.j == 2 ? (x0 + xi) * CF : ((x0 + xi) * C + y0 + yi) * CF;
-        a[r] = off[row + lo];
-        e[r] = off[row + hi + 1];
+        a[w] = off[row + lo];
+        e[w] = off[row + hi + 1];
     }
-    int nr = 0, acc = 0, gacc = 0;
-    q[9] = 0;
-    q[20] = 0;
-    q[21] = 0;
+    int acc = 0, gacc = 0;
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        if (r / 3 < nx && r % 3 < ny && e[r] > a[r]) {
-            if (r == own) q[20] = nr;
-            q[nr] = a[r];
-            acc += e[r] - a[r];
-            gacc += (e[r] - a[r] + 3) >> 2;
-            q[10 + nr] = acc;
-            q[22 + nr] = gacc;
-            ++nr;
+    for (int w = 0; w < 3; ++w) {
+        const int r = sub + 4 * w;
+        const int len = r < 9 && r / 3 < nx && r % 3 < ny ? max(e[w] - a[w], 0) : 0;
+        const int s = acc + quad_scan(len, sub), g = gacc + quad_scan((len + 3) >> 2, sub);
+        if (r < 9) {
+            q[r] = a[w];
+            q[10 + r] = s;
+            q[21 + r] = g;
         }
+        acc = __builtin_amdgcn_update_dpp(0, s, 0xFF, 0xF, 0xF, false);  // quad_perm [3,3,3,3]
+        gacc = __builtin_amdgcn_update_dpp(0, g, 0xFF, 0xF, 0xF, false);
     }
-    q[19] = nr;
+    if (sub == 0) {
+        q[9] = 0;
+        q[19] = G.j == 1 ? 0 : 3 * (c0 - x0) + (G.j == 3 ? c1 - y0 : 0);
+        q[20] = 0;
+    }
 }
 
 __device__ __forceinline__ int run_pos(const int *q, int c, int &r) {
@@ -233,49 +250,45 @@ __device__ __forceinline__ void lds_layout(char *smem, int k, float2 *&sc, float
     qr = reinterpret_cast<int *>(smem + (sizeof(float2) + sizeof(float)) * QPB * (size_t) k);
 }
 
-// the query's coordinates (sorted position i) and, per checked dimension, the
-// interval [lower, upper) of the coordinates whose eps cell is within one of
-// its own, into LDS: the first 8 dimensions' loads are all issued before any
-// store (a store to LDS through a generic pointer would otherwise order each
-// load after the previous store, one memory round trip per dimension)
-// (the cells are computed from the coordinates with the discretisation's
-// formula, G.C being the number of eps cells: no scattered read by point id;
-// the intervals come from the table of cell edges, see cell_edge)
-__device__ __forceinline__ void stage_query_b(const BatchSub &B, const float *__restrict__ edge, int i, float *sy,
-                                              float2 *sc, int stride, int *ci) {
-    constexpr int kStage = 8;
+// The query at sorted position i into LDS, by its quad: the coordinates and,
+// per checked dimension, the interval [lower, upper) of the coordinates whose
+// eps cell is within one of its own (lane `sub` takes dimensions sub, sub + 4,
+// ...; the cells come from the coordinates with the discretisation's formula,
+// the intervals from the table of cell edges, see cell_edge), then its runs.
+// By one lane of the four it took four times a wave's instructions: n=100,000
+// d=20, the full link phase 34.1 -> 28.1 ms a run, the counts of k_b_count 45.7 ->
+// 43.0; n=25,000 d=15 1.2 -> 1.1 and 1.2 -> 1.2.
+__device__ __forceinline__ void stage_query_b(const BatchSub &B, const float *__restrict__ edge, int i, int sub,
+                                              float s_star, float *sy, float2 *sc, int stride, int *q) {
     const int k = B.S.k;
     const float ecs = ecell_width(B.G.C);
     const float inf = __builtin_inff();
-    float y[kStage];
-#pragma unroll
-    for (int t = 0; t < kStage; ++t) y[t] = t < k ? B.col[t][i] : 0.0f;
-    float2 c[kStage];
-#pragma unroll
-    for (int t = 0; t < kStage; ++t) {
-        c[t] = make_float2(-inf, inf);
-        if (t < k && ((B.G.checkmask >> t) & 1ull)) {
-            const int e = ecell_of(y[t], ecs, B.G.C);
-            c[t] = make_float2(edge[e], edge[e + 3]);
+    for (int t0 = 0; t0 < k; t0 += 2 * kBLanes) {
+        // two dimensions' loads are issued before any store (a store to LDS
+        // through a generic pointer would order the second load after it)
+        const int t1 = t0 + sub, t2 = t1 + kBLanes;
+        const float y1 = t1 < k ? B.col[t1][i] : 0.0f, y2 = t2 < k ? B.col[t2][i] : 0.0f;
+        float2 i1 = make_float2(-inf, inf), i2 = i1;
+        if (t1 < k && ((B.G.checkmask >> t1) & 1ull)) {
+            const int e = ecell_of(y1, ecs, B.G.C);
+            i1 = make_float2(edge[e], edge[e + 3]);
+        }
+        if (t2 < k && ((B.G.checkmask >> t2) & 1ull)) {
+            const int e = ecell_of(y2, ecs, B.G.C);
+            i2 = make_float2(edge[e], edge[e + 3]);
+        }
+        if (t1 < k) {
+            sy[t1 * stride] = y1;
+            sc[t1 * stride] = i1;
+        }
+        if (t2 < k) {
+            sy[t2 * stride] = y2;
+            sc[t2 * stride] = i2;
         }
     }
-#pragma unroll
-    for (int t = 0; t < kStage; ++t)
-        if (t < k) {
-            sy[t * stride] = y[t];
-            sc[t * stride] = c[t];
-        }
-    for (int t = kStage; t < k; ++t) {
-        const float v = B.col[t][i];
-        sy[t * stride] = v;
-        float2 cc = make_float2(-inf, inf);
-        if ((B.G.checkmask >> t) & 1ull) {
-            const int e = ecell_of(v, ecs, B.G.C);
-            cc = make_float2(edge[e], edge[e + 3]);
-        }
-        sc[t * stride] = cc;
-    }
-    for (int a = 0; a < B.G.j; ++a) ci[a] = ecell_of(sy[B.G.tI[a] * stride], ecs, B.G.C);
+    wave_sync();
+    build_runs(B.G, B.off, sy, stride, sub, s_star, q);
+    wave_sync();
 }
 
 // ------------------------------------------------------------ candidate walks of one query
@@ -298,7 +311,7 @@ struct QueryWalk {
 
 __device__ __forceinline__ int walk_rot(const QueryWalk &W, int total) {
     const int *q = W.q;
-    const int cs0 = q[9 + q[20]], clen = q[10 + q[20]] - cs0;
+    const int cs0 = q[9 + q[19]], clen = q[10 + q[19]] - cs0;
     return total > 0 ? cs0 + (int) (((uint32_t) W.p * 2654435761u) % (uint32_t) max(clen, 1)) : 0;
 }
 
@@ -366,7 +379,7 @@ __device__ __forceinline__ void cells_of_hits(const BatchSub &B, const float2 *q
 // The vector memory pipeline bounds these walks (its address and data units
 // are busy nearly all the time), and its cost grows with the number of load
 // instructions.  The runs are
-// concatenated in groups of four (q[21..30]); the last group of a run masks
+// concatenated in groups of four (q[20..29]); the last group of a run masks
 // the positions past the run's end, which are read (up to three past the
 // run: the batch's coordinate buffer ends with padding) but
 // never counted.  A lane's first group position is 4-byte aligned only;
@@ -379,12 +392,11 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
     const uint32_t checked = (uint32_t) B.G.checkmask;
     const int *q = W.q;
     const int sub = __lane_id() % LPQ;
-    const int nr = q[19];
-    const int gtotal = q[21 + nr], total = q[9 + nr];
+    const int gtotal = q[29], total = q[18];
     // start at a pseudo-random group of the query's own run (spreads the
     // sample edges), walk to the end, then from the start to there
-    const int own = q[20];
-    const int og = q[21 + own], olen = q[22 + own] - og;
+    const int own = q[19];
+    const int og = q[20 + own], olen = q[21 + own] - og;
     const int grot = gtotal > 0 ? og + (int) (((uint32_t) W.p * 2654435761u) % (uint32_t) max(olen, 1)) : 0;
     const float *col[K];
     float qv[K];
@@ -396,14 +408,14 @@ __device__ __forceinline__ void walk_vec(const QueryWalk &W, int &found, double 
     for (int segm = 0; segm < 2; ++segm) {
         const int gbeg = segm == 0 ? grot : 0, gend = segm == 0 ? gtotal : grot;
         int r = segm == 0 ? own : 0;
-        int rgend = q[22 + r];
+        int rgend = q[21 + r];
         for (int g0 = gbeg; g0 < gend && more; g0 += LPQ) {
             const int g = min(g0 + sub, gend - 1);
             while (g >= rgend) {
                 ++r;
-                rgend = q[22 + r];
+                rgend = q[21 + r];
             }
-            const int e0 = (g - q[21 + r]) << 2;  // the group's first element in run r
+            const int e0 = (g - q[20 + r]) << 2;  // the group's first element in run r
             const int len = q[10 + r] - q[9 + r];
             const int nv = g0 + sub < gend ? min(U, len - e0) : 0;  // its elements inside the run
             const int jj0 = q[r] + e0;
@@ -470,7 +482,7 @@ __device__ __forceinline__ void walk_generic(const QueryWalk &W, int &found, dou
     constexpr int LPQ = kBLanes, U = 4, STEP = LPQ * U;
     const int *q = W.q;
     const int sub = __lane_id() % LPQ;
-    const int total = q[9 + q[19]];
+    const int total = q[18];
     const int rot = walk_rot(W, total);
     int r = 0;
     bool wrapped = false;
@@ -563,12 +575,7 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
         }
     }
     int *q = qr + lq * kRangeWords;
-    if (sub == 0 && active) {
-        int ci[3];
-        stage_query_b(B, edge, i, sy + lq, sc + lq, QPB, ci);
-        build_runs(B.G, B.off, ci, sy + lq, QPB, s_star, q);
-    }
-    __syncthreads();
+    if (active) stage_query_b(B, edge, i, sub, s_star, sy + lq, sc + lq, QPB, q);
     long long seen = 0;
     int found = 0;
     if (active) {
@@ -656,11 +663,6 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
 // dependent loads per query), a quarter the candidates, a third VALU work on
 // the neighbours; hence slots for masks of few children instead of idle lanes
 // (49 -> 43 ms; by child, k_b_count took 63 ms).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <bool PHI, int K, int CW, int NC>
 __global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ groups, const FanJob *__restrict__ jobs,
                                                   const int *__restrict__ blk_off, int njob, FanTable T, int d,
@@ -1308,16 +1310,11 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
     // r0 stands for the point in every union: its parent is read while the
     // query is staged
     int rp = active ? uf_find(pr, r0) : -1;
-    if (sub == 0 && active) {
-        int ci[3];
-        stage_query_b(B, edge, i, sy + lq, sc + lq, QPB, ci);
-        build_runs(B.G, B.off, ci, sy + lq, QPB, s_star, q);
-    }
-    __syncthreads();
+    if (active) stage_query_b(B, edge, i, sub, s_star, sy + lq, sc + lq, QPB, q);
     if (!active) return;
     const float *qy = sy + lq;
     const float2 *qcl = sc + lq;
-    const int total = q[9 + q[19]];
+    const int total = q[18];
     if constexpr (K > 0) {
         // each lane four consecutive candidates of one run per group (the
         // groups of walk_vec)
@@ -1325,9 +1322,8 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
         typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
         constexpr int U = 4, W = kLinkGroups;
         const uint32_t checked = (uint32_t) B.G.checkmask;
-        const int nr = q[19];
-        const int gtotal = q[21 + nr];
-        int r = 0, rgend = q[22];
+        const int gtotal = q[29];
+        int r = 0, rgend = q[21];
         for (int g0 = 0; g0 < gtotal; g0 += W * LPQ) {
             int at[W], nv[W];
             i4u rt[W];
@@ -1337,9 +1333,9 @@ __global__ __launch_bounds__(kBlock) void k_b_link_full(const BatchSub *__restri
                 const int g = min(gw, gtotal - 1);
                 while (g >= rgend) {
                     ++r;
-                    rgend = q[22 + r];
+                    rgend = q[21 + r];
                 }
-                const int e0 = (g - q[21 + r]) << 2;
+                const int e0 = (g - q[20 + r]) << 2;
                 nv[w] = gw < gtotal ? min(U, q[10 + r] - q[9 + r] - e0) : 0;
                 at[w] = q[r] + e0;
                 rt[w] = *reinterpret_cast<const i4u *>(rts + (uint32_t) at[w]);
