@@ -942,18 +942,18 @@ __global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ g
 // ------------------------------------------------------------ dense components of a batch
 // (k_dense_init .. k_uf_flatten per subspace; grid.y = subspace)
 
-// The whole sample phase of one subspace (its dense flags, the unions of the
-// sample edges, compressed parents, the giant component) in one block, with the
-// union-find in LDS: a device-scope swap goes past the XCD's L2 and their rate
-// bounded the same unions on global parents (n=100,000 d=20, 27 batches: 41.5 ms
-// there, 29.5 ms here, bound by the chains of dependent reads of one block; four
-// points a thread in flight, one took 32.0 ms).
-// Above kUfCap points every point first takes the smallest of itself and its
-// dense sample neighbours as parent (each thread writes its own entry, a forest
-// without a swap, about a third of the points are left as roots), and the roots
-// are numbered in id order for the LDS (smaller number = smaller id, so roots
-// stay the smallest ids); a subspace with more roots than fit clears fit[s] and
-// is left to the global passes.
+// The sample phase of one subspace (the unions of the sample edges, compressed
+// parents, the giant component) in one block, with the union-find in LDS: a
+// device-scope swap goes past the XCD's L2 and their rate bounded the same
+// unions on global parents (n=100,000 d=20, 29 batches: 41.5 ms there).  One
+// block's loads in flight bound it, so every pass takes kUfItems points a thread
+// (one 32.0 ms, four 28.4), and what needs no LDS runs on the whole chip: above
+// kUfCap points every point first takes the smallest of itself and its dense
+// sample neighbours as parent (k_b_dense_init; each thread writes its own entry,
+// a forest without a swap, about a third of the points are left as roots), and
+// the block numbers the roots in id order for the LDS (smaller number = smaller
+// id, so roots stay the smallest ids): 13.3 ms and 10.6 around it.  A subspace
+// with more roots than fit clears fit[s] and is left to the global passes.
 constexpr int kUfCap = 39936;
 constexpr int kUfThreads = 1024, kUfWaves = kUfThreads / 64, kUfItems = 4;
 __device__ __forceinline__ int lds_find(volatile int *up, int x) {
@@ -1009,57 +1009,21 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
     constexpr int M = kUfItems, STEP = kUfThreads * M;
     const int2 *nb2 = reinterpret_cast<const int2 *>(nb) + B.nbase;
     static_assert(kSampleEdges == 2, "a point's sample edges are one int2");
-    for (int i0 = t; i0 < n; i0 += STEP) {
-        int c[M];
-        int2 q[M];
-        int cq[M][2];
-#pragma unroll
-        for (int u = 0; u < M; ++u) {
-            const int i = min(i0 + u * kUfThreads, n - 1);
-            c[u] = B.cnt[i];
-            q[u] = numbered ? nb2[i] : make_int2(-1, -1);
-        }
-#pragma unroll
-        for (int u = 0; u < M; ++u) {
-            cq[u][0] = q[u].x >= 0 && q[u].x < n ? B.cnt[q[u].x] : 0;
-            cq[u][1] = q[u].y >= 0 && q[u].y < n ? B.cnt[q[u].y] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < M; ++u) {
-            const int i = i0 + u * kUfThreads;
-            if (i >= n) continue;
-            int root = -1;
-            if (meets(c[u], B.thr_dense, B.dbit)) {
-                root = i;
-                if (q[u].x >= 0 && q[u].x < root && meets(cq[u][0], B.thr_dense, B.dbit)) root = q[u].x;
-                if (q[u].y >= 0 && q[u].y < root && meets(cq[u][1], B.thr_dense, B.dbit)) root = q[u].y;
-                if (!numbered) up[i] = i;
-            }
-            pr[i] = root;
-        }
-    }
-    if (numbered) {
-        __syncthreads();
+    if (!numbered) {
         for (int i0 = t; i0 < n; i0 += STEP) {
-            int r[M], p[M];
+            int c[M];
 #pragma unroll
-            for (int u = 0; u < M; ++u) r[u] = i0 + u * kUfThreads < n ? pr[i0 + u * kUfThreads] : -1;
-            bool moved = true;
-            while (moved) {
-                moved = false;
+            for (int u = 0; u < M; ++u) c[u] = B.cnt[min(i0 + u * kUfThreads, n - 1)];
 #pragma unroll
-                for (int u = 0; u < M; ++u) p[u] = r[u] >= 0 ? pr[r[u]] : -1;
-#pragma unroll
-                for (int u = 0; u < M; ++u) {
-                    moved |= p[u] != r[u];
-                    r[u] = p[u];
-                }
+            for (int u = 0; u < M; ++u) {
+                const int i = i0 + u * kUfThreads;
+                if (i >= n) continue;
+                const bool dense = meets(c[u], B.thr_dense, B.dbit);
+                pr[i] = dense ? i : -1;
+                up[i] = i;
             }
-#pragma unroll
-            for (int u = 0; u < M; ++u)
-                if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
         }
-        __syncthreads();
+    } else {
         // roots of the wave's share (a multiple of 64), then their numbers:
         // csize[root] = number, comp[number] = root
         const int share = ((n + kUfWaves - 1) / kUfWaves + 63) & ~63;
@@ -1144,7 +1108,7 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
             if (r[u] >= 0) pr[i0 + u * kUfThreads] = r[u];
     }
     __syncthreads();  // the ids by number are read, the parents written
-    for (int i0 = t; i0 < n; i0 += STEP) {
+    for (int i0 = t; !numbered && i0 < n; i0 += STEP) {
         int o[M];
 #pragma unroll
         for (int u = 0; u < M; ++u) o[u] = B.order[min(i0 + u * kUfThreads, n - 1)];
@@ -1187,17 +1151,16 @@ __global__ __launch_bounds__(kUfThreads) void k_b_sample(const BatchSub *__restr
     }
 }
 
-// The same on global parents, for the subspaces that do not fit (fit null: all).
+// First parents (hooked) of tables above kUfCap points.
 __global__ void k_b_dense_init(const BatchSub *__restrict__ subs, int n, const int *__restrict__ nb,
-                               const int *__restrict__ fit, int *__restrict__ par) {
-    if (fit && fit[blockIdx.y]) return;
+                               int *__restrict__ par) {
     const BatchSub &B = subs[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    par[B.base + i] = hooked(B, nb, i);
-    B.csize[i] = 0;
+    if (i < n) par[B.base + i] = hooked(B, nb, i);
 }
 
+// The sample edges on global parents, for the subspaces whose first parents do
+// not fit (fit null: all).
 // Sample phase of the components: every dense point links to the dense ones
 // among the first kSampleEdges neighbours its count pass recorded (any edges would do:
 // the full phase below links every point outside the giant component to all
@@ -1234,16 +1197,22 @@ __global__ void k_b_uf_compress(const BatchSub *__restrict__ subs, int n, const 
     if (fit && fit[blockIdx.y]) return;
     int *pr = par + subs[blockIdx.y].base;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && pr[i] >= 0) pr[i] = uf_find(pr, i);
+    if (i >= n || pr[i] < 0) return;
+    // only the own entry is written, and once (uf_find shortens the entries it
+    // passes: a late one of its writes could undo a root written here)
+    int r = i;
+    for (int p = ld_relaxed(&pr[r]); p != r; p = ld_relaxed(&pr[r])) r = p;
+    st_relaxed(&pr[i], r);
 }
 
-// the parents in sorted order, for the full phase
-__global__ void k_b_rootpos(const BatchSub *__restrict__ subs, int n, const int *__restrict__ fit,
-                            const int *__restrict__ par, int *__restrict__ rootpos) {
-    if (fit && fit[blockIdx.y]) return;
+// the parents in sorted order, for the full phase; zeroed sizes
+__global__ void k_b_rootpos(const BatchSub *__restrict__ subs, int n, const int *__restrict__ par,
+                            int *__restrict__ rootpos) {
     const BatchSub &B = subs[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) rootpos[B.base + i] = par[B.base + B.order[i]];
+    if (i >= n) return;
+    rootpos[B.base + i] = par[B.base + B.order[i]];
+    B.csize[i] = 0;
 }
 
 // one block of 256 per subspace: the most frequent root among 256 evenly
@@ -2332,20 +2301,22 @@ hipError_t launch_b_components(const BatchSub *subs, int nsub, int n, int kmax, 
     if (nsub <= 0) return hipSuccess;
     // In LDS (one block per subspace) while one block's pass over a subspace is
     // shorter than the swaps of all blocks on global parents.  Whole runs, d=8,
-    // about 100 subspaces, LDS against global: n=10,000 2.4 / 2.6 ms, 39,936
-    // 6.0 / 7.4, 60,000 9.5 / 11.3, 100,000 21.8 / 24.7, 150,000 39.1 / 41.4,
-    // 200,000 67.1 / 62.3
+    // about 100 subspaces, LDS against global: n=39,936 5.9 / 6.7 ms, 60,000
+    // 8.6 / 10.4, 100,000 18.9 / 22.6, 150,000 33.2 / 38.7, 200,000 57.7 / 57.3,
+    // 300,000 108.8 / 103.2
     const bool lds_pass = n <= 4 * kUfCap;
     const int *fit = lds_pass ? X.fit : nullptr;
+    const dim3 all(blocks_for(n), nsub);
+    if (n > kUfCap) {
+        LAUNCH(k_b_dense_init, all, dim3(kBlock), 0, st, subs, n, X.nb, X.par);
+        LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, (const int *) nullptr, X.par);
+    }
     if (lds_pass)
         LAUNCH(k_b_sample, dim3(nsub), dim3(kUfThreads), 0, st, subs, n, X.nb, X.rootpos, X.par, X.giant, X.fit);
     if (n > kUfCap) {
-        const dim3 all(blocks_for(n), nsub);
-        LAUNCH(k_b_dense_init, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.par);
-        LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
         LAUNCH(k_b_link_sample, all, dim3(kBlock), 0, st, subs, n, X.nb, fit, X.par);
         LAUNCH(k_b_uf_compress, all, dim3(kBlock), 0, st, subs, n, fit, X.par);
-        LAUNCH(k_b_rootpos, all, dim3(kBlock), 0, st, subs, n, fit, X.par, X.rootpos);
+        LAUNCH(k_b_rootpos, all, dim3(kBlock), 0, st, subs, n, X.par, X.rootpos);
         LAUNCH(k_b_giant, dim3(nsub), dim3(256), 0, st, subs, n, fit, X.par, X.giant);
     }
     const dim3 grid(query_blocks_n(n), nsub);
