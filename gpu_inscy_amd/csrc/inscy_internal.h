@@ -126,6 +126,7 @@ struct Entry {
     int *mem;          // [n] points of the kept components, nmem of them
     int nkept;
     int nmem;
+    int maxk;          // points of the largest kept component
 };
 
 // Optional event pair bracketing the neighbour-count kernel of a launch.

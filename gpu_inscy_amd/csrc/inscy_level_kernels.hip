@@ -1708,13 +1708,13 @@ struct RowPlan {
 // loads rows [seg, seg + ns) of the list and their chunk prefix (of the items
 // past the first `head`); returns the number of chunks.  by_mem: walk the row's
 // members (else the tree's points, when nW is shorter; nW < 0 walks members
-// always)
+// always).  A row without a kept cluster of at least `floor` points is not walked.
 __device__ int plan_rows(const Entry *__restrict__ E, const int *__restrict__ list, int seg, int ns, int nW, int head,
-                         RowPlan &R, int *wtmp) {
+                         double floor, RowPlan &R, int *wtmp) {
     for (int i = threadIdx.x; i < ns; i += blockDim.x) {
         const Entry e = E[list[seg + i]];
         const bool bm = nW < 0 || e.nmem <= nW;
-        R.len[i] = e.nkept > 0 ? (bm ? e.nmem : nW) : 0;
+        R.len[i] = e.nkept > 0 && !(floor > (double) e.maxk) ? (bm ? e.nmem : nW) : 0;
         R.by_mem[i] = bm ? 1 : 0;
     }
     __syncthreads();
@@ -1771,10 +1771,13 @@ __device__ __forceinline__ int flag_drop(int J) { return -(3 + 3 * J); }
 __device__ __forceinline__ int flag_fresh(int J) { return -(4 + 3 * J); }
 
 // pruneRedundancy of every step with a tree (the step's own block range stands
-// for the grid).  A row is decided by one touched cluster smaller than |T| r, and
-// most rows that the tree touches show one among their first items: every row
-// is probed first, a wave per row, and only the rows left over are walked on
-// in chunks (n=100,000 d=20: 25.4 -> 20.7 ms a run; n=10,000 d=15: 1.15 -> 1.09).
+// for the grid).  A row drops the tree when the tree touches it and no cluster
+// touched is smaller than |T| r: a row whose largest kept cluster is smaller
+// cannot and is left out (n=100,000 d=20: 20.7 -> 8.5 ms a run; n=25,000 d=15:
+// 1.10 -> 0.58).  Of the others most that the tree touches show a
+// smaller cluster among their first items: every row is probed first, a wave per
+// row, and only the rows left over are walked on in chunks (n=100,000 d=20:
+// 25.4 -> 20.7 ms, before rows were left out).
 constexpr int kProbe = 256;
 __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__restrict__ blk_off, int nops,
                                 const Entry *__restrict__ E, float r, int *__restrict__ keepv) {
@@ -1807,7 +1810,7 @@ __global__ void k_rep_red_multi(const RepOp *__restrict__ ops, const int *__rest
     };
     for (int seg = 0; seg < nlist; seg += kSegRows) {
         const int ns = min(kSegRows, nlist - seg);
-        const int total = plan_rows(E, list, seg, ns, nW, kProbe, R, wtmp);
+        const int total = plan_rows(E, list, seg, ns, nW, kProbe, lhs, R, wtmp);
         constexpr int W = kBlock / 64;
         for (int i = bi * W + (int) (threadIdx.x / 64); i < ns; i += nb * W) {
             const int len = min(R.len[i], kProbe);
@@ -1905,7 +1908,7 @@ __global__ void k_rep_check_multi(const RepOp *__restrict__ ops, const int *__re
     const int cj = flag_cand(Op.J), dj = flag_drop(Op.J);
     for (int seg = 0; seg < Op.nlist; seg += kSegRows) {
         const int ns = min(kSegRows, Op.nlist - seg);
-        const int total = plan_rows(E, Op.list, seg, ns, -1, 0, R, wtmp);
+        const int total = plan_rows(E, Op.list, seg, ns, -1, 0, 0.0, R, wtmp);
         for (int w = bi; w < total; w += nb) {
             const int i = row_of(R, ns, w);
             const Entry e = E[Op.list[seg + i]];
@@ -1924,27 +1927,40 @@ __global__ void k_rep_check_multi(const RepOp *__restrict__ ops, const int *__re
 // the surviving candidates of every join step join the result of its
 // subspace (one block per step)
 __global__ void k_rep_apply_multi(const RepOp *__restrict__ ops, Entry *__restrict__ E) {
-    __shared__ int wtmp[kBlock / 64];
+    __shared__ int wtmp[kBlock / 64], wmax[kBlock / 64];
     const RepOp &Op = ops[blockIdx.x];
     if (Op.kind == 1) return;
     const int nc = min(Op.words[0], Op.ccap);
     const int cj = flag_cand(Op.J), fj = flag_fresh(Op.J);
-    int added = 0;
+    int added = 0, most = 0;
     for (int k = threadIdx.x; k < nc; k += blockDim.x) {
         const int K = Op.clist[k];
         if (Op.flag[K] == cj && !Op.inres[K]) {
             Op.inres[K] = 1;
             Op.flag[K] = fj;
             ++added;
+            most = max(most, Op.csize[K]);
         }
     }
-    for (int o = 32; o > 0; o >>= 1) added += __shfl_down(added, o);
-    if (__lane_id() == 0) wtmp[threadIdx.x / 64] = added;
+    for (int o = 32; o > 0; o >>= 1) {
+        added += __shfl_down(added, o);
+        most = max(most, __shfl_down(most, o));
+    }
+    if (__lane_id() == 0) {
+        wtmp[threadIdx.x / 64] = added;
+        wmax[threadIdx.x / 64] = most;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         int tot = 0;
-        for (int w = 0; w < kBlock / 64; ++w) tot += wtmp[w];
-        if (tot) E[Op.entry].nkept += tot;
+        for (int w = 0; w < kBlock / 64; ++w) {
+            tot += wtmp[w];
+            most = max(most, wmax[w]);
+        }
+        if (tot) {
+            E[Op.entry].nkept += tot;
+            E[Op.entry].maxk = max(E[Op.entry].maxk, most);
+        }
         Op.words[1] = tot;
     }
 }
