@@ -89,12 +89,22 @@ __global__ void k_hist1(const uint16_t *__restrict__ cellE, int n, int d, int ec
     atomicAdd(&hist[(size_t) k * ecells + cellE[i]], 1);
 }
 
-__global__ void k_histc(const uint8_t *__restrict__ cellC, int n, int d, int cells, int *__restrict__ hist) {
-    size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t) n * d) return;
-    int k = (int) (i / n);
-    atomicAdd(&hist[(size_t) k * cells + cellC[i]], 1);
+// grid.y = dimension.  A few cells take all counts, so every block counts in LDS
+// (n=3,001 d=9, 6 cells: 63 us with an atomic per value, 4.9 so).
+constexpr int kHistItems = 8;
+__global__ void k_histc(const uint8_t *__restrict__ cellC, int n, int cells, int *__restrict__ hist) {
+    __shared__ int h[256];
+    const int k = blockIdx.y;
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    for (int u = 0; u < kHistItems; ++u) {
+        const int i = (blockIdx.x * kHistItems + u) * kBlock + threadIdx.x;
+        if (i < n) atomicAdd(&h[cellC[(size_t) k * n + i]], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < cells && h[threadIdx.x]) atomicAdd(&hist[(size_t) k * cells + threadIdx.x], h[threadIdx.x]);
 }
+static_assert(kBlock == 256, "one thread per possible cell");
 
 // ------------------------------------------------------------ epsilon neighbourhood: subspace grid pass
 // Candidate rule of get_possible_neighbors_from (ScyTreeNode.cu:896-946) on
@@ -406,9 +416,9 @@ hipError_t launch_hist1(const uint16_t *cellE, int n, int d, int ecells, int *hi
 }
 
 hipError_t launch_histc(const uint8_t *cellC, int n, int d, int cells, int *hist, hipStream_t st) {
-    size_t nd = (size_t) n * d;
     LAUNCH(k_fill<int>, dim3(fill_blocks((size_t) d * cells, sizeof(int))), dim3(kBlock), 0, st, hist, 0, (size_t) d * cells);
-    LAUNCH(k_histc, dim3(blocks_for(nd)), dim3(kBlock), 0, st, cellC, n, d, cells, hist);
+    LAUNCH(k_histc, dim3((n + kBlock * kHistItems - 1) / (kBlock * kHistItems), d), dim3(kBlock), 0, st, cellC, n,
+           cells, hist);
     return hipGetLastError();
 }
 
