@@ -9,18 +9,17 @@ workload is n=100,000 d=20 (20 Zipf-sized clusters, eps=0.02, c=8, mu=4,
 min_size=1000, rectangular).  The reported value is restricted (subspace,
 region) trees evaluated per second, the throughput unit of the reference's
 depth-first search; ms_per_step is the end-to-end time of one run (labels of
-every result subspace back in host memory).  The default path is the
-level-synchronous driver (`batched`, exact results); the depth-first driver
-(`exact`, one restricted tree at a time) is timed beside it outside the timed
-region and reported as depth_first_ms.
+every result subspace back in host memory).  Every exact mode runs the
+level-synchronous driver (trees in the reference's depth-first order for the
+decisions); the mode that is not timed (`exact` beside the default `batched`) is
+run outside the timed region as depth_first_ms, a check that both agree.
 
 Also reported:
   parity        the last timed run equals the committed golden digests of the
                 oracle (tests/golden/config<N>.json), when present.
-  roofline      the neighbour-count kernel (the dominant one; k_b_count in the
-                level-synchronous driver, k_grid_count in the depth-first one):
-                its algorithmic bytes (per counted point 4k+4, per neighbour
-                established 4+4k) over its device time measured with HIP events
+  roofline      the neighbour-count kernels (k_b_count, and k_b_fan where one
+                walk counts all children of a mask): their algorithmic bytes (per counted point 4k+4, per neighbour
+                established 4+4k) over their device time measured with HIP events
                 on the engine's stream in a separate pass of up to 3 runs after
                 the timed steps (ms_per_step_with_events shows their overhead),
                 against 8 TB/s HBM; `traffic` comes from the committed rocprofv3
@@ -59,7 +58,7 @@ def parse():
     ap.add_argument("--mode", choices=["exact", "batched", "learned"], default="batched",
                     help="learned: the learned pruner (gpu_inscy_amd/pruner_weights.npz) against the exact run")
     ap.add_argument("--depth-first-steps", type=int, default=1,
-                    help="untimed runs of the depth-first driver for the comparison (0: skip)")
+                    help="untimed runs of the other exact mode for the comparison (0: skip)")
     ap.add_argument("--config", type=int, default=2,
                     help="workload index (2: n=100000 d=20, the default; 1: n=25000 d=15; 4: n=200000 d=32; "
                          "3: 64 data sets)")
@@ -209,7 +208,7 @@ def main():
     ebytes = sum(st["count_examined_bytes"] for st in pstats)
     avg_launch_ms = kernel_ms / max(launches, 1)
     achieved = (kbytes / max(launches, 1)) / (avg_launch_ms * 1e-3) / 1e9 if avg_launch_ms > 0 else 0.0
-    kernel = "k_b_count" if args.mode == "batched" else "k_grid_count"
+    kernel = "k_b_count"
     roofline = {
         "bound": "hbm",
         "kernel": kernel,
@@ -221,15 +220,15 @@ def main():
         "algorithmic_bytes_per_launch": round(kbytes / max(launches, 1), 1),
         "avg_launch_us": round(avg_launch_ms * 1e3, 3),
         "launches_per_step": launches // nprof,
-        # the candidates' packed cells and coordinates the walks read (mostly
-        # L2 hits): what the kernel moves through the caches, beside the
+        # the candidates' coordinates the walks read (mostly L2 hits): what the
+        # kernel moves through the caches, beside the
         # algorithmic bytes of the neighbours it establishes
         "examined_bytes_per_launch": round(ebytes / max(launches, 1), 1),
         "examined_GBs": round((ebytes / max(launches, 1)) / (avg_launch_ms * 1e-3) / 1e9, 2) if avg_launch_ms > 0 else 0.0,
         "kernel_share_of_step": round(kernel_ms / nprof / ms_step, 4),
     }
 
-    # the depth-first driver (one restricted tree at a time) on the same data
+    # the other exact mode on the same data
     other = same = None
     if args.depth_first_steps > 0:
         omode = _lib.MODE_EXACT if mode == _lib.MODE_BATCHED else _lib.MODE_BATCHED
@@ -242,7 +241,7 @@ def main():
         other = (time.perf_counter() - t1) / args.depth_first_steps * 1e3
         same = ores.subspaces == res.subspaces and np.array_equal(ores.labels, res.labels)
         del ores
-        say(f"other driver: {other:.1f} ms/run, same result: {same}")
+        say(f"other mode: {other:.1f} ms/run, same result: {same}")
 
     # the drop-in call (python/inscy.py GPU5: host tensor in, Python lists out)
     dropin = None

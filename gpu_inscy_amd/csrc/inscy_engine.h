@@ -123,8 +123,8 @@ inline int count_threshold(float t) {
 }
 
 // ------------------------------------------------------------ memory
-// Stack-disciplined bump allocator for the per-tree lists of the depth-first
-// recursion (a child's lists are released when its subtree is done).
+// Stack-disciplined bump allocator for the scratch of the set-up and of the
+// single-subspace passes (released to a mark when a pass is done).
 struct Arena {
     char *base = nullptr;
     size_t cap = 0, top = 0;

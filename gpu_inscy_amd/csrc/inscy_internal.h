@@ -220,7 +220,7 @@ struct QuerySeg {
     int len, b;
 };
 
-// Partition of one tree by the cell groups of dimension m (k_part_* per pair).
+// Partition of one tree by the cell groups of dimension m.
 struct PartPair {
     const int *P;
     const int *spx;

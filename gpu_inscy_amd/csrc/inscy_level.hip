@@ -1,4 +1,5 @@
-// Level-synchronous driver of the MI355X INSCY engine (INSCY_MODE_BATCHED).
+// Level-synchronous driver of the MI355X INSCY engine (every mode; the trees'
+// paths or, in a permuted level order, chains: inscy_perm.hip).
 //
 // In the reference's depth-first recursion (INSCYCPU3Weak,
 // src/algorithms/inscy/InscyNodeCpu.cu:159-235) only pruneRedundancy and join
@@ -14,7 +15,7 @@
 //     subspaces their dense components, a handful of launches for all of them.
 // pruneRedundancy and join are then replayed on the device in stages that keep
 // the reference's depth-first order wherever it matters (steps on subspaces
-// one of which contains the other), which gives the depth-first driver's
+// one of which contains the other), which gives the depth-first recursion's
 // result exactly.
 
 #include "inscy_engine.h"

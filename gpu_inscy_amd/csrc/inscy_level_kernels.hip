@@ -1,7 +1,6 @@
 // Level-synchronous passes of the MI355X INSCY engine (gfx950, wave64).
 //
-// The same per-tree and per-subspace work as the depth-first kernels in
-// inscy_kernels.hip, but every launch covers a whole batch: all trees of one
+// Every launch covers a whole batch: all trees of one
 // recursion level (merge flags, partition, path prune) or many subspaces (grid
 // index, neighbour counts, dense components).  A block belongs to exactly one
 // segment, found by a binary search of its block offsets, so a wave never
@@ -31,7 +30,7 @@ static_assert(QPB == kQueriesPerBlock, "queries per block of the host and the ke
 __device__ __forceinline__ int origin(int x) { return x >= 0 ? x : ~x; }
 
 // ------------------------------------------------------------ merge flags of every tree of a level
-// (k_flags_all per tree: ScyTreeNode.cu:837-851 with restrict_node :262-267)
+// (ScyTreeNode.cu:837-851 with restrict_node :262-267)
 __global__ void k_b_flags(const FlagTree *__restrict__ T, const int *__restrict__ blk_off, int nt,
                           const uint8_t *__restrict__ cellC, int n, int cells, int *__restrict__ flags) {
     const int t = seg_of(blk_off, nt, blockIdx.x);
@@ -519,9 +518,9 @@ __device__ __forceinline__ void walk_generic(const QueryWalk &W, int &found, dou
 }
 
 // ------------------------------------------------------------ neighbour counts
-// k_grid_count over a batch: LIST = the compacted queries of each subspace
-// (blocks by segment), else every sorted position of subspace blockIdx.y whose
-// count is still missing (components pass, with the subset bound).
+// LIST = the compacted queries of each subspace (blocks by segment), else every
+// sorted position of subspace blockIdx.y whose count is still missing
+// (components pass, with the subset bound).
 template <bool LIST, bool PHI, int K>
 __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__ subs, const int *__restrict__ blk_off,
                                                     int nsub, int n, const float *__restrict__ edge,
@@ -940,7 +939,7 @@ __global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ g
 }
 
 // ------------------------------------------------------------ dense components of a batch
-// (k_dense_init .. k_uf_flatten per subspace; grid.y = subspace)
+// (grid.y = subspace)
 
 // The sample phase of one subspace (the unions of the sample edges, compressed
 // parents, the giant component) in one block, with the union-find in LDS: a
@@ -1370,7 +1369,7 @@ __global__ void k_b_uf_flatten(const BatchSub *__restrict__ subs, int n, int *__
 }
 
 // ------------------------------------------------------------ partition of every (tree, dimension) pair
-// k_part_count / k_part_scatter per pair.  Only the weak-dense points and the
+// Only the weak-dense points and the
 // paths are written; a path's origin keeps its "point of this tree" bit when
 // the origin survives the weak-density prune of the group.
 __global__ void k_b_part_count(const PartPair *__restrict__ pairs, const int *__restrict__ blk_off, int np,

@@ -1,5 +1,5 @@
-// Allocation-free neighbour counts: the grid-index pass of the depth-first
-// driver (k_grid_keys, scan, k_grid_scatter, k_grid_count) over buffers carved
+// Allocation-free neighbour counts: the grid-index pass of one subspace
+// (k_grid_keys, scan, k_grid_scatter, k_grid_count) over buffers carved
 // from one file-scope device array, for callers that cannot allocate device
 // memory (code under graph capture, serving loops).
 //

@@ -4,7 +4,7 @@
                                         [--out experiments_data]
 
 Same command line, parameter grids and per-run records as
-experiments/run.py:1-175: METHOD is INSCY (exact, depth-first driver),
+experiments/run.py:1-175: METHOD is INSCY (exact mode),
 GPU-INSCY (level-batched), GPU-INSCY* or GPU-INSCY-memory (level-batched, the
 reference's variants of its GPU driver), or GPU-INSCY-learned (the learned
 pruner, gpu_inscy_amd/pruner_weights.npz).  EXPERIMENT (and EXPERIMENT_2ND)

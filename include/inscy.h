@@ -53,7 +53,7 @@ typedef struct inscy_params {
     float r;                 /* redundancy factor */
     int32_t number_of_cells; /* c: grid cells per dimension */
     int32_t rectangular;     /* 1: neighbour-count density, 0: Epanechnikov density */
-    int32_t entropy_order;   /* 0: identity level order (the only order this build runs) */
+    int32_t entropy_order;   /* SCY-tree levels: 0 identity, 1 / -1 by ascending / descending entropy */
 } inscy_params;
 
 /* Counters of one run (the reference prints `calls` only, InscyNodeCpu.cu:166). */
