@@ -123,7 +123,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             // one driver serves every mode and level order: the level-synchronous
             // one gives the depth-first recursion's result, trees and decisions
             // in a fraction of its launches (n=4,999 d=11: 12,556 dispatches and
-            // 58 ms one tree at a time, 240 and 3.9 ms)
+            // 58 ms one tree at a time, 186 and 2.9 ms)
             eng.collect = mode == INSCY_MODE_COLLECT;
             if (mode == INSCY_MODE_LEARNED) {
                 eng.pruner = pruner_on_device(eng.prune_thr, eng.prune_min_depth);

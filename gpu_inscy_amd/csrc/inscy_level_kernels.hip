@@ -662,8 +662,12 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
 // dependent loads per query), a quarter the candidates, a third VALU work on
 // the neighbours; hence slots for masks of few children instead of idle lanes
 // (49 -> 43 ms; by child, k_b_count took 63 ms).
+// Six waves a SIMD where that costs few or no spills (count mode, K <= 6, up to two
+// children a lane: 91 -> 79 VGPRs at K = 2, eight children): n=100,000 d=20
+// eps=0.02 583 -> 576 ms a run, n=25,000 d=15 9.96 -> 9.80 of kernels; seven
+// waves 591, eight 623, and four children a lane spill 21 registers or more at six.
 template <bool PHI, int K, int CW, int NC>
-__global__ __launch_bounds__(kBlock) void k_b_fan(const BatchSub *__restrict__ groups, const FanJob *__restrict__ jobs,
+__global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fan(const BatchSub *__restrict__ groups, const FanJob *__restrict__ jobs,
                                                   const int *__restrict__ blk_off, int njob, FanTable T, int d,
                                                   const float *__restrict__ X, const float *__restrict__ edge,
                                                   const int *__restrict__ qlist, const int *__restrict__ qstart,
