@@ -467,8 +467,8 @@ int inscy_debug_phi_exact(int on) {
 }
 
 // Test hook (not in the public header): run every neighbour walk of the
-// level-synchronous driver for k known only at run time, as for a batch that
-// mixes dimensionalities (no launch compiled for its k).
+// level-synchronous driver for k known only at run time, one walk per child
+// subspace (no launch compiled for its k, no k_b_fan).
 int inscy_debug_generic_walk(int on) {
     g_generic_walk = on != 0;
     return INSCY_OK;

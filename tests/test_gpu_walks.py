@@ -150,3 +150,45 @@ def test_permuted_order_in_batches_matches_oracle(max_batch, order):
         for a, b in zip(ref.labels, got.labels):
             assert np.array_equal(O.canonical(a), b)
         assert np.array_equal(trace, ref.trace)
+
+
+def clumps(n, d, eps, dims, seed):
+    """Uniform points with three groups that are dense in `dims` dimensions each."""
+    rng = np.random.default_rng(seed)
+    X = rng.random((n, d)).astype(np.float32)
+    for c in range(3):
+        rows = np.arange(c * n // 4, (c + 1) * n // 4)[:, None]
+        at = np.sort(rng.choice(d, dims, replace=False)) if c else np.r_[0:dims - 1, d - 1]
+        size = (c + 1) * n // 4 - c * n // 4
+        X[rows, at] = (rng.uniform(0.2, 0.8, dims) + 0.4 * eps * rng.standard_normal((size, dims))).astype(np.float32)
+    return np.clip(X, 0.0, 1.0)
+
+
+def traced(X, args):
+    _lib.debug_trace(True)
+    try:
+        got = INSCY.run(torch.from_numpy(X).cuda(), *args, mode=_lib.MODE_BATCHED)
+        return got, _lib.debug_trace_rows()
+    finally:
+        _lib.debug_trace(False)
+
+
+# one walk per mask (compiled for its k), one per child (any k): the hook must
+# reach the masks' walks too, and both give the same trees and labels
+@pytest.mark.parametrize("n,d,eps,dims", [(350, 9, 0.04, 5), (1203, 7, 0.01, 4)])
+@pytest.mark.parametrize("rect", [True, False])
+def test_walks_per_mask_and_per_child_agree(n, d, eps, dims, rect):
+    print("walk routes", n, d, eps, rect, flush=True)
+    X = clumps(n, d, eps, dims, n * d)
+    args = (eps, 1.0, 4, n // 6, 1.0, 4, rect, 0)
+    a, ta = traced(X, args)
+    _lib.debug_generic_walk(True)
+    try:
+        b, tb = traced(X, args)
+    finally:
+        _lib.debug_generic_walk(False)
+    # a walk per child leaves out the points that the counts of smaller
+    # subspaces decide, a walk per mask does not look them up
+    assert b.stats["queries"] < a.stats["queries"]
+    assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
+    assert np.array_equal(ta, tb)
