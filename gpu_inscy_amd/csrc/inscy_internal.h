@@ -404,9 +404,10 @@ hipError_t launch_b_sort(const DevData &D, const SortJob *jobs, int njob, int hm
                          int *rank, int *hist, int *off, void *scan_temp, size_t scan_bytes, hipStream_t st);
 hipError_t launch_b_gather(const ColJob *jobs, int njob, int n, hipStream_t st);
 // queries in sorted order: flag the points of the segments (X.qflag zeroed by the
-// caller), compact per subspace
+// caller), compact per subspace; seg (may be null) receives each query's segment
+// at its sorted position
 hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySeg *segs, const int *blk_off,
-                            int nseg, int nblk, const BatchIndex &X, hipStream_t st);
+                            int nseg, int nblk, const BatchIndex &X, int *seg, hipStream_t st);
 // neighbour counts of the listed queries (blk_off over subspaces), or of every
 // uncounted point when blk_off is null (grid.y = subspace)
 // phi: rectangular = false, the stored values are decision bits (1 weak-dense,
@@ -429,14 +430,20 @@ hipError_t launch_phi_exact(const DevData &D, const BatchSub *sub, const int2 *f
 // the caller clears *X.nfb before and recomputes the listed pairs after
 // (launch_phi_exact over the children)
 struct FanJob {
-    int g, ch0, nch, pad;  // group, its first child in the batch, number of children
+    int g, ch0, nch, part;  // group, its first child in the batch, number of children; which kFanMost of the group's
 };
 struct FanTable {  // per child of the batch: its counts, dimension m and first sample edge
     int *const *cnt;
     const int *dim;
     const long long *nbase;
+    // the learned mode's skips (null: none): per query segment two words, bit u of
+    // word w set when the pair of its tree and the group's child 64 w + u is live;
+    // the segment of the query at each sorted position (as qflag)
+    const unsigned long long *live;
+    const int *seg;
 };
-constexpr int kFanMost = 64;  // children of one walk
+constexpr int kFanPoints = (1 << 28) - 1;  // points of a table with fanned counts, at most
+constexpr int kFanMost = 64;  // children of one walk (one word of FanTable::live)
 hipError_t launch_b_fan(const BatchSub *groups, const FanJob *jobs, const int *blk_off, int njob, int nblk, int width,
                         int kS, const FanTable &T, const BatchIndex &X, float s_star, float eps, bool phi,
                         bool phi_all_exact, int cap, float phi_w, float phi_d, const DevData &D,

@@ -296,8 +296,9 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
             // 16, k coordinate columns: 4k, grid histogram and offsets), the
             // phi pass's queue (8)
             size_t est = (size_t) n * (41 + 4 * (size_t) S.k + (phi_mode ? 8 : 0)) + (size_t) ncell * 12;
-            // the index and the queries of a fanned mask
-            if (fan && (j == i || cs[j - 1].t0 != c.t0)) est += (size_t) n * (21 + 4 * (size_t) S.k) + (size_t) ncell * 12;
+            // the index and the queries (learned: and their trees) of a fanned mask
+            if (fan && (j == i || cs[j - 1].t0 != c.t0))
+                est += (size_t) n * (21 + (pruner ? 4 : 0) + 4 * (size_t) S.k) + (size_t) ncell * 12;
             for (int a = c.t0; a < c.t1; ++a) {
                 if (!pair_on(a, c.m)) continue;
                 const LTree &t = lt[lv_act[a]];
@@ -433,7 +434,7 @@ void Engine::index_of(std::vector<BatchSub> &hs, std::vector<const float *> &cta
 // far fewer: n=100,000 d=20, masks of two dimensions 16.8 ms by child, 39 ms by
 // mask; n=25,000 d=15, eps=0.015 (two index dimensions at most) 2.19 and 1.74.
 bool Engine::fan_level(const std::vector<ChildSub> &cs) const {
-    if (cs.empty() || (long long) n * d >= 1ll << 30) return false;  // 32-bit offsets into X
+    if (cs.empty() || n >= kFanPoints || (long long) n * d >= 1ll << 30) return false;  // 32-bit offsets into X
     if (permuted) return false;  // the children match different dimensions of one mask
     if (generic_walk) return false;  // the fan is compiled for its masks' k
     const SubspaceArg S = arg_of(cs[0].s & ~dbit(cs[0].m));
@@ -478,18 +479,16 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     std::vector<FanJob> jobs[5];    // by the width of their walk
     std::vector<QuerySeg> qs;
     std::vector<int> qblk{0};
+    std::vector<unsigned long long> live;  // fan: FanTable::live of the segments
+    bool skips = false;                    // fan: some segment has a pair that is not
     long long qoff = 0;
-    auto add_queries = [&](BatchSub &x, int w, int t0, int t1, int m) {  // m < 0: of any dimension
-        long long qmax = 0;
-        for (int a = t0; a < t1; ++a) {
-            const LTree &t = lt[lv_act[a]];
-            if (t.nW <= 0 || (m >= 0 && !pair_on(a, m))) continue;
-            qs.push_back({t.W, t.nW, w});
-            qblk.push_back(qblk.back() + nblocks(t.nW));
-            qmax += t.nW;
-        }
-        x.qmax = (int) qmax;
-        qoff += qmax;
+    auto add_segment = [&](int w, int a) {
+        const LTree &t = lt[lv_act[a]];
+        if (t.nW <= 0) return false;
+        qs.push_back({t.W, t.nW, w});
+        qblk.push_back(qblk.back() + nblocks(t.nW));
+        qoff += t.nW;
+        return true;
     };
     if (fan) {
         for (int b = 0; b < B;) {
@@ -501,18 +500,40 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             g.S = arg_of(c.s & ~dbit(c.m));
             g.G = grid_of(g.S, -1, true);
             g.base = (long long) gs.size() * n;
-            add_queries(g, (int) gs.size(), c.t0, c.t1, -1);
+            long long qmax = 0;
+            for (int a = c.t0; a < c.t1; ++a) {
+                // the tree's live pairs among the mask's children
+                unsigned long long on[2] = {0, 0};
+                bool all = true;
+                for (int x = b; x < e; ++x) {
+                    if (pair_on(a, cs[i0 + x].m))
+                        on[(x - b) / kFanMost] |= 1ull << ((x - b) % kFanMost);
+                    else
+                        all = false;
+                }
+                if (!(on[0] | on[1]) || !add_segment((int) gs.size(), a)) continue;
+                qmax += lt[lv_act[a]].nW;
+                live.insert(live.end(), on, on + 2);
+                skips |= !all;
+            }
+            g.qmax = (int) qmax;
             for (int at = b; at < e; at += kFanMost) {
                 const int nch = std::min(kFanMost, e - at);
                 int w = 0;
                 while (kWidths[w] < nch) ++w;
-                jobs[w].push_back({(int) gs.size(), at, nch, 0});
+                jobs[w].push_back({(int) gs.size(), at, nch, (at - b) / kFanMost});
             }
             gs.push_back(g);
             b = e;
         }
     } else {
-        for (int b = 0; b < B; ++b) add_queries(hs[b], b, cs[i0 + b].t0, cs[i0 + b].t1, cs[i0 + b].m);
+        for (int b = 0; b < B; ++b) {
+            const ChildSub &c = cs[i0 + b];
+            long long qmax = 0;
+            for (int a = c.t0; a < c.t1; ++a)
+                if (pair_on(a, c.m) && add_segment(b, a)) qmax += lt[lv_act[a]].nW;
+            hs[b].qmax = (int) qmax;
+        }
     }
     std::vector<BatchSub> &ws = fan ? gs : hs;
     const int nw = (int) ws.size();
@@ -616,7 +637,8 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             td[b] = cs[i0 + b].m;
             tbase[b] = hs[b].nbase;
         }
-        ft = FanTable{upload(batch, tc), upload(batch, td), upload(batch, tbase)};
+        ft = FanTable{upload(batch, tc), upload(batch, td), upload(batch, tbase), skips ? upload(batch, live) : nullptr,
+                      skips ? batch.take<int>((size_t) nw * n) : nullptr};
         for (int w = 0; w < 5; ++w) {
             if (jobs[w].empty()) continue;
             std::vector<int> blk{0};
@@ -631,7 +653,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         dcb = upload(batch, cblk);
     }
     flush_uploads();
-    HIP_OK(launch_b_queries(dws, nw, n, dqs, dqb, (int) qs.size(), qblk.back(), X, st));
+    HIP_OK(launch_b_queries(dws, nw, n, dqs, dqb, (int) qs.size(), qblk.back(), X, const_cast<int *>(ft.seg), st));
     const bool dbg = batch_trace;
     std::chrono::steady_clock::time_point tq0, tq1;
     if (dbg) {

@@ -125,14 +125,17 @@ __global__ void k_b_gather(const ColJob *__restrict__ jobs, int n, int nblk) {
 
 // ------------------------------------------------------------ query lists in sorted order
 __global__ void k_b_qmark(const BatchSub *__restrict__ subs, const QuerySeg *__restrict__ segs,
-                          const int *__restrict__ blk_off, int nseg, uint8_t *__restrict__ qflag) {
+                          const int *__restrict__ blk_off, int nseg, uint8_t *__restrict__ qflag,
+                          int *__restrict__ seg) {
     const int s = seg_of(blk_off, nseg, blockIdx.x);
     const QuerySeg Q = segs[s];
     const int i = (blockIdx.x - blk_off[s]) * blockDim.x + threadIdx.x;
     if (i >= Q.len) return;
     const BatchSub &B = subs[Q.b];
     const int p = Q.P[i];
-    qflag[B.base + B.pos[p]] = 1;
+    const long long at = B.base + B.pos[p];
+    qflag[at] = 1;
+    if (seg) seg[at] = s;
 }
 
 // ------------------------------------------------------------ candidate walk
@@ -655,6 +658,8 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
 // children and one of kFanLanes / CW slots, adds m's term of the slot's
 // neighbours: the lanes read consecutive coordinates of a neighbour's row of X.
 // The walk ends when every child is decided (cap, phi) or the runs are done.
+// A pair that the learned pruner skips is no child of its tree's points: they
+// are not counted in it, and points without a live child make no walk.
 // The children's bounds (k_b_count) are not looked up: one undecided child
 // makes the walk anyway, and the look-up costs a scattered read per child and
 // bound (n=100,000 d=20, masks of three dimensions: 54 ms with it, 49 without).
@@ -690,13 +695,24 @@ __global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fa
     const int slot = l / CW, cl = l % CW;
     const int gshift = __lane_id() & ~(L - 1);
     const int qi = qstart[J.g] + (blockIdx.x - blk_off[ji]) * Q + lq;
-    const bool active = qi < qstart[J.g + 1];
+    bool active = qi < qstart[J.g + 1];
     int seen = 0, nhits = 0;
+    // a lane without a live child in place c starts its count at kNone, more than
+    // any count and its sum over the slots in range (n <= kFanPoints; the host
+    // checks): the walk does not wait for it and records no edges
+    constexpr int kNone = kFanPoints;
+    static_assert((long long) kNone * (HS + 1) < INT_MAX, "the slots' counts are summed");
     int found[NC];
+    const int at = active ? qlist[qi] : 0;
+    {
+        unsigned long long live = J.nch < 64 ? (1ull << J.nch) - 1ull : ~0ull;
+        if (T.live && active) live &= T.live[2 * T.seg[at] + J.part];
+        active = active && live != 0;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) found[c] = 0;
+        for (int c = 0; c < NC; ++c) found[c] = (live >> (cl + CW * c)) & 1ull ? 0 : kNone;
+    }
     if (active) {
-        const int i = (int) (qlist[qi] - B.base);
+        const int i = (int) (at - B.base);
         const int p = B.order[i];
         // the query's coordinates and cell intervals in S: lane t holds dimension t
         const float inf = __builtin_inff();
@@ -848,8 +864,7 @@ __global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fa
                             const float acc = __uint_as_float(e[u].y) + sq;
                             if (acc <= s_star && z[u][c] >= lo[c] && z[u][c] < hi[c]) {
                                 // sample edges: the first of slots 0 and 1, or the first two of the only slot
-                                if (cl + CW * c < J.nch &&
-                                    (HS > 1 ? (slot < kSampleEdges && found[c] == 0) : found[c] < kSampleEdges))
+                                if (HS > 1 ? (slot < kSampleEdges && found[c] == 0) : found[c] < kSampleEdges)
                                     nb[kSampleEdges * (T.nbase[ch[c]] + p) + (HS > 1 ? slot : found[c])] =
                                         (int) (e[u].x / (uint32_t) d);
                                 ++found[c];
@@ -864,12 +879,12 @@ __global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fa
                     if (PHI) {
                         double ds = dsum[c];
                         for (int o = CW; o < L; o <<= 1) ds += __shfl_xor(ds, o);
-                        open |= (cl + CW * c < J.nch) &
+                        open |= (found[c] < kNone) &
                                 (ds * (1.0 - (double) total * phirel) < (double) fmaxf(phi_w, phi_d));
                     } else {
                         int f = found[c];
                         for (int o = CW; o < L; o <<= 1) f += __shfl_xor(f, o);
-                        open |= (cl + CW * c < J.nch) & (f < cap);
+                        open |= f < cap;
                     }
                 }
                 more = ((__ballot(open) >> gshift) & 0xFFFFull) != 0;
@@ -881,8 +896,8 @@ __global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fa
             for (int o = CW; o < L; o <<= 1) found[c] += __shfl_xor(found[c], o);
             if (PHI)
                 for (int o = CW; o < L; o <<= 1) dsum[c] += __shfl_xor(dsum[c], o);
-            if (slot != 0 || cl + CW * c >= J.nch) {
-                found[c] = -1;  // counted by another lane
+            if (slot != 0 || found[c] >= kNone) {
+                found[c] = -1;  // counted by another lane, or a skipped pair
                 continue;
             }
             if (PHI) {
@@ -2201,11 +2216,11 @@ hipError_t launch_flag_compact(const uint8_t *flags, size_t nb, void *temp, size
 }
 
 hipError_t launch_b_queries(const BatchSub *subs, int nsub, int n, const QuerySeg *segs, const int *blk_off,
-                            int nseg, int nblk, const BatchIndex &X, hipStream_t st) {
+                            int nseg, int nblk, const BatchIndex &X, int *seg, hipStream_t st) {
     if (nsub <= 0) return hipSuccess;
     const size_t nb = (size_t) nsub * n;
     if (nblk > 0)
-        LAUNCH(k_b_qmark, dim3(nblk), dim3(kBlock), 0, st, subs, segs, blk_off, nseg, X.qflag);
+        LAUNCH(k_b_qmark, dim3(nblk), dim3(kBlock), 0, st, subs, segs, blk_off, nseg, X.qflag, seg);
     return launch_flag_compact(X.qflag, nb, X.select_temp, X.select_bytes, X.qlist, X.nsel, n, X.qstart, st);
 }
 

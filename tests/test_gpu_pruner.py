@@ -242,3 +242,81 @@ def test_pruning_bound_from_the_exact_pair_labels():
     # the counts of pairs that reach the result are most of the work
     assert kept / total > 0.5
     assert bound < 3.0
+
+
+def _split_trees(n, d, c, seed):
+    """Points that leave the c-grid's cell edges free, so that every cell of a
+    dimension is a restricted tree of its own."""
+    rng = np.random.default_rng(seed)
+    cell = rng.integers(0, c, (n, d))
+    return ((cell + rng.uniform(0.06, 0.94, (n, d))) / c).astype(np.float32)
+
+
+@pytest.mark.parametrize("d", [4, 9, 20])
+def test_learned_mode_counts_live_pairs_only(d):
+    # one-dimensional trees only (min_size), whose children are counted by one
+    # walk per mask: a point is counted once per pair of its tree that the
+    # network keeps, and in no skipped one
+    n, c, eps, mu = 1100, 3, 0.01, 8
+    X = torch.from_numpy(_split_trees(n, d, c, d)).cuda()
+    args = (eps, 1.0, mu, 30, 1.0, c, True, 0)
+    _lib.debug_trace(True)
+    try:
+        ex = INSCY.run(X, *args, mode=_lib.MODE_BATCHED)
+        trace = _lib.debug_trace_rows()
+    finally:
+        _lib.debug_trace(False)
+    size = np.array([bin(int(m)).count("1") for m in trace[:, 0]])
+    assert (trace[size == 1, 5] == 1).sum() > d and not trace[size > 1, 5].any()
+    pairs = INSCY.run(X, *args, mode=_lib.MODE_COLLECT).pairs
+    one = pairs["info"][:, 0] == 1
+    own = pairs["cost"][:, 0].astype(np.int64)
+    assert ex.stats["queries"] == n * d + own[one].sum()
+    W = pruner.init_params(5)
+    prob = pruner.Trainer(W).forward(pairs["features"]).cpu().numpy()
+    for share in (0.02, 0.3, 0.7, 0.98):
+        s = np.sort(prob[one])
+        thr = float(s[max(1, int(share * len(s)))])
+        _lib.set_pruner(W, thr, 1)
+        le = INSCY.run(X, *args, mode=_lib.MODE_LEARNED)
+        say("live pairs", d, share, le.stats["pairs_skipped"], le.stats["queries"])
+        assert le.stats["pairs_skipped"] == (prob[one] < thr).sum() > 0
+        assert le.stats["queries"] == n * d + own[one & (prob >= np.float32(thr))].sum()
+    _lib.set_pruner(None, 0.0)
+
+
+@pytest.mark.parametrize("rect", [True, False])
+@pytest.mark.parametrize("d,eps", [(9, 0.03), (24, 0.02), (80, 0.01)])
+def test_learned_mode_by_mask_and_by_child_agree(d, eps, rect):
+    # skips that differ from tree to tree of one mask: the walk per mask and the
+    # walk per child (any k) give the same trees and labels
+    rng = np.random.default_rng(d)
+    n, c, dims = 700, 3, 4
+    X = _split_trees(n, d, c, d + 1)
+    for k in range(2):
+        rows = np.arange(k * n // 3, (k + 1) * n // 3)[:, None]
+        at = np.sort(rng.choice(d, dims, replace=False))
+        X[rows, at] = ((rng.integers(0, c, dims) + 0.5) / c + 0.5 * eps * rng.standard_normal((len(rows), dims)))
+    X = torch.from_numpy(np.clip(X, 0, 1)).cuda()
+    args = (eps, 1.0, 3, 15, 1.0, c, rect, 0)
+    P = INSCY.run(X, *args, mode=_lib.MODE_COLLECT).pairs
+    W = pruner.init_params(6)
+    prob = pruner.Trainer(W).forward(P["features"]).cpu().numpy()
+    _lib.set_pruner(W, float(np.quantile(prob[P["info"][:, 0] > 0], 0.5)), 1)
+    res = []
+    for generic in (False, True):
+        _lib.debug_generic_walk(generic)
+        _lib.debug_trace(True)
+        try:
+            r = INSCY.run(X, *args, mode=_lib.MODE_LEARNED)
+            res.append((r, _lib.debug_trace_rows()))
+        finally:
+            _lib.debug_trace(False)
+            _lib.debug_generic_walk(False)
+    (a, ta), (b, tb) = res
+    say("learned by mask / child", d, rect, a.stats["pairs_skipped"], a.stats["queries"], b.stats["queries"],
+        len(a.subspaces))
+    assert a.stats["pairs_skipped"] > 0 and max(len(s) for s in a.subspaces) >= 2
+    assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
+    assert np.array_equal(ta, tb)
+    _lib.set_pruner(None, 0.0)
