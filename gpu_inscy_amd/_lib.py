@@ -161,6 +161,8 @@ def lib():
     L.inscy_debug_phi_exact.argtypes = [ctypes.c_int]
     L.inscy_debug_generic_walk.argtypes = [ctypes.c_int]
     L.inscy_debug_keep_budget.argtypes = [ctypes.c_int64]
+    L.inscy_debug_batch_budget.argtypes = [ctypes.c_int64]
+    L.inscy_debug_batch_most.restype = ctypes.c_int64
     L.inscy_debug_thresholds.argtypes = [ctypes.c_int32, ctypes.c_float, ctypes.c_int32, ctypes.POINTER(ctypes.c_float)]
     L.inscy_debug_thresholds.restype = ctypes.c_int
     L.inscy_debug_scan_temp.argtypes = [ctypes.c_int64]
@@ -337,6 +339,16 @@ def debug_generic_walk(on: bool) -> None:
 def debug_keep_budget(nbytes: int) -> None:
     """Test hook: bytes a run keeps for index sorts and for sorted columns (each; < 0: default)."""
     lib().inscy_debug_keep_budget(int(nbytes))
+
+
+def debug_batch_budget(nbytes: int) -> None:
+    """Test hook: device bytes of one batch of child subspaces (0: the default)."""
+    lib().inscy_debug_batch_budget(int(nbytes))
+
+
+def debug_batch_most() -> int:
+    """Test hook: the most device bytes that a batch of this thread's last run took."""
+    return int(lib().inscy_debug_batch_most())
 
 
 def debug_flag_compact_temp(nb: int) -> int:

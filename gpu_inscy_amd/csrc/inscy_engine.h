@@ -183,6 +183,16 @@ struct Pool {
     };
     std::vector<Chunk> chunks;
     size_t ci = 0, top = 0, chunk = 64u << 20;
+    size_t used = 0, most = 0;  // bytes taken since the reset, and the most of any moment
+    struct Mark {
+        size_t ci, top, used;
+    };
+    Mark mark() const { return {ci, top, used}; }
+    void release(const Mark &m) {
+        ci = m.ci;
+        top = m.top;
+        used = m.used;
+    }
     ~Pool() {
         for (auto &c : chunks) dev_free(c.p);
     }
@@ -202,12 +212,11 @@ struct Pool {
         }
         T *r = reinterpret_cast<T *>(chunks[ci].p + top);
         top += bytes;
+        used += bytes;
+        most = std::max(most, used);
         return r;
     }
-    void reset() {
-        ci = 0;
-        top = 0;
-    }
+    void reset() { release({0, 0, 0}); }
 };
 
 // Pinned host memory that grows on demand (contents are not kept).
@@ -390,6 +399,8 @@ public:
     bool generic_walk = false;   // test hook: no neighbour walk compiled for its k
     long long keep_budget_override = -1;  // test hook: bytes kept across batches (< 0: the batch budget)
     int mem_share = 1;  // engines running at once on the device (each budgets 1/mem_share of the free bytes)
+    long long batch_budget_override = 0;  // test hook: bytes of a batch (0: from the free memory)
+    size_t batch_most = 0;                // most bytes that a batch of the run took
     int max_batch_override = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
 
     // dense components of one subspace (kernel-level entry point)

@@ -11,6 +11,8 @@ static thread_local std::vector<Engine::TraceRow> g_trace;
 static bool g_trace_on = false;
 static bool g_phi_all_exact = false;
 static bool g_generic_walk = false;
+static int64_t g_batch_budget = 0;
+static thread_local int64_t g_batch_most = 0;
 static long long g_keep_budget = -1;
 static bool g_profile_on = false;
 static int g_max_batch = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
@@ -116,6 +118,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.trace_on = g_trace_on;
             eng.phi_all_exact = g_phi_all_exact;
             eng.generic_walk = g_generic_walk;
+            eng.batch_budget_override = g_batch_budget;
             eng.keep_budget_override = g_keep_budget;
             eng.max_batch_override = g_max_batch;
             eng.profile_on = g_profile_on;
@@ -132,6 +135,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.setup(d_X);
             eng.run_levels(*res);
             res->stats = eng.stats;
+            g_batch_most = (int64_t) eng.batch_most;
             if (g_trace_on) g_trace = eng.trace;
         }
         if (own) stream_pool().put(st);
@@ -481,6 +485,16 @@ int inscy_debug_keep_budget(int64_t bytes) {
     g_keep_budget = bytes;
     return INSCY_OK;
 }
+
+// Test hooks (not in the public header): bytes that a batch of child subspaces
+// may take (0: from the free memory), and the most that a batch of this thread's
+// last run took.
+int inscy_debug_batch_budget(int64_t bytes) {
+    g_batch_budget = std::max<int64_t>(bytes, 0);
+    return INSCY_OK;
+}
+
+int64_t inscy_debug_batch_most(void) { return g_batch_most; }
 
 // Test hook (not in the public header): the ordered compaction of the query
 // flags.  out[0, *nsel) receives the positions of the nonzero bytes of

@@ -91,6 +91,7 @@ void Engine::run_levels(inscy_result &out) {
     keptp.reset();
     kept_used = 0;
     kept_budget = keep_budget_override >= 0 ? (size_t) keep_budget_override : batch_budget;
+    if (batch_budget_override > 0) batch_budget = (size_t) batch_budget_override;
     colp.reset();
     cols_used = 0;
 
@@ -136,6 +137,7 @@ void Engine::run_levels(inscy_result &out) {
             return lt[a].m != lt[b].m ? lt[a].m < lt[b].m : lt[a].lo < lt[b].lo;
         });
     sync();
+    batch_most = batch.most;
     auto t1 = std::chrono::steady_clock::now();
     // superset rows of every subspace with a row: AND of per-dimension bitsets
     {
@@ -817,8 +819,6 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                         pc.weakcnt = pairs[j].weakcnt;
                         const size_t slots = path_slots(2 * nSP);
                         pc.tmask = (uint64_t) (slots - 1);
-                        pc.rx = batch.take<int>(nSP);
-                        pc.rw = batch.take<uint64_t>(nSP);
                         pc.outx = ch.spx;
                         pc.outw = ch.spm;
                         pc.nout = lv_next_counts + ch.slot;
@@ -826,8 +826,6 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                         pc.nP = t.nW;
                         pc.nr = nSP;
                         pc.g = g;
-                        prune_slots.push_back(table_total);
-                        table_total += slots;
                         pprune.push_back(pc);
                     } else if (nSP > 0) {
                         PruneChild pc;
@@ -860,27 +858,87 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
         }
     }
 
+    // ---- permuted order: a chain passes to every surviving group, so what the
+    // children's prunes take is known only here; as many children at a time as
+    // fit a batch's bytes
+    struct ChainPrune {
+        std::vector<PermChild> c;
+        std::vector<int> br{0}, bw{0}, bp{0};
+        PermChild *dc;
+        int *dbr, *dbw, *dbp;
+    };
+    auto chain_prune = [&](size_t c0, size_t c1, FillMany &f) {
+        ChainPrune cp;
+        cp.c.assign(pprune.begin() + c0, pprune.begin() + c1);
+        size_t slots = 0, chains = 0;
+        for (const PermChild &pc : cp.c) {
+            slots += pc.tmask + 1;
+            chains += pc.nr;
+        }
+        uint64_t *table = f.add(batch.take<uint64_t>(slots), ~0u, slots * sizeof(uint64_t));
+        uint8_t *marks = f.add(batch.take<uint8_t>(2 * slots), 0, 2 * slots);
+        dmask_t *bits = f.add(batch.take<dmask_t>(cp.c.size()), 0, cp.c.size() * sizeof(dmask_t));
+        int *nr = f.add(batch.take<int>(cp.c.size()), 0, cp.c.size() * sizeof(int));
+        int *rx = batch.take<int>(chains);
+        uint64_t *rw = batch.take<uint64_t>(chains);
+        for (PermChild &pc : cp.c) {
+            pc.table = table;
+            pc.marks = marks;
+            pc.bits = bits++;
+            pc.nr_at = nr++;
+            pc.rx = rx;
+            pc.rw = rw;
+            table += pc.tmask + 1;
+            marks += 2 * (pc.tmask + 1);
+            rx += pc.nr;
+            rw += pc.nr;
+            cp.br.push_back(cp.br.back() + nblocks(pc.nsp));
+            cp.bw.push_back(cp.bw.back() + nblocks((long long) pc.nP + pc.nr));
+            cp.bp.push_back(cp.bp.back() + nblocks(pc.nr));
+        }
+        return cp;
+    };
+    auto upload_chains = [&](ChainPrune &cp) {
+        cp.dc = upload(batch, cp.c);
+        cp.dbr = upload(batch, cp.br);
+        cp.dbw = upload(batch, cp.bw);
+        cp.dbp = upload(batch, cp.bp);
+    };
+    auto prune_chains = [&](const ChainPrune &cp) {
+        HIP_OK(launch_p_prune(D, cp.dc, (int) cp.c.size(), cp.dbr, cp.br.back(), cp.dbw, cp.bw.back(), cp.dbp,
+                              cp.bp.back(), weak_thr, phi_mode ? 1 : 0, st));
+    };
+    size_t chains_from = 0;  // children whose prunes are left to the batch's last launches
+    {
+        size_t bytes = 0;
+        for (size_t c = 0; c < pprune.size(); ++c) {
+            const PermChild &pc = pprune[c];
+            const size_t need = (size_t) pc.nr * 12 + (pc.tmask + 1) * 10 + sizeof(PermChild) + 32;
+            if (c > chains_from && bytes + need > batch_budget) {
+                const Pool::Mark mark = batch.mark();
+                FillMany f;
+                ChainPrune cp = chain_prune(chains_from, c, f);
+                defer_uploads();
+                upload_chains(cp);
+                flush_uploads();
+                HIP_OK(launch_fill_many(f, st));
+                prune_chains(cp);
+                batch.release(mark);  // stream order keeps the memory for the queued kernels
+                chains_from = c;
+                bytes = 0;
+            }
+            bytes += need;
+        }
+    }
+
     // ---- path prune of the surviving children, their point lists, and the
     // dense components of the subspaces that gained one: descriptors in one copy
     FillMany post;
-    const int nprune = (int) prune.size(), npprune = (int) pprune.size();
-    std::vector<int> bw(nprune + npprune + 1, 0), bp(nprune + npprune + 1, 0), br(npprune + 1, 0);
-    if (npprune) {
-        uint64_t *tables = post.add(batch.take<uint64_t>(table_total), ~0u, table_total * sizeof(uint64_t));
-        uint8_t *marks = post.add(batch.take<uint8_t>(2 * table_total), 0, 2 * table_total);
-        dmask_t *bits = post.add(batch.take<dmask_t>(npprune), 0, (size_t) npprune * sizeof(dmask_t));
-        int *nr = post.add(batch.take<int>(npprune), 0, (size_t) npprune * sizeof(int));
-        for (int c = 0; c < npprune; ++c) {
-            PermChild &pc = pprune[c];
-            pc.table = tables + prune_slots[c];
-            pc.marks = marks + 2 * prune_slots[c];
-            pc.bits = bits + c;
-            pc.nr_at = nr + c;
-            br[c + 1] = br[c] + nblocks(pc.nsp);
-            bw[c + 1] = bw[c] + nblocks((long long) pc.nP + pc.nr);
-            bp[c + 1] = bp[c] + nblocks(pc.nr);
-        }
-    }
+    const int nprune = (int) prune.size();
+    std::vector<int> bw(nprune + 1, 0), bp(nprune + 1, 0);
+    ChainPrune chains;
+    const bool any_chains = chains_from < pprune.size();
+    if (any_chains) chains = chain_prune(chains_from, pprune.size(), post);
     if (nprune) {
         uint64_t *tables = post.add(batch.take<uint64_t>(table_total), ~0u, table_total * sizeof(uint64_t));
         dmask_t *bits = post.add(batch.take<dmask_t>(nprune), 0, (size_t) nprune * sizeof(dmask_t));
@@ -943,10 +1001,9 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     for (size_t c = 0; c < copies.size(); ++c) cb[c + 1] = cb[c] + nblocks(copies[c].len);
     defer_uploads();
     PruneChild *dpc = nprune ? upload(batch, prune) : nullptr;
-    PermChild *dpch = npprune ? upload(batch, pprune) : nullptr;
-    int *dbr = npprune ? upload(batch, br) : nullptr;
-    int *dbw = nprune + npprune ? upload(batch, bw) : nullptr;
-    int *dbp = nprune + npprune ? upload(batch, bp) : nullptr;
+    int *dbw = nprune ? upload(batch, bw) : nullptr;
+    int *dbp = nprune ? upload(batch, bp) : nullptr;
+    if (any_chains) upload_chains(chains);
     CopySeg *dcs = copies.empty() ? nullptr : upload(batch, copies);
     int *dcb2 = copies.empty() ? nullptr : upload(batch, cb);
     if (ncomp > 0 && fan) columns(hc, ctab2);
@@ -954,9 +1011,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
     if (ncomp > 0) put(entries + nentries, ents.data(), ents.size() * sizeof(Entry));
     flush_uploads();
     HIP_OK(launch_fill_many(post, st));
-    if (npprune)
-        HIP_OK(launch_p_prune(D, dpch, npprune, dbr, br[npprune], dbw, bw[npprune], dbp, bp[npprune], weak_thr,
-                              phi_mode ? 1 : 0, st));
+    if (any_chains) prune_chains(chains);
     if (nprune) HIP_OK(launch_b_prune(D, dpc, nprune, dbw, bw[nprune], dbp, bp[nprune], st));
     if (!copies.empty()) HIP_OK(launch_b_copy(dcs, dcb2, (int) copies.size(), cb.back(), st));
     if (ncomp > 0) {

@@ -192,3 +192,44 @@ def test_walks_per_mask_and_per_child_agree(n, d, eps, dims, rect):
     assert b.stats["queries"] < a.stats["queries"]
     assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
     assert np.array_equal(ta, tb)
+
+
+def many_groups(n, d, c, eps, seed):
+    """Half of the points at the upper edge of each dimension's first cell (all of
+    them on s-connection chains), the others in the middles of the other cells: every
+    tree splits into c - 1 groups, and a chain passes to most."""
+    rng = np.random.default_rng(seed)
+    # the larger the first cell's share, the smaller the dimension's entropy
+    cell = np.where(rng.random((n, d)) < np.linspace(0.4, 0.6, d), 0, rng.integers(1, c, (n, d)))
+    off = np.where(cell == 0, 1 - (0.5 + 0.4 * rng.uniform(-1, 1, (n, d))) * eps * c,
+                   0.5 + 0.1 * rng.uniform(-1, 1, (n, d)))
+    return ((cell + off) / c).astype(np.float32)
+
+
+# permuted level orders where a chain passes to most groups: a batch keeps to its
+# bytes (and as many again for its children's prunes), whatever they come to
+@pytest.mark.parametrize("order", [1, -1])
+@pytest.mark.parametrize("n,d,c,budget", [(1500, 4, 20, 1 << 20), (1500, 4, 20, 1 << 19), (900, 5, 10, 1 << 19)])
+def test_permuted_batches_keep_to_their_budget(n, d, c, budget, order):
+    print("permuted budget", n, d, c, budget, order, flush=True)
+    # levels against the dimensions: chains lie above the levels restricted first
+    X = np.ascontiguousarray(many_groups(n, d, c, 0.01, n)[:, ::order])
+    args = (0.01, 1.0, 4, 30, 1.0, c, True, order)
+    ref = O.run_ref(X, *args[:7], order, trace=True)
+    whole = None
+    for b in (0, budget):
+        _lib.debug_batch_budget(b)
+        try:
+            got, trace = traced(X, args)
+            most = _lib.debug_batch_most()
+        finally:
+            _lib.debug_batch_budget(0)
+        print("bytes of a batch", b, most, flush=True)
+        assert got.subspaces == ref.subspaces
+        for r, g in zip(ref.labels, got.labels):
+            assert np.array_equal(O.canonical(r), g)
+        assert np.array_equal(trace, ref.trace)
+        if whole is None:
+            whole = most
+        else:
+            assert most <= 2 * budget + (1 << 18) < whole
