@@ -163,6 +163,9 @@ def lib():
     L.inscy_debug_keep_budget.argtypes = [ctypes.c_int64]
     L.inscy_debug_batch_budget.argtypes = [ctypes.c_int64]
     L.inscy_debug_batch_most.restype = ctypes.c_int64
+    L.inscy_debug_path_slots.argtypes = [ctypes.c_int64]
+    L.inscy_debug_path_slots.restype = ctypes.c_int64
+    L.inscy_debug_chain_limit.argtypes = [ctypes.c_int32]
     L.inscy_debug_thresholds.argtypes = [ctypes.c_int32, ctypes.c_float, ctypes.c_int32, ctypes.POINTER(ctypes.c_float)]
     L.inscy_debug_thresholds.restype = ctypes.c_int
     L.inscy_debug_scan_temp.argtypes = [ctypes.c_int64]
@@ -349,6 +352,16 @@ def debug_batch_budget(nbytes: int) -> None:
 def debug_batch_most() -> int:
     """Test hook: the most device bytes that a batch of this thread's last run took."""
     return int(lib().inscy_debug_batch_most())
+
+
+def debug_path_slots(levels: int) -> int:
+    """Test hook: slots of a path prune's table for that many prefixes."""
+    return int(lib().inscy_debug_path_slots(int(levels)))
+
+
+def debug_chain_limit(chains: int) -> None:
+    """Test hook: the most chains of a permuted level order's root tree (0: the default)."""
+    lib().inscy_debug_chain_limit(int(chains))
 
 
 def debug_flag_compact_temp(nb: int) -> int:

@@ -400,6 +400,7 @@ public:
     long long keep_budget_override = -1;  // test hook: bytes kept across batches (< 0: the batch budget)
     int mem_share = 1;  // engines running at once on the device (each budgets 1/mem_share of the free bytes)
     long long batch_budget_override = 0;  // test hook: bytes of a batch (0: from the free memory)
+    int chain_limit = INT_MAX;            // most chains of a permuted order's root tree (test hook: less)
     size_t batch_most = 0;                // most bytes that a batch of the run took
     int max_batch_override = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
 
@@ -441,7 +442,7 @@ public:
 
 private:
     // ---------------------------------------------------------- helpers
-    // `small` device words (zeroed by the set-up): [0] input check flag, [1] the root's paths,
+    // `small` device words (zeroed by the set-up): [0] input check flag, [1] the root's paths, [2] its chains,
     // [kStatAt..) 64 slot pairs (16 words apart) of neighbour-count statistics
     static constexpr int kStatAt = 32;
     static constexpr int kSmallWords = kStatAt + 16 * 64;

@@ -13,6 +13,7 @@ static bool g_phi_all_exact = false;
 static bool g_generic_walk = false;
 static int64_t g_batch_budget = 0;
 static thread_local int64_t g_batch_most = 0;
+static int g_chain_limit = INT_MAX;
 static long long g_keep_budget = -1;
 static bool g_profile_on = false;
 static int g_max_batch = 0;  // inscy_set_tuning: child subspaces per batch (0: the default)
@@ -119,6 +120,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.phi_all_exact = g_phi_all_exact;
             eng.generic_walk = g_generic_walk;
             eng.batch_budget_override = g_batch_budget;
+            eng.chain_limit = g_chain_limit;
             eng.keep_budget_override = g_keep_budget;
             eng.max_batch_override = g_max_batch;
             eng.profile_on = g_profile_on;
@@ -495,6 +497,16 @@ int inscy_debug_batch_budget(int64_t bytes) {
 }
 
 int64_t inscy_debug_batch_most(void) { return g_batch_most; }
+
+// Test hooks (not in the public header): the slots of a path prune's table for
+// that many prefixes (host arithmetic), and the most chains of a permuted level
+// order's root tree (0: what the lists' positions hold).
+int64_t inscy_debug_path_slots(int64_t levels) { return (int64_t) path_slots((size_t) std::max<int64_t>(levels, 0)); }
+
+int inscy_debug_chain_limit(int32_t chains) {
+    g_chain_limit = chains > 0 ? chains : INT_MAX;
+    return INSCY_OK;
+}
 
 // Test hook (not in the public header): the ordered compaction of the query
 // flags.  out[0, *nsel) receives the positions of the nonzero bytes of

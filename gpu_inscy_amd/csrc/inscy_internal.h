@@ -228,7 +228,7 @@ struct PartPair {
     const int *gid;      // [cells]
     const int *weakcnt;  // counts of S ∪ {m}
     const uint8_t *keep; // [nP] the points that count (null: all)
-    int *cnt;            // [7G]: points, weak-dense points, paths per group; 3 cursors; the paths' branch levels
+    int *cnt;            // [8G]: points, weak-dense points, paths per group; 3 cursors; the paths' branch levels in 64 bits
     int *outW;
     int *outx;
     uint64_t *outm;
@@ -302,6 +302,14 @@ struct PermChild {
     int *nout;
     int nsp, nP, nr, g;
 };
+
+// slots of a path prune's table (all bits set when free) for at most `levels`
+// prefixes, at most half full
+inline size_t path_slots(size_t levels) {
+    size_t s = 64;
+    while (s < 2 * levels) s <<= 1;
+    return s;
+}
 
 // pad < 0: dst[i] = src[i]; else dst[src[i]] = pad (the tree stamps of the replay)
 struct CopySeg {
@@ -388,6 +396,8 @@ hipError_t launch_b_root(const dmask_t *nearm, int n, int *P, int *outx, uint64_
 // the same in a permuted level order: one chain per near-edge dimension of a point
 hipError_t launch_p_root(const dmask_t *nearm, int n, int d, int *P, int *cx, uint64_t *cw, int *nout, int C,
                          float *edge, hipStream_t st);
+// *total += the near-edge dimensions of all points (the chains of launch_p_root)
+hipError_t launch_p_chains(const dmask_t *nearm, int n, unsigned long long *total, hipStream_t st);
 hipError_t launch_p_flags(const FlagTree *T, const int *blk_off, int nt, int nblk, const uint8_t *cellC, int n,
                           int cells, int *flags, hipStream_t st);
 hipError_t launch_p_filter(const DevData &D, const PermFilter *F, const int *blk_off, int nf, int nblk, hipStream_t st);

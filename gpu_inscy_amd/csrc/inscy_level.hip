@@ -30,13 +30,6 @@ namespace {
 // launches, a wait and a read-back (n=20,011 d=70, 49,000 child subspaces:
 // batches of 1024 118.3 ms, 2048 112.2, 4096 107.6, 8192 107.3)
 constexpr size_t kMaxBatch = 4096;
-// slots of a path prune's table (all bits set when free) for at most `levels`
-// prefixes, at most half full
-inline size_t path_slots(int levels) {
-    size_t s = 64;
-    while (s < 2 * (size_t) levels) s <<= 1;
-    return s;
-}
 inline int nblocks(long long count) { return (int) ((count + kBlockThreads - 1) / kBlockThreads); }
 }  // namespace
 
@@ -107,7 +100,18 @@ void Engine::run_levels(inscy_result &out) {
     root.nW = n;
     root.pre = n;
     // identity order: a path per point; permuted: a chain per near-edge dimension
-    const size_t most = permuted ? std::min<size_t>((size_t) n * d, INT_MAX) : (size_t) n;
+    // (positions in the lists are ints: tables that could hold more chains are counted first)
+    size_t most = permuted ? (size_t) n * d : (size_t) n;
+    if (most > (size_t) chain_limit) {
+        unsigned long long *total = small + 2;  // zeroed by the set-up
+        HIP_OK(launch_p_chains(nearm, n, total, st));
+        unsigned long long *h = reinterpret_cast<unsigned long long *>(down.get(sizeof(*h)));
+        HIP_OK(hipMemcpyAsync(h, total, sizeof(*h), hipMemcpyDeviceToHost, st));
+        sync();
+        if (*h > (unsigned long long) chain_limit)
+            throw Failure(INSCY_ERR_UNSUPPORTED, "more than 2^31 - 1 s-connection chains in a permuted level order");
+        most = (size_t) *h;
+    }
     root.spx = L0.take<int>(most);
     root.spm = L0.take<uint64_t>(most * pw);
     root.nsp_max = (int) most;
@@ -305,7 +309,7 @@ void Engine::expand_level(const std::vector<int> &frontier, const int *counts) {
                 if (!pair_on(a, c.m)) continue;
                 const LTree &t = lt[lv_act[a]];
                 // lists, and the path prune's table (a few branch levels per path)
-                est += (size_t) t.nW * 8 + (size_t) t.nsp * (12 + 32 * std::min<size_t>(d - 1 - c.m, 4)) + 7 * 256 * 4;
+                est += (size_t) t.nW * 8 + (size_t) t.nsp * (12 + 32 * std::min<size_t>(d - 1 - c.m, 4)) + 8 * 256 * 4;
                 // the point filter's table and flags, the routed chains and their table
                 if (permuted) est += (size_t) t.nW * 33 + (size_t) t.nsp * 96;
             }
@@ -567,7 +571,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             const LTree &t = lt[lv_act[a]];
             const int G = (int) lv_groups[a][c.m - t.first].size();
             pinfo.push_back({a, b, G, pc_total});
-            pc_total += 7 * G;
+            pc_total += 8 * G;
         }
     }
     int *pcnt = batch.take<int>(std::max(pc_total, 1));
@@ -775,6 +779,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             col_G[gp] = G;
         }
         const int *c3 = hcnt.data() + pi.cnt_off;
+        const unsigned long long *levels = reinterpret_cast<const unsigned long long *>(c3 + 6 * G);
         int offW = 0, offS = 0, others = 0;
         for (int g = 0; permuted && g < G; ++g) others += c3[6 * G + g];
         for (int g = 0; g < G; ++g) {
@@ -817,7 +822,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                         pc.P = t.W;
                         pc.keep = pairs[j].keep;
                         pc.weakcnt = pairs[j].weakcnt;
-                        const size_t slots = path_slots(2 * nSP);
+                        const size_t slots = path_slots(2 * (size_t) nSP);
                         pc.tmask = (uint64_t) (slots - 1);
                         pc.outx = ch.spx;
                         pc.outw = ch.spm;
@@ -831,7 +836,7 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
                         PruneChild pc;
                         std::memset(&pc, 0, sizeof(pc));
                         pc.smask = c.s;
-                        const size_t slots = path_slots(c3[6 * G + g]);
+                        const size_t slots = path_slots((size_t) levels[g]);
                         pc.tmask = (uint64_t) (slots - 1);
                         pc.W = pairs[j].outW + offW;
                         pc.spx = pairs[j].outx + offS;

@@ -1426,8 +1426,14 @@ __global__ void k_b_part_count(const PartPair *__restrict__ pairs, const int *__
     }
     __syncthreads();
     // the paths' branch levels (the size of their prune's table) follow the cursors
-    for (int t = threadIdx.x; t < 4 * G; t += blockDim.x)
-        if (h[t]) atomicAdd(&A.cnt[t < 3 * G ? t : t + 3 * G], h[t]);
+    unsigned long long *levels = reinterpret_cast<unsigned long long *>(A.cnt + 6 * G);
+    for (int t = threadIdx.x; t < 4 * G; t += blockDim.x) {
+        if (!h[t]) continue;
+        if (t < 3 * G)
+            atomicAdd(&A.cnt[t], h[t]);
+        else
+            atomicAdd(&levels[t - 3 * G], (unsigned long long) h[t]);
+    }
 }
 
 // Only the groups whose weak-dense points reach min_size become surviving

@@ -123,6 +123,13 @@ __global__ void k_p_root(const dmask_t *__restrict__ nearm, int n, int d, int *_
     }
 }
 
+__global__ void k_p_chains(const dmask_t *__restrict__ nearm, int n, unsigned long long *__restrict__ total) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int c = i < n ? dcount(nearm[i]) : 0;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o);
+    if (__lane_id() == 0 && c) atomicAdd(total, (unsigned long long) c);
+}
+
 // merge flags of every dimension >= first of every tree
 __global__ void k_p_flags(const FlagTree *__restrict__ T, const int *__restrict__ blk_off, int nt,
                           const uint8_t *__restrict__ cellC, int n, int cells, int *__restrict__ flags) {
@@ -298,6 +305,11 @@ hipError_t launch_p_root(const dmask_t *nearm, int n, int d, int *P, int *cx, ui
                          float *edge, hipStream_t st) {
     LAUNCH(k_p_root, dim3(blocks_for((size_t) std::max(n, C + 3))), dim3(kBlock), 0, st, nearm, n, d, P, cx, cw, nout, C,
            edge);
+    return hipGetLastError();
+}
+
+hipError_t launch_p_chains(const dmask_t *nearm, int n, unsigned long long *total, hipStream_t st) {
+    LAUNCH(k_p_chains, dim3(blocks_for(n)), dim3(kBlock), 0, st, nearm, n, total);
     return hipGetLastError();
 }
 

@@ -233,3 +233,31 @@ def test_permuted_batches_keep_to_their_budget(n, d, c, budget, order):
             whole = most
         else:
             assert most <= 2 * budget + (1 << 18) < whole
+
+
+# a permuted order's root lists, where points times dimensions pass what their
+# positions hold: sized by the chains there are, refused past the limit
+def test_permuted_root_lists_at_the_limit():
+    n, d, c = 900, 5, 10
+    X = many_groups(n, d, c, 0.01, n)
+    args = (0.01, 1.0, 4, 30, 1.0, c, True, 1)
+    ref = O.run_ref(X, *args[:7], 1)
+    # near-edge marks: within eps of a cell's upper edge, the last cell's apart
+    cell = np.minimum((X.astype(np.float64) * c).astype(int), c - 1)
+    chains = int(((cell < c - 1) & ((cell + 1) / c - X < 0.01)).sum())
+    assert n * d // 4 < chains < n * d
+    try:
+        for limit, fits in ((n * d, True), (chains + 40, True), (chains - 40, False)):
+            print("chain limit", limit, chains, flush=True)
+            _lib.debug_chain_limit(limit)
+            if fits:
+                got = INSCY.run(torch.from_numpy(X).cuda(), *args, mode=_lib.MODE_BATCHED)
+                assert got.subspaces == ref.subspaces
+                for r, g in zip(ref.labels, got.labels):
+                    assert np.array_equal(O.canonical(r), g)
+            else:
+                with pytest.raises(_lib.InscyError) as e:
+                    INSCY.run(torch.from_numpy(X).cuda(), *args, mode=_lib.MODE_BATCHED)
+                assert e.value.code == _lib.INSCY_ERR_UNSUPPORTED
+    finally:
+        _lib.debug_chain_limit(0)

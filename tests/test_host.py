@@ -203,3 +203,12 @@ def test_tuning_rejects_bad_arguments_and_applies_saved_files(tmp_path):
         assert autotune.apply(str(path)) == {"max_batch": 512, "workers": 2}
     finally:
         _lib.set_tuning(0, 0)
+
+
+def test_path_table_slots_past_32_bits():
+    # a power of two, at least twice the prefixes: no sum of 32 bits on the way
+    for levels in (0, 1, 31, 32, 33, 1 << 20, (1 << 30) + 1, (1 << 31) - 1, 1 << 31, (1 << 31) + 1, 1 << 32,
+                   (1 << 36) + 5):
+        s = _lib.debug_path_slots(levels)
+        assert s >= max(64, 2 * levels) and s & (s - 1) == 0
+        assert s == 64 or s < 4 * levels
