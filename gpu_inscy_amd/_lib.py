@@ -166,6 +166,7 @@ def lib():
     L.inscy_debug_path_slots.argtypes = [ctypes.c_int64]
     L.inscy_debug_path_slots.restype = ctypes.c_int64
     L.inscy_debug_chain_limit.argtypes = [ctypes.c_int32]
+    L.inscy_debug_fill_many.argtypes = [ctypes.c_int32]
     L.inscy_debug_thresholds.argtypes = [ctypes.c_int32, ctypes.c_float, ctypes.c_int32, ctypes.POINTER(ctypes.c_float)]
     L.inscy_debug_thresholds.restype = ctypes.c_int
     L.inscy_debug_scan_temp.argtypes = [ctypes.c_int64]

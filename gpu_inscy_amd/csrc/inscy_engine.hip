@@ -54,11 +54,8 @@ static int check_params(int64_t n, int32_t d, const inscy_params *p, int32_t mod
     // A permuted SCY-tree level order has its trees hold s-connection chains
     // (inscy_perm.hip), with neighbour-count density or, for rectangular =
     // false, phi summed in the neighbourhood tree's leaf order.
-    if (p->entropy_order != 0) {
-        if (mode == INSCY_MODE_LEARNED || mode == INSCY_MODE_COLLECT)
-            return fail(INSCY_ERR_UNSUPPORTED, "entropy_order != 0 runs the exact drivers only");
-        if (d > 255) return fail(INSCY_ERR_ARGUMENT, "d must be at most 255");
-    }
+    if (p->entropy_order != 0 && (mode == INSCY_MODE_LEARNED || mode == INSCY_MODE_COLLECT))
+        return fail(INSCY_ERR_UNSUPPORTED, "entropy_order != 0 runs in the exact modes only");
     return INSCY_OK;
 }
 
@@ -502,6 +499,18 @@ int64_t inscy_debug_batch_most(void) { return g_batch_most; }
 // that many prefixes (host arithmetic), and the most chains of a permuted level
 // order's root tree (0: what the lists' positions hold).
 int64_t inscy_debug_path_slots(int64_t levels) { return (int64_t) path_slots((size_t) std::max<int64_t>(levels, 0)); }
+
+// (and whether that many arrays can be cleared together: INSCY_OK or an error)
+int inscy_debug_fill_many(int32_t arrays) {
+    try {
+        FillMany f;
+        uint32_t word = 0;
+        for (int i = 0; i < arrays; ++i) f.add(&word, 0, sizeof(word));
+        return INSCY_OK;
+    } catch (...) {
+        return fail_current();
+    }
+}
 
 int inscy_debug_chain_limit(int32_t chains) {
     g_chain_limit = chains > 0 ? chains : INT_MAX;

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <stdexcept>
 #include <string>
 
 namespace inscy {
@@ -379,6 +380,7 @@ struct FillMany {
     template <class T>
     T *add(T *dst, uint32_t word, size_t bytes) {
         if (bytes) {
+            if (n == kMost) throw std::length_error("FillMany holds kMost arrays");
             p[n] = reinterpret_cast<uint32_t *>(dst);
             words[n] = (bytes + 3) / 4;  // whole words: the arrays' allocations are rounded to 256 bytes
             v[n++] = word;
@@ -474,11 +476,6 @@ size_t rank_order_temp_bytes(int n);
 hipError_t launch_b_prune(const DevData &D, const PruneChild *C, int nc, const int *blk_w, int nblk_w,
                           const int *blk_p, int nblk_p, hipStream_t st);
 hipError_t launch_b_copy(const CopySeg *segs, const int *blk_off, int nseg, int nblk, hipStream_t st);
-// replay: pruneRedundancy of one tree (keepv[tree] = decision; rowflag: 2 *
-// nlist zeroed words and done: one zeroed word, both left zeroed by the
-// launch), join of one (parent, dimension) pair (added: one scratch word)
-hipError_t launch_rep_redundancy(const Entry *E, const int *list, int nlist, const int *tstamp, const int *W,
-                                 int tree, int nW, float r, int *rowflag, unsigned *done, int *keepv, hipStream_t st);
 // One step of the staged replay: pruneRedundancy of `tree` (kind 0 and 1),
 // and/or the join J of the kept trees [t_lo, t_hi) into subspace S (kind 0:
 // the pair's only surviving child is `tree`; kind 2: a pair with several).

@@ -212,3 +212,10 @@ def test_path_table_slots_past_32_bits():
         s = _lib.debug_path_slots(levels)
         assert s >= max(64, 2 * levels) and s & (s - 1) == 0
         assert s == 64 or s < 4 * levels
+
+
+def test_arrays_cleared_together_are_bounded():
+    L = _lib.lib()
+    assert L.inscy_debug_fill_many(8) == _lib.INSCY_OK
+    assert L.inscy_debug_fill_many(9) != _lib.INSCY_OK
+    assert b"kMost" in L.inscy_last_error()
