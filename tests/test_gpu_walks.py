@@ -261,3 +261,32 @@ def test_permuted_root_lists_at_the_limit():
                 assert e.value.code == _lib.INSCY_ERR_UNSUPPORTED
     finally:
         _lib.debug_chain_limit(0)
+
+
+# every route of one run gives one result: a walk per mask and per child, compiled
+# and not; one child subspace at a time, a few and all of a level; no index kept
+# from one batch for the next; small batches
+@pytest.mark.parametrize("rect,order", [(True, 0), (False, 0), (True, 1), (False, -1)])
+def test_routes_give_one_result(rect, order):
+    print("routes", rect, order, flush=True)
+    w = datagen.small(5, n=4000, d=8, n_clusters=4, eps=0.02, cells=5, num_obj=4, min_size=60, sub_dims=(3, 5))
+    args = (w.eps, w.F, w.num_obj, w.min_size, w.r, w.cells, rect, order)
+    a, ta = traced(w.X, args)
+    assert max(len(s) for s in a.subspaces) >= 3
+    for generic, max_batch, keep, budget in ((True, 0, -1, 0), (False, 1, -1, 0), (True, 1, -1, 0), (False, 3, 0, 0),
+                                             (True, 0, 0, 0), (False, 0, 1 << 20, 2 << 20)):
+        print("route", generic, max_batch, keep, budget, flush=True)
+        _lib.debug_generic_walk(generic)
+        _lib.set_tuning(max_batch=max_batch)
+        _lib.debug_keep_budget(keep)
+        _lib.debug_batch_budget(budget)
+        try:
+            b, tb = traced(w.X, args)
+        finally:
+            _lib.debug_batch_budget(0)
+            _lib.debug_keep_budget(-1)
+            _lib.set_tuning()
+            _lib.debug_generic_walk(False)
+        assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
+        assert np.array_equal(ta, tb)
+        assert a.stats["trees"] == b.stats["trees"] and a.stats["calls"] == b.stats["calls"]
