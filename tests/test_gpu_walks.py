@@ -290,3 +290,86 @@ def test_routes_give_one_result(rect, order):
         assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
         assert np.array_equal(ta, tb)
         assert a.stats["trees"] == b.stats["trees"] and a.stats["calls"] == b.stats["calls"]
+
+
+# the same sizes in the phi density (the groups' points meet its thresholds too;
+# the oracle says so for the small ones)
+@pytest.mark.parametrize("n,per", [(75, 3), (1025, 3), (39936, 3), (39937, 3), (159744, 3), (159744, 4), (159745, 3)])
+def test_sample_phase_sizes_phi(n, per):
+    print("sample phase phi", n, per, flush=True)
+    X, eps, want = groups(n, per)
+    args = (eps, 1.0, 1, 2, 1.0, 4, False)
+    if n < 5000:
+        ref = O.run_ref(X, *args)
+        assert ref.subspaces == [[0], [1], [0, 1]]
+        for a, b in zip(ref.labels, want):
+            assert np.array_equal(O.canonical(a), O.canonical(b))
+    got = INSCY.run(torch.from_numpy(X).cuda(), *args, 0, mode=_lib.MODE_BATCHED)
+    assert got.subspaces == [[0], [1], [0, 1]]
+    for a, b in zip(got.labels, want):
+        assert np.array_equal(a, O.canonical(b))
+
+
+# walks of up to 32 children against the oracle, and of up to 64 and (in two
+# walks) 79 against the walk per child
+@pytest.mark.parametrize("n,d,eps,dims", [(90, 20, 0.03, 3), (301, 33, 0.02, 4), (250, 60, 0.02, 3),
+                                          (240, 80, 0.02, 3)])
+@pytest.mark.parametrize("rect", [True, False])
+def test_walks_of_more_than_16_children(n, d, eps, dims, rect):
+    print("many children", n, d, eps, dims, rect, flush=True)
+    X = clumps(n, d, eps, dims, n * d)
+    args = (eps, 1.0, 4, n // 6, 1.0, 4, rect, 0)
+    got, trace = traced(X, args)
+    assert max(len(s) for s in got.subspaces) >= dims - 1
+    if d == 20:
+        ref = O.run_ref(X, *args[:7], 0, trace=True)
+        assert got.subspaces == ref.subspaces
+        for a, b in zip(ref.labels, got.labels):
+            assert np.array_equal(O.canonical(a), b)
+        assert np.array_equal(trace, ref.trace)
+    _lib.debug_generic_walk(True)
+    try:
+        b, tb = traced(X, args)
+    finally:
+        _lib.debug_generic_walk(False)
+    assert got.subspaces == b.subspaces and np.array_equal(got.labels, b.labels)
+    assert np.array_equal(trace, tb)
+
+
+def test_threads_share_streams_while_memory_is_released():
+    # callers without a stream take one from the pool and give it back, from
+    # several threads at once, while another returns the pools' idle contents
+    import threading
+    jobs = []
+    for seed, n in enumerate((150, 700, 1501)):
+        w = datagen.small(seed + 20, n=n, d=5, n_clusters=3, eps=0.04, min_size=max(5, n // 40))
+        args = (w.eps, w.F, w.num_obj, w.min_size, w.r, w.cells, True, 0)
+        jobs.append((w.X, args, INSCY.run(w.X, *args)))
+    bad, stop = [], threading.Event()
+
+    def work(k):
+        try:
+            for i in range(12):
+                X, args, want = jobs[(k + i) % len(jobs)]
+                got = INSCY.run(X if i % 2 else torch.from_numpy(X).cuda(), *args)
+                if got.subspaces != want.subspaces or not np.array_equal(got.labels, want.labels):
+                    bad.append((k, i))
+        except Exception as e:  # noqa: BLE001
+            bad.append((k, repr(e)))
+
+    def release():
+        while not stop.is_set():
+            _lib.lib().inscy_release_memory()
+            stop.wait(0.002)
+
+    print("threads", flush=True)
+    th = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    rel = threading.Thread(target=release)
+    rel.start()
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    stop.set()
+    rel.join()
+    assert not bad, bad
