@@ -27,6 +27,7 @@ static int fail(int code, const std::string &msg) {
 // The exception in flight as a return code and message: nothing thrown inside
 // the library crosses the C ABI.
 static int fail_current() {
+    (void) hipGetLastError();  // reported here: the next call's launches must not report it as theirs
     try {
         throw;
     } catch (const Failure &f) {

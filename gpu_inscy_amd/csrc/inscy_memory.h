@@ -45,6 +45,8 @@ public:
             (void) hipGetLastError();
             release(dev);
             e = raw_alloc(p, sz);
+            // returned, and not left for a later launch to report as its own
+            if (e != hipSuccess) (void) hipGetLastError();
         }
         if (e == hipSuccess) {
             std::lock_guard<std::mutex> g(mu_);

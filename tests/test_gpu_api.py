@@ -75,3 +75,21 @@ def test_autotune_settings_do_not_change_results():
         assert len(rec3["results"]) == 2
     finally:
         _lib.set_tuning(0, 0)
+
+
+def test_a_call_after_one_out_of_memory_runs():
+    # an allocation larger than the device is refused before anything is read;
+    # the error is that call's alone
+    import ctypes
+    say("after out of memory")
+    w = datagen.small(3, n=300, d=4)
+    X = torch.from_numpy(w.X).cuda()
+    want = INSCY.run(X, mode=_lib.MODE_BATCHED, **w.params())
+    L = _lib.lib()
+    p = _lib.make_params(w.eps, w.F, w.num_obj, w.min_size, w.r, w.cells, True, 0)
+    h = ctypes.c_void_p()
+    for _ in range(2):
+        assert L.inscy_run_device(X.data_ptr(), (1 << 30) - 1, 128, ctypes.byref(p), _lib.MODE_BATCHED, None,
+                                  ctypes.byref(h)) == _lib.INSCY_ERR_MEMORY
+        got = INSCY.run(X, mode=_lib.MODE_BATCHED, **w.params())
+        assert got.subspaces == want.subspaces and np.array_equal(got.labels, want.labels)
