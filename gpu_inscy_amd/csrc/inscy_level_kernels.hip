@@ -378,9 +378,9 @@ __device__ __forceinline__ void cells_of_hits(const BatchSub &B, const float2 *q
 // column with one 16-byte load per lane instead of four 4-byte loads, and
 // nothing else: the eps cells of the checked dimensions are tested on the
 // coordinates of the step's hits (cells_of_hits).
-// The vector memory pipeline bounds these walks (its address and data units
-// are busy nearly all the time), and its cost grows with the number of load
-// instructions.  The runs are
+// Load instructions are what these walks pay for most (the CUs' address unit is busy
+// for 63 to 79% of the cycles, at 24 to 29 cycles and 12 to 21 cache lines a load;
+// n=100,000 d=20).  The runs are
 // concatenated in groups of four (q[20..29]); the last group of a run masks
 // the positions past the run's end, which are read (up to three past the
 // run: the batch's coordinate buffer ends with padding) but
@@ -663,14 +663,19 @@ __global__ __launch_bounds__(kBlock) void k_b_count(const BatchSub *__restrict__
 // The children's bounds (k_b_count) are not looked up: one undecided child
 // makes the walk anyway, and the look-up costs a scattered read per child and
 // bound (n=100,000 d=20, masks of three dimensions: 54 ms with it, 49 without).
-// Bound: about two fifths of the time is the set-up of the walks (a chain of
-// dependent loads per query), a quarter the candidates, a third VALU work on
-// the neighbours; hence slots for masks of few children instead of idle lanes
-// (49 -> 43 ms; by child, k_b_count took 63 ms).
-// Six waves a SIMD where that costs few or no spills (count mode, K <= 6, up to two
-// children a lane: 91 -> 79 VGPRs at K = 2, eight children): n=100,000 d=20
-// eps=0.02 583 -> 576 ms a run, n=25,000 d=15 9.96 -> 9.80 of kernels; seven
-// waves 591, eight 623, and four children a lane spill 21 registers or more at six.
+// Bound: no unit alone (n=100,000 d=20 eps=0.02): waves wait for 60 to 68% of
+// their cycles (a query's set-up is a chain of dependent loads), while the CUs'
+// address units are busy for 73 to 81% (18 cycles and 8 to 14 cache lines a load)
+// and VALU instructions issue at 0.67 to 0.81 of one a SIMD per four cycles.
+// Masks of few children have slots instead of idle lanes (49 -> 43 ms; by
+// child, k_b_count took 63 ms).
+// Six waves a SIMD in count mode with up to two children a lane, up to K = 6:
+// 91 -> 79 VGPRs at K = 2, eight children.  The 80 registers of six waves are enough
+// or two short up to K = 4; at K = 5 up to 10 are spilled, at K = 6 8 to 17.  Whole
+// runs at n=100,000 d=20 eps=0.02: without it 583 ms, up to K = 4 583 and 578, K = 5
+// 575 and 574, K = 6 576 and 575 (the last neither gains nor costs); n=25,000 d=15
+// 9.96 -> 9.80 ms of kernels; seven waves 591, eight 623, and four children a lane
+// spill 21 registers or more at six.
 template <bool PHI, int K, int CW, int NC>
 __global__ __launch_bounds__(kBlock, PHI || NC > 2 || K > 6 ? 3 : 6) void k_b_fan(const BatchSub *__restrict__ groups, const FanJob *__restrict__ jobs,
                                                   const int *__restrict__ blk_off, int njob, FanTable T, int d,

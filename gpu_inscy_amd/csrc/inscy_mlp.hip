@@ -154,7 +154,7 @@ __device__ __forceinline__ Split8 split8(const float (&v)[8]) {
 // order (its weights are laid out to match), so activations stay in registers.
 // The weights lie in LDS in operand order (16 bytes a lane, no bank conflicts),
 // loaded once per block; the blocks walk the tiles.
-// 200,003 rows: 695 us with VALU sums, 43 now; bound by the
+// 200,003 rows: 695 us with VALU sums, 41 now alone and 35 among others; bound by the
 // matrix cores (144 instructions a tile) and the activation splits, at two waves
 // per SIMD.
 constexpr int kMfTiles = kH / 32;         // 32-unit tiles of a layer
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_predict(const float *__restric
 // the 32 samples) as 4 tiles of dW2 and 2 of dW1 per wave, kept in registers
 // over the block's tiles.  The minibatch's tiles fill half the CUs at most, so
 // the time is the chain of one tile: 4,096 rows 114 us with VALU sums by 4 waves,
-// 24 now.
+// 24 now, alone (a step with the reduction and Adam 26 among others).
 constexpr int kGradThreads = 1024;
 constexpr int kXs = kIn + 4, kHs = kH + 4;  // padded rows (LDS banks)
 constexpr int kWs = kH + 16;
@@ -542,7 +542,7 @@ hipError_t launch_mlp_round(const float *master, uint16_t *P, hipStream_t st) {
 hipError_t launch_mlp_predict(const float *X, long long N, const uint16_t *P, float *prob, hipStream_t st) {
     if (N <= 0) return hipSuccess;
     // four tiles of 32 samples per block at a time; two blocks fill a CU (200,003
-    // rows: 43 us with 512 blocks, 51 with 768 and 54 with 256)
+    // rows, alone: 41 to 43 us with 512 blocks, 51 with 768 and 54 with 256)
     const long long blocks = (N + 4 * 32 - 1) / (4 * 32);
     const unsigned grid = (unsigned) std::min<long long>(blocks, 2 * 256);
     hipLaunchKernelGGL(k_mlp_predict, dim3(grid), dim3(kThreads), 0, st, X, N, P, prob);

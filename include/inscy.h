@@ -72,8 +72,7 @@ typedef struct inscy_stats {
     int64_t count_bytes;    /* its algorithmic bytes: per counted point 4k+4, per neighbour found 4+4k */
     /* wall time of the phases of the run (seconds): growing the restricted
      * trees (restrict, prunes, counts, dense components), the replay of
-     * pruneRedundancy and join (inside the first phase with a permuted level
-     * order), and reading the result back */
+     * pruneRedundancy and join, and reading the result back */
     double expand_seconds;
     double replay_seconds;
     double emit_seconds;
@@ -85,7 +84,9 @@ typedef struct inscy_stats {
      * earlier batch of the run (same index dimensions) instead of sorted */
     int64_t sorts_kept;
     /* level-synchronous driver: bytes of the candidates the neighbour-count
-     * kernel examined (packed cells and coordinates), most of them cache hits */
+     * kernels examined (their coordinates; walks of all children of a mask: also
+     * the neighbours' ids and coordinates in the children's dimensions), most of
+     * them cache hits */
     int64_t count_examined_bytes;
 } inscy_stats;
 
