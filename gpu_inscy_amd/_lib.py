@@ -160,6 +160,7 @@ def lib():
     L.inscy_debug_trace.argtypes = [ctypes.c_int]
     L.inscy_debug_phi_exact.argtypes = [ctypes.c_int]
     L.inscy_debug_generic_walk.argtypes = [ctypes.c_int]
+    L.inscy_debug_walk_per_child.argtypes = [ctypes.c_int]
     L.inscy_debug_keep_budget.argtypes = [ctypes.c_int64]
     L.inscy_debug_batch_budget.argtypes = [ctypes.c_int64]
     L.inscy_debug_batch_most.restype = ctypes.c_int64
@@ -338,6 +339,11 @@ def debug_phi_exact(on: bool) -> None:
 def debug_generic_walk(on: bool) -> None:
     """Test hook: run the neighbour walks for k known only at run time."""
     lib().inscy_debug_generic_walk(int(on))
+
+
+def debug_walk_per_child(on: bool) -> None:
+    """Test hook: count every level by one walk per child subspace."""
+    lib().inscy_debug_walk_per_child(int(on))
 
 
 def debug_keep_budget(nbytes: int) -> None:

@@ -396,7 +396,8 @@ public:
     int prune_min_depth = 1;
     bool collect = false;
     bool phi_all_exact = false;  // test hook: every phi by the leaf-order recomputation
-    bool generic_walk = false;   // test hook: no neighbour walk compiled for its k
+    bool generic_walk = false;   // test hook: no neighbour walk per child compiled for its k
+    bool walk_per_child = false;  // test hook: no walk per mask
     long long keep_budget_override = -1;  // test hook: bytes kept across batches (< 0: the batch budget)
     int mem_share = 1;  // engines running at once on the device (each budgets 1/mem_share of the free bytes)
     long long batch_budget_override = 0;  // test hook: bytes of a batch (0: from the free memory)

@@ -11,6 +11,7 @@ static thread_local std::vector<Engine::TraceRow> g_trace;
 static bool g_trace_on = false;
 static bool g_phi_all_exact = false;
 static bool g_generic_walk = false;
+static bool g_walk_per_child = false;
 static int64_t g_batch_budget = 0;
 static thread_local int64_t g_batch_most = 0;
 static int g_chain_limit = INT_MAX;
@@ -117,6 +118,7 @@ static int run_impl(const float *d_X, int64_t n, int32_t d, const inscy_params *
             eng.trace_on = g_trace_on;
             eng.phi_all_exact = g_phi_all_exact;
             eng.generic_walk = g_generic_walk;
+            eng.walk_per_child = g_walk_per_child;
             eng.batch_budget_override = g_batch_budget;
             eng.chain_limit = g_chain_limit;
             eng.keep_budget_override = g_keep_budget;
@@ -470,11 +472,18 @@ int inscy_debug_phi_exact(int on) {
     return INSCY_OK;
 }
 
-// Test hook (not in the public header): run every neighbour walk of the
-// level-synchronous driver for k known only at run time, one walk per child
-// subspace (no launch compiled for its k, no k_b_fan).
+// Test hook (not in the public header): run every neighbour walk per child
+// subspace for k known only at run time (no k_b_count or k_b_link_full compiled
+// for its k).
 int inscy_debug_generic_walk(int on) {
     g_generic_walk = on != 0;
+    return INSCY_OK;
+}
+
+// Test hook (not in the public header): count every level by one walk per child
+// subspace (no k_b_fan).
+int inscy_debug_walk_per_child(int on) {
+    g_walk_per_child = on != 0;
     return INSCY_OK;
 }
 

@@ -442,7 +442,7 @@ void Engine::index_of(std::vector<BatchSub> &hs, std::vector<const float *> &cta
 bool Engine::fan_level(const std::vector<ChildSub> &cs) const {
     if (cs.empty() || n >= kFanPoints || (long long) n * d >= 1ll << 30) return false;  // 32-bit offsets into X
     if (permuted) return false;  // the children match different dimensions of one mask
-    if (generic_walk) return false;  // the fan is compiled for its masks' k
+    if (walk_per_child) return false;
     const SubspaceArg S = arg_of(cs[0].s & ~dbit(cs[0].m));
     if (S.k < 1 || S.k > kMaxFastK) return false;
     return grid_of(S, -1, true).j >= grid_of(arg_of(cs[0].s), -1, true).j;

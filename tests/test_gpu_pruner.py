@@ -289,7 +289,7 @@ def test_learned_mode_counts_live_pairs_only(d):
 @pytest.mark.parametrize("d,eps", [(9, 0.03), (24, 0.02), (80, 0.01)])
 def test_learned_mode_by_mask_and_by_child_agree(d, eps, rect):
     # skips that differ from tree to tree of one mask: the walk per mask and the
-    # walk per child (any k) give the same trees and labels
+    # walk per child give the same trees and labels
     rng = np.random.default_rng(d)
     n, c, dims = 700, 3, 4
     X = _split_trees(n, d, c, d + 1)
@@ -304,15 +304,15 @@ def test_learned_mode_by_mask_and_by_child_agree(d, eps, rect):
     prob = pruner.Trainer(W).forward(P["features"]).cpu().numpy()
     _lib.set_pruner(W, float(np.quantile(prob[P["info"][:, 0] > 0], 0.5)), 1)
     res = []
-    for generic in (False, True):
-        _lib.debug_generic_walk(generic)
+    for child in (False, True):
+        _lib.debug_walk_per_child(child)
         _lib.debug_trace(True)
         try:
             r = INSCY.run(X, *args, mode=_lib.MODE_LEARNED)
             res.append((r, _lib.debug_trace_rows()))
         finally:
             _lib.debug_trace(False)
-            _lib.debug_generic_walk(False)
+            _lib.debug_walk_per_child(False)
     (a, ta), (b, tb) = res
     say("learned by mask / child", d, rect, a.stats["pairs_skipped"], a.stats["queries"], b.stats["queries"],
         len(a.subspaces))

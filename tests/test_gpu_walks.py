@@ -173,8 +173,19 @@ def traced(X, args):
         _lib.debug_trace(False)
 
 
-# one walk per mask (compiled for its k), one per child (any k): the hook must
-# reach the masks' walks too, and both give the same trees and labels
+def by_child(X, args, generic):
+    """The run with one walk per child, compiled for its k or not."""
+    _lib.debug_walk_per_child(True)
+    _lib.debug_generic_walk(generic)
+    try:
+        return traced(X, args)
+    finally:
+        _lib.debug_generic_walk(False)
+        _lib.debug_walk_per_child(False)
+
+
+# one walk per mask, one per child (compiled for its k, and for any k): the same
+# trees and labels
 @pytest.mark.parametrize("n,d,eps,dims", [(350, 9, 0.04, 5), (1203, 7, 0.01, 4)])
 @pytest.mark.parametrize("rect", [True, False])
 def test_walks_per_mask_and_per_child_agree(n, d, eps, dims, rect):
@@ -182,16 +193,13 @@ def test_walks_per_mask_and_per_child_agree(n, d, eps, dims, rect):
     X = clumps(n, d, eps, dims, n * d)
     args = (eps, 1.0, 4, n // 6, 1.0, 4, rect, 0)
     a, ta = traced(X, args)
-    _lib.debug_generic_walk(True)
-    try:
-        b, tb = traced(X, args)
-    finally:
-        _lib.debug_generic_walk(False)
-    # a walk per child leaves out the points that the counts of smaller
-    # subspaces decide, a walk per mask does not look them up
-    assert b.stats["queries"] < a.stats["queries"]
-    assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
-    assert np.array_equal(ta, tb)
+    for generic in (False, True):
+        b, tb = by_child(X, args, generic)
+        # a walk per child leaves out the points that the counts of smaller
+        # subspaces decide, a walk per mask does not look them up
+        assert b.stats["queries"] < a.stats["queries"]
+        assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
+        assert np.array_equal(ta, tb)
 
 
 def many_groups(n, d, c, eps, seed):
@@ -273,9 +281,12 @@ def test_routes_give_one_result(rect, order):
     args = (w.eps, w.F, w.num_obj, w.min_size, w.r, w.cells, rect, order)
     a, ta = traced(w.X, args)
     assert max(len(s) for s in a.subspaces) >= 3
-    for generic, max_batch, keep, budget in ((True, 0, -1, 0), (False, 1, -1, 0), (True, 1, -1, 0), (False, 3, 0, 0),
-                                             (True, 0, 0, 0), (False, 0, 1 << 20, 2 << 20)):
-        print("route", generic, max_batch, keep, budget, flush=True)
+    for child, generic, max_batch, keep, budget in ((True, False, 0, -1, 0), (True, True, 0, -1, 0),
+                                                    (False, True, 0, -1, 0), (False, False, 1, -1, 0),
+                                                    (True, False, 1, -1, 0), (False, False, 3, 0, 0),
+                                                    (True, True, 0, 0, 0), (False, False, 0, 1 << 20, 2 << 20)):
+        print("route", child, generic, max_batch, keep, budget, flush=True)
+        _lib.debug_walk_per_child(child)
         _lib.debug_generic_walk(generic)
         _lib.set_tuning(max_batch=max_batch)
         _lib.debug_keep_budget(keep)
@@ -287,6 +298,7 @@ def test_routes_give_one_result(rect, order):
             _lib.debug_keep_budget(-1)
             _lib.set_tuning()
             _lib.debug_generic_walk(False)
+            _lib.debug_walk_per_child(False)
         assert a.subspaces == b.subspaces and np.array_equal(a.labels, b.labels)
         assert np.array_equal(ta, tb)
         assert a.stats["trees"] == b.stats["trees"] and a.stats["calls"] == b.stats["calls"]
@@ -327,11 +339,7 @@ def test_walks_of_more_than_16_children(n, d, eps, dims, rect):
         for a, b in zip(ref.labels, got.labels):
             assert np.array_equal(O.canonical(a), b)
         assert np.array_equal(trace, ref.trace)
-    _lib.debug_generic_walk(True)
-    try:
-        b, tb = traced(X, args)
-    finally:
-        _lib.debug_generic_walk(False)
+    b, tb = by_child(X, args, False)
     assert got.subspaces == b.subspaces and np.array_equal(got.labels, b.labels)
     assert np.array_equal(trace, tb)
 
