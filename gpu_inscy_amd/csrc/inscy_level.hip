@@ -508,19 +508,21 @@ void Engine::process_batch(const std::vector<ChildSub> &cs, size_t i0, size_t i1
             g.base = (long long) gs.size() * n;
             long long qmax = 0;
             for (int a = c.t0; a < c.t1; ++a) {
-                // the tree's live pairs among the mask's children
-                unsigned long long on[2] = {0, 0};
-                bool all = true;
-                for (int x = b; x < e; ++x) {
-                    if (pair_on(a, cs[i0 + x].m))
-                        on[(x - b) / kFanMost] |= 1ull << ((x - b) % kFanMost);
-                    else
-                        all = false;
+                if (!lv_skip.empty()) {
+                    // the tree's live pairs among the mask's children
+                    unsigned long long on[2] = {0, 0};
+                    int dead = 0;
+                    for (int x = b; x < e; ++x) {
+                        if (pair_on(a, cs[i0 + x].m))
+                            on[(x - b) / kFanMost] |= 1ull << ((x - b) % kFanMost);
+                        else
+                            ++dead;
+                    }
+                    if (dead == e - b || lt[lv_act[a]].nW <= 0) continue;
+                    live.insert(live.end(), on, on + 2);
+                    skips |= dead > 0;
                 }
-                if (!(on[0] | on[1]) || !add_segment((int) gs.size(), a)) continue;
-                qmax += lt[lv_act[a]].nW;
-                live.insert(live.end(), on, on + 2);
-                skips |= !all;
+                if (add_segment((int) gs.size(), a)) qmax += lt[lv_act[a]].nW;
             }
             g.qmax = (int) qmax;
             for (int at = b; at < e; at += kFanMost) {
